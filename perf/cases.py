@@ -144,35 +144,50 @@ def _captured(forward):
     return graph, outputs
 
 
-def prepare(case, seed):
-    kind, rows = case["kind"], case["rows"]
-    make = _Inputs(seed)
-    if kind == "mxfp4":
-        n, k = case["n"], case["k"]
-        kernel = tl.matmul_bf16_mxfp4(rows, n, k, with_bias=case["bias"], weight_format="e2m1", scale_bias=127)
-        weight = make.packed(n, k // 2).view(torch.uint8)
-        scale = make.ints(127 - 8, 127, n, k // 32, dtype=torch.uint8)
-        bias = make.normal(rows, n, dtype=torch.bfloat16)
-        return {"kernel": kernel, "args": (make.normal(rows, k, dtype=torch.bfloat16), weight, scale, bias)}
-    if kind == "w4a8":
-        n, k = case["n"], case["k"]
-        kernel = tl.matmul_int8xint4(rows, n, k)
-        return {"kernel": kernel, "args": (make.ints(-128, 127, rows, k, dtype=torch.int8), make.packed(n, k // 2).view(torch.uint8))}
+def _drawn(case, make):
+    """The inputs of a kernel case, in the order that its call takes them."""
+    rows, n, k = case["rows"], case["n"], case["k"]
+    if case["kind"] == "w4a8":
+        return make.ints(-128, 127, rows, k, dtype=torch.int8), make.packed(n, k // 2).view(torch.uint8)
+    weight = make.packed(n, k // 2).view(torch.uint8)
+    scale = make.ints(127 - 8, 127, n, k // 32, dtype=torch.uint8)
+    bias = make.normal(rows, n, dtype=torch.bfloat16)
+    return make.normal(rows, k, dtype=torch.bfloat16), weight, scale, bias
 
-    layers, inputs = [], []
+
+def _drawn_layers(case, make, seed):
+    """For every layer of a case of layers: the tensors that it holds, and its activations."""
     for n, k in _shapes(case):
-        if kind == "w4a16":
-            layer = W4A16Linear(k, n, group_size=case["group"], with_zeros=case["zeros"])
+        if case["kind"] == "w4a16":
             held = {"qweight": make.packed(n, k // 2), "scales": make.uniform(0.002, 0.01, n, k // case["group"])}
             if case["zeros"]:
                 held["zeros"] = make.ints(6, 10, n, k // case["group"], dtype=torch.int8).half()
-            layer = layer.to(make.dev)
+        else:
+            held = {"qweight": make.ternary(n, k), "sw": 1.0 + (seed % 7) / 4}
+        yield n, k, held, make.normal(case["rows"], k, dtype=torch.float16)
+
+
+def prepare(case, seed):
+    kind, rows = case["kind"], case["rows"]
+    make = _Inputs(seed)
+    if kind in ("mxfp4", "w4a8"):
+        n, k = case["n"], case["k"]
+        if kind == "w4a8":
+            kernel = tl.matmul_int8xint4(rows, n, k)
+        else:
+            kernel = tl.matmul_bf16_mxfp4(rows, n, k, with_bias=case["bias"], weight_format="e2m1", scale_bias=127)
+        return {"kernel": kernel, "args": _drawn(case, make)}
+
+    layers, inputs = [], []
+    for n, k, held, x in _drawn_layers(case, make, seed):
+        if kind == "w4a16":
+            layer = W4A16Linear(k, n, group_size=case["group"], with_zeros=case["zeros"]).to(make.dev)
             layer.load_state_dict(held)
         else:
             layer = BitLinear(k, n, prefill_fragments=case["fragments"]).to(make.dev)
-            layer.load_packed_weight(make.ternary(n, k), 1.0 + (seed % 7) / 4)
+            layer.load_packed_weight(held["qweight"], held["sw"])
         layers.append(layer)
-        inputs.append(make.normal(rows, k, dtype=torch.float16))
+        inputs.append(x)
     state = {"layers": layers, "inputs": inputs}
     if case["block"]:
         with torch.no_grad():
@@ -218,3 +233,46 @@ def tolerance(case):
         "bitlinear": {"rel": 8e-4, "max": 2e-3},
         "w4a8": "exact",
     }[case["kind"]]
+
+
+def _nibbles(packed):
+    """Codes 0 .. 15 of packed bytes, the even column in the low nibble."""
+    b = packed.view(torch.uint8)
+    return torch.stack((b & 15, b >> 4), dim=-1).reshape(b.shape[0], -1)
+
+
+def _ternary_codes(packed):
+    """Codes of words whose element e lies at bit 8 * (e % 4) + 2 * (e // 4)."""
+    b = packed.view(torch.uint8).reshape(packed.shape[0], -1, 1, 4)
+    shift = torch.tensor([0, 2, 4, 6], dtype=torch.uint8, device=b.device).view(1, 1, 4, 1)
+    return ((b >> shift) & 3).reshape(packed.shape[0], -1)
+
+
+def exact(case, seed):
+    """The result in 64 bits.  A BitLinear layer's activations are whole numbers that 32-bit arithmetic defines (127 over
+    the row's largest magnitude, to the nearest): they are taken so, and all after them in 64 bits."""
+    kind = case["kind"]
+    make = _Inputs(seed)
+    if kind == "w4a8":
+        a, packed = _drawn(case, make)
+        codes = _nibbles(packed).to(torch.int16)
+        return (torch.where(codes > 7, codes - 16, codes).double() @ a.double().t()).to(torch.int32)
+    if kind == "mxfp4":
+        a, packed, scale, bias = _drawn(case, make)
+        values = torch.tensor([0.0, 0.5, 1.0, 1.5, 2.0, 3.0, 4.0, 6.0], dtype=torch.float64, device=make.dev)
+        weight = torch.cat((values, -values))[_nibbles(packed).int()]
+        weight = weight * torch.exp2(scale.double() - 127).repeat_interleave(32, dim=1)
+        out = a.double() @ weight.t()
+        return out + bias.double() if case["bias"] else out
+
+    outputs = []
+    for _, k, held, x in _drawn_layers(case, make, seed):
+        if kind == "w4a16":
+            codes = _nibbles(held["qweight"]).double()
+            zeros = held["zeros"].double().repeat_interleave(case["group"], dim=1) if case["zeros"] else 8.0
+            outputs.append(x.double() @ ((codes - zeros) * held["scales"].double().repeat_interleave(case["group"], dim=1)).t())
+        else:
+            s = 127 / x.float().abs().amax(dim=1, keepdim=True).clamp(min=1e-5)
+            whole = (x.float() * s).round().clamp(-128, 127).double()
+            outputs.append(whole @ (_ternary_codes(held["qweight"]).double() - 2).t() / s.double() / held["sw"])
+    return outputs if case["block"] else outputs[0]
