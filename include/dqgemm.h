@@ -150,6 +150,17 @@ enum dq_fp4_format {
 int call_dequant_gemm_bf16_mxfp4(const void* A, const void* B, const void* Scale, const void* Bias, void* C, int M,
                                  int N, int K, int scale_size, int fp4_format, int scale_bias, dq_stream_t stream);
 
+/* The same product with a workspace for partial sums (the form of call_dequantize_gemv_w4a16_ws): where M x N gives
+ * the CUs too few tiles, K is cut into slices, their fp32 sums go to the workspace and a second kernel adds them in
+ * slice order, with the bias, and rounds once.  split: 0 the library's choice (then dq_mxfp4_workspace_bytes(M, N, K)
+ * bytes are what it asks for; 0: no slices), 1 none, up to 16 that many where the shape allows it.  A smaller workspace
+ * lowers the count.  Workspace: 16-byte aligned, contents undefined afterwards, not to be shared by calls that overlap
+ * in time. */
+size_t dq_mxfp4_workspace_bytes(int M, int N, int K);
+int call_dequant_gemm_bf16_mxfp4_ws(const void* A, const void* B, const void* Scale, const void* Bias, void* C,
+                                    void* Workspace, size_t workspace_bytes, int M, int N, int K, int scale_size,
+                                    int fp4_format, int scale_bias, int split, dq_stream_t stream);
+
 /* ---- further dequantize GEMMs (same 256x256 MFMA kernel, different decoders) ------------------ */
 
 /* bf16 x fp4 without block scales: C[M,N] bf16 = A[M,K] bf16 . bf16(fp4(B[N,K/2]))^T, fp32 accumulation.

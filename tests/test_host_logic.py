@@ -50,6 +50,17 @@ def test_w4a16_workspace_query():
         assert K // 256 // (nbytes // (M * N * 4)) >= 4  # every slice at least 1024 k long
 
 
+def test_mxfp4_workspace_query():
+    """Room for K slices: nothing up to 80 rows, where the tiles fill the chip, where the slices' rows would be
+    misaligned or K is no multiple of 128; otherwise a whole number of [M, N] fp32 slices of at least 512 k."""
+    q = _lib.load_library().dq_mxfp4_workspace_bytes
+    for shape in ((1, 8192, 8192), (16, 8192, 8192), (80, 8192, 8192), (4096, 8192, 8192), (99, 8191, 8192), (96, 5760, 2880), (0, 8, 8), (96, 8192, 256)):
+        assert q(*shape) == 0
+    for M, N, K in ((96, 8192, 8192), (512, 8192, 8192), (128, 4096, 14336), (128, 28672, 8192)):
+        nbytes = q(M, N, K)
+        assert nbytes % (M * N * 4) == 0 and 2 <= nbytes // (M * N * 4) <= 12 and K * M * N * 4 // nbytes >= 512
+
+
 def test_entry_points_reject_bad_arguments_before_any_launch():
     """NULL pointers and impossible sizes return -1 with a message; no GPU is touched."""
     lib = _lib.load_library()

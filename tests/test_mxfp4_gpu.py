@@ -206,3 +206,43 @@ def test_unscaled_bf16_fp4_reads_back_the_reference_vectors(cuda):
         torch.cuda.synchronize()
         got = C.float().cpu().numpy().T  # [N, K]
         np.testing.assert_array_equal(got, orc.bf16_bits_to_f32(want_bits))
+
+
+@pytest.mark.parametrize("fmt", ["e2m1", "twiddling", "simple"])
+@pytest.mark.parametrize("M,N,K,split,with_bias", [
+    (17, 256, 256, 2, False),    # one unit of 128 k per slice: the pipeline's shortest walk
+    (129, 260, 1152, 2, True),   # ragged edges, slices of four and five units
+    (40, 1028, 1664, 12, True),  # slices of one and two units
+    (300, 516, 384, 8, False),   # more slices asked for than units: the kernel is not cut
+    (7, 262, 512, 4, True),      # M * N no multiple of four: not cut
+    (257, 1284, 1024, 3, False),
+])
+def test_k_slices(cuda, fmt, M, N, K, split, with_bias):
+    """K cut over workgroups, through the C-ABI with the slice count named; and a workspace with room for one slice
+    fewer.  Same tolerance as the uncut kernel: the fp32 sums are only grouped otherwise."""
+    from tilelang_amd import _lib, kernels
+
+    lib = _lib.get_library()
+    d = workloads.mxfp4(M, N, K, seed=3, scale_bias=127)
+    B = orc.twiddle_pack_fp4(orc.unpack_u4(d["B"])) if fmt == "twiddling" else d["B"]
+    bias_bits = orc.f32_to_bf16_bits(np.random.default_rng(4).standard_normal((M, N), dtype=np.float32) * 4)
+    A, Bd, S = _dev(d["A"], cuda), _dev(B, cuda), _dev(d["Scale"], cuda)
+    bias = _dev(bias_bits, cuda) if with_bias else None
+    ref = orc.bf16_bits_to_f32(orc.ref_mxfp4(d["A"], B, d["Scale"], bias_bits if with_bias else None, fmt=fmt, scale_bias=127))
+    for slices in (split, split - 1):
+        room = slices * M * N * 4
+        ws = torch.full((room,), 255, dtype=torch.uint8, device=cuda)  # NaN wherever a sum were left out
+        C = torch.empty((M, N), dtype=torch.bfloat16, device=cuda)
+        rc = lib.call_dequant_gemm_bf16_mxfp4_ws(A.data_ptr(), Bd.data_ptr(), S.data_ptr(), bias.data_ptr() if with_bias else None,
+                                                 C.data_ptr(), ws.data_ptr(), room, M, N, K, 32, kernels._FP4_FORMATS[fmt], 127,
+                                                 split, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0, _lib.last_error()
+        torch.cuda.synchronize()
+        np.testing.assert_allclose(C.float().cpu().numpy(), ref, rtol=RTOL, atol=ATOL)
+
+
+@pytest.mark.parametrize("M,N,K", [(81, 4096, 4096), (96, 8192, 8192), (200, 4104, 4224)])
+def test_k_slices_by_default(cuda, M, N, K):
+    """Shapes that the default cuts: through the kernel object, which brings the workspace."""
+    assert any(p.name == "Workspace" for p in tl.matmul_bf16_mxfp4(M, N, K, weight_format="e2m1", scale_bias=127).params)
+    _check(cuda, M, N, K, "e2m1", scale_bias=127, with_bias=True)

@@ -32,6 +32,7 @@ SIGNATURES = {
     "call_unpack_qzeros": [_vp, _vp, _i, _i, _i, _vp],
     "call_dequantize_w4": [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp],
     "call_dequant_gemm_bf16_mxfp4": [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp],
+    "call_dequant_gemm_bf16_mxfp4_ws": [_vp, _vp, _vp, _vp, _vp, _vp, ctypes.c_size_t, _i, _i, _i, _i, _i, _i, _i, _vp],
     "call_dequant_gemm_bf16_fp4": [_vp, _vp, _vp, _i, _i, _i, _i, _vp],
     "call_dequant_gemm_fp16_fp4": [_vp, _vp, _vp, _i, _i, _i, _i, _vp],
     "call_dequant_gemm_fp16_fp4_splitk": [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp],
@@ -50,6 +51,7 @@ SIGNATURES = {
 #: name -> argtypes of the functions that return a byte count (size_t) and launch nothing
 SIZE_QUERIES = {
     "dq_w4a16_workspace_bytes": [_i, _i, _i, _i, _i],
+    "dq_mxfp4_workspace_bytes": [_i, _i, _i],
 }
 
 

@@ -38,6 +38,9 @@ int mxfp4_gemm(const void* A, const void* B, const void* S, const void* Bias, vo
 
 int mxfp4_gemm_regres(const void* A, const void* B, const void* S, const void* Bias, void* C, int M, int N, int K, int fmt,
                       int scale_bias, int max_rows, hipStream_t stream);
+int mxfp4_gemm_ksplit(const void* A, const void* B, const void* S, const void* Bias, void* C, void* parts, int M, int N, int K,
+                      int fmt, int scale_bias, int split, hipStream_t stream);
+double mxfp4_regres_time(int M, int N, int K);
 int bf16_fp4_gemm(const void* A, const void* B, void* C, int M, int N, int K, int fmt, hipStream_t stream);
 int fp16_fp4_gemm(const void* A, const void* B, void* C, int M, int N, int K, int transposed, hipStream_t stream);
 int w4_f16_gemm(const void* A, const void* B, const void* S, const void* Z, void* C, int M, int N, int K, int group,
@@ -343,10 +346,37 @@ extern "C" int call_unpack_qzeros(const void* QZeros, void* Zeros, int N, int gr
   return unpack_qzeros(QZeros, Zeros, N, groups, format == DQ_QZEROS_PACKED4, (hipStream_t)stream);
 }
 
-extern "C" int call_dequant_gemm_bf16_mxfp4(const void* A, const void* B, const void* Scale, const void* Bias, void* C,
-                                            int M, int N, int K, int scale_size, int fp4_format, int scale_bias,
-                                            dq_stream_t stream) {
-  const char* fn = "call_dequant_gemm_bf16_mxfp4";
+// Into how many slices of K the tiled MXFP4 GEMM is cut when the caller brought a workspace; 1: not cut.  The times (us)
+// are fits to N x K = 8192 x 8192, 13824 x 5120, 4096 x 14336, 4096 x 4096 and 28672 x 8192 at 24 to 800 rows, each at
+// one, two, three, four, six and eight slices: a tile of 128 x 256 walks K at 8.5 ns per k while at most 192 of the CUs
+// have one and at 11.8 ns from there on (two tiles on a CU share that rate).  Sliced only where the fit is ahead by an
+// eighth: it is off by up to 10 % (M = 300, N = 13824, K = 5120: three slices 68.6 against 70.3 us, two 78.9; not cut).
+// Up to 80 rows nothing is cut although it would pay (M = 64, N = K = 8192: 48 us, six slices 27): a decode batch that
+// runs on the tiled kernel gives the bits that its rows give inside a large product, which programs may compare
+// (tests do), and sums grouped by slice round otherwise.
+static int mxfp4_ksplit(int M, int N, int K) {
+  if (M <= 80 || K % 128 != 0 || ((size_t)M * N) % 4 != 0) return 1;
+  const long tiles = (long)((M + 127) / 128) * ((N + 255) / 256);
+  if (tiles > 224) return 1;
+  const int units = K / 128;
+  // unsliced: from 96 such tiles on the same tile, below that the register-staged kernel's smaller ones, at a decode
+  // batch the register-resident kernel where that is ahead
+  double best = tiles >= 96 ? 4.0 + 1e-3 * K * (tiles <= 128 ? 11.2 : 13.0) : 2.0 + 1e-3 * K * (tiles <= 32 ? 7.2 : 8.0);
+  if (M <= 128) best = min(best, mxfp4_regres_time(M, N, K));
+  best *= 0.88;
+  int split = 1;
+  for (int s = 2; s <= 12 && units / s >= 4; ++s) {
+    const long wgs = tiles * s;
+    const double rate = wgs <= 192 ? 8.5 : 11.8 * (double)((wgs + 255) / 256);
+    const double t = 13.5 + 1e-3 * rate * 128 * ((units + s - 1) / s) + (double)s * M * N * 4 / 5.2e6;
+    if (t < best) best = t, split = s;
+  }
+  return split;
+}
+
+static int gemm_bf16_mxfp4(const char* fn, const void* A, const void* B, const void* Scale, const void* Bias, void* C, int M, int N,
+                           int K, int scale_size, int fp4_format, int scale_bias, int split, void* workspace,
+                           size_t workspace_bytes, dq_stream_t stream) {
   if (!A) DQ_FAIL("%s: A is expected to have non-NULL data pointer", fn);
   if (!B) DQ_FAIL("%s: B is expected to have non-NULL data pointer", fn);
   if (!Scale) DQ_FAIL("%s: Scale is expected to have non-NULL data pointer", fn);
@@ -358,6 +388,12 @@ extern "C" int call_dequant_gemm_bf16_mxfp4(const void* A, const void* B, const 
   if (scale_bias < 0 || scale_bias > 255) DQ_FAIL("%s: scale_bias must be in 0..255 (got %d)", fn, scale_bias);
   if (!aligned16(A) || !aligned16(B) || !aligned16(C) || (Bias && !aligned16(Bias)))
     DQ_FAIL("%s: A, B, Bias and C must be 16-byte aligned", fn);
+  if (workspace && split == 0) split = mxfp4_ksplit(M, N, K);
+  while (split > 1 && (size_t)split * M * N * sizeof(float) > workspace_bytes) --split;
+  if (split > 1) {
+    const int rc = mxfp4_gemm_ksplit(A, B, Scale, Bias, C, workspace, M, N, K, fp4_format, scale_bias, split, (hipStream_t)stream);
+    if (rc <= 0) return rc;
+  }
   // a decode batch: activations resident in registers, the weights streamed once per 16 rows (K % 64 == 0, beyond 8192 K % 128 == 0;
   // beyond 16 rows while the passes stay ahead of the tiled kernel: the kernel's launcher decides)
   if (M <= 128) {
@@ -365,6 +401,30 @@ extern "C" int call_dequant_gemm_bf16_mxfp4(const void* A, const void* B, const 
     if (rc <= 0) return rc;
   }
   return mxfp4_gemm(A, B, Scale, Bias, C, M, N, K, fp4_format, scale_bias, (hipStream_t)stream);
+}
+
+extern "C" int call_dequant_gemm_bf16_mxfp4(const void* A, const void* B, const void* Scale, const void* Bias, void* C,
+                                            int M, int N, int K, int scale_size, int fp4_format, int scale_bias,
+                                            dq_stream_t stream) {
+  return gemm_bf16_mxfp4("call_dequant_gemm_bf16_mxfp4", A, B, Scale, Bias, C, M, N, K, scale_size, fp4_format, scale_bias, 1, nullptr,
+                         0, stream);
+}
+
+extern "C" size_t dq_mxfp4_workspace_bytes(int M, int N, int K) {
+  if (M <= 0 || N <= 0 || K <= 0 || K % 64 != 0) return 0;
+  const int split = mxfp4_ksplit(M, N, K);
+  return split > 1 ? (size_t)split * M * N * sizeof(float) : 0;
+}
+
+extern "C" int call_dequant_gemm_bf16_mxfp4_ws(const void* A, const void* B, const void* Scale, const void* Bias, void* C,
+                                               void* Workspace, size_t workspace_bytes, int M, int N, int K, int scale_size,
+                                               int fp4_format, int scale_bias, int split, dq_stream_t stream) {
+  const char* fn = "call_dequant_gemm_bf16_mxfp4_ws";
+  if (workspace_bytes && !Workspace) DQ_FAIL("%s: Workspace is expected to have non-NULL data pointer", fn);
+  if (Workspace && !aligned16(Workspace)) DQ_FAIL("%s: Workspace must be 16-byte aligned", fn);
+  if (split < 0 || split > 16) DQ_FAIL("%s: split must be in 0..16 (got %d)", fn, split);
+  return gemm_bf16_mxfp4(fn, A, B, Scale, Bias, C, M, N, K, scale_size, fp4_format, scale_bias, split,
+                         workspace_bytes ? Workspace : nullptr, workspace_bytes, stream);
 }
 
 static int check_gemm_args(const char* fn, const void* A, const void* B, const void* C, int M, int N, int K, int kmult) {

@@ -71,6 +71,7 @@ struct Params {
   int M, N, K;       // K: contraction length of this launch (of one K slice when split > 1)
   int ldk;           // k elements per stored row of A and B (= K unless the launch covers K slices)
   int split;         // K slices, each its own set of workgroups and its own M x N output behind C
+  int kunit;         // > 0: slices are runs of whole units of this many k, as even as they come, and K is all of ldk
   int tiles_m, tiles_n;
   int p0, p1;        // policy specific integers (e.g. scale exponent offset, group shift)
   float f0;          // policy specific float (e.g. 1 / weight scale)
@@ -95,14 +96,29 @@ __device__ __forceinline__ void tile_of_block(int bid, int tiles_m, int tiles_n,
 // Split-K (examples/dequantize_gemm/example_dequant_gemm_fp4_hopper.py:136-167): workgroup ids beyond the first
 // tiles_m x tiles_n belong to further K slices.  Slice z reads columns [z K, (z + 1) K) of A and B and writes the
 // z-th M x N (or N x M) partial result behind C; a second kernel sums the partial results.  Plain (unpacked) A only.
+template <class P, class = void>
+struct UnevenSlices : std::false_type {};
+template <class P>
+struct UnevenSlices<P, std::void_t<decltype(P::kUnevenSlices)>> : std::integral_constant<bool, P::kUnevenSlices> {};
+
 template <class P>
 __device__ __forceinline__ void take_k_slice(Params& p, int& bid) {
   if (p.split > 1) {
     const int tiles = p.tiles_m * p.tiles_n;
     const int z = bid / tiles;
     bid -= z * tiles;
-    p.A = (const unsigned char*)p.A + (size_t)z * p.K * (kARowBytes / P::kKPerBlock);
-    p.B = (const unsigned char*)p.B + (size_t)z * p.K * P::kBRowBytes / P::kKPerBlock;
+    int k0 = z * p.K;
+    if constexpr (UnevenSlices<P>::value) {
+      const int units = p.ldk / p.kunit;
+      const int u0 = units * z / p.split, u1 = units * (z + 1) / p.split;
+      k0 = u0 * p.kunit;
+      p.K = (u1 - u0) * p.kunit;
+      // a slice starts where a dword of a row's scale bytes does (kunit is a multiple of 128 k)
+      static_assert(P::kScaleDma <= 1, "slices of fp16 group scales are not built");
+      if constexpr (P::kScaleDma == 1) p.S = (const unsigned char*)p.S + (k0 >> 5);
+    }
+    p.A = (const unsigned char*)p.A + (size_t)k0 * (kARowBytes / P::kKPerBlock);
+    p.B = (const unsigned char*)p.B + (size_t)k0 * P::kBRowBytes / P::kKPerBlock;
     p.C = (unsigned char*)p.C + (size_t)z * p.M * p.N * sizeof(typename P::out_t);
   }
 }
@@ -582,7 +598,7 @@ __global__ __launch_bounds__(64 * kWavesM * (8 / kNBW), 32 * kMBW * kWavesM == 1
   // need the scales issued with every tile: not the kPairB form, which dma_eligible keeps them away from
   const int s_gshift = P::kScaleDma >= 2 ? p.p0 : 7;
   const int s_ps = s_gshift - 5;
-  const unsigned s_voff = (unsigned)min(n0 + (tid & 255), N - 1) * (unsigned)(P::kScaleDma == 1 ? (K >> 5) : ((K >> s_gshift) << 1));  // waves 4..7 repeat 0..3
+  const unsigned s_voff = (unsigned)min(n0 + (tid & 255), N - 1) * (unsigned)(P::kScaleDma == 1 ? (p.ldk >> 5) : ((p.ldk >> s_gshift) << 1));  // waves 4..7 repeat 0..3
 
   // One tile = kSOps + kAOps + kBOps DMA instructions per thread: first the scale dword(s) (row tid; issued
   // with every tile although a dword serves two or four, which keeps the loop branch-free), then the A
@@ -1015,12 +1031,15 @@ bool dma_eligible(const Params& p) {
 // against 48.8 us; M = 640: 61 against 49 us).
 constexpr int kHalfTileMin = 96;
 template <class P>
-bool dma_half_eligible(const Params& p, int min_tiles = kHalfTileMin) {
-  const long tiles = (long)((p.M + 127) / 128) * ((p.N + BN - 1) / BN) * p.split;
+bool dma_half_takes(const Params& p) {
   const size_t a_bytes = (size_t)p.M * (p.ldk / P::kKPerBlock) * kARowBytes;
   const size_t b_bytes = (size_t)p.N * (p.ldk / P::kKPerBlock) * P::kBRowBytes;
-  return !dma_eligible<P>(p) && P::dma_ok(p) && (p.K % (2 * P::kKPerBlock) == 0) && tiles >= min_tiles &&
-         a_bytes < (1ull << 32) && b_bytes < (1ull << 32);
+  return P::dma_ok(p) && (p.K % (2 * P::kKPerBlock) == 0) && a_bytes < (1ull << 32) && b_bytes < (1ull << 32);
+}
+template <class P>
+bool dma_half_eligible(const Params& p, int min_tiles = kHalfTileMin) {
+  const long tiles = (long)((p.M + 127) / 128) * ((p.N + BN - 1) / BN) * p.split;
+  return !dma_eligible<P>(p) && dma_half_takes<P>(p) && tiles >= min_tiles;
 }
 
 template <class P, int kMBW, int kNBW, int kWavesM = 2>
@@ -1065,6 +1084,57 @@ int launch_best(const Params& p, hipStream_t stream, int half_tile_min = kHalfTi
   if (dma_eligible<P>(p)) return launch_dma<P>(p, stream);
   if (dma_half_eligible<P>(p, half_tile_min)) return launch_dma_half<P>(p, stream);
   return launch_auto<P>(p, stream);
+}
+
+// ---- K sliced over workgroups, fp32 sums in between --------------------------------------------------
+// A few dozen to a few hundred rows: M x N gives a fraction of the CUs a tile of 128 x 256, and each of them then runs
+// all of K at the rate of its ring (8 to 12 ns per k).  Sliced, the same tiles fill the chip; what it costs is the
+// slices' sums (4 bytes an element and slice, written and read: about 5 TB/s together) and a second kernel (with the
+// pipeline's start and end about 13 us).  MXFP4, N = K = 8192: M = 96 61 -> 29 us, M = 512 96 -> 75 us; N = 4096,
+// K = 14336, M = 128: 114 -> 32 us.
+// The policy with its accumulators stored as they are: one slice's partial result.
+template <class P>
+struct PartialSums : P {
+  static constexpr bool kUnevenSlices = true;
+  using out_t = float;
+  __device__ static __forceinline__ out_t finish(uint32_t raw, const Params&, int, int) { return __builtin_bit_cast(float, raw); }
+};
+
+// C = out_t(parts[0] + parts[1] + ... (+ Bias)), the slices in that order.  count % 4 == 0.
+template <class OUT, bool HAS_BIAS>
+__global__ __launch_bounds__(256) void ksplit_sum_kernel(const float* __restrict__ parts, const OUT* __restrict__ bias,
+                                                         OUT* __restrict__ C, size_t count, int split) {
+  typedef OUT out4_t __attribute__((ext_vector_type(4)));
+  const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i >= count) return;
+  float4_t v = *reinterpret_cast<const float4_t*>(parts + i);
+  for (int z = 1; z < split; ++z) v = v + *reinterpret_cast<const float4_t*>(parts + (size_t)z * count + i);
+  if constexpr (HAS_BIAS) {
+    const out4_t b = *reinterpret_cast<const out4_t*>(bias + i);
+    v = v + float4_t{(float)b[0], (float)b[1], (float)b[2], (float)b[3]};
+  }
+  *reinterpret_cast<out4_t*>(C + i) = out4_t{(OUT)v[0], (OUT)v[1], (OUT)v[2], (OUT)v[3]};
+}
+
+// p: the whole problem.  1: a shape that the 128 x 256 direct-to-LDS tile or the cut does not take.
+template <class P>
+int launch_ksplit(Params p, void* parts, int split, hipStream_t stream) {
+  if (split < 2 || !dma_half_takes<P>(p)) return 1;
+  const size_t count = (size_t)p.M * p.N;
+  p.kunit = 2 * P::kKPerBlock;
+  if (p.K % p.kunit != 0 || p.K / p.kunit < split || count % 4 != 0) return 1;
+  p.split = split;
+  using out_t = typename P::out_t;
+  out_t* const C = (out_t*)p.C;
+  p.C = parts;
+  if (launch_dma_tile<PartialSums<P>, 2, 4>(p, stream)) return -1;
+  const dim3 blocks((unsigned)((count + 1023) / 1024));
+  if (p.Bias)
+    hipLaunchKernelGGL((ksplit_sum_kernel<out_t, true>), blocks, dim3(256), 0, stream, (const float*)parts, (const out_t*)p.Bias, C, count, split);
+  else
+    hipLaunchKernelGGL((ksplit_sum_kernel<out_t, false>), blocks, dim3(256), 0, stream, (const float*)parts, (const out_t*)nullptr, C, count, split);
+  DQ_CHECK_HIP(hipGetLastError());
+  return 0;
 }
 
 inline Params make_params(const void* A, const void* B, const void* S, const void* Z, const void* Bias, void* C, int M,

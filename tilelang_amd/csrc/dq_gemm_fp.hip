@@ -123,6 +123,19 @@ int mxfp4_gemm(const void* A, const void* B, const void* S, const void* Bias, vo
 #undef DQ_MX
 }
 
+// K in `split` slices with fp32 sums in parts[split][M][N]; 1: not a shape of that kernel
+int mxfp4_gemm_ksplit(const void* A, const void* B, const void* S, const void* Bias, void* C, void* parts, int M, int N, int K,
+                      int fmt, int scale_bias, int split, hipStream_t stream) {
+  Params p = gemm::make_params(A, B, S, nullptr, Bias, C, M, N, K);
+  p.p0 = 127 - scale_bias;
+  switch (fmt) {  // the bias is added with the slices
+    case FP4_E2M1: return gemm::launch_ksplit<MxPolicy<FP4_E2M1, false>>(p, parts, split, stream);
+    case FP4_SIMPLE: return gemm::launch_ksplit<MxPolicy<FP4_SIMPLE, false>>(p, parts, split, stream);
+    case FP4_TWIDDLING: return gemm::launch_ksplit<MxPolicy<FP4_TWIDDLING, false>>(p, parts, split, stream);
+    default: DQ_FAIL("mxfp4 gemm: unknown weight format %d", fmt);
+  }
+}
+
 int bf16_fp4_gemm(const void* A, const void* B, void* C, int M, int N, int K, int fmt, hipStream_t stream) {
   Params p = gemm::make_params(A, B, nullptr, nullptr, nullptr, C, M, N, K);
 #define DQ_F4(FMT_) return gemm::launch_best<Bf16Fp4Policy<FMT_>>(p, stream)

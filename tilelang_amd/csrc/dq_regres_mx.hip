@@ -694,6 +694,20 @@ int launch_mx_gemv_long(const void* A, const void* B, const void* S, const void*
 
 }  // namespace
 
+// More than 16 rows run as passes of 16, each streaming the weights again: worth it while that stays ahead of the
+// tiled kernel, whose time up to 128 rows is one round of workgroups with all of K behind each (60 us at K = 8192,
+// 92 us from N = 16384 on).  Here the passes' workgroups come in rounds of one per CU, and a workgroup takes its
+// prologue (2 us + 2.5 us per 8192 k, once per slice of K) and 0.3 us + 2.8 us per 8192 k for every block of 16
+// weight rows it visits (measured at K = 8192: N = 8192 at 16 / 32 / 48 rows 13 / 24 / 35 us, N = 28672 at 16 rows
+// 26.6 us; N = K = 2880, where the passes share a round, 16 / 32 / 64 / 128 rows 6.7 / 11 / 16 / 29 us against 24.6 us).
+double mxfp4_regres_time(int M, int N, int K) {
+  const double kfrac = (double)K / 8192.0;
+  const int nslices = K > kWaves * kMaxChunks * 128 ? ((K >> 7) + kWaves * 6 - 1) / (kWaves * 6) : 1;
+  const long grid = (N + 15) / 16 < 256 ? (N + 15) / 16 : 256, blocks_each = ((N + 15) / 16 + grid - 1) / grid;
+  const long rounds = (grid * ((M + 15) / 16) + 255) / 256;
+  return 2.0 + 1.1 * (double)rounds * (2.0 * nslices + 2.5 * kfrac + (double)blocks_each * (0.3 * nslices + 2.8 * kfrac));
+}
+
 // 0: launched; 1: this shape is not the kernel's (the caller goes on to the tiled GEMM); -1: error.
 // max_rows: the most activation rows to take (passes of 16, each streaming the weights again).
 int mxfp4_gemm_regres(const void* A, const void* B, const void* S, const void* Bias, void* C, int M, int N, int K, int fmt,
@@ -701,20 +715,9 @@ int mxfp4_gemm_regres(const void* A, const void* B, const void* S, const void* B
   // 128-k chunks (the last one may be half: K % 128 == 64), at most eight per wave
   const bool longk = K > kWaves * kMaxChunks * 128;
   if (M < 1 || M > max_rows || K % 64 != 0 || (longk && K % 128 != 0)) return 1;
-  // More than 16 rows run as passes of 16, each streaming the weights again: worth it while that stays ahead of the
-  // tiled kernel, whose time up to 128 rows is one round of workgroups with all of K behind each (60 us at K = 8192,
-  // 92 us from N = 16384 on).  Here the passes' workgroups come in rounds of one per CU, and a workgroup takes its
-  // prologue (2 us + 2.5 us per 8192 k, once per slice of K) and 0.3 us + 2.8 us per 8192 k for every block of 16
-  // weight rows it visits (measured at K = 8192: N = 8192 at 16 / 32 / 48 rows 13 / 24 / 35 us, N = 28672 at 16 rows
-  // 26.6 us; N = K = 2880, where the passes share a round, 16 / 32 / 64 / 128 rows 6.7 / 11 / 16 / 29 us against 24.6 us).
   if (M > 16) {
-    const double kfrac = (double)K / 8192.0;
-    const int nslices = longk ? ((K >> 7) + kWaves * 6 - 1) / (kWaves * 6) : 1;
-    const long grid = (N + 15) / 16 < 256 ? (N + 15) / 16 : 256, blocks_each = ((N + 15) / 16 + grid - 1) / grid;
-    const long rounds = (grid * ((M + 15) / 16) + 255) / 256;
-    const double t_here = 2.0 + 1.1 * (double)rounds * (2.0 * nslices + 2.5 * kfrac + (double)blocks_each * (0.3 * nslices + 2.8 * kfrac));
-    const double t_tiled = (N > 16384 ? 92.0 : 60.0) * kfrac + 3.0;
-    if (t_here > 0.9 * t_tiled) return 1;
+    const double t_tiled = (N > 16384 ? 92.0 : 60.0) * ((double)K / 8192.0) + 3.0;
+    if (mxfp4_regres_time(M, N, K) > 0.9 * t_tiled) return 1;
   }
   const int exp_off = 127 - scale_bias;
   if (M == 1 && K <= 8192) {  // one row: the dot-product kernel

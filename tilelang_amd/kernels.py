@@ -444,12 +444,20 @@ def matmul_bf16_mxfp4(
         KernelParam("C", torch.bfloat16, (M, N)),
     ]
 
+    # some dozens to hundreds of rows: the library cuts K over workgroups when it is given room for the slices' sums
+    ws_bytes = int(_lib.load_library().dq_mxfp4_workspace_bytes(M, N, K))
+    if ws_bytes:
+        params.append(KernelParam("Workspace", torch.uint8, (ws_bytes,)))
+
     def launch(ptrs, stream):
         lib = _lib.get_library()
         bias = ptrs[3] if with_bias else None
+        if ws_bytes:
+            return lib.call_dequant_gemm_bf16_mxfp4_ws(ptrs[0], ptrs[1], ptrs[2], bias, ptrs[4], ptrs[5], ws_bytes, M, N, K, scale_size,
+                                                       fmt, scale_bias, 0, stream)
         return lib.call_dequant_gemm_bf16_mxfp4(ptrs[0], ptrs[1], ptrs[2], bias, ptrs[4], M, N, K, scale_size, fmt, scale_bias, stream)
 
-    return KernelAdapter("matmul_bf16_mxfp4", params, [-1], launch, _lib.last_error)
+    return KernelAdapter("matmul_bf16_mxfp4", params, [4], launch, _lib.last_error, workspace_idx=[5] if ws_bytes else [])
 
 
 def matmul_bf16_fp4(
