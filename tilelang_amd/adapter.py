@@ -69,6 +69,19 @@ class KernelAdapter:
 
     # -- validation, same order and wording as the reference ------------------------------
     def _check(self, tensors: list):
+        # One look per tensor settles a good call; what it does not settle goes through the five passes below, which say
+        # what is wrong.  (With __call__ asking the runtime for a GPU no more: W4A16 one row through a layer 23.9 -> 17.7
+        # us, MXFP4 one row 19.6 -> 12.4.)  Contiguous with no dimension of zero is every stride as expected.
+        device_type = self.device_type
+        for p, t in zip(self.params, tensors):
+            if isinstance(t, torch.Tensor) and not (
+                t.device.type == device_type
+                and (t.dtype == p.dtype or (p.packed and t.dtype in (torch.int8, torch.uint8)))
+                and t.shape == p.shape and 0 not in p.shape and t.is_contiguous()
+            ):
+                break
+        else:
+            return
         for p, t in zip(self.params, tensors):
             if not isinstance(t, torch.Tensor):
                 continue
@@ -121,13 +134,18 @@ class KernelAdapter:
                 break
         if device is None:
             device = torch.device(self.device_type)
-        on_gpu = device.type == "cuda" and torch.cuda.is_available()
+        # a tensor on the GPU says that there is one and the runtime need not be asked
+        has_cuda_input = device.type == "cuda" and device.index is not None
+        on_gpu = has_cuda_input or (device.type == "cuda" and torch.cuda.is_available())
         # the library launches on the CURRENT device: make the operands' device current for the length of the call
         guard = contextlib.nullcontext()
         if on_gpu and device.index is not None and device.index != torch.cuda.current_device():
             guard = torch.cuda.device(device)
         with guard:
-            current = current_stream_handle(self.device_type)
+            if has_cuda_input and self.device_type == "cuda":
+                current = torch._C._cuda_getCurrentRawStream(device.index)
+            else:
+                current = current_stream_handle(self.device_type)
             if stream == -1:
                 stream = current
             # Outputs and scratch come from torch's caching allocator, which hands a freed block back to work on
