@@ -246,3 +246,32 @@ def test_k_slices_by_default(cuda, M, N, K):
     """Shapes that the default cuts: through the kernel object, which brings the workspace."""
     assert any(p.name == "Workspace" for p in tl.matmul_bf16_mxfp4(M, N, K, weight_format="e2m1", scale_bias=127).params)
     _check(cuda, M, N, K, "e2m1", scale_bias=127, with_bias=True)
+
+
+@pytest.mark.parametrize("offset", [1, 2, 3])
+@pytest.mark.parametrize("M,N,K,split", [
+    (96, 4100, 1024, 2),   # would be cut
+    (1500, 2000, 256, 0),  # 96 tiles of 128 x 256
+    (4096, 3072, 128, 0),  # 192 tiles of 256 x 256
+])
+def test_scales_that_start_at_any_byte(cuda, M, N, K, split, offset):
+    """Scale is bytes and need not start at a multiple of four: the kernels that fetch it by dwords leave such a call to
+    the one that reads bytes, with the bits of the aligned, uncut call."""
+    from tilelang_amd import _lib
+
+    lib = _lib.get_library()
+    d = workloads.mxfp4(M, N, K, seed=5, scale_bias=127)
+    A, B, S = (_dev(d[k], cuda) for k in ("A", "B", "Scale"))
+    shifted = torch.zeros(S.numel() + 4, dtype=torch.uint8, device=cuda)[offset:offset + S.numel()]
+    shifted.copy_(S.reshape(-1))
+    ws = torch.full((2 * M * N * 4,), 255, dtype=torch.uint8, device=cuda)
+    results = []
+    for scale, slices in ((S, 1), (shifted, split)):
+        C = torch.empty((M, N), dtype=torch.bfloat16, device=cuda)
+        rc = lib.call_dequant_gemm_bf16_mxfp4_ws(A.data_ptr(), B.data_ptr(), scale.data_ptr(), None, C.data_ptr(), ws.data_ptr(), ws.numel(),
+                                                 M, N, K, 32, 0, 127, slices, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0, _lib.last_error()
+        results.append(C)
+    torch.cuda.synchronize()
+    assert bool((ws == 255).all())  # neither call was cut
+    assert torch.equal(results[0].view(torch.int16), results[1].view(torch.int16))

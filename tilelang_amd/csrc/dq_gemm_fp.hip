@@ -36,7 +36,8 @@ struct MxPolicy : Bf16Mfma, gemm::PlainA {
   using out_t = bf16_t;
   using ScaleRaw = int;
   static constexpr int kScaleDma = 1;  // one scale byte per 32 k travels by DMA in the direct-to-LDS kernel
-  static bool dma_ok(const Params&) { return true; }
+  // by dwords, so only from where a dword lies: Scale may start at any byte, and the register-staged kernel reads bytes
+  static bool dma_ok(const Params& p) { return ((size_t)p.S & 3) == 0; }
   struct Scale { float f; uint32_t add; };
   __device__ static __forceinline__ ScaleRaw fetch_scale(const Params& p, int row, int kb, int g) {
     return ((const uint8_t*)p.S)[(size_t)row * (p.K >> 5) + kb * 2 + g];
