@@ -184,6 +184,23 @@ def test_adapter_out_idx_allocates_outputs():
     assert C.shape == (2, 4) and C.dtype == torch.float16 and calls[0][0][2] == C.data_ptr()
 
 
+@pytest.mark.parametrize("workspace_idx,result_idx", [([1], [2]), ([-1], [-2]), ([0, 3], []), ([], [-1])])
+def test_profiler_supplies_what_a_caller_passes(workspace_idx, result_idx):
+    """Scratch is allocated by the adapter: the profiler's inputs are those of the call, scratch in neither form."""
+    from tilelang_amd.profiler import TensorSupplyType, get_tensor_supply
+
+    calls = []
+    params = [KernelParam(name, torch.float16, (2, 4 + i)) for i, name in enumerate("ABCD")]
+    k = KernelAdapter("k", params, result_idx, lambda ptrs, s: calls.append(len(ptrs)) or 0, lambda: "boom", device_type="cpu",
+                      workspace_idx=workspace_idx)
+    prof = k.get_profiler()
+    prof.supply = get_tensor_supply(TensorSupplyType.Auto, device="cpu")
+    prof.run_once()
+    assert calls == [4]
+    assert len(prof._get_inputs()) == 4 - len(workspace_idx) - len(result_idx)
+    assert len(prof._get_inputs(with_output=True)) == 4 - len(workspace_idx)
+
+
 @pytest.mark.parametrize("case,match", [
     ("count", r"Expected 3 inputs, got 2 with 2 inputs and 0 outputs"),
     ("dtype", r"Buffer dtype mismatch for parameter A: expected torch.float16, got torch.float32"),

@@ -80,6 +80,17 @@ def test_explicit_stream_gets_its_own_outputs(cuda):
     assert len({o.data_ptr() for o in outs}) == 4
 
 
+def test_profiler_of_a_kernel_with_scratch(cuda):
+    """A shape that the library cuts over K: the profiler's calls leave the workspace to the kernel object."""
+    M, N, K = 96, 4096, 4096
+    kern = tl.matmul_bf16_mxfp4(M, N, K, weight_format="e2m1", scale_bias=127)
+    assert kern.workspace_idx
+    prof = kern.get_profiler()
+    assert prof.run_once().shape == (M, N)
+    prof.assert_consistent(repeat=3)
+    assert prof.do_bench(warmup=1, rep=2) > 0
+
+
 @pytest.mark.parametrize("dtype, peak", [("bfloat16", 2.5e15), ("float16", 2.5e15), ("int8", 5.0e15), ("fp4", 10.1e15)])
 def test_mfma_sustained_rate_is_a_plausible_ceiling(cuda, dtype, peak):
     """``call_mfma_rate`` through ``profiler.mfma_sustained_rate``: the matrix pipe alone, on random operands, runs at

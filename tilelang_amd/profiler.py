@@ -235,7 +235,12 @@ class Profiler:
         self.result_idx = adapter.result_idx
 
     def _get_inputs(self, with_output: bool = False):
-        return [self.supply(p) for i, p in enumerate(self.adapter.params) if with_output or i not in self.result_idx]
+        # scratch is the adapter's own: no caller passes it
+        return [
+            self.supply(p)
+            for i, p in enumerate(self.adapter.params)
+            if i not in self.adapter.workspace_idx and (with_output or i not in self.result_idx)
+        ]
 
     def run_once(self):
         return self.adapter(*self._get_inputs())
