@@ -33,13 +33,14 @@ class KernelParam:
     packed: bool = False
 
 
-def current_stream_handle(device_type: str = "cuda") -> int:
-    """Raw handle of torch's current stream (tilelang/jit/adapter/cython/cython_wrapper.pyx:178-185)."""
-    if device_type == "cuda" and torch.cuda.is_available():
+def current_stream_handle(device_type: str = "cuda", index: int | None = None) -> int:
+    """Raw handle of torch's current stream (tilelang/jit/adapter/cython/cython_wrapper.pyx:178-185).  ``index``: the
+    GPU that an operand lies on, which the runtime then need not be asked for."""
+    if device_type == "cuda" and (index is not None or torch.cuda.is_available()):
         try:
-            return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+            return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
         except (ImportError, AttributeError):
-            return torch.cuda.current_stream().cuda_stream
+            return torch.cuda.current_stream(index).cuda_stream
     return 0
 
 
@@ -142,10 +143,7 @@ class KernelAdapter:
         if on_gpu and device.index is not None and device.index != torch.cuda.current_device():
             guard = torch.cuda.device(device)
         with guard:
-            if has_cuda_input and self.device_type == "cuda":
-                current = torch._C._cuda_getCurrentRawStream(device.index)
-            else:
-                current = current_stream_handle(self.device_type)
+            current = current_stream_handle(self.device_type, device.index if has_cuda_input else None)
             if stream == -1:
                 stream = current
             # Outputs and scratch come from torch's caching allocator, which hands a freed block back to work on
