@@ -61,6 +61,32 @@ def test_mxfp4_workspace_query():
         assert nbytes % (M * N * 4) == 0 and 2 <= nbytes // (M * N * 4) <= 12 and K * M * N * 4 // nbytes >= 512
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (384, 13824, 8192), (320, 13824, 8192), (384, 13824, 14336), (512, 11008, 14336),  # a second round of unsorted tiles
+    (640, 8192, 8192),    # a second round that gains nothing
+    (128, 2048, 4096),    # the register-resident kernel is ahead
+    (160, 28672, 28672),  # 224 tiles
+])
+def test_mxfp4_is_not_cut_where_that_is_slower(M, N, K):
+    """Shapes measured slower, or no faster, with K cut: no workspace is asked for."""
+    assert _lib.load_library().dq_mxfp4_workspace_bytes(M, N, K) == 0
+
+
+def test_mxfp4_cut_over_its_range():
+    """The estimates are compared as they are, not as whole microseconds; slices are whole, at least 512 k long and at
+    most twelve, and their room stays bounded, also beyond the sizes that were measured."""
+    q = _lib.load_library().dq_mxfp4_workspace_bytes
+    assert q(128, 28672, 4096) == 2 * 128 * 28672 * 4
+    rng = np.random.default_rng(0)
+    for _ in range(20000):
+        M, N, K = (int(v) for v in np.exp(rng.uniform(np.log((64, 8, 512)), np.log((8192, 40000, 40000)))))
+        K = K // 128 * 128
+        slices, rest = divmod(q(M, N, K), M * N * 4)
+        assert rest == 0 and slices <= 12 and slices * M * N * 4 < 200 << 20, (M, N, K)
+        assert slices != 1 and (slices == 0 or K // 128 // slices >= 4), (M, N, K)
+    assert q(2**31 - 1, 8, 1024) == q(2**31 - 1, 2**31 - 1, 1024) == 0
+
+
 def test_entry_points_reject_bad_arguments_before_any_launch():
     """NULL pointers and impossible sizes return -1 with a message; no GPU is touched."""
     lib = _lib.load_library()

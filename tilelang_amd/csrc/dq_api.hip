@@ -7,6 +7,8 @@
 #include "../../include/dqgemm.h"
 #include "dq_common.h"
 
+#include <algorithm>
+
 namespace dq {
 
 static char g_error_buf[kErrorBufSize];
@@ -347,26 +349,30 @@ extern "C" int call_unpack_qzeros(const void* QZeros, void* Zeros, int N, int gr
 }
 
 // Into how many slices of K the tiled MXFP4 GEMM is cut when the caller brought a workspace; 1: not cut.  The times (us)
-// are fits to N x K = 8192 x 8192, 13824 x 5120, 4096 x 14336, 4096 x 4096 and 28672 x 8192 at 24 to 800 rows, each at
-// one, two, three, four, six and eight slices: a tile of 128 x 256 walks K at 8.5 ns per k while at most 192 of the CUs
-// have one and at 11.8 ns from there on (two tiles on a CU share that rate).  Sliced only where the fit is ahead by an
-// eighth: it is off by up to 10 % (M = 300, N = 13824, K = 5120: three slices 68.6 against 70.3 us, two 78.9; not cut).
-// Up to 80 rows nothing is cut although it would pay (M = 64, N = K = 8192: 48 us, six slices 27): a decode batch that
-// runs on the tiled kernel gives the bits that its rows give inside a large product, which programs may compare
-// (tests do), and sums grouped by slice round otherwise.
+// are fits, and cut is what they put ahead by a twelfth.  Measured both ways at 1372 shapes (81 to 4096 rows, N 8 to
+// 28672, K 1024 to 28672, odd ones and close calls among them): the 901 that are cut take 0.6 of the uncut time in the
+// median (M = 96, N = K = 8192: 65 -> 27 us; M = 384, N = K = 8192: 90 -> 61; M = 2048, N = 2048, K = 8192: 96 -> 71),
+// one more than it (M = 3000, N = 2048, K = 14336: 174.5 against 173.6 us).
+// * Uncut from 96 tiles of 128 x 256 on: 10.4 ns per k there, 12.8 at 224 (the tiles share the memory's bandwidth).
+//   Below that the register-staged kernel's smaller tiles; at a decode batch the register-resident kernel, which up to
+//   K = 4096 takes 0.7 of its estimate (M = 128, N = 2048: 16.5 us, cut 17.2).
+// * More than one round of 256 workgroups is cut only where the tile count is a multiple of the XCDs: only then does an
+//   XCD walk neighbouring tiles (M = 1000, N = 5120, K = 14336, 160 tiles: 169 -> 146 us; M = 384, N = 13824, K = 8192,
+//   162 tiles: 96 -> 112).  Beyond 192 tiles nothing gained more than 6 %, with a workspace of 100 MB and more.
+// Up to 80 rows nothing is cut.  That is a promise of the header and no crossover: up to there a call that runs on the
+// tiled kernel gives the bits that its rows have in a large product (cut, M = 80, N = K = 8192 would take 27 us, not 63).
 static int mxfp4_ksplit(int M, int N, int K) {
   if (M <= 80 || K % 128 != 0 || ((size_t)M * N) % 4 != 0) return 1;
-  const long tiles = (long)((M + 127) / 128) * ((N + 255) / 256);
-  if (tiles > 224) return 1;
+  const long tiles = (((long)M + 127) / 128) * (((long)N + 255) / 256);
+  if (tiles > 192) return 1;
   const int units = K / 128;
-  // unsliced: from 96 such tiles on the same tile, below that the register-staged kernel's smaller ones, at a decode
-  // batch the register-resident kernel where that is ahead
-  double best = tiles >= 96 ? 4.0 + 1e-3 * K * (tiles <= 128 ? 11.2 : 13.0) : 2.0 + 1e-3 * K * (tiles <= 32 ? 7.2 : 8.0);
-  if (M <= 128) best = min(best, mxfp4_regres_time(M, N, K));
-  best *= 0.88;
+  double best = tiles >= 96 ? 4.0 + 1e-3 * K * (8.6 + 0.0186 * (double)tiles) : 2.0 + 1e-3 * K * (tiles <= 32 ? 7.2 : 8.0);
+  if (M <= 128) best = std::min(best, mxfp4_regres_time(M, N, K) * (K <= 4096 ? 0.7 : 1.0));
+  best *= 0.92;
   int split = 1;
   for (int s = 2; s <= 12 && units / s >= 4; ++s) {
     const long wgs = tiles * s;
+    if (wgs > 256 && tiles % 8 != 0) break;
     const double rate = wgs <= 192 ? 8.5 : 11.8 * (double)((wgs + 255) / 256);
     const double t = 13.5 + 1e-3 * rate * 128 * ((units + s - 1) / s) + (double)s * M * N * 4 / 5.2e6;
     if (t < best) best = t, split = s;
