@@ -72,6 +72,16 @@ def test_mxfp4_is_not_cut_where_that_is_slower(M, N, K):
     assert _lib.load_library().dq_mxfp4_workspace_bytes(M, N, K) == 0
 
 
+def test_mxfp4_factory_without_a_library(monkeypatch):
+    """A kernel object's parameters do not need the built library; its call does, and says so."""
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib, "LIB_PATH", "/nonexistent/libdqgemm.so")
+    kern = tl.matmul_bf16_mxfp4(96, 8192, 8192)
+    assert [p.name for p in kern.params] == ["A", "B", "Scale", "Bias", "C"] and kern.result_idx == [4]
+    with pytest.raises(_lib.LibraryNotBuiltError, match="no fallback"):
+        kern._launch([0] * 5, 0)
+
+
 def test_mxfp4_cut_over_its_range():
     """The estimates are compared as they are, not as whole microseconds; slices are whole, at least 512 k long and at
     most twelve, and their room stays bounded, also beyond the sizes that were measured."""

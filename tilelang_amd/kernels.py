@@ -445,7 +445,10 @@ def matmul_bf16_mxfp4(
     ]
 
     # some dozens to hundreds of rows: the library cuts K over workgroups when it is given room for the slices' sums
-    ws_bytes = int(_lib.load_library().dq_mxfp4_workspace_bytes(M, N, K))
+    try:
+        ws_bytes = int(_lib.load_library().dq_mxfp4_workspace_bytes(M, N, K))
+    except _lib.LibraryNotBuiltError:  # the kernel's parameters can be had without a library; its call raises this
+        ws_bytes = 0
     if ws_bytes:
         params.append(KernelParam("Workspace", torch.uint8, (ws_bytes,)))
 
