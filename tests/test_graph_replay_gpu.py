@@ -223,3 +223,40 @@ def test_graph_replays_match_eager_mxfp4_decode_kernels(cuda):
         torch.cuda.synchronize()
         for got, want in zip(outs, eager):
             assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+def test_graph_replays_match_eager_mxfp4_cut_over_k(cuda):
+    """MXFP4 with K cut over workgroups (two kernels, the slices' sums between them in a workspace of each call): the
+    same bits from a second call, and from every replay, with eager calls of the same kernels in between."""
+    runs = []
+    for i, (M, N, K, with_bias) in enumerate([(96, 4096, 4096, True), (200, 1030, 8192, True), (300, 2048, 5120, False)]):
+        d = workloads.mxfp4(M, N, K, seed=50 + i, scale_bias=127)
+        kern = tl.matmul_bf16_mxfp4(M, N, K, weight_format="e2m1", scale_bias=127, with_bias=with_bias)
+        assert kern.workspace_idx
+        gen = torch.Generator(device=cuda).manual_seed(i)
+        bias = torch.randn((M, N), device=cuda, generator=gen).to(torch.bfloat16)
+        runs.append((kern, (_dev(d["A"], cuda).view(torch.bfloat16), _dev(d["B"], cuda), _dev(d["Scale"], cuda), bias)))
+
+    def run():
+        return [k(*a) for k, a in runs]
+
+    eager = run()
+    again = run()
+    torch.cuda.synchronize()
+    for got, want in zip(again, eager):
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            outs = run()
+    for _ in range(4):
+        for t in outs:
+            t.fill_(float("nan"))
+        between = run()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for got, want, other in zip(outs, eager, between):
+            assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+            assert torch.equal(other.view(torch.int16), want.view(torch.int16))

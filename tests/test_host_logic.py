@@ -51,8 +51,9 @@ def test_w4a16_workspace_query():
 
 
 def test_mxfp4_workspace_query():
-    """Room for K slices: nothing up to 80 rows, where the tiles fill the chip, where the slices' rows would be
-    misaligned or K is no multiple of 128; otherwise a whole number of [M, N] fp32 slices of at least 512 k."""
+    """Room for K slices: nothing up to 80 rows, where the tiles fill the chip, where a slice would start misaligned
+    (M * N no multiple of four; the rows inside it may be) or K is no multiple of 128; otherwise a whole number of
+    [M, N] fp32 slices of at least 512 k."""
     q = _lib.load_library().dq_mxfp4_workspace_bytes
     for shape in ((1, 8192, 8192), (16, 8192, 8192), (80, 8192, 8192), (4096, 8192, 8192), (99, 8191, 8192), (96, 5760, 2880), (0, 8, 8), (96, 8192, 256)):
         assert q(*shape) == 0
@@ -308,6 +309,46 @@ def test_adapter_validation_errors(case, match):
         if args:
             k(*args, skip_tensor_validation=True)
             assert len(calls) == 1
+
+
+def _form(shape, stride=None, offset=0, dtype=torch.float16):
+    t = torch.zeros(64, dtype=dtype)[offset:]
+    return t[:int(np.prod(shape))].reshape(shape) if stride is None else t.as_strided(shape, stride)
+
+
+@pytest.mark.parametrize("shape,packed,tensor,message", [
+    ((1, 8), True, _form((1, 8), dtype=torch.int8), None),
+    ((1, 8), True, _form((1, 8), dtype=torch.uint8), None),
+    ((1, 8), True, _form((1, 8), dtype=torch.int16), "dtype mismatch"),
+    ((1, 8), False, _form((1, 8), dtype=torch.int8), "dtype mismatch"),
+    ((1, 8), False, _form((1, 8), (5, 1)), None),     # a dimension of one has any stride
+    ((1, 8), False, _form((1, 8), offset=3), None),   # a view that starts anywhere
+    ((1, 8), False, _form((1, 8), (8, 2)), "stride mismatch"),
+    ((3, 1, 4), False, _form((3, 1, 4), (4, 17, 1)), None),
+    ((3, 1, 4), False, _form((3, 1, 4), (0, 4, 1)), "stride mismatch"),  # expanded
+    ((3, 1, 4), False, _form((3, 1, 4), (1, 1, 3)), "stride mismatch"),  # transposed
+    ((3, 1, 4), False, _form((3, 4)), "expected 3 dimensions, got 2"),
+    ((3, 1, 4), False, _form((3, 1, 5)), "expected 4 at index 2, got 5"),
+    ((3, 1, 4), False, torch.zeros(3, 1, 4, dtype=torch.float16, device="meta"), "device mismatch"),
+    ((3, 1, 4), False, None, None),
+    ((3, 1, 4), False, 4096, None),  # a raw pointer
+    ((0, 4), False, _form((0, 4)), None),
+    ((0, 4), False, _form((1, 4)), "expected 0 at index 0, got 1"),
+    ((2, 0), False, torch.zeros(2, 0, dtype=torch.float16), "stride mismatch"),
+    ((-1, 4), False, _form((2, 4)), None),
+])
+def test_adapter_one_look_settles_what_the_five_passes_accept(shape, packed, tensor, message):
+    """The walk that settles a good call alone, and the passes behind it (to which a second parameter with an open
+    dimension sends every call), say the same of every form."""
+    param = KernelParam("X", torch.int8 if packed else torch.float16, shape, packed=packed)
+    opened = KernelParam("open", torch.float16, (-1,))
+    for params, tensors in (([param], [tensor]), ([param, opened], [tensor, torch.zeros(5, dtype=torch.float16)])):
+        k = KernelAdapter("k", params, [], lambda ptrs, s: 0, lambda: "", device_type="cpu")
+        if message is None:
+            k._check(tensors)
+        else:
+            with pytest.raises(ValueError, match=message):
+                k._check(tensors)
 
 
 def test_adapter_error_code_raises_runtime_error():

@@ -208,44 +208,102 @@ def test_unscaled_bf16_fp4_reads_back_the_reference_vectors(cuda):
         np.testing.assert_array_equal(got, orc.bf16_bits_to_f32(want_bits))
 
 
-@pytest.mark.parametrize("fmt", ["e2m1", "twiddling", "simple"])
-@pytest.mark.parametrize("M,N,K,split,with_bias", [
-    (17, 256, 256, 2, False),    # one unit of 128 k per slice: the pipeline's shortest walk
-    (129, 260, 1152, 2, True),   # ragged edges, slices of four and five units
-    (40, 1028, 1664, 12, True),  # slices of one and two units
-    (300, 516, 384, 8, False),   # more slices asked for than units: the kernel is not cut
-    (7, 262, 512, 4, True),      # M * N no multiple of four: not cut
-    (257, 1284, 1024, 3, False),
-])
-def test_k_slices(cuda, fmt, M, N, K, split, with_bias):
-    """K cut over workgroups, through the C-ABI with the slice count named; and a workspace with room for one slice
-    fewer.  Same tolerance as the uncut kernel: the fp32 sums are only grouped otherwise."""
+def _cut_call(A, B, S, bias, C, ws, room, M, N, K, fmt, split):
     from tilelang_amd import _lib, kernels
 
-    lib = _lib.get_library()
+    return _lib.get_library().call_dequant_gemm_bf16_mxfp4_ws(
+        A.data_ptr(), B.data_ptr(), S.data_ptr(), None if bias is None else bias.data_ptr(), C.data_ptr(),
+        None if ws is None else ws.data_ptr(), room, M, N, K, 32, kernels._FP4_FORMATS[fmt], 127, split,
+        torch.cuda.current_stream().cuda_stream)
+
+
+@pytest.mark.parametrize("fmt", ["e2m1", "twiddling", "simple"])
+@pytest.mark.parametrize("M,N,K,split,with_bias,cut", [
+    (17, 256, 256, 2, False, True),     # one unit of 128 k per slice: the pipeline's shortest walk
+    (129, 260, 1152, 2, True, True),    # ragged edges, slices of four and five units
+    (40, 1028, 1664, 12, True, True),   # slices of one and two units
+    (8, 262, 512, 4, True, True),       # rows of the partial sums that start off 16 bytes: stored by elements
+    (100, 1027, 1152, 3, True, True),   # and off 8 bytes: the sum kernel's quadruples straddle rows
+    (300, 516, 384, 8, False, False),   # more slices asked for than units: the kernel is not cut
+    (7, 262, 512, 4, True, False),      # M * N no multiple of four: not cut
+    (257, 1284, 1024, 3, False, True),
+])
+def test_k_slices(cuda, fmt, M, N, K, split, with_bias, cut):
+    """K cut over workgroups, through the C-ABI with the slice count named; and a workspace with room for one slice
+    fewer.  Same tolerance as the uncut kernel: the fp32 sums are only grouped otherwise.  The workspace says whether the
+    call was cut: its slices' sums, added in order with the bias and rounded once, are the result, and nothing around
+    them is written; an uncut call writes none of it."""
+    from tilelang_amd import _lib
+
     d = workloads.mxfp4(M, N, K, seed=3, scale_bias=127)
     B = orc.twiddle_pack_fp4(orc.unpack_u4(d["B"])) if fmt == "twiddling" else d["B"]
     bias_bits = orc.f32_to_bf16_bits(np.random.default_rng(4).standard_normal((M, N), dtype=np.float32) * 4)
     A, Bd, S = _dev(d["A"], cuda), _dev(B, cuda), _dev(d["Scale"], cuda)
     bias = _dev(bias_bits, cuda) if with_bias else None
     ref = orc.bf16_bits_to_f32(orc.ref_mxfp4(d["A"], B, d["Scale"], bias_bits if with_bias else None, fmt=fmt, scale_bias=127))
+    guard = 1024
     for slices in (split, split - 1):
         room = slices * M * N * 4
-        ws = torch.full((room,), 255, dtype=torch.uint8, device=cuda)  # NaN wherever a sum were left out
+        around = torch.full((guard + room + guard,), 255, dtype=torch.uint8, device=cuda)  # NaN wherever a sum were left out
+        ws = around[guard:guard + room]
         C = torch.empty((M, N), dtype=torch.bfloat16, device=cuda)
-        rc = lib.call_dequant_gemm_bf16_mxfp4_ws(A.data_ptr(), Bd.data_ptr(), S.data_ptr(), bias.data_ptr() if with_bias else None,
-                                                 C.data_ptr(), ws.data_ptr(), room, M, N, K, 32, kernels._FP4_FORMATS[fmt], 127,
-                                                 split, torch.cuda.current_stream().cuda_stream)
-        assert rc == 0, _lib.last_error()
+        assert _cut_call(A, Bd, S, bias, C, ws, room, M, N, K, fmt, split) == 0, _lib.last_error()
         torch.cuda.synchronize()
         np.testing.assert_allclose(C.float().cpu().numpy(), ref, rtol=RTOL, atol=ATOL)
+        assert bool((around[:guard] == 255).all()) and bool((around[guard + room:] == 255).all())
+        if not cut or slices < 2:
+            assert bool((ws == 255).all())
+            continue
+        parts = ws.view(torch.float32).view(slices, M, N)
+        total = parts[0].clone()
+        for z in range(1, slices):
+            total += parts[z]
+        if with_bias:
+            total += bias.view(torch.bfloat16).float()
+        assert bool(torch.isfinite(parts).all())
+        assert torch.equal(total.to(torch.bfloat16).view(torch.int16), C.view(torch.int16))
 
 
-@pytest.mark.parametrize("M,N,K", [(81, 4096, 4096), (96, 8192, 8192), (200, 4104, 4224)])
+@pytest.mark.parametrize("M,N,K", [(81, 4096, 4096), (96, 8192, 8192), (200, 4104, 4224), (100, 8190, 4096)])
 def test_k_slices_by_default(cuda, M, N, K):
     """Shapes that the default cuts: through the kernel object, which brings the workspace."""
     assert any(p.name == "Workspace" for p in tl.matmul_bf16_mxfp4(M, N, K, weight_format="e2m1", scale_bias=127).params)
     _check(cuda, M, N, K, "e2m1", scale_bias=127, with_bias=True)
+
+
+def test_k_slice_workspace_through_c_abi(cuda):
+    """The library's own choice with its full room, with less, with none: fewer slices and in the end the plain entry
+    point's bits; what is refused."""
+    from tilelang_amd import _lib
+
+    lib = _lib.get_library()
+    M, N, K = 200, 1028, 8192
+    d = workloads.mxfp4(M, N, K, seed=6, scale_bias=127)
+    A, B, S = (_dev(d[k], cuda) for k in ("A", "B", "Scale"))
+    full = int(lib.dq_mxfp4_workspace_bytes(M, N, K))
+    assert full >= 4 * M * N * 4
+    ws = torch.empty(full + 16, dtype=torch.uint8, device=cuda)
+    C = torch.empty((M, N), dtype=torch.bfloat16, device=cuda)
+    plain = torch.empty((M, N), dtype=torch.bfloat16, device=cuda)
+    rc = lib.call_dequant_gemm_bf16_mxfp4(A.data_ptr(), B.data_ptr(), S.data_ptr(), None, plain.data_ptr(), M, N, K, 32, 0, 127,
+                                          torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, _lib.last_error()
+    ref = orc.bf16_bits_to_f32(orc.ref_mxfp4(d["A"], d["B"], d["Scale"], None, fmt="e2m1", scale_bias=127))
+    for room, slices in ((full, full // (M * N * 4)), (3 * M * N * 4 + 8, 3), (2 * M * N * 4, 2), (M * N * 4, 1), (8, 1), (0, 1)):
+        ws.fill_(255)
+        C.fill_(float("nan"))
+        assert _cut_call(A, B, S, None, C, ws if room else None, room, M, N, K, "e2m1", 0) == 0, _lib.last_error()
+        torch.cuda.synchronize()
+        used = slices * M * N * 4 if slices > 1 else 0
+        assert bool((ws[used:] == 255).all()) and bool(torch.isfinite(ws[:used].view(torch.float32)).all())
+        np.testing.assert_allclose(C.float().cpu().numpy(), ref, rtol=RTOL, atol=ATOL)
+        if slices == 1:
+            assert torch.equal(C.view(torch.int16), plain.view(torch.int16))
+    for workspace, room, split, message in ((None, full, 0, "Workspace is expected to have non-NULL data pointer"),
+                                            (ws[4:], full, 0, "16-byte aligned"), (ws, full, -1, "split must be in 0..16"),
+                                            (ws, full, 17, "split must be in 0..16")):
+        assert _cut_call(A, B, S, None, C, workspace, room, M, N, K, "e2m1", split) == -1
+        assert message in _lib.last_error()
 
 
 @pytest.mark.parametrize("offset", [1, 2, 3])
@@ -259,7 +317,6 @@ def test_scales_that_start_at_any_byte(cuda, M, N, K, split, offset):
     the one that reads bytes, with the bits of the aligned, uncut call."""
     from tilelang_amd import _lib
 
-    lib = _lib.get_library()
     d = workloads.mxfp4(M, N, K, seed=5, scale_bias=127)
     A, B, S = (_dev(d[k], cuda) for k in ("A", "B", "Scale"))
     shifted = torch.zeros(S.numel() + 4, dtype=torch.uint8, device=cuda)[offset:offset + S.numel()]
@@ -268,9 +325,7 @@ def test_scales_that_start_at_any_byte(cuda, M, N, K, split, offset):
     results = []
     for scale, slices in ((S, 1), (shifted, split)):
         C = torch.empty((M, N), dtype=torch.bfloat16, device=cuda)
-        rc = lib.call_dequant_gemm_bf16_mxfp4_ws(A.data_ptr(), B.data_ptr(), scale.data_ptr(), None, C.data_ptr(), ws.data_ptr(), ws.numel(),
-                                                 M, N, K, 32, 0, 127, slices, torch.cuda.current_stream().cuda_stream)
-        assert rc == 0, _lib.last_error()
+        assert _cut_call(A, B, scale, None, C, ws, ws.numel(), M, N, K, "e2m1", slices) == 0, _lib.last_error()
         results.append(C)
     torch.cuda.synchronize()
     assert bool((ws == 255).all())  # neither call was cut
