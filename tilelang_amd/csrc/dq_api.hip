@@ -351,7 +351,7 @@ extern "C" int call_unpack_qzeros(const void* QZeros, void* Zeros, int N, int gr
 // Into how many slices of K the tiled MXFP4 GEMM is cut when the caller brought a workspace; 1: not cut.  The times (us)
 // are fits, and cut is what they put ahead by a twelfth.  Measured both ways at 1372 shapes (81 to 4096 rows, N 8 to
 // 28672, K 1024 to 28672, odd ones and close calls among them): the 901 that are cut take 0.6 of the uncut time in the
-// median (M = 96, N = K = 8192: 65 -> 27 us; M = 384, N = K = 8192: 90 -> 61; M = 2048, N = 2048, K = 8192: 96 -> 71),
+// median (M = 96, N = K = 8192: 64 -> 29 us; M = 384, N = K = 8192: 90 -> 61; M = 2048, N = 2048, K = 8192: 96 -> 71),
 // one more than it (M = 3000, N = 2048, K = 14336: 174.5 against 173.6 us).
 // * Uncut from 96 tiles of 128 x 256 on: 10.4 ns per k there, 12.8 at 224 (the tiles share the memory's bandwidth).
 //   Below that the register-staged kernel's smaller tiles; at a decode batch the register-resident kernel, which up to

@@ -71,7 +71,7 @@ struct Params {
   int M, N, K;       // K: contraction length of this launch (of one K slice when split > 1)
   int ldk;           // k elements per stored row of A and B (= K unless the launch covers K slices)
   int split;         // K slices, each its own set of workgroups and its own M x N output behind C
-  int kunit;         // > 0: slices are runs of whole units of this many k, as even as they come, and K is all of ldk
+  int kunit;         // k per unit of which a slice is a run; read by policies with kUnevenSlices alone
   int tiles_m, tiles_n;
   int p0, p1;        // policy specific integers (e.g. scale exponent offset, group shift)
   float f0;          // policy specific float (e.g. 1 / weight scale)
@@ -93,14 +93,16 @@ __device__ __forceinline__ void tile_of_block(int bid, int tiles_m, int tiles_n,
   tn = in_band / gm;
 }
 
-// Split-K (examples/dequantize_gemm/example_dequant_gemm_fp4_hopper.py:136-167): workgroup ids beyond the first
-// tiles_m x tiles_n belong to further K slices.  Slice z reads columns [z K, (z + 1) K) of A and B and writes the
-// z-th M x N (or N x M) partial result behind C; a second kernel sums the partial results.  Plain (unpacked) A only.
+// P::kUnevenSlices: K slices as even as whole units of kunit k allow, instead of equal ones
 template <class P, class = void>
 struct UnevenSlices : std::false_type {};
 template <class P>
 struct UnevenSlices<P, std::void_t<decltype(P::kUnevenSlices)>> : std::integral_constant<bool, P::kUnevenSlices> {};
 
+// Split-K (examples/dequantize_gemm/example_dequant_gemm_fp4_hopper.py:136-167): workgroup ids beyond the first
+// tiles_m x tiles_n belong to further K slices.  Slice z reads columns [z K, (z + 1) K) of A and B, with uneven slices
+// (where K comes in as all of ldk) the z-th of `split` runs of whole units, and writes the z-th M x N (or N x M) partial
+// result behind C; a second kernel sums the partial results.  Plain (unpacked) A only.
 template <class P>
 __device__ __forceinline__ void take_k_slice(Params& p, int& bid) {
   if (p.split > 1) {
@@ -130,7 +132,8 @@ __device__ __forceinline__ void take_k_slice(Params& p, int& bid) {
 // bytes.  Each wave owns a 32 x (128 + 4) slab of 32-bit values; LDS operations of one wave execute
 // in order, so no workgroup barrier is needed between the phases.  Each wave owns a 32 x (32 kNBW + 4) slab.
 // C is written once and not read again by the kernel: the 16-byte stores are nontemporal, which keeps the
-// output from displacing operand lines in the L2 (MXFP4 GEMM 361 -> 358 us, block-scaled GEMM 147 -> 138 us).
+// output from displacing operand lines in the L2 (MXFP4 GEMM 361 -> 358 us, block-scaled GEMM 147 -> 138 us).  The
+// partial sums of K slices, which the next kernel reads, leave the same way (not measured otherwise).
 #define DQ_GEMM_EPILOGUE \
   using out_t = typename P::out_t; \
   constexpr int kSlabStride = 32 * kNBW + 4; \
@@ -1088,10 +1091,10 @@ int launch_best(const Params& p, hipStream_t stream, int half_tile_min = kHalfTi
 
 // ---- K sliced over workgroups, fp32 sums in between --------------------------------------------------
 // A few dozen to a few hundred rows: M x N gives a fraction of the CUs a tile of 128 x 256, and each of them then runs
-// all of K at the rate of its ring (8 to 12 ns per k).  Sliced, the same tiles fill the chip; what it costs is the
+// all of K at the rate of its ring (8 to 13 ns per k).  Sliced, the same tiles fill the chip; what it costs is the
 // slices' sums (4 bytes an element and slice, written and read: about 5 TB/s together) and a second kernel (with the
-// pipeline's start and end about 13 us).  MXFP4, N = K = 8192: M = 96 61 -> 29 us, M = 512 96 -> 75 us; N = 4096,
-// K = 14336, M = 128: 114 -> 32 us.
+// pipeline's start and end about 13 us).  MXFP4, N = K = 8192: M = 96 64 -> 29 us, M = 512 93 -> 71 us; N = 4096,
+// K = 14336, M = 128: 117 -> 31 us.
 // The policy with its accumulators stored as they are: one slice's partial result.
 template <class P>
 struct PartialSums : P {
