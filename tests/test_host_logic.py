@@ -66,7 +66,8 @@ def test_mxfp4_workspace_query():
     (384, 13824, 8192), (320, 13824, 8192), (384, 13824, 14336), (512, 11008, 14336),  # a second round of unsorted tiles
     (640, 8192, 8192),    # a second round that gains nothing
     (128, 2048, 4096),    # the register-resident kernel is ahead
-    (160, 28672, 28672),  # 224 tiles
+    (768, 8192, 14336), (160, 28672, 28672),  # 192 and 224 tiles
+    (1242, 1560, 3712),   # 70 tiles whose narrow last column leaves one round of the smaller ones
 ])
 def test_mxfp4_is_not_cut_where_that_is_slower(M, N, K):
     """Shapes measured slower, or no faster, with K cut: no workspace is asked for."""

@@ -271,6 +271,24 @@ def test_k_slices_by_default(cuda, M, N, K):
     _check(cuda, M, N, K, "e2m1", scale_bias=127, with_bias=True)
 
 
+@pytest.mark.parametrize("M,N,K,cut", [(166, 5818, 3072, ("e2m1", "twiddling")), (256, 4096, 8192, ("e2m1", "twiddling", "simple"))])
+def test_default_cut_by_format(cuda, M, N, K, cut):
+    """The "simple" format, whose decoder is the longest, is cut where that is faster with it and not with the others."""
+    from tilelang_amd import _lib
+
+    room = int(_lib.load_library().dq_mxfp4_workspace_bytes(M, N, K))
+    assert room
+    d = workloads.mxfp4(M, N, K, seed=7, scale_bias=127)
+    A, B, S = (_dev(d[k], cuda) for k in ("A", "B", "Scale"))
+    C = torch.empty((M, N), dtype=torch.bfloat16, device=cuda)
+    ws = torch.empty(room, dtype=torch.uint8, device=cuda)
+    for fmt in ("e2m1", "twiddling", "simple"):
+        ws.fill_(255)
+        assert _cut_call(A, B, S, None, C, ws, room, M, N, K, fmt, 0) == 0, _lib.last_error()
+        torch.cuda.synchronize()
+        assert bool((ws == 255).all()) == (fmt not in cut)
+
+
 def test_k_slice_workspace_through_c_abi(cuda):
     """The library's own choice with its full room, with less, with none: fewer slices and in the end the plain entry
     point's bits; what is refused."""

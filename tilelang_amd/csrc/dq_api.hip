@@ -349,26 +349,32 @@ extern "C" int call_unpack_qzeros(const void* QZeros, void* Zeros, int N, int gr
 }
 
 // Into how many slices of K the tiled MXFP4 GEMM is cut when the caller brought a workspace; 1: not cut.  The times (us)
-// are fits, and cut is what they put ahead by a twelfth.  Measured both ways at 1372 shapes (81 to 4096 rows, N 8 to
-// 28672, K 1024 to 28672, odd ones and close calls among them): the 901 that are cut take 0.6 of the uncut time in the
-// median (M = 96, N = K = 8192: 64 -> 29 us; M = 384, N = K = 8192: 90 -> 61; M = 2048, N = 2048, K = 8192: 96 -> 71),
-// one more than it (M = 3000, N = 2048, K = 14336: 174.5 against 173.6 us).
+// are fits, and cut is what they put ahead by a twelfth.  Measured both ways at 1712 shapes (81 to 4096 rows, N 64 to
+// 28672, K 1024 to 28672, odd ones and close calls among them) in the three formats: the 1389 that are cut ("simple"
+// 999) take two thirds of the uncut time in the median (M = 96, N = K = 8192: 64 -> 29 us; M = 384, N = K = 8192:
+// 90 -> 61; M = 2048, N = 2048, K = 8192: 96 -> 71); four calls take 1 to 4 % more (M = 110, N = 818, K = 11520: 25.6
+// against 26.6 us).
 // * Uncut from 96 tiles of 128 x 256 on: 10.4 ns per k there, 12.8 at 224 (the tiles share the memory's bandwidth).
-//   Below that the register-staged kernel's smaller tiles; at a decode batch the register-resident kernel, which up to
-//   K = 4096 takes 0.7 of its estimate (M = 128, N = 2048: 16.5 us, cut 17.2).
+//   Below that the register-staged kernel's tiles of 128 x 64 (beyond 256 of them a second round); at a decode batch
+//   the register-resident kernel, which up to K = 4096 takes 0.7 of its estimate (M = 128, N = 2048: 16.5 us, cut 17.2).
+// * The "simple" format's decoder is longer, and the 128 x 256 tile spills with it: its times are 1.65 of the above there,
+//   1.3 on the other kernels (M = 166, N = 5818, K = 3072: 35.2 us, in four slices 43; e2m1 27.9 and 27.3).
 // * More than one round of 256 workgroups is cut only where the tile count is a multiple of the XCDs: only then does an
 //   XCD walk neighbouring tiles (M = 1000, N = 5120, K = 14336, 160 tiles: 169 -> 146 us; M = 384, N = 13824, K = 8192,
-//   162 tiles: 96 -> 112).  Beyond 192 tiles nothing gained more than 6 %, with a workspace of 100 MB and more.
+//   162 tiles: 96 -> 112).  From 192 tiles on it is even (M = 768, N = 8192, K = 14336: 174 us, in four slices 178), with
+//   a workspace of 100 MB.
 // Up to 80 rows nothing is cut.  That is a promise of the header and no crossover: up to there a call that runs on the
 // tiled kernel gives the bits that its rows have in a large product (cut, M = 80, N = K = 8192 would take 27 us, not 63).
-static int mxfp4_ksplit(int M, int N, int K) {
+static int mxfp4_ksplit(int M, int N, int K, int fp4_format) {
   if (M <= 80 || K % 128 != 0 || ((size_t)M * N) % 4 != 0) return 1;
   const long tiles = (((long)M + 127) / 128) * (((long)N + 255) / 256);
-  if (tiles > 192) return 1;
+  if (tiles >= 192) return 1;
   const int units = K / 128;
-  double best = tiles >= 96 ? 4.0 + 1e-3 * K * (8.6 + 0.0186 * (double)tiles) : 2.0 + 1e-3 * K * (tiles <= 32 ? 7.2 : 8.0);
+  const long small_tiles = (((long)M + 127) / 128) * (((long)N + 63) / 64);  // of the register-staged kernel
+  double best = tiles >= 96 ? 4.0 + 1e-3 * K * (8.6 + 0.0186 * (double)tiles)
+                            : 2.0 + 1e-3 * K * (tiles <= 32 ? 7.2 : tiles <= 64 ? 8.0 : small_tiles <= 256 ? 7.6 : 9.5);
   if (M <= 128) best = std::min(best, mxfp4_regres_time(M, N, K) * (K <= 4096 ? 0.7 : 1.0));
-  best *= 0.92;
+  best *= fp4_format == DQ_FP4_SIMPLE && tiles < 96 ? 0.92 / 1.25 : 0.92;
   int split = 1;
   for (int s = 2; s <= 12 && units / s >= 4; ++s) {
     const long wgs = tiles * s;
@@ -394,7 +400,7 @@ static int gemm_bf16_mxfp4(const char* fn, const void* A, const void* B, const v
   if (scale_bias < 0 || scale_bias > 255) DQ_FAIL("%s: scale_bias must be in 0..255 (got %d)", fn, scale_bias);
   if (!aligned16(A) || !aligned16(B) || !aligned16(C) || (Bias && !aligned16(Bias)))
     DQ_FAIL("%s: A, B, Bias and C must be 16-byte aligned", fn);
-  if (workspace && split == 0) split = mxfp4_ksplit(M, N, K);
+  if (workspace && split == 0) split = mxfp4_ksplit(M, N, K, fp4_format);
   while (split > 1 && (size_t)split * M * N * sizeof(float) > workspace_bytes) --split;
   if (split > 1) {
     const int rc = mxfp4_gemm_ksplit(A, B, Scale, Bias, C, workspace, M, N, K, fp4_format, scale_bias, split, (hipStream_t)stream);
@@ -418,7 +424,7 @@ extern "C" int call_dequant_gemm_bf16_mxfp4(const void* A, const void* B, const 
 
 extern "C" size_t dq_mxfp4_workspace_bytes(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0 || K % 64 != 0) return 0;
-  const int split = mxfp4_ksplit(M, N, K);
+  const int split = mxfp4_ksplit(M, N, K, DQ_FP4_E2M1);
   return split > 1 ? (size_t)split * M * N * sizeof(float) : 0;
 }
 
