@@ -222,43 +222,47 @@ def test_adapter_out_idx_allocates_outputs():
     assert C.shape == (2, 4) and C.dtype == torch.float16 and calls[0][0][2] == C.data_ptr()
 
 
-@pytest.mark.parametrize("has_private", [True, False])
-def test_current_stream_of_an_operands_device(monkeypatch, has_private):
-    """The stream of the GPU that an operand lies on, from torch's private call or, where a build of torch has none,
-    from the public one; never whether there is a GPU at all."""
+def _with_streams(monkeypatch, has_private):
+    """GPU i's current stream is 100 + i, GPU 2 the current one; returns the list of how it was asked for."""
     import types
 
     from tilelang_amd import adapter
 
     asked = []
-    private = types.SimpleNamespace(**({"_cuda_getCurrentRawStream": lambda i: 100 + i} if has_private else {}))
-    cuda = types.SimpleNamespace(is_available=lambda: asked.append("available") or True, current_device=lambda: 2,
-                                 current_stream=lambda i=None: types.SimpleNamespace(cuda_stream=100 + (2 if i is None else i)))
-    monkeypatch.setattr(adapter, "torch", types.SimpleNamespace(_C=private, cuda=cuda))
-    assert adapter.current_stream_handle("cuda", 3) == 103 and not asked
-    assert adapter.current_stream_handle("cuda") == 102 and asked
-    assert adapter.current_stream_handle("cpu", 3) == 0
+    monkeypatch.setattr(adapter, "_raw_stream", (lambda i: asked.append("private") or 100 + i) if has_private else None)
+    monkeypatch.setattr(torch.cuda, "is_available", lambda: asked.append("available") or True)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 2)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda i=None: asked.append("public")
+                        or types.SimpleNamespace(cuda_stream=100 + (2 if i is None else i)))
+    return asked
 
 
-def test_a_call_asks_for_the_stream_through_the_fallback(monkeypatch):
-    """The kernel call itself uses that function, with the operand's device."""
-    import types
-
+@pytest.mark.parametrize("has_private", [True, False])
+def test_current_stream_of_an_operands_device(monkeypatch, has_private):
+    """The stream of the GPU that an operand lies on, from torch's private call or, where a build of torch has none,
+    from the public one; never whether there is a GPU at all."""
     from tilelang_amd import adapter
 
-    seen = []
-    monkeypatch.setattr(adapter, "current_stream_handle", lambda device_type, index=None: seen.append((device_type, index)) or 7)
-    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
-    k, calls = _cpu_adapter()
-    k.device_type = "cuda"
-    operand = torch.zeros(2, 8, dtype=torch.float16)
+    how = "private" if has_private else "public"
+    asked = _with_streams(monkeypatch, has_private)
+    assert adapter.current_stream_handle("cuda", 3) == 103 and asked == [how]
+    assert adapter.current_stream_handle("cuda") == 102 and asked == [how, "available", how]
+    assert adapter.current_stream_handle("cpu", 3) == 0 and len(asked) == 3
+
+
+@pytest.mark.parametrize("has_private", [True, False])
+def test_a_call_launches_on_the_stream_of_its_operands_device(monkeypatch, has_private):
+    """The kernel call itself, either way."""
+    asked = _with_streams(monkeypatch, has_private)
 
     class OnGpu(torch.Tensor):
-        device = torch.device("cuda", 1)
+        device = torch.device("cuda", 2)
 
-    A, B, C = (t.as_subclass(OnGpu) for t in (operand, torch.zeros(4, 4, dtype=torch.int8), torch.zeros(2, 4, dtype=torch.float16)))
-    k(A, B, C)
-    assert seen == [("cuda", 1)] and calls[0][1] == 7
+    k, calls = _cpu_adapter()
+    k.device_type = "cuda"
+    operands = [torch.zeros(2, 8, dtype=torch.float16), torch.zeros(4, 4, dtype=torch.int8), torch.zeros(2, 4, dtype=torch.float16)]
+    k(*(t.as_subclass(OnGpu) for t in operands))
+    assert calls[0][1] == 102 and asked == ["private" if has_private else "public"]
 
 
 @pytest.mark.parametrize("workspace_idx,result_idx", [([1], [2]), ([-1], [-2]), ([0, 3], []), ([], [-1])])
