@@ -1,0 +1,120 @@
+"""The 128 x 256 tile of the direct-to-LDS GEMM (dq_gemm_core.h) at the edges of its walk over K and of the matrix, and the
+stores of rows that are no whole cache lines.  Operands are small integers and powers of two, so that every product and every
+fp32 sum is exact and the result is one rounding of the float64 product, whatever order the kernel adds in."""
+
+import pytest
+import torch
+
+import tilelang_amd as tl
+from tilelang_amd import _lib, quantize
+
+pytestmark = pytest.mark.gpu
+
+
+def _ints(gen, lo, hi, *shape, dtype, device):
+    return torch.randint(lo, hi + 1, shape, generator=gen, device=device).to(dtype)
+
+
+def _nibbles(packed):
+    b = packed.view(torch.uint8)
+    return torch.stack((b & 15, b >> 4), dim=-1).reshape(b.shape[0], -1)
+
+
+@pytest.mark.parametrize("zeros", [False, True])
+@pytest.mark.parametrize("M,N,K,group", [
+    (1025, 3076, 384, 64),    # three stages of 128 k, the fewest on eight waves; one row and four columns in the last tiles
+    (1100, 3500, 256, 128),   # two: four waves
+    (1100, 3500, 640, 64),    # five
+    (1100, 3500, 1024, 128),  # a dword of scales every other stage
+    (1100, 3500, 3072, 512),  # every eighth
+    (1100, 3500, 512, 32),    # one per 64 k: four waves
+    (897, 4104, 1024, 256),   # rows of C that are no whole lines
+])
+def test_uint4(cuda, M, N, K, group, zeros):
+    gen = torch.Generator(device=cuda).manual_seed(K + group)
+    A = _ints(gen, -2, 2, M, K, dtype=torch.float16, device=cuda)
+    B = _ints(gen, -128, 127, N, K // 2, dtype=torch.int8, device=cuda)
+    S = torch.exp2(_ints(gen, -4, 0, N, K // group, dtype=torch.float16, device=cuda))
+    Z = _ints(gen, 5, 11, N, K // group, dtype=torch.float16, device=cuda)
+    kern = tl.matmul_w4a16(M, N, K, group_size=group, source_format="uint" if zeros else "int", with_zeros=zeros)
+    C = torch.full((M, N), float("nan"), dtype=torch.float16, device=cuda)
+    kern(A, B, S, *([Z] if zeros else []), C)
+    zero = Z.double().repeat_interleave(group, dim=1) if zeros else 8.0
+    W = (_nibbles(B).double() - zero) * S.double().repeat_interleave(group, dim=1)
+    assert torch.equal(C, (A.double() @ W.t()).half())
+
+
+@pytest.mark.parametrize("K", [384, 640, 256])
+def test_fp4(cuda, K):
+    M, N = 1100, 3500
+    gen = torch.Generator(device=cuda).manual_seed(K)
+    A = _ints(gen, -2, 2, M, K, dtype=torch.bfloat16, device=cuda)
+    B = _ints(gen, 0, 255, N, K // 2, dtype=torch.uint8, device=cuda)
+    C = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=cuda)
+    rc = _lib.get_library().call_dequant_gemm_bf16_fp4(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, 0,
+                                                       torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, _lib.last_error()
+    values = torch.tensor([0.0, 0.5, 1.0, 1.5, 2.0, 3.0, 4.0, 6.0], dtype=torch.float64, device=cuda)
+    W = torch.cat((values, -values))[_nibbles(B).int()]
+    assert torch.equal(C, (A.double() @ W.t()).bfloat16())
+
+
+@pytest.mark.parametrize("M,N,K", [(1100, 3500, 640), (1100, 3500, 128), (2600, 6200, 384)])
+def test_mxfp4_rows_keep_their_bits(cuda, M, N, K):
+    """Uncut, a row's products are added in one order whatever tile the call runs on: the rows of a large product against
+    a call of 80 of them (real-valued operands, so that another order would show)."""
+    gen = torch.Generator(device=cuda).manual_seed(N + K)
+    A = torch.randn((M, K), generator=gen, device=cuda).bfloat16()
+    B = _ints(gen, 0, 255, N, K // 2, dtype=torch.uint8, device=cuda)
+    S = _ints(gen, 119, 127, N, K // 32, dtype=torch.uint8, device=cuda)
+    out = []
+    for a in (A, A[M - 80:].contiguous()):
+        C = torch.empty((a.shape[0], N), dtype=torch.bfloat16, device=cuda)
+        rc = _lib.get_library().call_dequant_gemm_bf16_mxfp4(a.data_ptr(), B.data_ptr(), S.data_ptr(), None, C.data_ptr(),
+                                                             a.shape[0], N, K, 32, 0, 127, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0, _lib.last_error()
+        out.append(C)
+    assert torch.equal(out[0][M - 80:].view(torch.int16), out[1].view(torch.int16))
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (1000, 3500, 768),   # 128 x 256; columns of Ct that are no whole lines
+    (1001, 3500, 256),   # and no multiple of 16 bytes: stored by elements; two k-blocks: four waves
+    (1002, 3333, 512),   # 128 x 256 on eight waves
+    (1024, 3500, 1024),
+    (999, 11008, 512),   # 256 x 256
+    (131, 200, 384),     # register-staged
+    (36, 130, 256),
+])
+@pytest.mark.parametrize("transposed", [True, False])
+def test_int8_int4(cuda, M, N, K, transposed):
+    gen = torch.Generator(device=cuda).manual_seed(M)
+    A = _ints(gen, -128, 127, M, K, dtype=torch.int8, device=cuda)
+    B = _ints(gen, 0, 255, N, K // 2, dtype=torch.uint8, device=cuda)
+    C = torch.full((N, M) if transposed else (M, N), -7, dtype=torch.int32, device=cuda)
+    rc = _lib.get_library().call_gemm_int8xint4(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, 1, 0, int(transposed),
+                                                torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, _lib.last_error()
+    codes = _nibbles(B).short()
+    W = torch.where(codes > 7, codes - 16, codes).double()
+    ref = (W @ A.double().t()) if transposed else (A.double() @ W.t())
+    assert torch.equal(C, ref.int())
+
+
+@pytest.mark.parametrize("fragments", [False, True])
+@pytest.mark.parametrize("M,N,K", [(1300, 4000, 768), (1300, 4000, 512), (1281, 4072, 1280)])  # three stages, two, five
+def test_bitnet(cuda, M, N, K, fragments):
+    gen = torch.Generator(device=cuda).manual_seed(K)
+    A = _ints(gen, -128, 127, M, K, dtype=torch.int8, device=cuda)
+    codes = _ints(gen, 1, 3, N, K // 16, 4, 4, dtype=torch.uint8, device=cuda)  # element e of a word at bit 8 (e % 4) + 2 (e / 4)
+    packed = sum(codes[:, :, j] << (2 * j) for j in range(4)).reshape(N, K // 4).view(torch.int8)
+    s_a = torch.exp2(_ints(gen, -1, 2, M, dtype=torch.float32, device=cuda))
+    B = quantize.prepack_i2_fragments(packed) if fragments else packed
+    out = torch.full((M, N), float("nan"), dtype=torch.float16, device=cuda)
+    layout = 1 | (2 if fragments else 0)  # interleaved words, in the operand order or row-major
+    rc = _lib.get_library().call_gemm_int8xint2(A.data_ptr(), B.data_ptr(), out.data_ptr(), M, N, K, 1, layout, s_a.data_ptr(), 4.0,
+                                                1, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, _lib.last_error()
+    W = codes.reshape(N, K).double() - 2
+    ref = (A.double() @ W.t()) / s_a.double()[:, None] / 4.0
+    assert torch.equal(out, ref.half())

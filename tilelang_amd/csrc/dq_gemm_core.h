@@ -125,34 +125,48 @@ __device__ __forceinline__ void take_k_slice(Params& p, int& bid) {
   }
 }
 
-// Epilogue shared by both kernel variants (a macro: it uses the kernel's locals).
+// Epilogue shared by both kernel variants (a macro: it uses the kernel's locals), over the first BLOCKS_ of the wave's kMBW
+// blocks of rows.
 // acc[mb][nb][i] = C[m0 + (wm*kMBW + mb)*32 + 8*(i/4) + 4*g + i%4][n0 + (wn*kNBW + nb)*32 + r], with kMBW x kNBW
 // blocks of 32 x 32 per wave (constants of the kernel that expands the macro).  Staged through
 // LDS (every tile is consumed: the loop ended with a barrier) so that each lane stores 16 contiguous
-// bytes.  Each wave owns a 32 x (128 + 4) slab of 32-bit values; LDS operations of one wave execute
-// in order, so no workgroup barrier is needed between the phases.  Each wave owns a 32 x (32 kNBW + 4) slab.
-// C is written once and not read again by the kernel: the 16-byte stores are nontemporal, which keeps the
-// output from displacing operand lines in the L2 (MXFP4 GEMM 361 -> 358 us, block-scaled GEMM 147 -> 138 us).  The
-// partial sums of K slices, which the next kernel reads, leave the same way (not measured otherwise).
-#define DQ_GEMM_EPILOGUE \
+// bytes.  Each wave owns a slab of 32-bit values, 32 x (32 kNBW + 4) for a block of rows or, transposed, 32 x (32 kMBW + 4)
+// for a block of columns; LDS operations of one wave execute in order, so no workgroup barrier is needed between the phases.
+// The stores: C is written once and not read again by the kernel.  Where its rows (transposed: columns) are whole cache
+// lines they are nontemporal, which keeps the output from displacing operand lines in the L2 (MXFP4 GEMM 361 -> 358 us,
+// block-scaled GEMM 147 -> 138 us).  Where they are not, a line is shared by two pieces that a nontemporal store would
+// each write to memory by itself: ordinary stores, which meet in the L2 (int8 x int4, M = 1000, N = 11008, K = 1024:
+// 34 -> 26 us; int8 x 2-bit, M = 2048, N = 8200, K = 4096 118 -> 92; MXFP4 there 159 -> 140).  Which of the two is asked
+// once per tile: asked per store it cost BitLinear at M = 2048, N = K = 8192 1 %.
+// Transposed, the four consecutive rows that a lane holds are one LDS write, and a wave stores whole runs of its rows; a
+// column that does not start at 16 bytes goes out by elements, consecutive lanes on consecutive elements (M = 1001,
+// N = 11008, K = 4096: 73 -> 59 us, with the better tile of that shape).
+#define DQ_GEMM_EPILOGUE DQ_GEMM_EPILOGUE_OF(kMBW)
+#define DQ_GEMM_EPILOGUE_OF(BLOCKS_) \
+  if ((P::kTransposed ? M : N) * (int)sizeof(typename P::out_t) % 128 == 0) { \
+    DQ_GEMM_EPILOGUE_STORING(BLOCKS_, true) \
+  } else { \
+    DQ_GEMM_EPILOGUE_STORING(BLOCKS_, false) \
+  }
+#define DQ_GEMM_EPILOGUE_STORING(BLOCKS_, WHOLE_LINES_) \
   using out_t = typename P::out_t; \
-  constexpr int kSlabStride = 32 * kNBW + 4; \
   constexpr int kOutPerPiece = 16 / sizeof(out_t); \
-  uint32_t* slab = reinterpret_cast<uint32_t*>(smem) + wave * (32 * kSlabStride); \
+  if constexpr (!P::kTransposed) { \
+    constexpr int kSlabStride = 32 * kNBW + 4; \
+    uint32_t* slab = reinterpret_cast<uint32_t*>(smem) + wave * (32 * kSlabStride); \
   _Pragma("unroll") \
-  for (int mb = 0; mb < kMBW; ++mb) { \
+    for (int mb = 0; mb < BLOCKS_; ++mb) { \
   _Pragma("unroll") \
-    for (int nb = 0; nb < kNBW; ++nb) \
+      for (int nb = 0; nb < kNBW; ++nb) \
   _Pragma("unroll") \
-      for (int i = 0; i < 16; ++i) { \
-        const int row = 8 * (i >> 2) + 4 * g + (i & 3); \
-        const decltype(acc[0][0][0] + 0) elem = acc[mb][nb][i]; \
-        uint32_t bits; \
-        __builtin_memcpy(&bits, &elem, 4); \
-        slab[row * kSlabStride + nb * 32 + r] = bits; \
-      } \
-    __builtin_amdgcn_wave_barrier(); \
-    if constexpr (!P::kTransposed) { \
+        for (int i = 0; i < 16; ++i) { \
+          const int row = 8 * (i >> 2) + 4 * g + (i & 3); \
+          const decltype(acc[0][0][0] + 0) elem = acc[mb][nb][i]; \
+          uint32_t bits; \
+          __builtin_memcpy(&bits, &elem, 4); \
+          slab[row * kSlabStride + nb * 32 + r] = bits; \
+        } \
+      __builtin_amdgcn_wave_barrier(); \
       constexpr int kPiecesPerRow = 32 * kNBW / kOutPerPiece; \
       constexpr int kIters = 32 * kPiecesPerRow / 64; \
   _Pragma("unroll") \
@@ -175,7 +189,8 @@ __device__ __forceinline__ void take_k_slice(Params& p, int& bid) {
           if ((n + kOutPerPiece <= N) && ((N % kOutPerPiece) == 0)) { \
             uint4_t pk; \
             __builtin_memcpy(&pk, o, 16); \
-            __builtin_nontemporal_store(pk, reinterpret_cast<uint4_t*>(dst)); \
+            if constexpr (WHOLE_LINES_) __builtin_nontemporal_store(pk, reinterpret_cast<uint4_t*>(dst)); \
+            else *reinterpret_cast<uint4_t*>(dst) = pk; \
           } else { \
   _Pragma("unroll") \
             for (int e = 0; e < kOutPerPiece; ++e) \
@@ -183,34 +198,59 @@ __device__ __forceinline__ void take_k_slice(Params& p, int& bid) {
           } \
         } \
       } \
-    } else { \
-      constexpr int kPiecesPerCol = 32 / kOutPerPiece; \
-      constexpr int kIters = 32 * kNBW * kPiecesPerCol / 64; \
+      __builtin_amdgcn_wave_barrier(); \
+    } \
+  } else { \
+    constexpr int kRows = 32 * BLOCKS_; \
+    constexpr int kSlabStride = kRows + 4; \
+    uint32_t* slab = reinterpret_cast<uint32_t*>(smem) + wave * (32 * kSlabStride); \
+    const int m_wave = m0 + wm * (32 * kMBW); \
   _Pragma("unroll") \
-      for (int it = 0; it < kIters; ++it) { \
-        const int q = lane + 64 * it; \
-        const int col = q / kPiecesPerCol, piece = q % kPiecesPerCol; \
-        const int n = n0 + wn * (32 * kNBW) + col; \
-        const int m = m0 + wm * (32 * kMBW) + mb * 32 + piece * kOutPerPiece; \
-        if (n < N && m < M) { \
-          out_t o[kOutPerPiece]; \
+    for (int nb = 0; nb < kNBW; ++nb) { \
   _Pragma("unroll") \
-          for (int e = 0; e < kOutPerPiece; ++e) \
-            o[e] = P::finish(slab[(piece * kOutPerPiece + e) * kSlabStride + col], p, min(m + e, M - 1), n); \
-          out_t* dst = (out_t*)p.C + (size_t)n * M + m; \
-          if ((m + kOutPerPiece <= M) && ((M % kOutPerPiece) == 0)) { \
+      for (int mb = 0; mb < BLOCKS_; ++mb) \
+  _Pragma("unroll") \
+        for (int v = 0; v < 4; ++v) { \
+          const decltype(acc[0][0][0] + 0) elem[4] = {acc[mb][nb][4 * v], acc[mb][nb][4 * v + 1], acc[mb][nb][4 * v + 2], acc[mb][nb][4 * v + 3]}; \
+          uint4_t bits; \
+          __builtin_memcpy(&bits, elem, 16); \
+          *reinterpret_cast<uint4_t*>(slab + r * kSlabStride + mb * 32 + 8 * v + 4 * g) = bits; \
+        } \
+      __builtin_amdgcn_wave_barrier(); \
+      const int n_block = n0 + wn * (32 * kNBW) + nb * 32; \
+      if ((M % kOutPerPiece) == 0) { \
+        constexpr int kPiecesPerCol = kRows / kOutPerPiece; \
+  _Pragma("unroll") \
+        for (int it = 0; it < 32 * kPiecesPerCol / 64; ++it) { \
+          const int q = lane + 64 * it; \
+          const int col = q / kPiecesPerCol, piece = q % kPiecesPerCol; \
+          const int n = n_block + col, m = m_wave + piece * kOutPerPiece; \
+          uint32_t raw[kOutPerPiece]; \
+  _Pragma("unroll") \
+          for (int e = 0; e < kOutPerPiece; e += 4) { \
+            const uint4_t v = *reinterpret_cast<const uint4_t*>(slab + col * kSlabStride + piece * kOutPerPiece + e); \
+            raw[e] = v[0]; raw[e + 1] = v[1]; raw[e + 2] = v[2]; raw[e + 3] = v[3]; \
+          } \
+          if (n < N && m < M) { \
+            out_t o[kOutPerPiece]; \
+  _Pragma("unroll") \
+            for (int e = 0; e < kOutPerPiece; ++e) o[e] = P::finish(raw[e], p, m + e, n); \
             uint4_t pk; \
             __builtin_memcpy(&pk, o, 16); \
-            __builtin_nontemporal_store(pk, reinterpret_cast<uint4_t*>(dst)); \
-          } else { \
-  _Pragma("unroll") \
-            for (int e = 0; e < kOutPerPiece; ++e) \
-              if (m + e < M) dst[e] = o[e]; \
+            uint4_t* const dst = reinterpret_cast<uint4_t*>((out_t*)p.C + (size_t)n * M + m); \
+            if constexpr (WHOLE_LINES_) __builtin_nontemporal_store(pk, dst); \
+            else *dst = pk; \
           } \
         } \
+      } else { \
+        for (int it = 0; it < 32 * kRows / 64; ++it) { \
+          const int q = lane + 64 * it; \
+          const int col = q / kRows, m = m_wave + q % kRows, n = n_block + col; \
+          if (n < N && m < M) ((out_t*)p.C)[(size_t)n * M + m] = P::finish(slab[col * kSlabStride + q % kRows], p, m, n); \
+        } \
       } \
+      __builtin_amdgcn_wave_barrier(); \
     } \
-    __builtin_amdgcn_wave_barrier(); \
   } \
   /* end of epilogue */
 
@@ -454,7 +494,7 @@ __global__ __launch_bounds__(kThreads * kKSplit, 1) void gemm_kernel(const Param
 
   if constexpr (kKSplit == 2) {
     // the second copy hands its accumulators to the first: [wave][mb][nb][lane] behind the epilogue's slabs
-    constexpr int kSlabBytes = 4 * 32 * (32 * kNBW + 4) * 4;
+    constexpr int kSlabBytes = 4 * 32 * (32 * (kNBW > kMBW ? kNBW : kMBW) + 4) * 4;
     typename P::acc_t* red = reinterpret_cast<typename P::acc_t*>(smem_all + ((kSlabBytes + 63) & ~63)) + wave * (kMBW * kNBW * 64) + lane;
     if (kh == 1) {
 #pragma unroll
@@ -983,7 +1023,7 @@ int launch(Params p, hipStream_t stream) {
   constexpr int kTileM = 64 * kMBW, kTileN = 64 * kNBW;
   constexpr int kPipe = kKSplit * 3 * (kTileM * kARowBytes + kTileN * P::kBRowBytes);
   // epilogue staging, and behind it the accumulators the second copy of the pipeline hands over
-  constexpr int kSlabs = ((4 * 32 * (32 * kNBW + 4) * 4 + 63) & ~63) + (kKSplit - 1) * 4 * kMBW * kNBW * 64 * 64;
+  constexpr int kSlabs = ((4 * 32 * (32 * (kNBW > kMBW ? kNBW : kMBW) + 4) * 4 + 63) & ~63) + (kKSplit - 1) * 4 * kMBW * kNBW * 64 * 64;
   constexpr int kLds = kPipe > kSlabs ? kPipe : kSlabs;
   static_assert(kLds <= 160 * 1024, "LDS budget");
   p.tiles_m = (p.M + kTileM - 1) / kTileM;
@@ -1051,7 +1091,7 @@ int launch_dma_tile(Params p, hipStream_t stream) {
   constexpr int kTileM = 32 * kMBW * kWavesM;
   constexpr bool kPairB = P::kBRowBytes == 32 && kTileM == 256 && kWaves == 4;  // as in the kernel: a fourth B slot
   constexpr int kPipe = 3 * (kTileM * kARowBytes + BN * P::kBRowBytes) + (kPairB ? BN * P::kBRowBytes : 0) + 8 * 1024;
-  constexpr int kSlabs = kWaves * 32 * (32 * kNBW + 4) * 4;  // epilogue staging
+  constexpr int kSlabs = kWaves * 32 * (32 * (kNBW > kMBW ? kNBW : kMBW) + 4) * 4;  // epilogue staging
   constexpr int kLds = kPipe > kSlabs ? kPipe : kSlabs;
   p.tiles_m = (p.M + kTileM - 1) / kTileM;
   p.tiles_n = (p.N + BN - 1) / BN;
