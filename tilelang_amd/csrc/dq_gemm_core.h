@@ -34,13 +34,6 @@
 #define DQ_SWZ_SHIFT 1
 #endif
 
-#ifndef DQ_DMA_NBW
-#define DQ_DMA_NBW 4  // wave tile columns / 32 of the direct-to-LDS kernel (2 = eight waves, two per SIMD)
-#endif
-#ifndef DQ_DMA_MBW
-#define DQ_DMA_MBW 4  // wave tile rows / 32 of the direct-to-LDS kernel (2 = 128 x 256 tiles, two workgroups per CU)
-#endif
-
 namespace dq {
 namespace gemm {
 
@@ -375,7 +368,7 @@ __global__ __launch_bounds__(kThreads * kKSplit, 1) void gemm_kernel(const Param
     a_row_sw[mb] = a_swz(row);
   }
   // packed B of n-block nb: row wn*128 + nb*32 + r, the half of the row that belongs to group g
-  int b_off[kNBW][kBPiecesPerRow / 2];
+  int b_off[kNBW][kBWords / 4];
   int w_row[kNBW];
 #pragma unroll
   for (int nb = 0; nb < kNBW; ++nb) {
@@ -548,63 +541,80 @@ __device__ __forceinline__ void dma4(unsigned lds_addr, unsigned voff, const voi
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2\n\t" ::"s"(lds_addr), "v"(voff), "s"(sbase) : "memory");
 }
 
-// kMBW = 4: 256 x 256 tile, one workgroup per CU (the default).  kMBW = 2: 128 x 256 tile, two
-// workgroups per CU (76 KiB of LDS and 256 registers each) that fill each other's barrier stalls;
-// measured 13 % slower on the 4096 x 8192 x 8192 MXFP4 problem (twice the decode work per MFMA,
-// and the 256-register budget spills), so it is kept as a build option only.  kNBW = 2: the same
-// 256 x 256 tile on eight waves (two per SIMD, wave tile 128 x 64): no spills and the same decode work,
-// but every A fragment is read from LDS by twice as many waves; measured 4 % slower on that
-// problem (410 us against 393 us), also a build option only (-DDQ_DMA_NBW=2).  Eight waves of 64 x 128
-// (four along the rows, which keeps the LDS traffic of the four-wave form) measured the same 410 us: a
-// second wave per SIMD does not buy MFMA issue slots here.
-//
-// kWavesM = 1 (with kMBW = 8, kNBW = 2): the same 256 x 256 tile on four waves side by side, each 256 rows x 64
-// columns.  A wave then decodes only the 64 weight rows it alone multiplies (with two rows of waves every packed
-// word is decoded twice per workgroup) and reads every A fragment of the tile instead: half the decode
-// instructions, twice the LDS reads of A.  For policies whose decode keeps a lone wave's instruction issue busier
-// than its matrix pipe (P::kTallWaves).
-template <class P, int kMBW, int kNBW, int kWavesM = 2>
-__global__ __launch_bounds__(64 * kWavesM * (8 / kNBW), 32 * kMBW * kWavesM == 128 ? 2 : 1) void gemm_kernel_dma(const Params p_in) {
+// The same where `not_due` (wave-uniform) is zero.  The jump stays inside the statement: a branch of its own
+// would cut the region that the scheduler spreads over the matrix instructions.
+__device__ __forceinline__ void dma4_unless(int not_due, unsigned lds_addr, unsigned voff, const void* sbase) {
+  asm volatile("s_cmp_lg_u32 %0, 0\n\ts_cbranch_scc1 .Lnot_due%=\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %2, %3\n.Lnot_due%=:" ::"s"(__builtin_amdgcn_readfirstlane(not_due)), "s"(lds_addr), "v"(voff), "s"(sbase) : "memory", "scc");
+}
+
+// Three forms, on a tile of 256 columns:
+// * kMBW = 4, kNBW = 4, kWavesM = 2: 256 rows on 2 x 2 waves of 128 x 128, one workgroup per CU.
+// * kMBW = 8, kNBW = 2, kWavesM = 1: 256 rows on four waves side by side, each 256 rows x 64 columns.  A wave then
+//   decodes only the 64 weight rows it alone multiplies (with two rows of waves every packed word is decoded twice per
+//   workgroup) and reads every A fragment of the tile instead: half the decode instructions, twice the LDS reads of A.
+//   For policies whose decode keeps a lone wave's instruction issue busier than its matrix pipe (P::kTallWaves).
+// * kMBW = 4, kNBW = 2, kWavesM = 1: 128 rows on four waves side by side of 128 x 64, for problems with too few tiles
+//   of 256 rows.  With kKHalves = 2 on eight waves, two per SIMD: waves 4 .. 7 multiply the other half of every stage
+//   (a second k-block, or with 64-byte rows of B the other two steps of the one k-block) into accumulators of their own,
+//   and the two halves exchange sums through LDS before the epilogue, of which each does half.
+// What bounds the 128-row form is the CU's load unit, which takes about two cycles per 64 bytes or per row piece, if that
+// is shorter: with a 32-byte piece of B and a dword of scales and of zeros per weight row and k-block (two workgroups of
+// four waves, 2 x 2) it was busy 87 % of the time and the matrix pipe 45 %.  So scales come only when their dword is due,
+// a stage brings B in pieces of 64 bytes, and eight waves share one stage (load unit 43 %, matrix pipe 73 %).  fp16 x
+// uint4 with zeros at M = 2048, N = 4096, K = 14336: 260 -> 233 (scales when due, waves side by side) -> 211 us; M = 300,
+// N = 13824, K = 5120: 86 -> 73 -> 60; MXFP4 at M = 768, N = K = 8192: 102 -> 92 -> 83; int8 x 2-bit, M = 1024,
+// N = K = 8192: 58 -> 53.5; int8 x int4, M = 1024, N = K = 8192: 64 -> 59.5.
+template <class P, int kMBW, int kNBW, int kWavesM = 2, int kKHalves = 1>
+__global__ __launch_bounds__(256 * kKHalves, 32 * kMBW * kWavesM == 128 ? 2 : 1) void gemm_kernel_dma(const Params p_in) {
   Params p = p_in;
   int bid = blockIdx.x;
   take_k_slice<P>(p, bid);
   extern __shared__ __align__(16) unsigned char smem[];
   static_assert(P::kBRowBytes == 32 || P::kBRowBytes == 64, "direct-to-LDS variant: 32 or 64 packed bytes per weight row per tile");
-  static_assert(kWavesM == 2 ? (kMBW == 2 || kMBW == 4) : (kWavesM == 1 && kMBW == 8 && kNBW == 2), "wave tile of 64, 128 or 256 rows");
-  static_assert(kNBW == 2 || kNBW == 4, "wave tile of 64 or 128 columns");
+  static_assert(kWavesM == 2 ? (kMBW == 4 && kNBW == 4) : (kWavesM == 1 && (kMBW == 8 || kMBW == 4) && kNBW == 2), "one of the three forms");
+  static_assert(kKHalves == 1 || (kKHalves == 2 && kWavesM == 1 && kMBW == 4), "two halves of a stage: the 128-row form");
   constexpr int kWavesN = 8 / kNBW;            // waves across the 256 tile columns
-  constexpr int kWaves = kWavesM * kWavesN;    // 4, or 8 (two per SIMD)
+  constexpr int kWaves = 4;                    // of one half
   constexpr int BM = 32 * kMBW * kWavesM;      // shadows the 256-row default
-  constexpr int kAStage = BM * kARowBytes;     // 32 or 16 KiB
-  constexpr int kAOps = BM / 8 / kWaves;       // A DMA instructions per wave per tile
+  constexpr bool kHalves = kKHalves == 2;
+  constexpr int kStageTiles = kHalves && P::kBRowBytes == 32 ? 2 : 1;  // k-blocks in a stage
+  constexpr int kSteps = kHalves && P::kBRowBytes == 64 ? 2 : 4;       // of a wave in a k-block
+  constexpr int kAStage = BM * kARowBytes * kStageTiles;  // 32 KiB (16 for 128 rows and one k-block)
+  constexpr int kDmaWaves = kWaves * kKHalves;
+  constexpr int kAOps = BM * kStageTiles / 8 / kDmaWaves;  // A DMA instructions per wave per stage
   constexpr int kBPiecesPerRow = P::kBRowBytes / 16;          // 2 or 4
-  constexpr int kBRot = kBPiecesPerRow == 2 ? 3 : 2;          // piece rotation advances every 8 or 4 rows
-  constexpr int kBOps = BN * kBPiecesPerRow / 64 / kWaves;    // packed-B DMA instructions per wave per tile
-  constexpr int kBStage = BN * P::kBRowBytes;  // 8 KiB
-  constexpr int kStage = kAStage + kBStage;    // 40 or 24 KiB
+  constexpr bool kBFrag = BFragments<P>::value;
+  constexpr int kBLoadPieces = kBPiecesPerRow * kStageTiles;  // of a row in one stage
+  constexpr int kBRot = kBLoadPieces == 2 ? 3 : 2;            // piece rotation advances every 8 or 4 rows
+  constexpr int kBOps = BN * kBPiecesPerRow * kStageTiles / 64 / kDmaWaves;    // packed-B DMA instructions per wave per tile
+  constexpr int kBStage = BN * P::kBRowBytes * kStageTiles;  // 8 or 16 KiB
+  constexpr int kStage = kAStage + kBStage;
   constexpr int kStages = 3;
   // A packed-B row of one tile is 32 bytes, a quarter of a cache line, and the next tile's row is the next 32:
   // the B loads of tiles t and t + 1 (t even) are issued as pairs, the same instruction for t and then for t + 1,
   // which halves the lines the B stream asks the L2 for.  Tile t + 1 then lands three iterations before it is
-  // read, which takes a fourth B slot, so B gets a ring of its own behind the three A stages: kPairB.  Policies
-  // with 64-byte rows keep A and B side by side in three stages (a fourth 16 KiB slot would not fit).
-  constexpr bool kPairB = P::kBRowBytes == 32 && BM == 256 && kWaves == 4;
+  // read, which takes a fourth B slot, so B gets a ring of its own behind the three A stages: kPairB.  (One 64-byte piece
+  // of a row for both tiles, half the load unit's steps: 357.3 -> 357.8 us for MXFP4 at M = 4096, N = K = 8192, which the
+  // load unit does not bind.)  Policies with 64-byte rows keep A and B side by side in three stages (a fourth 16 KiB
+  // slot would not fit).
+  constexpr bool kPairB = P::kBRowBytes == 32 && BM == 256;
   constexpr int kBRing = kPairB ? kStages * kAStage : kAStage;       // where B of slot 0 starts
   constexpr int kBSlot = kPairB ? kBStage : kStage;                  // distance between B slots
   constexpr int kAStride = kPairB ? kAStage : kStage;                // distance between A stages
   // Scales that travel by DMA (P::kScaleDma): 1 = one byte per 32 k (a dword per row covers a pair of tiles),
   // 2 = one fp16 per group of 64 .. 4096 k (a dword per row covers two groups: four tiles at group 128), 3 = the same
-  // for scales and for zeros.
+  // for scales and for zeros.  A dword is asked for with the first tile it serves (and with the first tile of all).
   // Ring: 4 slots x 1 KiB (256 rows x one dword), a second ring for the zeros.
   constexpr int kRing = kPairB ? kStages * kAStage + 4 * kBStage : kStages * kStage;
-  constexpr int kSOps = P::kScaleDma == 0 ? 0 : (P::kScaleDma == 3 ? 2 : 1);  // scale DMA instructions per wave per tile
-  constexpr int kBWords = P::kBRowBytes / 8;   // dwords per lane and 32-row block: 4 or 8
-  constexpr bool kBFrag = BFragments<P>::value;
-  static_assert(!kBFrag || (P::kBRowBytes == 32 && kWaves == 4), "fragment-ordered B: 32-byte rows, four waves");
+  constexpr int kSOps = P::kScaleDma == 0 ? 0 : (P::kScaleDma == 3 ? 2 : 1);  // scale DMA instructions per wave per tile, at most
+  constexpr int kBWords = P::kBRowBytes / 8 * kSteps / 4;   // dwords per lane and 32-row block: 4 or 8
+  static_assert(!kBFrag || P::kBRowBytes == 32, "fragment-ordered B: 32-byte rows");
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int dma_wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kh = kHalves ? dma_wave / kWaves : 0;  // which half of a stage the wave multiplies
+  const int wave = kHalves ? dma_wave % kWaves : dma_wave;
   const int wm = wave / kWavesN, wn = wave % kWavesN;
   const int g = lane >> 5, r = lane & 31;
   const int M = p.M, N = p.N, K = p.K;
@@ -612,28 +622,31 @@ __global__ __launch_bounds__(64 * kWavesM * (8 / kNBW), 32 * kMBW * kWavesM == 1
   int tm, tn;
   tile_of_block(bid, p.tiles_m, p.tiles_n, tm, tn);
   const int m0 = tm * BM, n0 = tn * BN;
-  const int KB = K / P::kKPerBlock;
+  const int KB = K / P::kKPerBlock / kStageTiles;  // tiles, or stages of two of them
   const unsigned lds0 = (unsigned)(size_t)smem;  // LDS byte address of the dynamic segment
 
   // ---- per-lane source offsets: LDS chunk c (16 bytes) of a tile <- which global 16 bytes --------
   unsigned a_voff[kAOps], b_voff[kBOps];
 #pragma unroll
   for (int i = 0; i < kAOps; ++i) {
-    const int c = (wave * kAOps + i) * 64 + lane;  // A chunk: row c / 8, physical piece c % 8
-    const int row = c >> 3, pp = c & 7;
-    a_voff[i] = (unsigned)min(m0 + row, M - 1) * (unsigned)(p.ldk * (kARowBytes / P::kKPerBlock)) + (unsigned)((pp ^ a_swz(row)) << 4);
+    const int c = (dma_wave * kAOps + i) * 64 + lane;  // A chunk: row c / 8 (of half c / 1024), physical piece c % 8
+    const int row = (c >> 3) % BM, pp = c & 7;
+    a_voff[i] = (unsigned)min(m0 + row, M - 1) * (unsigned)(p.ldk * (kARowBytes / P::kKPerBlock)) + (unsigned)((pp ^ a_swz(row)) << 4) +
+                (unsigned)((c >> 3) / BM * kARowBytes);
   }
 #pragma unroll
   for (int i = 0; i < kBOps; ++i) {
-    const int c = (wave * kBOps + i) * 64 + lane;  // B chunk: row c / pieces per row, physical piece c % pieces per row
-    const int row = c / kBPiecesPerRow, pp = c % kBPiecesPerRow;
+    const int c = (dma_wave * kBOps + i) * 64 + lane;  // B chunk: row c / pieces per row, physical piece c % pieces per row
+    const int row = c / kBLoadPieces, pp = c % kBLoadPieces;
     // LDS position (piece + rotation) % pieces holds source piece `piece`
     b_voff[i] = (unsigned)min(n0 + row, N - 1) * (unsigned)(p.ldk * P::kBRowBytes / P::kKPerBlock) +
-                (unsigned)(((pp - (row >> kBRot)) & (kBPiecesPerRow - 1)) << 4);
+                (unsigned)(((pp - (row >> kBRot)) & (kBLoadPieces - 1)) << 4);
     if constexpr (kBFrag) {
       // instruction (wave, i) brings the 32-row block wave * kBOps + i of the tile: 1 KiB as stored, lane-linear
-      const int blk = min((n0 >> 5) + wave * kBOps + i, ((N + 31) >> 5) - 1);
-      b_voff[i] = (unsigned)blk * (unsigned)(p.ldk / P::kKPerBlock) * 1024u + (unsigned)lane * 16u;
+      // (a stage of two tiles: 2 KiB)
+      const int at = dma_wave * kBOps + i;
+      const int blk = min((n0 >> 5) + at / kStageTiles, ((N + 31) >> 5) - 1);
+      b_voff[i] = (unsigned)blk * (unsigned)(p.ldk / P::kKPerBlock) * 1024u + (unsigned)(at % kStageTiles) * 1024u + (unsigned)lane * 16u;
     }
   }
   // fp16 scales (kScaleDma >= 2): one per 2^p0 k (p.p0 = 5 .. 12, the policy's dma_ok checks it), so a dword of a row
@@ -643,74 +656,79 @@ __global__ __launch_bounds__(64 * kWavesM * (8 / kNBW), 32 * kMBW * kWavesM == 1
   const int s_ps = s_gshift - 5;
   const unsigned s_voff = (unsigned)min(n0 + (tid & 255), N - 1) * (unsigned)(P::kScaleDma == 1 ? (p.ldk >> 5) : ((p.ldk >> s_gshift) << 1));  // waves 4..7 repeat 0..3
 
-  // One tile = kSOps + kAOps + kBOps DMA instructions per thread: first the scale dword(s) (row tid; issued
-  // with every tile although a dword serves two or four, which keeps the loop branch-free), then the A
-  // chunks, then the packed-B chunks.
+  // One tile = kSOps + kAOps + kBOps DMA instructions per thread: first the scale dword(s) (row tid) if one is due,
+  // then the A chunks, then the packed-B chunks.  Two halves: waves 0 .. 3 bring the scales and waves 4 .. 7 the zeros.
+  // Two tiles of a stage share its dwords: no groups of 32 k there.
   constexpr int kTileOps = kSOps + kAOps + kBOps;
-  auto issue_op = [&](int op, int kb, int stage) {
+  auto issue_op = [&](int op, int kb, int stage, bool first_tile = false) {
     const unsigned sbase = lds0 + stage * kAStride;
     const unsigned bbase = lds0 + kBRing + (kPairB ? (kb & 3) : stage) * kBSlot;
     if (op < kSOps) {
       if constexpr (P::kScaleDma == 1) {
-        const int pair = kb >> 1;
-        dma4(lds0 + kRing + (pair & 3) * 1024 + (wave & 3) * 256, s_voff, (const unsigned char*)p.S + (size_t)pair * 4);
+        const int pair = kHalves ? kb : kb >> 1;
+        dma4_unless(kHalves ? kh : (first_tile ? 0 : kb & 1), lds0 + kRing + (pair & 3) * 1024 + (wave & 3) * 256, s_voff, (const unsigned char*)p.S + (size_t)pair * 4);
       } else if constexpr (P::kScaleDma >= 2) {
-        const int quad = kb >> s_ps;
-        dma4(lds0 + kRing + op * 4096 + (quad & 3) * 1024 + (wave & 3) * 256, s_voff,
-             (const unsigned char*)(op == 0 ? p.S : p.Z) + (size_t)quad * 4);
+        const int quad = (kb * kStageTiles) >> s_ps;
+        dma4_unless(kHalves && kh != op ? 1 : (first_tile ? 0 : (kb * kStageTiles) & ((1 << s_ps) - 1)),
+                    lds0 + kRing + op * 4096 + (quad & 3) * 1024 + (wave & 3) * 256, s_voff,
+                    (const unsigned char*)(op == 0 ? p.S : p.Z) + (size_t)quad * 4);
       }
     } else if (op < kSOps + kAOps) {
       const int i = op - kSOps;
-      dma16(sbase + (wave * kAOps + i) * 1024, a_voff[i], (const unsigned char*)p.A + (size_t)kb * 128);
+      dma16(sbase + (dma_wave * kAOps + i) * 1024, a_voff[i], (const unsigned char*)p.A + (size_t)kb * (128 * kStageTiles));
     } else {
       const int i = op - kSOps - kAOps;
-      dma16(bbase + (wave * kBOps + i) * 1024, b_voff[i], (const unsigned char*)p.B + (size_t)kb * (kBFrag ? 1024 : P::kBRowBytes));
+      dma16(bbase + (dma_wave * kBOps + i) * 1024, b_voff[i], (const unsigned char*)p.B + (size_t)kb * ((kBFrag ? 1024 : P::kBRowBytes) * kStageTiles));
     }
   };
-  constexpr int kWaitOps = kTileOps;  // outstanding DMA instructions of one tile
+  // DMA instructions of one tile that may be outstanding while the one before is waited for: the scales come first in a
+  // tile and only with some tiles, so a wait that counts without them is right with and without them
+  constexpr int kWaitOps = kTileOps - kSOps;
 
   // ---- fragment read offsets (same LDS geometry as the register-staged kernel) --------------------
-  int a_row_off[kMBW], a_row_sw[kMBW], b_off[kNBW][kBPiecesPerRow / 2], s_off[kNBW];
+  int a_row_off[kMBW], a_row_sw[kMBW], b_off[kNBW][kBWords / 4], s_off[kNBW];
 #pragma unroll
   for (int mb = 0; mb < kMBW; ++mb) {
     const int row = wm * (32 * kMBW) + mb * 32 + r;
-    a_row_off[mb] = row * 128;
+    a_row_off[mb] = row * 128 + (kStageTiles == 2 ? kh * (BM * kARowBytes) : 0);
     a_row_sw[mb] = a_swz(row);
   }
 #pragma unroll
   for (int nb = 0; nb < kNBW; ++nb) {
     const int row = wn * (32 * kNBW) + nb * 32 + r;
 #pragma unroll
-    for (int h = 0; h < kBPiecesPerRow / 2; ++h) {
-      const int piece = g * (kBPiecesPerRow / 2) + h;
-      b_off[nb][h] = row * P::kBRowBytes + (((piece + (row >> kBRot)) & (kBPiecesPerRow - 1)) << 4);  // in its B slot
+    for (int h = 0; h < kBWords / 4; ++h) {
+      const int piece = (kStageTiles == 2 ? kh * kBPiecesPerRow : 0) + g * (kBPiecesPerRow / 2) + (kSteps == 2 ? kh : h);
+      b_off[nb][h] = row * (16 * kBLoadPieces) + (((piece + (row >> kBRot)) & (kBLoadPieces - 1)) << 4);  // in its B slot
       // fragment order: block row / 32 of the tile, then the lanes as the matrix instruction numbers them
-      if constexpr (kBFrag) b_off[nb][h] = (row >> 5) * 1024 + lane * 16;
+      if constexpr (kBFrag) b_off[nb][h] = (row >> 5) * (1024 * kStageTiles) + (kStageTiles == 2 ? kh * 1024 : 0) + lane * 16;
     }
     s_off[nb] = kRing + row * 4 + (P::kScaleDma == 1 ? g : (P::kScaleDma >= 2 && s_gshift == 5 ? 2 * g : 0));
   }
   using frag_t = typename P::frag_t;
   auto read_a1 = [&](const unsigned char* base, int j, int mb) -> frag_t {
-    return P::fix_a(*reinterpret_cast<const frag_t*>(base + a_row_off[mb] + ((((g << 2) + j) ^ a_row_sw[mb]) << 4)));
+    return P::fix_a(*reinterpret_cast<const frag_t*>(base + a_row_off[mb] + ((((g << 2) + (kSteps == 2 ? 2 * kh : 0) + j) ^ a_row_sw[mb]) << 4)));
   };
   // 32 rows further down the rotation of the packed-B pieces repeats ((32 >> kBRot) % kBPiecesPerRow == 0)
   // and the scale rows are 4 bytes apart: block nb sits at a constant distance from block 0, so one
   // address per tile serves all kNBW reads through their immediate offsets
-  static_assert((32 >> kBRot) % kBPiecesPerRow == 0, "B rotation must repeat every 32 rows");
+  static_assert((32 >> kBRot) % kBLoadPieces == 0, "B rotation must repeat every 32 rows");
   auto read_b1 = [&](const unsigned char* base, int nb, uint32_t (&bw)[kBWords]) {
 #pragma unroll
-    for (int h = 0; h < kBPiecesPerRow / 2; ++h) {
-      const uint4_t v = *reinterpret_cast<const uint4_t*>(base + b_off[0][h] + nb * (32 * P::kBRowBytes));
+    for (int h = 0; h < kBWords / 4; ++h) {
+      const uint4_t v = *reinterpret_cast<const uint4_t*>(base + b_off[0][h] + nb * (32 * 16 * kBLoadPieces));
       bw[4 * h + 0] = v[0]; bw[4 * h + 1] = v[1]; bw[4 * h + 2] = v[2]; bw[4 * h + 3] = v[3];
     }
   };
   // the LDS read of a scale and the arithmetic on it are separate steps, so that the read can be issued a
   // chunk ahead of its first use
-  auto read_scale_byte = [&](int kb, int nb) -> int {
+  auto read_scale_byte = [&](int step_kb, int nb) -> int {
+    const int kb = step_kb * kStageTiles + (kStageTiles == 2 ? kh : 0);
     if constexpr (P::kScaleDma == 1) return (smem + s_off[0] + ((kb >> 1) & 3) * 1024 + (kb & 1) * 2)[nb * 128];
     else return 0;
   };
-  auto read_scale1 = [&](int kb, int nb) -> typename P::Scale {
+  auto read_scale1 = [&](int step_kb, int nb) -> typename P::Scale {
+    const int kb = step_kb * kStageTiles + (kStageTiles == 2 ? kh : 0);  // the 64-k tile
     if constexpr (P::kScaleDma >= 2) {
       // which of the dword's two groups: with groups of 32 k the lane's half of the tile (in s_off), else the tile's
       const unsigned char* at = smem + s_off[0] + ((kb >> s_ps) & 3) * 1024 + (s_gshift == 5 ? 0 : (((kb << 6) >> s_gshift) & 1) * 2) + nb * 128;
@@ -731,7 +749,7 @@ __global__ __launch_bounds__(64 * kWavesM * (8 / kNBW), 32 * kMBW * kWavesM == 1
   // ---- prologue: tiles 0 and 1 (and their scales) in flight; only tile 0 has to have landed -------
   if constexpr (kPairB) {  // scales, A of tile 0, the B pairs of tiles 0 and 1, then A of tile 1
 #pragma unroll
-    for (int op = 0; op < kSOps + kAOps; ++op) issue_op(op, 0, 0);
+    for (int op = 0; op < kSOps + kAOps; ++op) issue_op(op, 0, 0, true);
 #pragma unroll
     for (int i = 0; i < kBOps; ++i) {
       issue_op(kSOps + kAOps + i, 0, 0);
@@ -742,7 +760,7 @@ __global__ __launch_bounds__(64 * kWavesM * (8 / kNBW), 32 * kMBW * kWavesM == 1
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kAOps) : "memory");
   } else {
 #pragma unroll
-    for (int op = 0; op < kTileOps; ++op) issue_op(op, 0, 0);
+    for (int op = 0; op < kTileOps; ++op) issue_op(op, 0, 0, true);
 #pragma unroll
     for (int op = 0; op < kTileOps; ++op) issue_op(op, 1, 1);  // KB >= 2 because K % 128 == 0
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kWaitOps) : "memory");
@@ -793,8 +811,8 @@ __global__ __launch_bounds__(64 * kWavesM * (8 / kNBW), 32 * kMBW * kWavesM == 1
     const int stage2 = stage == 0 ? 2 : stage - 1;  // (stage + 2) % 3
     const unsigned char* base = smem + stage * kAStride;
     const unsigned char* bbase = smem + kBRing + (kPairB ? (kb & 3) : stage) * kBSlot;
-    constexpr int kIterOps = !kPairB ? kTileOps : (odd ? kAOps : kSOps + kAOps + 2 * kBOps);  // issued per iteration
-    if constexpr ((kMBW == 4 && kNBW == 4) || kWavesM == 1) {
+    constexpr int kIterOps = !kPairB ? kTileOps : (odd ? kAOps : kSOps + kAOps + 2 * kBOps);  // issued per iteration at most
+    {
       using DoMfma = std::integral_constant<bool, !first>;
       auto dma = [&](int chunk) {
         if constexpr (!kPairB) {
@@ -823,7 +841,7 @@ __global__ __launch_bounds__(64 * kWavesM * (8 / kNBW), 32 * kMBW * kWavesM == 1
         // Eight matrix instructions (four A fragments against the wave's two B fragments) and their side work per
         // scheduling region, as a pipeline of one matrix instruction, at most one LDS read and a few vector
         // instructions.  Skewed by one step like the 2 x 2 form below.
-        constexpr int kValu = 3;
+        constexpr int kValu = kMBW == 4 ? 4 : 3;
         auto region = [&](int q0, auto do_mfma_tag, auto&& side) {
           if constexpr (decltype(do_mfma_tag)::value) {
 #pragma unroll
@@ -841,30 +859,56 @@ __global__ __launch_bounds__(64 * kWavesM * (8 / kNBW), 32 * kMBW * kWavesM == 1
 #undef DQ_SPREAD_GROUP
           __builtin_amdgcn_sched_barrier(0);
         };
-        region(0, DoMfma{}, [&] {
-          fetch_b(0);
-          fetch_b(1);
-          dma(0);
-          dma(1);
+        if constexpr (kMBW == 4) {
+          // 128 rows: a step of the wave is one region
+          region(0, DoMfma{}, [&] {
+            fetch_b(0);
+            fetch_b(1);
 #pragma unroll
-          for (int q = 0; q < 4; ++q) af_n[q] = read_a1(base, 0, q);
-        });
-        region(4, DoMfma{}, [&] {
+            for (int q = 0; q < 4; ++q) af_n[q] = read_a1(base, 0, q);
+            dma(0);
+            dma(1);
+            finish_scale(0);
+            finish_scale(1);
+            bf_n[0] = P::decode(bw_c[0], 0, sc_c[0]);
+            bf_n[1] = P::decode(bw_c[1], 0, sc_c[1]);
+          });
+        } else {
+          region(0, DoMfma{}, [&] {
+            fetch_b(0);
+            fetch_b(1);
+            dma(0);
+            dma(1);
 #pragma unroll
-          for (int q = 4; q < 8; ++q) af_n[q] = read_a1(base, 0, q);
-          finish_scale(0);
-          finish_scale(1);
-          dma(2);
-          dma(3);
-          bf_n[0] = P::decode(bw_c[0], 0, sc_c[0]);
-          bf_n[1] = P::decode(bw_c[1], 0, sc_c[1]);
-        });
+            for (int q = 0; q < 4; ++q) af_n[q] = read_a1(base, 0, q);
+          });
+          region(4, DoMfma{}, [&] {
 #pragma unroll
-        for (int q = 0; q < 8; ++q) af_c[q] = af_n[q];
+            for (int q = 4; q < 8; ++q) af_n[q] = read_a1(base, 0, q);
+            finish_scale(0);
+            finish_scale(1);
+            dma(2);
+            dma(3);
+            bf_n[0] = P::decode(bw_c[0], 0, sc_c[0]);
+            bf_n[1] = P::decode(bw_c[1], 0, sc_c[1]);
+          });
+        }
+#pragma unroll
+        for (int q = 0; q < kMBW; ++q) af_c[q] = af_n[q];
         bf_c[0] = bf_n[0];
         bf_c[1] = bf_n[1];
 #pragma unroll
-        for (int j = 0; j < 3; ++j) {
+        for (int j = 0; j < kSteps - 1; ++j) {
+          if constexpr (kMBW == 4) {
+            region(0, std::true_type{}, [&] {
+#pragma unroll
+              for (int q = 0; q < 4; ++q) af_n[q] = read_a1(base, j + 1, q);
+              dma(2 + 2 * j);
+              dma(3 + 2 * j);
+              bf_n[0] = P::decode(bw_c[0], j + 1, sc_c[0]);
+              bf_n[1] = P::decode(bw_c[1], j + 1, sc_c[1]);
+            });
+          } else if constexpr (kMBW == 8) {
           region(0, std::true_type{}, [&] {
 #pragma unroll
             for (int q = 0; q < 4; ++q) af_n[q] = read_a1(base, j + 1, q);
@@ -879,8 +923,9 @@ __global__ __launch_bounds__(64 * kWavesM * (8 / kNBW), 32 * kMBW * kWavesM == 1
             dma(7 + 4 * j);
             bf_n[1] = P::decode(bw_c[1], j + 1, sc_c[1]);
           });
+          }
 #pragma unroll
-          for (int q = 0; q < 8; ++q) af_c[q] = af_n[q];
+          for (int q = 0; q < kMBW; ++q) af_c[q] = af_n[q];
           bf_c[0] = bf_n[0];
           bf_c[1] = bf_n[1];
         }
@@ -911,76 +956,10 @@ __global__ __launch_bounds__(64 * kWavesM * (8 / kNBW), 32 * kMBW * kWavesM == 1
         }
       }
       }
-    } else {
-#pragma unroll
-    for (int q = 0; q < kMBW; ++q) {
-      if constexpr (kMBW == 4) {
-        if (q == 0) {
-#pragma unroll
-          for (int nb = 0; nb < kNBW; ++nb) {
-            read_b1(bbase, nb, bw_c[nb]);
-            sc_c[nb] = read_scale1(kb, nb);
-          }
-        } else if (q == 1) {
-          af_n[0] = read_a1(base, 0, 0);
-          af_n[1] = read_a1(base, 0, 1);
-        } else if (q == 2) {
-          af_n[2] = read_a1(base, 0, 2);
-          af_n[3] = read_a1(base, 0, 3);
-#pragma unroll
-          for (int nb = 0; nb < kNBW / 2; ++nb) bf_n[nb] = P::decode(bw_c[nb], 0, sc_c[nb]);
-        } else {
-#pragma unroll
-          for (int nb = kNBW / 2; nb < kNBW; ++nb) bf_n[nb] = P::decode(bw_c[nb], 0, sc_c[nb]);
-        }
-      } else {
-        if (q == 0) {
-#pragma unroll
-          for (int nb = 0; nb < kNBW; ++nb) {
-            read_b1(bbase, nb, bw_c[nb]);
-            sc_c[nb] = read_scale1(kb, nb);
-          }
-          af_n[0] = read_a1(base, 0, 0);
-          af_n[1] = read_a1(base, 0, 1);
-        } else {
-#pragma unroll
-          for (int nb = 0; nb < kNBW; ++nb) bf_n[nb] = P::decode(bw_c[nb], 0, sc_c[nb]);
-        }
-      }
-      if (has_next2 && q < kTileOps) issue_op(q, kb + 2, stage2);
-      if (!first) {
-#pragma unroll
-        for (int nb = 0; nb < kNBW; ++nb) acc[q][nb] = P::mfma(af_c[q], bf_c[nb], acc[q][nb]);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-#pragma unroll
-    for (int q = 0; q < kMBW; ++q) af_c[q] = af_n[q];
-#pragma unroll
-    for (int q = 0; q < kNBW; ++q) bf_c[q] = bf_n[q];
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-#pragma unroll
-      for (int q = 0; q < kMBW; ++q) {
-        const int chunk = kMBW + j * kMBW + q;
-        af_n[q] = read_a1(base, j + 1, q);
-#pragma unroll
-        for (int nb = 0; nb < kNBW; ++nb)  // the kNBW decodes of a step spread evenly over its kMBW chunks
-          if (nb * kMBW / kNBW == q) bf_n[nb] = P::decode(bw_c[nb], j + 1, sc_c[nb]);
-        if (has_next2 && chunk < kTileOps) issue_op(chunk, kb + 2, stage2);
-#pragma unroll
-        for (int nb = 0; nb < kNBW; ++nb) acc[q][nb] = P::mfma(af_c[q], bf_c[nb], acc[q][nb]);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-#pragma unroll
-      for (int q = 0; q < kMBW; ++q) af_c[q] = af_n[q];
-#pragma unroll
-      for (int q = 0; q < kNBW; ++q) bf_c[q] = bf_n[q];
-    }
     }
     // tile kb+1 must have landed before the next iteration reads it; tile kb+2 (issued during this
     // iteration) may still be in flight
-    if (has_next2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kIterOps) : "memory");
+    if (has_next2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(!kPairB || !odd ? kIterOps - kSOps : kIterOps) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
   };
@@ -991,7 +970,17 @@ __global__ __launch_bounds__(64 * kWavesM * (8 / kNBW), 32 * kMBW * kWavesM == 1
   int stage = 0;
   int kb = 0;
   auto next_stage = [&] { stage = stage == 2 ? 0 : stage + 1; };
-  if (KB > 2) {
+  if constexpr (kHalves) {  // KB >= 3, any number
+    iteration(0, 0, T{}, T{}, F{});
+    stage = 1;
+    for (kb = 1; kb + 2 < KB; ++kb) {
+      iteration(kb, stage, F{}, T{}, F{});
+      next_stage();
+    }
+    iteration(kb, stage, F{}, F{}, F{});  // kb = KB - 2
+    next_stage();
+    iteration(kb + 1, stage, F{}, F{}, F{});
+  } else if (KB > 2) {
     iteration(0, 0, T{}, T{}, F{});
     stage = 1;
     for (kb = 1; kb + 3 < KB; kb += 2) {
@@ -1015,7 +1004,52 @@ __global__ __launch_bounds__(64 * kWavesM * (8 / kNBW), 32 * kMBW * kWavesM == 1
 #pragma unroll
     for (int nb = 0; nb < kNBW; ++nb) acc[q][nb] = P::mfma(af_c[q], bf_c[nb], acc[q][nb]);
 
-  DQ_GEMM_EPILOGUE
+  if constexpr (kKHalves == 2) {
+    // Each half hands two of its four 32-row blocks over and finishes the other two: [half][wave][block][nb][i / 4][lane]
+    typedef decltype(acc[0][0][0] + 0) elem_t;
+    typedef elem_t elem4_t __attribute__((ext_vector_type(4)));
+    elem4_t* const red = reinterpret_cast<elem4_t*>(smem) + wave * (2 * 2 * 4 * 64) + lane;
+    constexpr int kHalfPieces = 4 * 2 * 2 * 4 * 64;
+    auto hand_over = [&](auto first_block) {
+      constexpr int q0 = decltype(first_block)::value;
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int nb = 0; nb < kNBW; ++nb)
+#pragma unroll
+          for (int v = 0; v < 4; ++v)
+            red[kh * kHalfPieces + ((q * kNBW + nb) * 4 + v) * 64] =
+                elem4_t{acc[q0 + q][nb][4 * v], acc[q0 + q][nb][4 * v + 1], acc[q0 + q][nb][4 * v + 2], acc[q0 + q][nb][4 * v + 3]};
+    };
+    if (kh == 0) {
+      hand_over(std::integral_constant<int, 2>{});
+    } else {
+      hand_over(std::integral_constant<int, 0>{});
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int nb = 0; nb < kNBW; ++nb) acc[q][nb] = acc[q + 2][nb];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int nb = 0; nb < kNBW; ++nb)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const elem4_t other = red[(1 - kh) * kHalfPieces + ((q * kNBW + nb) * 4 + v) * 64];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[q][nb][4 * v + e] += other[e];
+        }
+    __syncthreads();  // the epilogue's slabs lie where the sums were handed over
+    const int first_row = m0 + 64 * kh, slab_wave = wave + kWaves * kh;
+    {
+      const int m0 = first_row, wave = slab_wave;
+      DQ_GEMM_EPILOGUE_OF(2)
+    }
+  } else {
+    DQ_GEMM_EPILOGUE
+  }
 }
 
 template <class P, int kMBW = 4, int kNBW = 4, int kKSplit = 1>
@@ -1053,52 +1087,63 @@ int launch_auto(const Params& p, hipStream_t stream) {
   return launch<P, 2, 1>(p, stream);
 }
 
+// Whether the direct-to-LDS kernel takes the problem at all
 template <class P>
-bool dma_eligible(const Params& p) {
-  // the direct-to-LDS kernel has one tile shape (256 x 256): small problems go to the tile-size choice above
-  const long tiles = (long)((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN) * p.split;
+bool dma_takes(const Params& p) {
   // 32-bit lane offsets: A rows are 128 bytes per K block, packed B rows kBRowBytes
-  const size_t a_bytes = (size_t)p.M * (p.ldk / P::kKPerBlock) * kARowBytes;
-  const size_t b_bytes = (size_t)p.N * (p.ldk / P::kKPerBlock) * P::kBRowBytes;
-  // fp16 scales of groups of 32 k go with every tile: not with the pairwise issue of the 32-byte-row form of this tile
-  const bool scales_per_tile = P::kScaleDma >= 2 && P::kBRowBytes == 32 && p.p0 == 5;
-  return P::dma_ok(p) && !scales_per_tile && (p.K % (2 * P::kKPerBlock) == 0) && tiles >= 192 && a_bytes < (1ull << 32) &&
-         b_bytes < (1ull << 32);
-}
-
-// Problems with too few 256 x 256 tiles for the kernel above but at least `min_tiles` tiles of 128 x 256: the same
-// kernel on the half-height tile (two workgroups fit a CU), which keeps the operands on the direct-to-LDS path.
-// Measured at N = K = 8192 against the register-staged 128 x 128 tiles, M = 1024: MXFP4 139 -> 114 us, fp16 x uint4
-// 213 -> 158 us, int8 x 2-bit 68 -> 57 us, int8 x int4 75 -> 60 us; M = 384 (96 tiles): MXFP4 90 -> 85.5 us, fp16 x
-// uint4 139 -> 117 us.  The int8 x 2-bit policy gains from 160 tiles on only (M = 512: 43.5 us register-staged
-// against 48.8 us; M = 640: 61 against 49 us).
-constexpr int kHalfTileMin = 96;
-template <class P>
-bool dma_half_takes(const Params& p) {
   const size_t a_bytes = (size_t)p.M * (p.ldk / P::kKPerBlock) * kARowBytes;
   const size_t b_bytes = (size_t)p.N * (p.ldk / P::kKPerBlock) * P::kBRowBytes;
   return P::dma_ok(p) && (p.K % (2 * P::kKPerBlock) == 0) && a_bytes < (1ull << 32) && b_bytes < (1ull << 32);
 }
-template <class P>
-bool dma_half_eligible(const Params& p, int min_tiles = kHalfTileMin) {
-  const long tiles = (long)((p.M + 127) / 128) * ((p.N + BN - 1) / BN) * p.split;
-  return !dma_eligible<P>(p) && dma_half_takes<P>(p) && tiles >= min_tiles;
+
+inline long tiles_of(const Params& p, int rows) { return (long)((p.M + rows - 1) / rows) * ((p.N + BN - 1) / BN) * p.split; }
+
+// Rounds of 256 workgroups, one per CU.  The last one takes two thirds of a full round however few tiles it has, the rest by
+// their share (a lone tile runs at a higher clock and has the caches to itself: fp16 x uint4, K = 4096, 270 tiles of 256
+// rows 176 us, 256 of them 108).
+inline double dma_rounds(long tiles) {
+  const long full = tiles / 256, rest = tiles % 256;
+  return (double)full + (rest ? 0.65 + 0.35 * (double)rest / 256.0 : 0.0);
 }
 
-template <class P, int kMBW, int kNBW, int kWavesM = 2>
+// 256 x 256 tiles, or 128 x 256.  A round of the first costs 1.85 of the second's (K = 8192: fp16 x uint4 215 and 116 us,
+// MXFP4 180 and 98, int8 x int4 84 and 57), so what decides is how either fills its rounds.  Measured on both, fp16 x uint4
+// with zeros, K = 4096: M = 700, N = 11008 75 us in tiles of 256 rows, 98 in tiles of 128; M = 1000 92 and 106; M = 600 76
+// and 56; M = 1100, N = 13824 176 and 119; M = 1300, N = 8192 92 and 102; M = 1500, N = 28672 300 and 338.
+template <class P>
+bool dma_eligible(const Params& p) {
+  // fp16 scales of groups of 32 k go with every tile: not with the pairwise issue of the 32-byte-row form of this tile
+  const bool scales_per_tile = P::kScaleDma >= 2 && P::kBRowBytes == 32 && p.p0 == 5;
+  const long tiles = tiles_of(p, 256);
+  return !scales_per_tile && tiles >= 96 && dma_takes<P>(p) && 1.85 * dma_rounds(tiles) <= dma_rounds(tiles_of(p, 128));
+}
+
+// Too few 256 x 256 tiles but at least `min_tiles` of 128 x 256: the same kernel on the half-height tile, which keeps the
+// operands on the direct-to-LDS path.  Below that the register-staged kernel's smaller tiles (N = 11008, 86 tiles, K = 5120:
+// int8 x int4 31.9 against 33.4 us).  The int8 x 2-bit policy gains from 160 tiles on only (N = 8192, K = 5120: 128 tiles
+// 32 against 30.3 us, 256 tiles 36 against 45).
+constexpr int kHalfTileMin = 96;
+template <class P>
+bool dma_half_eligible(const Params& p, int min_tiles = kHalfTileMin) {
+  return !dma_eligible<P>(p) && dma_takes<P>(p) && tiles_of(p, 128) >= min_tiles;
+}
+
+template <class P, int kMBW, int kNBW, int kWavesM = 2, int kKHalves = 1>
 int launch_dma_tile(Params p, hipStream_t stream) {
-  constexpr int kWaves = kWavesM * (8 / kNBW);
+  constexpr int kWaves = 4;
   constexpr int kTileM = 32 * kMBW * kWavesM;
-  constexpr bool kPairB = P::kBRowBytes == 32 && kTileM == 256 && kWaves == 4;  // as in the kernel: a fourth B slot
-  constexpr int kPipe = 3 * (kTileM * kARowBytes + BN * P::kBRowBytes) + (kPairB ? BN * P::kBRowBytes : 0) + 8 * 1024;
-  constexpr int kSlabs = kWaves * 32 * (32 * (kNBW > kMBW ? kNBW : kMBW) + 4) * 4;  // epilogue staging
+  constexpr bool kPairB = P::kBRowBytes == 32 && kTileM == 256;  // as in the kernel: a fourth B slot
+  constexpr int kPipe = 3 * (kKHalves == 2 && P::kBRowBytes == 32 ? 2 : 1) * (kTileM * kARowBytes + BN * P::kBRowBytes) + (kPairB ? BN * P::kBRowBytes : 0) + 8 * 1024;
+  // epilogue staging; with K in two halves the accumulators handed over before it
+  constexpr int kSlabs = kKHalves == 1 ? kWaves * 32 * (32 * (kNBW > kMBW ? kNBW : kMBW) + 4) * 4 : 128 * 1024;
   constexpr int kLds = kPipe > kSlabs ? kPipe : kSlabs;
   p.tiles_m = (p.M + kTileM - 1) / kTileM;
   p.tiles_n = (p.N + BN - 1) / BN;
-  auto kern = gemm_kernel_dma<P, kMBW, kNBW, kWavesM>;
+  static_assert(kLds <= 160 * 1024, "LDS budget");
+  auto kern = gemm_kernel_dma<P, kMBW, kNBW, kWavesM, kKHalves>;
   static bool lds_limit_raised[kMaxDevices];
   if (raise_lds_limit<kLds>(kern, lds_limit_raised)) return -1;
-  hipLaunchKernelGGL(kern, dim3(p.tiles_m * p.tiles_n * p.split), dim3(64 * kWaves), kLds, stream, p);
+  hipLaunchKernelGGL(kern, dim3(p.tiles_m * p.tiles_n * p.split), dim3(64 * kWaves * kKHalves), kLds, stream, p);
   DQ_CHECK_HIP(hipGetLastError());
   return 0;
 }
@@ -1112,12 +1157,29 @@ struct TallWaves<P, std::void_t<decltype(P::kTallWaves)>> : std::integral_consta
 template <class P>
 int launch_dma(const Params& p, hipStream_t stream) {
   if constexpr (TallWaves<P>::value) return launch_dma_tile<P, 8, 2, 1>(p, stream);
-  else return launch_dma_tile<P, DQ_DMA_MBW, DQ_DMA_NBW>(p, stream);
+  else return launch_dma_tile<P, 4, 4>(p, stream);
+}
+
+// P::kOneOrder: a row's products are added in one order whatever the tile
+template <class P, class = void>
+struct OneOrder : std::false_type {};
+template <class P>
+struct OneOrder<P, std::void_t<decltype(P::kOneOrder)>> : std::integral_constant<bool, P::kOneOrder> {};
+
+// Eight waves on the two halves of every stage: at least three stages, and no groups of 32 k (a dword of scales per tile)
+template <class P>
+bool dma_halves_take(const Params& p) {
+  if constexpr (OneOrder<P>::value) return false;
+  const int shortest = UnevenSlices<P>::value && p.split > 1 ? p.K / p.kunit / p.split * p.kunit : p.K;
+  const int stage_k = P::kKPerBlock * (P::kBRowBytes == 32 ? 2 : 1);
+  return shortest % stage_k == 0 && shortest / stage_k >= 3 && !(P::kScaleDma >= 2 && p.p0 == 5);
 }
 
 template <class P>
 int launch_dma_half(const Params& p, hipStream_t stream) {
-  return launch_dma_tile<P, 2, 4>(p, stream);
+  if constexpr (!OneOrder<P>::value)
+    if (dma_halves_take<P>(p)) return launch_dma_tile<P, 4, 2, 1, 2>(p, stream);
+  return launch_dma_tile<P, 4, 2, 1>(p, stream);
 }
 
 // The tile choice of every policy that can take the direct-to-LDS path: 256 x 256 tiles there when the problem has
@@ -1139,6 +1201,7 @@ int launch_best(const Params& p, hipStream_t stream, int half_tile_min = kHalfTi
 template <class P>
 struct PartialSums : P {
   static constexpr bool kUnevenSlices = true;
+  static constexpr bool kOneOrder = false;
   using out_t = float;
   __device__ static __forceinline__ out_t finish(uint32_t raw, const Params&, int, int) { return __builtin_bit_cast(float, raw); }
 };
@@ -1162,7 +1225,7 @@ __global__ __launch_bounds__(256) void ksplit_sum_kernel(const float* __restrict
 // p: the whole problem.  1: a shape that the 128 x 256 direct-to-LDS tile or the cut does not take.
 template <class P>
 int launch_ksplit(Params p, void* parts, int split, hipStream_t stream) {
-  if (split < 2 || !dma_half_takes<P>(p)) return 1;
+  if (split < 2 || !dma_takes<P>(p)) return 1;
   const size_t count = (size_t)p.M * p.N;
   p.kunit = 2 * P::kKPerBlock;
   if (p.K % p.kunit != 0 || p.K / p.kunit < split || count % 4 != 0) return 1;
@@ -1170,7 +1233,7 @@ int launch_ksplit(Params p, void* parts, int split, hipStream_t stream) {
   using out_t = typename P::out_t;
   out_t* const C = (out_t*)p.C;
   p.C = parts;
-  if (launch_dma_tile<PartialSums<P>, 2, 4>(p, stream)) return -1;
+  if (launch_dma_half<PartialSums<P>>(p, stream)) return -1;
   const dim3 blocks((unsigned)((count + 1023) / 1024));
   if (p.Bias)
     hipLaunchKernelGGL((ksplit_sum_kernel<out_t, true>), blocks, dim3(256), 0, stream, (const float*)parts, (const out_t*)p.Bias, C, count, split);

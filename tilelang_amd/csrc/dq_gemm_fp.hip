@@ -32,6 +32,7 @@ struct F16Mfma {
 template <int FMT, bool HAS_BIAS>
 struct MxPolicy : Bf16Mfma, gemm::PlainA {
   static constexpr int kBRowBytes = 32;
+  static constexpr bool kOneOrder = true;  // the header's promise of a row's bits
   static constexpr bool kTransposed = false;
   using out_t = bf16_t;
   using ScaleRaw = int;
