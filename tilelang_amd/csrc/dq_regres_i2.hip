@@ -277,7 +277,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void i2_regres_kernel(const int8_t*
 // The loads of the last three blocks' turns have nothing left to ask for and read block 0 instead (the same 32 KiB
 // for every workgroup, from L2, never used): a load under a condition would make the compiler wait for more than
 // the block it needs.
-constexpr int kDepth16 = 4;               // sets of weight registers
+constexpr int kMaxPairs16 = 8;            // pairs of 128-k blocks per wave (K <= 16384)
 constexpr int kPartial16 = 16 * 16 * 4;   // one wave's 16 x 16 sums
 constexpr int kLds16 = kWaves * 4096;     // the prologue's parking areas; the two buffers of partial sums reuse them
 
@@ -286,6 +286,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void i2_regres16_kernel(const int8_
                                                                      typename FIN::out_t* __restrict__ C, int M, int N, int K,
                                                                      int interleaved, FIN fin) {
   extern __shared__ __align__(16) unsigned char smem[];
+  constexpr int kDepth16 = NPW <= 6 ? 4 : NPW == 7 ? 3 : 2;  // sets of weight registers
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -339,8 +340,8 @@ __global__ __launch_bounds__(64 * kWaves, 1) void i2_regres16_kernel(const int8_
       for (int j = 0; j < 4; ++j)
         line[i][j] = *reinterpret_cast<const uint4_t*>(a_lane + (size_t)min(4 * j + (lane >> 4), M - 1) * K + 256 * pair_of(i));
     __builtin_amdgcn_sched_barrier(0);
-    load_w(w[1], nb0 + step, mine > 1);
-    load_w(w[2], nb0 + 2 * step, mine > 2);
+#pragma unroll
+    for (int d = 1; d < kDepth16 - 1; ++d) load_w(w[d], nb0 + d * step, mine > d);
     unsigned char* const park = smem + wave * 4096;
 #pragma unroll
     for (int i = 0; i < NPW; ++i) {
@@ -364,7 +365,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void i2_regres16_kernel(const int8_
   auto do_block = [&](auto q_tag, int k) __attribute__((always_inline)) {
     constexpr int q = decltype(q_tag)::value;
     const int nb = nb0 + k * step;
-    load_w(w[(q + 3) % kDepth16], nb + 3 * step, k + 3 < mine);
+    load_w(w[(q + kDepth16 - 1) % kDepth16], nb + (kDepth16 - 1) * step, k + kDepth16 - 1 < mine);
     int4_t acc = {0, 0, 0, 0};
 #pragma unroll
     for (int i = 0; i < NPW; ++i) {
@@ -412,14 +413,17 @@ __global__ __launch_bounds__(64 * kWaves, 1) void i2_regres16_kernel(const int8_
   for (; k + kDepth16 <= mine; k += kDepth16) {
     do_block(std::integral_constant<int, 0>{}, k);
     do_block(std::integral_constant<int, 1>{}, k + 1);
-    do_block(std::integral_constant<int, 2>{}, k + 2);
-    do_block(std::integral_constant<int, 3>{}, k + 3);
+    if constexpr (kDepth16 >= 3) do_block(std::integral_constant<int, 2>{}, k + 2);
+    if constexpr (kDepth16 == 4) do_block(std::integral_constant<int, 3>{}, k + 3);
   }
   if (k < mine) {
     do_block(std::integral_constant<int, 0>{}, k);
-    if (k + 1 < mine) {
-      do_block(std::integral_constant<int, 1>{}, k + 1);
-      if (k + 2 < mine) do_block(std::integral_constant<int, 2>{}, k + 2);
+    if constexpr (kDepth16 >= 3) {
+      if (k + 1 < mine) {
+        do_block(std::integral_constant<int, 1>{}, k + 1);
+        if constexpr (kDepth16 == 4)
+          if (k + 2 < mine) do_block(std::integral_constant<int, 2>{}, k + 2);
+      }
     }
   }
 }
@@ -493,7 +497,8 @@ int i2_gemm_regres(const void* A, const void* B, void* C, int M, int N, int K, i
   // blocks in flight (N = 28672, K = 8192: 15.8 against 19.0 us; N = K = 8192 at 16 rows 9.1 against 10.5 us; N = 2048,
   // K = 8192: 7.6 against 9.8 us; N = K = 4096: 5.3 against 6.6 us).  With K below 4096 only where a workgroup has more
   // than four of them: its longer prologue shows (N = 8192, K = 2048 at 4 and 8 rows: 4.8 against 4.5 us).
-  const bool rows16 = M <= 16 && (K >= 4096 || (N + 15) / 16 > 4 * 256);
+  const int npw16 = (npair + kWaves - 1) / kWaves;
+  const bool rows16 = M <= 16 && npw16 <= kMaxPairs16 && (K >= 4096 || (N + 15) / 16 > 4 * 256);
 #define DQ_I2R(CONV_, FRAG_, NPW_, CH_)                                                                                        \
   do {                                                                                                                         \
     if (bitnet_epilogue)                                                                                                       \
@@ -508,15 +513,19 @@ int i2_gemm_regres(const void* A, const void* B, void* C, int M, int N, int K, i
   } while (0)
 #define DQ_I2RN(CONV_, FRAG_)                           \
   do {                                                  \
-    if (chunked) DQ_I2R(CONV_, FRAG_, kChunkPairs, true); \
     if (rows16) {                                       \
-      switch (npw) {                                    \
+      switch (npw16) {                                  \
         case 1: DQ_I2R16(CONV_, FRAG_, 1);              \
         case 2: DQ_I2R16(CONV_, FRAG_, 2);              \
         case 3: DQ_I2R16(CONV_, FRAG_, 3);              \
-        default: DQ_I2R16(CONV_, FRAG_, 4);             \
+        case 4: DQ_I2R16(CONV_, FRAG_, 4);              \
+        case 5: DQ_I2R16(CONV_, FRAG_, 5);              \
+        case 6: DQ_I2R16(CONV_, FRAG_, 6);              \
+        case 7: DQ_I2R16(CONV_, FRAG_, 7);              \
+        default: DQ_I2R16(CONV_, FRAG_, 8);             \
       }                                                 \
     }                                                   \
+    if (chunked) DQ_I2R(CONV_, FRAG_, kChunkPairs, true); \
     switch (npw) {                                      \
       case 1: DQ_I2R(CONV_, FRAG_, 1, false);           \
       case 2: DQ_I2R(CONV_, FRAG_, 2, false);           \
