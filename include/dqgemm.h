@@ -257,6 +257,15 @@ int call_gemm_int8xint2(const void* A, const void* B, void* C, int M, int N, int
  * replaces.  Requires K % 8 == 0. */
 int call_bitnet_activation_quant(const void* X, void* Q, void* S, int M, int K, dq_stream_t stream);
 
+/* BitLinear's forward: the activation quantiser above and call_gemm_int8xint2 (DQ_I2_OFFSET, out_kind 1) in one call, with
+ * the bits of the two.  X[M,K] fp16, C[M,N] fp16, layout and s_w as there.  At a decode batch the GEMM kernel quantises the
+ * activations itself; else they go through the workspace, dq_bitlinear_workspace_bytes(M, N, K, layout) bytes (0: none
+ * needed, Workspace may be NULL), 16-byte aligned, contents undefined afterwards, not to be shared by calls that overlap in
+ * time.  Replaces BitLinearBitBLAS.forward without its bias (examples/bitnet-1.58b/utils_quant.py:188-209). */
+size_t dq_bitlinear_workspace_bytes(int M, int N, int K, int layout);
+int call_bitlinear_fp16(const void* X, const void* B, void* C, void* Workspace, size_t workspace_bytes, int M, int N, int K,
+                        int layout, float s_w, dq_stream_t stream);
+
 /* MXFP4 weight quantiser (the producer of call_dequant_gemm_bf16_mxfp4's B and Scale, which the reference's
  * example draws at random, examples/dequantize_gemm/example_dequant_gemm_bf16_mxfp4_cdna4.py:99-103,286-290):
  * W[N,K] bf16 -> B[N,K/2] e2m1 codes, two per byte, even k in the low nibble, and Scale[N,K/32] one byte per 32 k.

@@ -39,6 +39,7 @@ SIGNATURES = {
     "call_dequant_gemm_fp16_fp4_splitk_static": [_vp, _vp, _vp, _i, _i, _i, _i, _i, _vp],
     "call_dequant_gemm_w4_fp16": [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp],
     "call_gemm_int8xint2": [_vp, _vp, _vp, _i, _i, _i, _i, _i, _vp, ctypes.c_float, _i, _vp],
+    "call_bitlinear_fp16": [_vp, _vp, _vp, _vp, ctypes.c_size_t, _i, _i, _i, _i, ctypes.c_float, _vp],
     "call_bitnet_activation_quant": [_vp, _vp, _vp, _i, _i, _vp],
     "call_quantize_bf16_mxfp4": [_vp, _vp, _vp, _i, _i, _i, _vp],
     "call_gemm_int8xint4": [_vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp],
@@ -52,6 +53,7 @@ SIGNATURES = {
 SIZE_QUERIES = {
     "dq_w4a16_workspace_bytes": [_i, _i, _i, _i, _i],
     "dq_mxfp4_workspace_bytes": [_i, _i, _i],
+    "dq_bitlinear_workspace_bytes": [_i, _i, _i, _i],
 }
 
 

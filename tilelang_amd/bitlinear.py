@@ -2,9 +2,9 @@
 
 Twin of ``BitLinearBitBLAS`` of examples/bitnet-1.58b/utils_quant.py:34-209 with the BitBLAS operator replaced by
 ``libdqgemm.so``: the weights are quantised once to ternary codes (``weight_quant``, :149-154), packed four per
-byte (and interleaved for the fast decoder, as the reference's kernels expect), and ``forward`` is two kernel
-launches: the activation quantiser (:156-163) and the GEMM with the fused ``post_quant_process`` epilogue
-(:165-170).  BitBLAS's own weight transform (``transform_weight``) is third-party and absent; the packed layout
+byte (and interleaved for the fast decoder, as the reference's kernels expect), and ``forward`` is one call: the
+activation quantiser (:156-163), in a launch of its own or, at a decode batch, inside the GEMM kernel, and the GEMM with
+the fused ``post_quant_process`` epilogue (:165-170).  BitBLAS's own weight transform (``transform_weight``) is third-party and absent; the packed layout
 here is the reference examples' ``general_compress`` + ``interleave_weight``.
 """
 
@@ -97,12 +97,11 @@ class BitLinear(nn.Module):
         self._sw_value = float(self.sw)
         self._kernels.clear()
 
-    def _get_kernels(self, M: int):
+    def _get_kernel(self, M: int):
         k = self._kernels.get(M)
         if k is None:
-            k = (kernels.bitnet_activation_quant(M, self.in_features),
-                 kernels.bitlinear_int8xint2(M, self.out_features, self.in_features, self._sw_value, convention="offset",
-                                             interleaved=self.interleave, weight_fragments=self.prefill_fragments))
+            k = kernels.bitlinear_fp16(M, self.out_features, self.in_features, self._sw_value, interleaved=self.interleave,
+                                       weight_fragments=self.prefill_fragments)
             self._kernels[M] = k
         return k
 
@@ -110,9 +109,7 @@ class BitLinear(nn.Module):
         x = input.reshape(-1, self.in_features)
         if x.dtype != torch.float16:
             x = x.to(torch.float16)
-        quant, gemm = self._get_kernels(x.shape[0])
-        x_q, s_a = quant(x.contiguous())
-        out = gemm(x_q, self.qweight, s_a)
+        out = self._get_kernel(x.shape[0])(x.contiguous(), self.qweight)
         if self.bias is not None:
             out += self.bias.view(1, -1).expand_as(out)
         return out.reshape(*input.shape[:-1], self.out_features)

@@ -57,6 +57,8 @@ int i2_gemm_regres(const void* A, const void* B, void* C, int M, int N, int K, i
                    float s_w, int bitnet_epilogue, hipStream_t stream);
 int i2_gemv(const void* A, const void* B, void* C, int M, int N, int K, int convention, int layout, const void* s_a,
             float s_w, int out_kind, hipStream_t stream);
+int i2_bitlinear_gemv(const void* X, const void* B, void* C, int M, int N, int K, int layout, float s_w, hipStream_t stream);
+int i2_bitlinear_regres(const void* X, const void* B, void* C, int M, int N, int K, int layout, float s_w, hipStream_t stream);
 int i4_gemv(const void* A, const void* B, void* C, int M, int N, int K, int decode, hipStream_t stream);
 int i1_gemv(const void* A, const void* B, void* C, int M, int N, int K, int convention, int layout, hipStream_t stream);
 int activation_quant(const void* X, void* Q, void* S, int M, int K, hipStream_t stream);
@@ -577,6 +579,49 @@ extern "C" int call_bitnet_activation_quant(const void* X, void* Q, void* S, int
   if (K % 8 != 0) DQ_FAIL("%s: K=%d must be a multiple of 8", fn, K);
   if (!aligned16(X) || ((uintptr_t)Q & 7) != 0) DQ_FAIL("%s: X must be 16-byte and Q 8-byte aligned", fn);
   return activation_quant(X, Q, S, M, K, (hipStream_t)stream);
+}
+
+// BitLinear's forward in one launch: whether a GEMM kernel quantises the activations itself, in every workgroup.  Against two
+// launches (us): N = K = 4096, row-major words, M = 1 6.7 -> 4.6, M = 4 7.5 -> 6.5, M = 8 8.0 -> 7.3, M = 16 8.4 against 8.5;
+// fragments M = 4 7.2 -> 5.6, M = 8 7.5 -> 6.7; N = K = 8192, M = 8 11.9 -> 11.2; N = 11008, K = 6144, M = 16 10.6 against
+// 11.3; N = 11008, K = 2048, M = 16 7.8 -> 7.1.
+static bool bitlinear_by_gemv(int M, int K, int layout) {
+  return (layout & LAYOUT_FRAGMENTS) ? M == 1 && K <= 16384 : M <= 2 && (size_t)M * K <= 32768;
+}
+static bool bitlinear_in_one_kernel(int M, int N, int K, int layout) {
+  if (M < 1 || M > 16 || N < 1 || K < 128 || K % 128 != 0) return false;
+  if (bitlinear_by_gemv(M, K, layout)) return true;
+  if (K % 256 != 0 || (uint64_t)(N + 32) * (uint64_t)(K >> 2) >= (1ull << 32)) return false;
+  return K <= (M <= 4 ? 16384 : M <= 8 ? 10240 : 2048);
+}
+
+extern "C" size_t dq_bitlinear_workspace_bytes(int M, int N, int K, int layout) {
+  if (M <= 0 || N <= 0 || K <= 0 || bitlinear_in_one_kernel(M, N, K, layout)) return 0;
+  return (size_t)M * K + (size_t)M * sizeof(float);  // the int8 activations, where the workspace starts, and s_a
+}
+
+extern "C" int call_bitlinear_fp16(const void* X, const void* B, void* C, void* Workspace, size_t workspace_bytes, int M, int N, int K,
+                                   int layout, float s_w, dq_stream_t stream) {
+  const char* fn = "call_bitlinear_fp16";
+  if (!X) DQ_FAIL("%s: X is expected to have non-NULL data pointer", fn);
+  if (check_gemm_args(fn, X, B, C, M, N, K, 128)) return -1;
+  const int word_layout = layout & ~LAYOUT_FRAGMENTS;
+  if (word_layout != LAYOUT_PLAIN && word_layout != LAYOUT_INTERLEAVED) DQ_FAIL("%s: unknown weight layout %d", fn, layout);
+  if (!(s_w != 0.f)) DQ_FAIL("%s: s_w must be non-zero", fn);
+  if (bitlinear_in_one_kernel(M, N, K, layout)) {
+    const int rc = bitlinear_by_gemv(M, K, layout) ? i2_bitlinear_gemv(X, B, C, M, N, K, layout, s_w, (hipStream_t)stream)
+                                                   : i2_bitlinear_regres(X, B, C, M, N, K, layout, s_w, (hipStream_t)stream);
+    if (rc > 0) DQ_FAIL("%s: shape M=%d N=%d K=%d is not covered", fn, M, N, K);
+    return rc;
+  }
+  const size_t need = dq_bitlinear_workspace_bytes(M, N, K, layout);
+  if (!Workspace) DQ_FAIL("%s: Workspace is expected to have non-NULL data pointer", fn);
+  if (!aligned16(Workspace)) DQ_FAIL("%s: Workspace must be 16-byte aligned", fn);
+  if (workspace_bytes < need) DQ_FAIL("%s: Workspace holds %zu bytes, the quantised activations need %zu", fn, workspace_bytes, need);
+  int8_t* const q = (int8_t*)Workspace;  // K % 128 == 0: whole lines, and s_a behind them at a multiple of four bytes
+  float* const s_a = (float*)(q + (size_t)M * K);
+  if (activation_quant(X, q, s_a, M, K, (hipStream_t)stream)) return -1;
+  return call_gemm_int8xint2(q, B, C, M, N, K, I2_OFFSET, layout, s_a, s_w, 1, stream);
 }
 
 extern "C" int call_quantize_bf16_mxfp4(const void* W, void* B, void* Scale, int N, int K, int scale_bias,

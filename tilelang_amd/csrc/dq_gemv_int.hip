@@ -18,7 +18,7 @@
 //   * K is reduced over each 16-lane row with DPP row operations, all values of a batch of rows together (most levels
 //     halve the number of values), and over the 16-lane rows of a weight row through LDS; integer sums, so the result
 //     is exact whatever the order.
-#include "dq_common.h"
+#include "dq_act_quant.h"
 
 namespace dq {
 
@@ -86,8 +86,11 @@ __device__ __forceinline__ void load_activations(const int8_t* ap, bool valid, b
   }
 }
 
-template <int BITS, int MROWS, int NP, int R>
-__global__ __launch_bounds__(256) void int_gemv_kernel(const int8_t* __restrict__ A, const uint8_t* __restrict__ B,
+// QUANT: the activations come in fp16 (BitLinear's forward in one launch) and every workgroup quantises them itself
+// (dq_act_quant.h: the bits of the quantiser's own kernel), shared over its threads, into LDS, from where a thread takes its
+// chunks.
+template <int BITS, int MROWS, int NP, int R, bool QUANT = false>
+__global__ __launch_bounds__(256) void int_gemv_kernel(const void* __restrict__ A_any, const uint8_t* __restrict__ B,
                                                         void* __restrict__ C, const float* __restrict__ s_a, float s_w,
                                                         int out_kind, int M, int N, int K, int tpr_shift, int nb,
                                                         uint32_t flip_mask, int mul, int zsub, int interleaved) {
@@ -99,6 +102,9 @@ __global__ __launch_bounds__(256) void int_gemv_kernel(const int8_t* __restrict_
   static_assert(NV <= 16 && (NV & (NV - 1)) == 0, "a power of two of at most 16 values per lane row");
   // partial sums: [batch][16-lane row of the workgroup (16)][value]
   __shared__ int red[kMaxRowsPerWg * 16 * MROWS];
+  __shared__ __align__(16) int8_t act[QUANT ? MROWS * NP * 256 * kCodes : 16];
+  __shared__ float wave_amax[MROWS][4];
+  float scale[MROWS];  // QUANT: s_a
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -127,6 +133,42 @@ __global__ __launch_bounds__(256) void int_gemv_kernel(const int8_t* __restrict_
 #pragma unroll
   for (int u = 0; u < R; ++u) issue_row(u, 0);
 
+  if constexpr (QUANT) {
+    const half_t* const X = (const half_t*)A_any;
+    constexpr int kHeld = NP * kCodes / 8;  // 16-byte pieces of a row per thread, at most
+    const int nvec = K >> 3;
+    half8_t x[MROWS][kHeld];
+#pragma unroll
+    for (int m = 0; m < MROWS; ++m)
+#pragma unroll
+      for (int i = 0; i < kHeld; ++i) {
+        x[m][i] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+        if (256 * i < nvec) {  // uniform; a clamped piece counts twice in the maximum
+          x[m][i] = *reinterpret_cast<const half8_t*>(X + (size_t)min(m, M - 1) * K + (size_t)min(tid + 256 * i, nvec - 1) * 8);
+        }
+      }
+#pragma unroll
+    for (int m = 0; m < MROWS; ++m) {
+      float amax = 0.f;
+#pragma unroll
+      for (int i = 0; i < kHeld; ++i)
+        if (256 * i < nvec) amax = amax8(x[m][i], amax);
+      amax = wave_max(amax);
+      if (lane == 0) wave_amax[m][tid >> 6] = amax;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < MROWS; ++m) {
+      scale[m] = act_scale(fmaxf(fmaxf(wave_amax[m][0], wave_amax[m][1]), fmaxf(wave_amax[m][2], wave_amax[m][3])));
+#pragma unroll
+      for (int i = 0; i < kHeld; ++i) {
+        const int v = tid + 256 * i;
+        if (v < nvec) *reinterpret_cast<uint2_t*>(act + m * K + v * 8) = quantise8(x[m][i], scale[m]);
+      }
+    }
+    __syncthreads();
+  }
+
   // activations of this thread's chunk(s) in decoder order; their sum for the zero point
   uint32_t a[NP][MROWS][kDwords];
   int asum[NP][MROWS];
@@ -136,8 +178,9 @@ __global__ __launch_bounds__(256) void int_gemv_kernel(const int8_t* __restrict_
     const bool valid = chunk < c16;  // a clamped chunk is read (in bounds) and zeroed
 #pragma unroll
     for (int m = 0; m < MROWS; ++m) {
-      const int8_t* ap = A + (size_t)min(m, M - 1) * K + (size_t)min(chunk, c16 - 1) * kCodes;
-      load_activations<BITS>(ap, valid, interleaved != 0, a[p][m]);
+      const size_t at = (size_t)min(m, M - 1) * K + (size_t)min(chunk, c16 - 1) * kCodes;
+      if constexpr (QUANT) load_activations<BITS>(act + at, valid, interleaved != 0, a[p][m]);
+      else load_activations<BITS>((const int8_t*)A_any + at, valid, interleaved != 0, a[p][m]);
       int s = 0;
 #pragma unroll
       for (int i = 0; i < kDwords; ++i) s = __builtin_amdgcn_sdot4((int)a[p][m][i], 0x01010101, s, false);
@@ -203,7 +246,8 @@ __global__ __launch_bounds__(256) void int_gemv_kernel(const int8_t* __restrict_
       } else {
         // BitLinear epilogue: (float(acc) / s_a[m]) / s_w -> fp16
         float f = (float)v;
-        f = f / s_a[m];
+        if constexpr (QUANT) f = f / (MROWS == 1 || m == 0 ? scale[0] : scale[MROWS - 1]);
+        else f = f / s_a[m];
         f = f / s_w;
         ((half_t*)C)[(size_t)m * N + row] = (half_t)f;
       }
@@ -216,7 +260,7 @@ struct Decoder {
   int mul, zsub;
 };
 
-template <int BITS, int MROWS, int NP>
+template <int BITS, int MROWS, int NP, bool QUANT = false>
 int launch_int_gemv(const void* A, const void* B, void* C, const void* s_a, float s_w, int out_kind, int M, int N, int K,
                     int tpr_shift, Decoder dec, int interleaved, hipStream_t stream) {
   constexpr int R = NP >= 4 ? 1 : 4 / NP;
@@ -228,8 +272,8 @@ int launch_int_gemv(const void* A, const void* B, void* C, const void* s_a, floa
   while (nb > 1 && nb * R * rpp > kMaxRowsPerWg) --nb;
   if (nb < 1) nb = 1;
   const int rows_per_wg = nb * R * rpp;
-  hipLaunchKernelGGL((int_gemv_kernel<BITS, MROWS, NP, R>), dim3((N + rows_per_wg - 1) / rows_per_wg), dim3(256), 0,
-                     stream, (const int8_t*)A, (const uint8_t*)B, C, (const float*)s_a, s_w, out_kind, M, N, K, tpr_shift,
+  hipLaunchKernelGGL((int_gemv_kernel<BITS, MROWS, NP, R, QUANT>), dim3((N + rows_per_wg - 1) / rows_per_wg), dim3(256), 0,
+                     stream, A, (const uint8_t*)B, C, (const float*)s_a, s_w, out_kind, M, N, K, tpr_shift,
                      nb, dec.flip, dec.mul, dec.zsub, interleaved);
   DQ_CHECK_HIP(hipGetLastError());
   return 0;
@@ -275,14 +319,17 @@ int int_gemv(const void* A, const void* B, void* C, int M, int N, int K, Decoder
 constexpr int kFragWaves = 16;
 constexpr int kFragActBytes = 32768;  // staged activations: MROWS * K bytes
 
-template <int MROWS, int NP>
-__global__ __launch_bounds__(64 * kFragWaves) void i2_gemv_frag_kernel(const int8_t* __restrict__ A, const uint8_t* __restrict__ B,
+// QUANT: as in the kernel above.
+template <int MROWS, int NP, bool QUANT = false>
+__global__ __launch_bounds__(64 * kFragWaves) void i2_gemv_frag_kernel(const void* __restrict__ A_any, const uint8_t* __restrict__ B,
                                                                        void* __restrict__ C, const float* __restrict__ s_a,
                                                                        float s_w, int out_kind, int M, int N, int K,
                                                                        uint32_t flip_mask, int mul, int zsub, int interleaved) {
   __shared__ __align__(16) int8_t act[kFragActBytes];
   __shared__ int red[kFragWaves * 64 * MROWS];
   __shared__ int asum[MROWS];
+  __shared__ float wave_amax[MROWS][kFragWaves];
+  float scale[MROWS];  // QUANT: s_a
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -306,12 +353,39 @@ __global__ __launch_bounds__(64 * kFragWaves) void i2_gemv_frag_kernel(const int
   if (tid < MROWS) asum[tid] = 0;
   __syncthreads();
   const int pieces = K >> 4;  // 16-byte pieces per activation row
+  half8_t x[MROWS][2];  // the thread's piece of every row: K <= 16384 is at most 1024 pieces
+  if constexpr (QUANT) {
+    const int q = min(tid, pieces - 1);
+#pragma unroll
+    for (int m = 0; m < MROWS; ++m)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) x[m][i] = *reinterpret_cast<const half8_t*>((const half_t*)A_any + (size_t)min(m, M - 1) * K + q * 16 + i * 8);
+#pragma unroll
+    for (int m = 0; m < MROWS; ++m) {
+      const float amax = wave_max(amax8(x[m][1], amax8(x[m][0], 0.f)));
+      if (lane == 0) wave_amax[m][wave] = amax;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < MROWS; ++m) {
+      float amax = 0.f;
+#pragma unroll
+      for (int w = 0; w < kFragWaves; ++w) amax = fmaxf(amax, wave_amax[m][w]);
+      scale[m] = act_scale(amax);
+    }
+  }
 #pragma unroll
   for (int m = 0; m < MROWS; ++m) {
-    const int8_t* ap = A + (size_t)min(m, M - 1) * K;
+    const int8_t* ap = (const int8_t*)A_any + (size_t)min(m, M - 1) * K;
     int s = 0;
     for (int q = tid; q < pieces; q += 64 * kFragWaves) {
-      uint4_t d = *reinterpret_cast<const uint4_t*>(ap + q * 16);
+      uint4_t d;
+      if constexpr (QUANT) {
+        const uint2_t lo = quantise8(x[m][0], scale[m]), hi = quantise8(x[m][1], scale[m]);
+        d = uint4_t{lo[0], lo[1], hi[0], hi[1]};
+      } else {
+        d = *reinterpret_cast<const uint4_t*>(ap + q * 16);
+      }
       if (!interleaved) d = transpose4x4_bytes(d);  // plain words decode to elements (i, 4 + i, 8 + i, 12 + i)
       *reinterpret_cast<uint4_t*>(act + m * K + q * 16) = d;
 #pragma unroll
@@ -365,7 +439,14 @@ __global__ __launch_bounds__(64 * kFragWaves) void i2_gemv_frag_kernel(const int
           ((int32_t*)C)[(size_t)m * N + row] = v;
         } else {
           float f = (float)v;
-          f = f / s_a[m];
+          if constexpr (QUANT) {
+            float sa = scale[0];
+#pragma unroll
+            for (int k = 1; k < MROWS; ++k) sa = m == k ? scale[k] : sa;
+            f = f / sa;
+          } else {
+            f = f / s_a[m];
+          }
           f = f / s_w;
           ((half_t*)C)[(size_t)m * N + row] = (half_t)f;
         }
@@ -375,12 +456,12 @@ __global__ __launch_bounds__(64 * kFragWaves) void i2_gemv_frag_kernel(const int
   }
 }
 
-template <int MROWS, int NP>
+template <int MROWS, int NP, bool QUANT = false>
 int launch_i2_gemv_frag(const void* A, const void* B, void* C, const void* s_a, float s_w, int out_kind, int M, int N, int K,
                         Decoder dec, int interleaved, hipStream_t stream) {
   const int row_blocks = (N + 31) / 32;
   const int grid = row_blocks < 512 ? row_blocks : 512;
-  hipLaunchKernelGGL((i2_gemv_frag_kernel<MROWS, NP>), dim3(grid), dim3(64 * kFragWaves), 0, stream, (const int8_t*)A,
+  hipLaunchKernelGGL((i2_gemv_frag_kernel<MROWS, NP, QUANT>), dim3(grid), dim3(64 * kFragWaves), 0, stream, A,
                      (const uint8_t*)B, C, (const float*)s_a, s_w, out_kind, M, N, K, dec.flip, dec.mul, dec.zsub, interleaved);
   DQ_CHECK_HIP(hipGetLastError());
   return 0;
@@ -420,6 +501,33 @@ int i2_gemv(const void* A, const void* B, void* C, int M, int N, int K, int conv
 #undef DQ_GO
   }
   return int_gemv<2>(A, B, C, M, N, K, dec, interleaved, s_a, s_w, out_kind, stream);
+}
+
+// The same on fp16 activations (BitLinear's forward in one launch), offset-binary codes: one row, and on row-major words two
+// where they fit the LDS (in fragment order the register-resident kernel is ahead from two rows on: N = K = 4096 8.4 against
+// 5.6 us at three).  1: not these kernels'.
+int i2_bitlinear_gemv(const void* X, const void* B, void* C, int M, int N, int K, int layout, float s_w, hipStream_t stream) {
+  const Decoder dec{0u, 1, 2};
+  const int interleaved = (layout & ~LAYOUT_FRAGMENTS) == LAYOUT_INTERLEAVED;
+  if (layout & LAYOUT_FRAGMENTS) {
+    if (M != 1 || K % 128 != 0 || K > 16384) return 1;
+    const int np = ((K >> 7) + kFragWaves - 1) / kFragWaves;
+#define DQ_GO(NP_) return launch_i2_gemv_frag<1, NP_, true>(X, B, C, nullptr, s_w, 1, M, N, K, dec, interleaved, stream)
+    if (np <= 1) DQ_GO(1);
+    if (np <= 2) DQ_GO(2);
+    if (np <= 4) DQ_GO(4);
+    DQ_GO(8);
+#undef DQ_GO
+  }
+  if (M < 1 || M > 2 || K % 64 != 0) return 1;
+  const int c16 = K / 64;
+  int tpr_shift = 5;
+  while ((1 << tpr_shift) < c16 && tpr_shift < 8) ++tpr_shift;
+  const int np = (c16 + (1 << tpr_shift) - 1) >> tpr_shift;
+  if (M * np > 2) return 1;
+  if (M == 2) return launch_int_gemv<2, 2, 1, true>(X, B, C, nullptr, s_w, 1, M, N, K, tpr_shift, dec, interleaved, stream);
+  if (np == 2) return launch_int_gemv<2, 1, 2, true>(X, B, C, nullptr, s_w, 1, M, N, K, tpr_shift, dec, interleaved, stream);
+  return launch_int_gemv<2, 1, 1, true>(X, B, C, nullptr, s_w, 1, M, N, K, tpr_shift, dec, interleaved, stream);
 }
 
 // decode: the values of call_gemm_int8xint4 (0 unsigned nibbles, 1 two's complement, 2 / 3 the words of

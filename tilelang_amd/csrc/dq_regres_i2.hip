@@ -30,7 +30,7 @@
 // read as row M - 1; neither is stored.
 #include <type_traits>
 
-#include "dq_common.h"
+#include "dq_act_quant.h"
 #include "dq_i2_codes.h"
 
 namespace dq {
@@ -281,8 +281,16 @@ constexpr int kMaxPairs16 = 8;            // pairs of 128-k blocks per wave (K <
 constexpr int kPartial16 = 16 * 16 * 4;   // one wave's 16 x 16 sums
 constexpr int kLds16 = kWaves * 4096;     // the prologue's parking areas; the two buffers of partial sums reuse them
 
-template <int CONV, bool FRAG, int NPW, class FIN>
-__global__ __launch_bounds__(64 * kWaves, 1) void i2_regres16_kernel(const int8_t* __restrict__ A, const uint8_t* __restrict__ B,
+//
+// JN > 0: the activations come in fp16, as a BitLinear layer gets them, at most 2 JN rows, and every workgroup quantises
+// all of them itself (dq_act_quant.h: the bits of the quantiser's own kernel): a wave takes the maxima of its eighth of K,
+// the eight meet in LDS, and the int8 values go into the parking areas that the other form copies them into.  That costs a
+// CU five vector instructions per activation and twice the bytes of its prologue, and saves a launch: see
+// bitlinear_in_one_kernel for where it pays.
+constexpr int kRowMax16 = kWaves * 16 * 4;  // their rows' maxima, [16 rows][8 waves]
+
+template <int CONV, bool FRAG, int NPW, int JN, class FIN>
+__global__ __launch_bounds__(64 * kWaves, 1) void i2_regres16_kernel(const void* __restrict__ A_any, const uint8_t* __restrict__ B,
                                                                      typename FIN::out_t* __restrict__ C, int M, int N, int K,
                                                                      int interleaved, FIN fin) {
   extern __shared__ __align__(16) unsigned char smem[];
@@ -321,7 +329,8 @@ __global__ __launch_bounds__(64 * kWaves, 1) void i2_regres16_kernel(const int8_
   // ahead of the activations, see the kernel above)
   const int out_m = tid >> 2, out_p = tid & 3;
   const bool finisher = tid < 64 && out_m < M;
-  const typename FIN::row_t out_row = fin.row(finisher ? out_m : 0);
+  typename FIN::row_t out_row = {};
+  if constexpr (JN == 0) out_row = fin.row(finisher ? out_m : 0);
   uint4_t w[kDepth16][NPW];
   // Loads come back in the order they went out, and the first block's arithmetic needs the first block and the
   // activations: the two blocks ahead go out behind the activations.
@@ -331,8 +340,82 @@ __global__ __launch_bounds__(64 * kWaves, 1) void i2_regres16_kernel(const int8_
   // whole lines (instruction j: rows 4 j .. 4 j + 3, lane l the piece l % 16 of row 4 j + l / 16), parked in the
   // wave's 4 KiB of LDS (piece q of row m at position q ^ m) and read back in operand order
   int4_t af[NPW][4];
-  {
-    const int8_t* const a_lane = A + 16 * (lane & 15);
+  auto read_back = [&](int i, const unsigned char* park) __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      uint4_t a = *reinterpret_cast<const uint4_t*>(park + r * 256 + (((4 * g + s) ^ r) << 4));
+      if (!interleaved) a = transpose4x4_bytes(a);  // plain packing: the decoder's dword j holds elements j, 4 + j, 8 + j, 12 + j
+      af[i][s] = __builtin_bit_cast(int4_t, i < npw ? a : uint4_t{0u, 0u, 0u, 0u});
+    }
+  };
+  if constexpr (JN > 0) {
+    // instruction j: rows 2 j and 2 j + 1, half a wave and 512 bytes each (rows beyond M repeat row M - 1)
+    const half_t* const a_lane = (const half_t*)A_any + 8 * (lane & 31);
+    half8_t line[NPW][JN];
+#pragma unroll
+    for (int i = 0; i < NPW; ++i)
+#pragma unroll
+      for (int j = 0; j < JN; ++j)
+        line[i][j] = *reinterpret_cast<const half8_t*>(a_lane + (size_t)min(2 * j + (lane >> 5), M - 1) * K + 256 * pair_of(i));
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int d = 1; d < kDepth16 - 1; ++d) load_w(w[d], nb0 + d * step, mine > d);
+    // Maxima and rounding in the cheap form that infinities and NaN rule out; where a row has one, in the general form.
+    uint32_t* const row_max = reinterpret_cast<uint32_t*>(smem + kLds16);
+    auto quantise = [&](auto finite_tag) __attribute__((always_inline)) {
+      constexpr bool finite = decltype(finite_tag)::value;
+#pragma unroll
+      for (int j = 0; j < JN; ++j) {
+        uint32_t most;
+        if constexpr (finite) {
+          ushort2_t m = {0, 0};
+#pragma unroll
+          for (int i = 0; i < NPW; ++i) m = abits8(line[i][j], m);  // (a pair short: the last pair twice)
+          most = half_wave_max_bits(m);
+        } else {
+          float amax = 0.f;
+#pragma unroll
+          for (int i = 0; i < NPW; ++i) amax = amax8(line[i][j], amax);
+          most = __builtin_bit_cast(uint32_t, half_wave_max(amax));
+        }
+        if ((lane & 31) == 0) row_max[(2 * j + (lane >> 5)) * kWaves + wave] = most;
+      }
+      __syncthreads();
+      // lane m < 16 of every wave: the scale of row m (non-negative floats order like their bits)
+      uint32_t most = 0;
+#pragma unroll
+      for (int k = 0; k < kWaves; k += 4) {
+        const uint4_t p = *reinterpret_cast<const uint4_t*>(row_max + (lane & (2 * JN - 1)) * kWaves + k);
+        most = max(most, max(max(p[0], p[1]), max(p[2], p[3])));
+      }
+      if constexpr (finite)
+        if (__any(most > kLargestFinite)) return false;
+      const float row_scale = finite ? act_scale_of_bits(most) : act_scale(__builtin_bit_cast(float, most));
+      unsigned char* const park = smem + wave * 4096;
+      const int piece = lane & 31;  // eight int8: half of the 16-byte piece / 2
+      float scale[JN];
+#pragma unroll
+      for (int j = 0; j < JN; ++j) scale[j] = __shfl(row_scale, 2 * j + (lane >> 5));
+      out_row = (typename FIN::row_t)__shfl(row_scale, out_m & (2 * JN - 1));
+#pragma unroll
+      for (int i = 0; i < NPW; ++i) {
+#pragma unroll
+        for (int j = 0; j < JN; ++j) {
+          const int row = 2 * j + (lane >> 5);
+          const uint2_t q = finite ? quantise8_finite(line[i][j], scale[j]) : quantise8(line[i][j], scale[j]);
+          *reinterpret_cast<uint2_t*>(park + row * 256 + (((piece >> 1) ^ row) << 4) + (piece & 1) * 8) = q;
+        }
+        read_back(i, park);  // (rows from 2 JN on: what lies there; their sums are not stored)
+      }
+      return true;
+    };
+    if (!quantise(std::true_type{})) {
+      __syncthreads();  // the maxima are read
+      quantise(std::false_type{});
+    }
+    __syncthreads();  // the parking areas are where the partial sums go
+  } else {
+    const int8_t* const a_lane = (const int8_t*)A_any + 16 * (lane & 15);
     uint4_t line[NPW][4];
 #pragma unroll
     for (int i = 0; i < NPW; ++i)
@@ -350,12 +433,7 @@ __global__ __launch_bounds__(64 * kWaves, 1) void i2_regres16_kernel(const int8_
         const int row = 4 * j + (lane >> 4);
         *reinterpret_cast<uint4_t*>(park + row * 256 + (((lane & 15) ^ row) << 4)) = line[i][j];
       }
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        uint4_t a = *reinterpret_cast<const uint4_t*>(park + r * 256 + (((4 * g + s) ^ r) << 4));
-        if (!interleaved) a = transpose4x4_bytes(a);  // plain packing: the decoder's dword j holds elements j, 4 + j, 8 + j, 12 + j
-        af[i][s] = __builtin_bit_cast(int4_t, i < npw ? a : uint4_t{0u, 0u, 0u, 0u});
-      }
+      read_back(i, park);
     }
     __syncthreads();  // the parking areas are where the partial sums go
   }
@@ -428,11 +506,12 @@ __global__ __launch_bounds__(64 * kWaves, 1) void i2_regres16_kernel(const int8_
   }
 }
 
-template <int CONV, bool FRAG, int NPW, class FIN>
+template <int CONV, bool FRAG, int NPW, int JN, class FIN>
 int launch_i2_regres16(const void* A, const void* B, void* C, int M, int N, int K, int interleaved, FIN fin, hipStream_t stream) {
-  auto kern = i2_regres16_kernel<CONV, FRAG, NPW, FIN>;
+  auto kern = i2_regres16_kernel<CONV, FRAG, NPW, JN, FIN>;
+  constexpr int kLdsBytes = kLds16 + (JN > 0 ? kRowMax16 : 0);
   static bool raised[kMaxDevices] = {};
-  if (raise_lds_limit<kLds16>(kern, raised)) return -1;
+  if (raise_lds_limit<kLdsBytes>(kern, raised)) return -1;
   static int cus_of[kMaxDevices] = {};
   int device = 0;
   DQ_CHECK_HIP(hipGetDevice(&device));
@@ -440,7 +519,7 @@ int launch_i2_regres16(const void* A, const void* B, void* C, int M, int N, int 
   if (!cus_of[device]) DQ_CHECK_HIP(hipDeviceGetAttribute(&cus_of[device], hipDeviceAttributeMultiprocessorCount, device));
   const int row_blocks = (N + 15) / 16;
   const int grid = row_blocks < cus_of[device] ? row_blocks : cus_of[device];
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * kWaves), kLds16, stream, (const int8_t*)A, (const uint8_t*)B,
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * kWaves), kLdsBytes, stream, A, (const uint8_t*)B,
                      (typename FIN::out_t*)C, M, N, K, interleaved, fin);
   DQ_CHECK_HIP(hipGetLastError());
   return 0;
@@ -508,8 +587,8 @@ int i2_gemm_regres(const void* A, const void* B, void* C, int M, int N, int K, i
 #define DQ_I2R16(CONV_, FRAG_, NPW_)                                                                                     \
   do {                                                                                                                   \
     if (bitnet_epilogue)                                                                                                 \
-      return launch_i2_regres16<CONV_, FRAG_, NPW_>(A, B, C, M, N, K, il, BitnetFinish{(const float*)s_a, s_w}, stream); \
-    return launch_i2_regres16<CONV_, FRAG_, NPW_>(A, B, C, M, N, K, il, Int32Finish{}, stream);                          \
+      return launch_i2_regres16<CONV_, FRAG_, NPW_, 0>(A, B, C, M, N, K, il, BitnetFinish{(const float*)s_a, s_w}, stream); \
+    return launch_i2_regres16<CONV_, FRAG_, NPW_, 0>(A, B, C, M, N, K, il, Int32Finish{}, stream);                          \
   } while (0)
 #define DQ_I2RN(CONV_, FRAG_)                           \
   do {                                                  \
@@ -548,6 +627,51 @@ int i2_gemm_regres(const void* A, const void* B, void* C, int M, int N, int K, i
 #undef DQ_I2RN
 #undef DQ_I2R16
 #undef DQ_I2R
+}
+
+// The same kernel on fp16 activations (BitLinear's forward in one launch), offset-binary codes.  1: not the kernel's.
+int i2_bitlinear_regres(const void* X, const void* B, void* C, int M, int N, int K, int layout, float s_w, hipStream_t stream) {
+  if (M < 1 || M > 16 || K % 256 != 0) return 1;
+  if ((uint64_t)(N + 32) * (uint64_t)(K >> 2) >= (1ull << 32)) return 1;
+  const int npw = ((K >> 8) + kWaves - 1) / kWaves;
+  const int il = (layout & ~LAYOUT_FRAGMENTS) == LAYOUT_INTERLEAVED;
+  const BitnetFinish fin{nullptr, s_w};
+  // the rows' lines are held between the maximum and the rounding: 4 JN registers per pair of blocks
+#define DQ_GO(NPW_, JN_)                                                                                              \
+  do {                                                                                                                \
+    if (layout & LAYOUT_FRAGMENTS) return launch_i2_regres16<I2_OFFSET, true, NPW_, JN_>(X, B, C, M, N, K, il, fin, stream); \
+    return launch_i2_regres16<I2_OFFSET, false, NPW_, JN_>(X, B, C, M, N, K, il, fin, stream);                        \
+  } while (0)
+  if (M <= 4) {
+    switch (npw) {
+      case 1: DQ_GO(1, 2);
+      case 2: DQ_GO(2, 2);
+      case 3: DQ_GO(3, 2);
+      case 4: DQ_GO(4, 2);
+      case 5: DQ_GO(5, 2);
+      case 6: DQ_GO(6, 2);
+      case 7: DQ_GO(7, 2);
+      case 8: DQ_GO(8, 2);
+      default: return 1;
+    }
+  }
+  if (M <= 8) {
+    switch (npw) {
+      case 1: DQ_GO(1, 4);
+      case 2: DQ_GO(2, 4);
+      case 3: DQ_GO(3, 4);
+      case 4: DQ_GO(4, 4);
+      case 5: DQ_GO(5, 4);
+      default: return 1;  // (six pairs spill)
+    }
+  }
+  switch (npw) {
+    case 1: DQ_GO(1, 8);
+    case 2: DQ_GO(2, 8);
+    case 3: DQ_GO(3, 8);
+    default: return 1;  // (four pairs spill)
+  }
+#undef DQ_GO
 }
 
 }  // namespace dq

@@ -897,6 +897,34 @@ def bitlinear_int8xint2(M: int, N: int, K: int, s_w: float, convention: str = "o
     return KernelAdapter("bitlinear_int8xint2", params, [-1], launch, _lib.last_error)
 
 
+def bitlinear_fp16(M: int, N: int, K: int, s_w: float, interleaved: bool = False, weight_fragments: bool = False) -> KernelAdapter:
+    """BitLinear forward: ``out[M,N] fp16 = kernel(x, B)`` with ``x`` fp16 ``[M, K]``: :func:`bitnet_activation_quant` and
+    :func:`bitlinear_int8xint2` (offset-binary codes) in one call, with their bits.
+
+    ``forward`` of examples/bitnet-1.58b/utils_quant.py:188-209 without the bias.  At a decode batch it is one kernel; beyond,
+    the quantised activations go through a workspace that the kernel object allocates per call.
+    """
+    if K % 128 != 0:
+        raise ValueError(f"bitlinear_fp16: K={K} must be a multiple of 128")
+    layout = LAYOUT_INTERLEAVED if interleaved else LAYOUT_PLAIN
+    b_shape = (N, K // 4)
+    if weight_fragments:
+        _i2_fragments_ok("bitlinear_fp16", K, None)
+        layout |= LAYOUT_FRAGMENTS
+        b_shape = ((N + 31) // 32, K // 128, 64, 16)
+    room = int(_lib.load_library().dq_bitlinear_workspace_bytes(M, N, K, layout))
+    params = [KernelParam("x", torch.float16, (M, K)), KernelParam("B", torch.int8, b_shape, packed=True),
+              KernelParam("out", torch.float16, (M, N))]
+    if room:
+        params.append(KernelParam("Workspace", torch.uint8, (room,)))
+
+    def launch(ptrs, stream):
+        return _lib.get_library().call_bitlinear_fp16(ptrs[0], ptrs[1], ptrs[2], ptrs[3] if room else None, room, M, N, K, layout,
+                                                      float(s_w), stream)
+
+    return KernelAdapter("bitlinear_fp16", params, [2], launch, _lib.last_error, workspace_idx=[3] if room else [])
+
+
 def bitnet_activation_quant(M: int, K: int) -> KernelAdapter:
     """BitLinear activation quantiser: ``x_q, s = kernel(x)`` with ``x`` fp16 ``[M, K]``, ``x_q`` int8 ``[M, K]``,
     ``s`` fp32 ``[M]``: ``s = 127 / max(|x|.max(-1), 1e-5)``, ``x_q = clamp(round(x.float() * s), -128, 127)``.
