@@ -118,7 +118,30 @@ def get_library(device_index: int | None = None) -> ctypes.CDLL:
                 if lib.init() != 0:
                     raise RuntimeError(f"libdqgemm init failed: {lib.get_last_error().decode()}")
                 _initialised_devices.add(device_index)
+        host = host_call()  # (not under the lock, which loading the library takes)
+        if host is not None and device_index >= 0:
+            host.initialised(device_index)
     return lib
+
+
+_host_call = None  # None: not looked for; False: not there
+
+
+def host_call():
+    """The native call of kernel objects (csrc/host_call.cpp), bound to the library; None where it is not built."""
+    global _host_call
+    if _host_call is None:
+        try:
+            import torch
+
+            from . import _hostcall
+
+            load_library()
+            raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+            _host_call = _hostcall if raw_stream is not None and _hostcall.open(LIB_PATH, raw_stream) else False
+        except (ImportError, LibraryNotBuiltError):
+            return None
+    return _host_call or None
 
 
 def last_error() -> str:

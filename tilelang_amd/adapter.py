@@ -23,6 +23,8 @@ from typing import Callable, Sequence
 
 import torch
 
+from . import _lib
+
 
 @dataclass(frozen=True)
 class KernelParam:
@@ -57,7 +59,11 @@ class KernelAdapter:
         get_last_error: Callable[[], str],
         device_type: str = "cuda",
         workspace_idx: Sequence[int] = (),
+        native: tuple | None = None,
     ):
+        """``native``: ``(entry point, parameter per pointer argument (None: NULL), int arguments, float argument, workspace
+        bytes)`` of the C call that ``launch`` makes, where that is all that it does; a good call then goes to it without
+        passing through the interpreter's checks (csrc/host_call.cpp)."""
         self.name = name
         self.params = list(params)
         n = len(self.params)
@@ -70,6 +76,19 @@ class KernelAdapter:
         self._launch = launch
         self._get_last_error = get_last_error
         self.device_type = device_type
+        self._native_spec = native if device_type == "cuda" else None
+        self._native = self._bind(self.result_idx)
+        self._native_new: dict = {}
+
+    def _bind(self, result_idx):
+        """The native call with the parameters of ``result_idx`` allocated by it; None where there is none."""
+        host = _lib.host_call() if self._native_spec is not None and _raw_stream is not None and len(result_idx) <= 1 else None
+        if host is None:
+            return None
+        entry, slots, ints, f, ws_bytes = self._native_spec
+        roles = [2 if i in self.workspace_idx else 1 if i in result_idx else 0 for i in range(len(self.params))]
+        return host.bind(entry, tuple((p.dtype, int(p.packed), tuple(p.shape), role) for p, role in zip(self.params, roles)),
+                         tuple(-1 if i is None else i for i in slots), tuple(ints), float(f), ws_bytes)
 
     # -- validation, same order and wording as the reference ------------------------------
     def _check(self, tensors: list):
@@ -125,7 +144,26 @@ class KernelAdapter:
             if isinstance(t, torch.Tensor) and not t.is_contiguous():
                 raise ValueError(f"Expected parameter {p.name} to be a contiguous tensor")
 
+    def into_new(self, out_idx: int, *inputs):
+        """``kernel(*inputs, out)`` for a kernel whose output, parameter ``out_idx`` and the last one that the caller
+        brings, is the caller's: allocates it on the first input's device and returns it."""
+        native = self._native_new.get(out_idx)
+        if native is None and out_idx not in self._native_new:
+            native = self._native_new[out_idx] = self._bind([out_idx])
+        if native is not None:
+            out = native(*inputs)
+            if out is not NotImplemented:
+                return out
+        p = self.params[out_idx]
+        out = torch.empty(p.shape, dtype=p.dtype, device=inputs[0].device)
+        self(*inputs, out)
+        return out
+
     def __call__(self, *inputs, stream: int = -1, skip_tensor_validation: bool = False):
+        if self._native is not None and stream == -1 and not skip_tensor_validation:
+            out = self._native(*inputs)
+            if out is not NotImplemented:
+                return out
         n_params, n_in, n_out = len(self.params) - len(self.workspace_idx), len(inputs), len(self.result_idx)
         if n_params != n_in + n_out:
             raise ValueError(

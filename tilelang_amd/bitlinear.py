@@ -106,10 +106,13 @@ class BitLinear(nn.Module):
         return k
 
     def forward(self, input: torch.Tensor) -> torch.Tensor:
-        x = input.reshape(-1, self.in_features)
+        flat = input.dim() == 2 and input.shape[1] == self.in_features
+        x = input if flat else input.reshape(-1, self.in_features)
         if x.dtype != torch.float16:
             x = x.to(torch.float16)
-        out = self._get_kernel(x.shape[0])(x.contiguous(), self.qweight)
+        kern = self._kernels.get(x.shape[0]) or self._get_kernel(x.shape[0])
+        qweight = self._buffers.get("qweight")  # self.qweight without the module's attribute look-up
+        out = kern(x.contiguous(), self.qweight if qweight is None else qweight)
         if self.bias is not None:
             out += self.bias.view(1, -1).expand_as(out)
-        return out.reshape(*input.shape[:-1], self.out_features)
+        return out if flat else out.reshape(*input.shape[:-1], self.out_features)

@@ -209,7 +209,12 @@ def dequantize_gemv(
                                                      mode, layout, variant, stream)
         return lib.call_dequantize_gemv_w4a16(a, b, s, z, ptrs[c_idx], M, N, K, group_size, mode, layout, variant, stream)
 
-    return KernelAdapter("dequantize_gemv", params, [], launch, _lib.last_error, workspace_idx=workspace_idx)
+    native = None
+    if zwork is None:
+        pointers = (0, 1, 2 if with_scaling else None, 3 if with_zeros else None, c_idx) + ((c_idx + 1,) if ws_bytes else ())
+        native = ("call_dequantize_gemv_w4a16_ws" if ws_bytes else "call_dequantize_gemv_w4a16", pointers,
+                  (M, N, K, group_size, mode, layout, variant), 0.0, ws_bytes)
+    return KernelAdapter("dequantize_gemv", params, [], launch, _lib.last_error, workspace_idx=workspace_idx, native=native)
 
 
 def _dequantize_gemv_int8(M, N, K, out_dtype, accum_dtype, num_bits, storage_dtype, source_format, fast_decoding,
@@ -460,7 +465,10 @@ def matmul_bf16_mxfp4(
                                                        fmt, scale_bias, 0, stream)
         return lib.call_dequant_gemm_bf16_mxfp4(ptrs[0], ptrs[1], ptrs[2], bias, ptrs[4], M, N, K, scale_size, fmt, scale_bias, stream)
 
-    return KernelAdapter("matmul_bf16_mxfp4", params, [4], launch, _lib.last_error, workspace_idx=[5] if ws_bytes else [])
+    pointers = (0, 1, 2, 3 if with_bias else None, 4) + ((5,) if ws_bytes else ())
+    native = ("call_dequant_gemm_bf16_mxfp4_ws" if ws_bytes else "call_dequant_gemm_bf16_mxfp4", pointers,
+              (M, N, K, scale_size, fmt, scale_bias) + ((0,) if ws_bytes else ()), 0.0, ws_bytes)
+    return KernelAdapter("matmul_bf16_mxfp4", params, [4], launch, _lib.last_error, workspace_idx=[5] if ws_bytes else [], native=native)
 
 
 def matmul_bf16_fp4(
@@ -761,7 +769,8 @@ def matmul_int8xint4(
     def launch(ptrs, stream):
         return _lib.get_library().call_gemm_int8xint4(ptrs[0], ptrs[1], ptrs[2], M, N, K, 1, 0, 1, stream)
 
-    return KernelAdapter("matmul_int8xint4", params, [2], launch, _lib.last_error)
+    return KernelAdapter("matmul_int8xint4", params, [2], launch, _lib.last_error,
+                         native=("call_gemm_int8xint4", (0, 1, 2), (M, N, K, 1, 0, 1), 0.0, 0))
 
 
 def matmul_nt_int4(M: int, N: int, K: int, block_M: int = 128, block_N: int = 128, block_K: int = 64, threads: int = 128) -> KernelAdapter:
@@ -922,7 +931,8 @@ def bitlinear_fp16(M: int, N: int, K: int, s_w: float, interleaved: bool = False
         return _lib.get_library().call_bitlinear_fp16(ptrs[0], ptrs[1], ptrs[2], ptrs[3] if room else None, room, M, N, K, layout,
                                                       float(s_w), stream)
 
-    return KernelAdapter("bitlinear_fp16", params, [2], launch, _lib.last_error, workspace_idx=[3] if room else [])
+    return KernelAdapter("bitlinear_fp16", params, [2], launch, _lib.last_error, workspace_idx=[3] if room else [],
+                         native=("call_bitlinear_fp16", (0, 1, 2, 3 if room else None), (M, N, K, layout), float(s_w), room))
 
 
 def bitnet_activation_quant(M: int, K: int) -> KernelAdapter:

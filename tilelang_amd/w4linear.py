@@ -99,16 +99,18 @@ class W4A16Linear(nn.Module):
         return k
 
     def forward(self, input: torch.Tensor) -> torch.Tensor:
-        x = input.reshape(-1, self.in_features)
+        flat = input.dim() == 2 and input.shape[1] == self.in_features
+        x = input if flat else input.reshape(-1, self.in_features)
         if x.dtype != torch.float16:
             x = x.to(torch.float16)
         x = x.contiguous()
-        out = torch.empty((x.shape[0], self.out_features), dtype=torch.float16, device=x.device)
-        kern = self._get_kernel(x.shape[0])
-        if self.with_zeros:
-            kern(x, self.qweight, self.scales, self.zeros, out)
-        else:
-            kern(x, self.qweight, self.scales, out)
-        if self.bias is not None:
-            out += self.bias.view(1, -1).expand_as(out)
-        return out.reshape(*input.shape[:-1], self.out_features)
+        try:  # what self.qweight and the others are, without the module's attribute look-up
+            held = self._buffers
+            qweight, scales, zeros, bias = held["qweight"], held["scales"], held["zeros"], held["bias"]
+        except KeyError:  # something else in a buffer's place
+            qweight, scales, zeros, bias = self.qweight, self.scales, self.zeros, self.bias
+        kern = self._kernels.get(x.shape[0]) or self._get_kernel(x.shape[0])
+        out = kern.into_new(4, x, qweight, scales, zeros) if self.with_zeros else kern.into_new(3, x, qweight, scales)
+        if bias is not None:
+            out += bias.view(1, -1).expand_as(out)
+        return out if flat else out.reshape(*input.shape[:-1], self.out_features)
