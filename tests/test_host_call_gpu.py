@@ -34,8 +34,8 @@ def test_same_results(cuda, M, N, K, bias):
     args = _mxfp4(cuda, M, N, K, bias)
     kernel = tl.matmul_bf16_mxfp4(M, N, K, with_bias=bias, weight_format="e2m1", scale_bias=127)
     want = _python(kernel, *args)
-    assert kernel._native(*args) is not NotImplemented
     assert torch.equal(kernel(*args), want)
+    assert kernel._native(*args) is not NotImplemented
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(side):
@@ -61,6 +61,7 @@ def test_unsettled_calls(cuda):
     kernel = tl.matmul_bf16_mxfp4(3, 264, 512, weight_format="e2m1", scale_bias=127)
     a, b, s, bias = _mxfp4(cuda, 3, 264, 512, True)
     want = kernel(a, b, s, bias)
+    assert kernel._native(a, b, s, bias) is not NotImplemented
     for wrong, message in (((a.float(), b, s, bias), "dtype mismatch for parameter A"), ((a, b[:-1], s, bias), "shape mismatch for parameter B"),
                            ((a, b, s.cpu(), bias), "device mismatch for parameter Scale"),
                            ((a, b, s, torch.empty((3, 528), dtype=torch.bfloat16, device=cuda)[:, ::2]), "stride mismatch for parameter Bias"),

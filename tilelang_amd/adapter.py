@@ -49,6 +49,10 @@ def current_stream_handle(device_type: str = "cuda", index: int | None = None) -
     return 0
 
 
+#: a kernel object's native call that its first call has yet to bind
+_unbound = object()
+
+
 class KernelAdapter:
     def __init__(
         self,
@@ -77,7 +81,8 @@ class KernelAdapter:
         self._get_last_error = get_last_error
         self.device_type = device_type
         self._native_spec = native if device_type == "cuda" else None
-        self._native = self._bind(self.result_idx)
+        # bound by the first call: a kernel object that is only looked at, or made anew, pays for none
+        self._native = _unbound if self._native_spec is not None else None
         self._native_new: dict = {}
 
     def _bind(self, result_idx):
@@ -160,8 +165,11 @@ class KernelAdapter:
         return out
 
     def __call__(self, *inputs, stream: int = -1, skip_tensor_validation: bool = False):
-        if self._native is not None and stream == -1 and not skip_tensor_validation:
-            out = self._native(*inputs)
+        native = self._native
+        if native is not None and stream == -1 and not skip_tensor_validation:
+            if native is _unbound:
+                native = self._native = self._bind(self.result_idx)
+            out = native(*inputs) if native is not None else NotImplemented
             if out is not NotImplemented:
                 return out
         n_params, n_in, n_out = len(self.params) - len(self.workspace_idx), len(inputs), len(self.result_idx)

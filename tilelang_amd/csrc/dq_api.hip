@@ -351,38 +351,44 @@ extern "C" int call_unpack_qzeros(const void* QZeros, void* Zeros, int N, int gr
 }
 
 // Into how many slices of K the tiled MXFP4 GEMM is cut when the caller brought a workspace; 1: not cut.  The times (us)
-// are fits, and cut is what they put ahead by a twelfth.  Measured both ways at 1712 shapes (81 to 4096 rows, N 64 to
-// 28672, K 1024 to 28672, odd ones and close calls among them) in the three formats: the 1389 that are cut ("simple"
-// 999) take two thirds of the uncut time in the median (M = 96, N = K = 8192: 64 -> 29 us; M = 384, N = K = 8192:
-// 90 -> 61; M = 2048, N = 2048, K = 8192: 96 -> 71); four calls take 1 to 4 % more (M = 110, N = 818, K = 11520: 25.6
-// against 26.6 us).
-// * Uncut from 96 tiles of 128 x 256 on: 10.4 ns per k there, 12.8 at 224 (the tiles share the memory's bandwidth).
-//   Below that the register-staged kernel's tiles of 128 x 64 (beyond 256 of them a second round); at a decode batch
-//   the register-resident kernel, which up to K = 4096 takes 0.7 of its estimate (M = 128, N = 2048: 16.5 us, cut 17.2).
+// are fits over 131 shapes (81 to 4096 rows, N 2048 to 28672, K 1024 to 14336, odd ones among them) and ten slice counts
+// each, and cut is what they put ahead by a twelfth: the pick takes 1.0 % more than the best count on average, 17 % at most,
+// and no cut call more than uncut (M = 96, N = K = 8192: 64 -> 25.5 us; M = 384, N = K = 8192: 90 -> 55; M = 155, N = 18624,
+// K = 12672, 146 tiles: 149 -> 112).
+// * Cut: 9 us of two launches and a start and an end of the pipeline, 5.5 for every further round of 256 workgroups; a
+//   slice's k at 7.6 ns with 64 workgroups, 9.1 with 208 and 11.5 with all CUs taken (M = 96, N = K = 8192: six slices, 192
+//   workgroups, 26.9 us, eight 30.1), 10.6 per round beyond; and the sums' way through memory at 3.3 TB/s.
+// * Uncut, on tiles of 256 rows where the kernel takes those, else of 128 from 96 of them on.  Below that the register-staged
+//   kernel's tiles of 128 x 64 (beyond 256 of them a second round); at a decode batch the register-resident kernel, which
+//   up to K = 4096 takes 0.7 of its estimate (M = 128, N = 2048: 16.5 us, cut 17.2).
 // * The "simple" format's decoder is longer, and the 128 x 256 tile spills with it: its times are 1.65 of the above there,
 //   1.3 on the other kernels (M = 166, N = 5818, K = 3072: 35.2 us, in four slices 43; e2m1 27.9 and 27.3).
-// * More than one round of 256 workgroups is cut only where the tile count is a multiple of the XCDs: only then does an
-//   XCD walk neighbouring tiles (M = 1000, N = 5120, K = 14336, 160 tiles: 169 -> 146 us; M = 384, N = 13824, K = 8192,
-//   162 tiles: 96 -> 112).  From 192 tiles on it is even (M = 768, N = 8192, K = 14336: 174 us, in four slices 178), with
-//   a workspace of 100 MB.
+// * More than one round from 160 tiles on only where the tile count is a multiple of the XCDs: an XCD then walks neighbouring
+//   tiles (M = 384, N = 13824, K = 8192, 162 tiles: 95 us, in three slices 112 when those were slower than they are now).
+// From 192 tiles on nothing is gained (M = 768, N = 8192, K = 14336: 174 us, in four slices 178).
 // Up to 80 rows nothing is cut.  That is a promise of the header and no crossover: up to there a call that runs on the
-// tiled kernel gives the bits that its rows have in a large product (cut, M = 80, N = K = 8192 would take 27 us, not 63).
+// tiled kernel gives the bits that its rows have in a large product (cut, M = 80, N = K = 8192 would take 25 us, not 63).
 static int mxfp4_ksplit(int M, int N, int K, int fp4_format) {
   if (M <= 80 || K % 128 != 0 || ((size_t)M * N) % 4 != 0) return 1;
   const long tiles = (((long)M + 127) / 128) * (((long)N + 255) / 256);
   if (tiles >= 192) return 1;
   const int units = K / 128;
+  const long tall_tiles = (((long)M + 255) / 256) * (((long)N + 255) / 256);
   const long small_tiles = (((long)M + 127) / 128) * (((long)N + 63) / 64);  // of the register-staged kernel
-  double best = tiles >= 96 ? 4.0 + 1e-3 * K * (8.6 + 0.0186 * (double)tiles)
-                            : 2.0 + 1e-3 * K * (tiles <= 32 ? 7.2 : tiles <= 64 ? 8.0 : small_tiles <= 256 ? 7.6 : 9.5);
+  // as dq_gemm_core.h counts them: a last round of few workgroups takes two thirds of a full one
+  auto rounds = [](long wgs) { return (double)(wgs / 256) + (wgs % 256 ? 0.65 + 0.35 * (double)(wgs % 256) / 256.0 : 0.0); };
+  double best;
+  if (tall_tiles >= 96 && 1.85 * rounds(tall_tiles) <= rounds(tiles)) best = 11.3 + 1e-3 * K * 19.6 * rounds(tall_tiles);
+  else if (tiles >= 96) best = 5.1 + 1e-3 * K * (8.65 + 4.5 * (double)tiles / 256.0);
+  else best = 2.0 + 1e-3 * K * (tiles <= 32 ? 7.2 : tiles <= 64 ? 8.0 : small_tiles <= 256 ? 7.6 : 9.5);
   if (M <= 128) best = std::min(best, mxfp4_regres_time(M, N, K) * (K <= 4096 ? 0.7 : 1.0));
   best *= fp4_format == DQ_FP4_SIMPLE && tiles < 96 ? 0.92 / 1.25 : 0.92;
   int split = 1;
   for (int s = 2; s <= 12 && units / s >= 4; ++s) {
     const long wgs = tiles * s;
-    if (wgs > 256 && tiles % 8 != 0) break;
-    const double rate = wgs <= 192 ? 8.5 : 11.8 * (double)((wgs + 255) / 256);
-    const double t = 13.5 + 1e-3 * rate * 128 * ((units + s - 1) / s) + (double)s * M * N * 4 / 5.2e6;
+    if (wgs > 256 && tiles >= 160 && tiles % 8 != 0) break;
+    const double rate = wgs <= 256 ? 7.0 + 0.01 * (double)wgs + 0.04 * (double)std::max(0L, wgs - 208) : 10.6 * rounds(wgs);
+    const double t = 9.0 + 5.5 * (double)((wgs - 1) / 256) + 1e-3 * rate * 128 * ((units + s - 1) / s) + (double)s * M * N * 4 / 3.3e6;
     if (t < best) best = t, split = s;
   }
   return split;
