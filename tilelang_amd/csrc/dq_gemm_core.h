@@ -70,13 +70,14 @@ struct Params {
   float f0;          // policy specific float (e.g. 1 / weight scale)
 };
 
-// Workgroup id -> output tile.  With T tiles and 8 XCDs, XCD x (ids x, x+8, ...) gets the
-// contiguous range [x*T/8, (x+1)*T/8) of a sequence that walks the tile grid in bands of
-// kGroupM tile rows, column by column inside a band.
+// Workgroup id -> output tile.  With T tiles and 8 XCDs, XCD x (ids x, x+8, ...) gets a
+// contiguous range of T/8 tiles, the first T%8 XCDs one more, of a sequence that walks the tile grid in bands of
+// kGroupM tile rows, column by column inside a band.  (Up to 320 tiles that are no multiple of 8 go as they come (259: 26.9 us, sorted
+// 28.9); beyond, sorted: MXFP4 M = 1316, N = 22608, K = 6912 385 -> 342 us, int8 x int4 M = 2217, N = 18000, K = 3328 155 -> 140.)
 __device__ __forceinline__ void tile_of_block(int bid, int tiles_m, int tiles_n, int& tm, int& tn) {
   const int T = tiles_m * tiles_n;
   int pid = bid;
-  if ((T & 7) == 0) pid = (bid & 7) * (T >> 3) + (bid >> 3);
+  if ((T & 7) == 0 || T > 320) pid = (bid & 7) * (T >> 3) + min(bid & 7, T & 7) + (bid >> 3);
   constexpr int kGroupM = 4;
   const int band = kGroupM * tiles_n;
   const int first_m = (pid / band) * kGroupM;
@@ -125,23 +126,25 @@ __device__ __forceinline__ void take_k_slice(Params& p, int& bid) {
 // LDS (every tile is consumed: the loop ended with a barrier) so that each lane stores 16 contiguous
 // bytes.  Each wave owns a slab of 32-bit values, 32 x (32 kNBW + 4) for a block of rows or, transposed, 32 x (32 kMBW + 4)
 // for a block of columns; LDS operations of one wave execute in order, so no workgroup barrier is needed between the phases.
-// The stores: C is written once and not read again by the kernel.  Where its rows (transposed: columns) are whole cache
-// lines they are nontemporal, which keeps the output from displacing operand lines in the L2 (MXFP4 GEMM 361 -> 358 us,
-// block-scaled GEMM 147 -> 138 us).  Where they are not, a line is shared by two pieces that a nontemporal store would
-// each write to memory by itself: ordinary stores, which meet in the L2 (int8 x int4, M = 1000, N = 11008, K = 1024:
-// 34 -> 26 us; int8 x 2-bit, M = 2048, N = 8200, K = 4096 118 -> 92; MXFP4 there 159 -> 140).  Which of the two is asked
-// once per tile: asked per store it cost BitLinear at M = 2048, N = K = 8192 1 %.
+// The stores: C is written once and not read again by the kernel.  They are nontemporal, which keeps the output from
+// displacing operand lines in the L2 (MXFP4 GEMM 361 -> 358 us, block-scaled GEMM 147 -> 138 us), except where a memory
+// sector (32 bytes) is shared by two pieces, which a nontemporal store would each write to memory by itself: ordinary
+// stores there, which meet in the L2 (int8 x 2-bit, M = 2048, N = 8200, K = 4096 118 -> 92 us, MXFP4 159 -> 140; with rows
+// of whole sectors ordinary stores are the slower ones: M = 2664, N = 4560, K = 2304 39.8 against 44.6).  Columns of a
+// transposed output, which other workgroups continue, take them where they are no whole cache lines (int8 x int4, M = 1000,
+// N = 11008, K = 1024: 34 -> 21 us, nontemporal 24).  Which of the two is asked once per tile: asked per store it cost
+// BitLinear at M = 2048, N = K = 8192 1 %.
 // Transposed, the four consecutive rows that a lane holds are one LDS write, and a wave stores whole runs of its rows; a
 // column that does not start at 16 bytes goes out by elements, consecutive lanes on consecutive elements (M = 1001,
 // N = 11008, K = 4096: 73 -> 59 us, with the better tile of that shape).
 #define DQ_GEMM_EPILOGUE DQ_GEMM_EPILOGUE_OF(kMBW)
 #define DQ_GEMM_EPILOGUE_OF(BLOCKS_) \
-  if ((P::kTransposed ? M : N) * (int)sizeof(typename P::out_t) % 128 == 0) { \
+  if (P::kTransposed ? M * (int)sizeof(typename P::out_t) % 128 == 0 : N * (int)sizeof(typename P::out_t) % 32 == 0) { \
     DQ_GEMM_EPILOGUE_STORING(BLOCKS_, true) \
   } else { \
     DQ_GEMM_EPILOGUE_STORING(BLOCKS_, false) \
   }
-#define DQ_GEMM_EPILOGUE_STORING(BLOCKS_, WHOLE_LINES_) \
+#define DQ_GEMM_EPILOGUE_STORING(BLOCKS_, STREAMED_) \
   using out_t = typename P::out_t; \
   constexpr int kOutPerPiece = 16 / sizeof(out_t); \
   if constexpr (!P::kTransposed) { \
@@ -182,7 +185,7 @@ __device__ __forceinline__ void take_k_slice(Params& p, int& bid) {
           if ((n + kOutPerPiece <= N) && ((N % kOutPerPiece) == 0)) { \
             uint4_t pk; \
             __builtin_memcpy(&pk, o, 16); \
-            if constexpr (WHOLE_LINES_) __builtin_nontemporal_store(pk, reinterpret_cast<uint4_t*>(dst)); \
+            if constexpr (STREAMED_) __builtin_nontemporal_store(pk, reinterpret_cast<uint4_t*>(dst)); \
             else *reinterpret_cast<uint4_t*>(dst) = pk; \
           } else { \
   _Pragma("unroll") \
@@ -231,7 +234,7 @@ __device__ __forceinline__ void take_k_slice(Params& p, int& bid) {
             uint4_t pk; \
             __builtin_memcpy(&pk, o, 16); \
             uint4_t* const dst = reinterpret_cast<uint4_t*>((out_t*)p.C + (size_t)n * M + m); \
-            if constexpr (WHOLE_LINES_) __builtin_nontemporal_store(pk, dst); \
+            if constexpr (STREAMED_) __builtin_nontemporal_store(pk, dst); \
             else *dst = pk; \
           } \
         } \
@@ -1106,6 +1109,12 @@ inline double dma_rounds(long tiles) {
   return (double)full + (rest ? 0.65 + 0.35 * (double)rest / 256.0 : 0.0);
 }
 
+// P::kPairWorkgroups: 257 to 512 tiles of 128 x 256 run as two workgroups of four waves per CU, not as rounds of eight waves
+template <class P, class = void>
+struct PairWorkgroups : std::false_type {};
+template <class P>
+struct PairWorkgroups<P, std::void_t<decltype(P::kPairWorkgroups)>> : std::integral_constant<bool, P::kPairWorkgroups> {};
+
 // 256 x 256 tiles, or 128 x 256.  A round of the first costs 1.85 of the second's (K = 8192: fp16 x uint4 215 and 116 us,
 // MXFP4 180 and 98, int8 x int4 84 and 57), so what decides is how either fills its rounds.  Measured on both, fp16 x uint4
 // with zeros, K = 4096: M = 700, N = 11008 75 us in tiles of 256 rows, 98 in tiles of 128; M = 1000 92 and 106; M = 600 76
@@ -1115,7 +1124,7 @@ bool dma_eligible(const Params& p) {
   // fp16 scales of groups of 32 k go with every tile: not with the pairwise issue of the 32-byte-row form of this tile
   const bool scales_per_tile = P::kScaleDma >= 2 && P::kBRowBytes == 32 && p.p0 == 5;
   const long tiles = tiles_of(p, 256);
-  return !scales_per_tile && tiles >= 96 && dma_takes<P>(p) && 1.85 * dma_rounds(tiles) <= dma_rounds(tiles_of(p, 128));
+  return !scales_per_tile && tiles >= (PairWorkgroups<P>::value ? 192 : 96) && dma_takes<P>(p) && 1.85 * dma_rounds(tiles) <= dma_rounds(tiles_of(p, 128));
 }
 
 // Too few 256 x 256 tiles but at least `min_tiles` of 128 x 256: the same kernel on the half-height tile, which keeps the
@@ -1170,6 +1179,8 @@ struct OneOrder<P, std::void_t<decltype(P::kOneOrder)>> : std::integral_constant
 template <class P>
 bool dma_halves_take(const Params& p) {
   if constexpr (OneOrder<P>::value) return false;
+  if constexpr (PairWorkgroups<P>::value)
+    if (tiles_of(p, 128) > 256 && tiles_of(p, 128) <= 512) return false;
   const int shortest = UnevenSlices<P>::value && p.split > 1 ? p.K / p.kunit / p.split * p.kunit : p.K;
   const int stage_k = P::kKPerBlock * (P::kBRowBytes == 32 ? 2 : 1);
   return shortest % stage_k == 0 && shortest / stage_k >= 3 && !(P::kScaleDma >= 2 && p.p0 == 5);

@@ -33,6 +33,9 @@ namespace {
 template <int CONV, class EPI, bool INTERLEAVED, bool TOP = false, bool FRAG = false>
 struct I2Policy : I8Mfma, gemm::NoScale, EPI {
   static_assert(!TOP || CONV != I2_UNSIGNED, "unsigned codes are masked in place");
+  // the two-instruction decoder leaves a lone workgroup's waves little to overlap: M = 2477, N = 3920, K = 2560 (320 tiles of
+  // 128 x 256) 47 us on 160 tiles of 256 rows, 36.7 so; M = 965, N = 9992, K = 4096 58 -> 49
+  static constexpr bool kPairWorkgroups = true;
   static constexpr int kBRowBytes = 32;
   static constexpr bool kBFragments = FRAG;
   static constexpr bool kAPacked = false;
