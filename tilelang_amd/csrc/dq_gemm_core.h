@@ -136,7 +136,8 @@ __device__ __forceinline__ void take_k_slice(Params& p, int& bid) {
 // BitLinear at M = 2048, N = K = 8192 1 %.
 // Transposed, the four consecutive rows that a lane holds are one LDS write, and a wave stores whole runs of its rows; a
 // column that does not start at 16 bytes goes out by elements, consecutive lanes on consecutive elements (M = 1001,
-// N = 11008, K = 4096: 73 -> 59 us, with the better tile of that shape).
+// N = 11008, K = 4096: 73 -> 57 us, with the better tile of that shape), or, where fewer than 48 rows are left, a lane's
+// four rows one after the other (M = 5, N = K = 4096: 15.4 us by elements, 14.9 so).
 #define DQ_GEMM_EPILOGUE DQ_GEMM_EPILOGUE_OF(kMBW)
 #define DQ_GEMM_EPILOGUE_OF(BLOCKS_) \
   if (P::kTransposed ? M * (int)sizeof(typename P::out_t) % 128 == 0 : N * (int)sizeof(typename P::out_t) % 32 == 0) { \
@@ -201,6 +202,7 @@ __device__ __forceinline__ void take_k_slice(Params& p, int& bid) {
     constexpr int kSlabStride = kRows + 4; \
     uint32_t* slab = reinterpret_cast<uint32_t*>(smem) + wave * (32 * kSlabStride); \
     const int m_wave = m0 + wm * (32 * kMBW); \
+    if (m_wave < M) \
   _Pragma("unroll") \
     for (int nb = 0; nb < kNBW; ++nb) { \
   _Pragma("unroll") \
@@ -214,7 +216,7 @@ __device__ __forceinline__ void take_k_slice(Params& p, int& bid) {
         } \
       __builtin_amdgcn_wave_barrier(); \
       const int n_block = n0 + wn * (32 * kNBW) + nb * 32; \
-      if ((M % kOutPerPiece) == 0) { \
+      if ((M % kOutPerPiece) == 0 || M - m_wave < 48) { \
         constexpr int kPiecesPerCol = kRows / kOutPerPiece; \
   _Pragma("unroll") \
         for (int it = 0; it < 32 * kPiecesPerCol / 64; ++it) { \
@@ -230,15 +232,22 @@ __device__ __forceinline__ void take_k_slice(Params& p, int& bid) {
           if (n < N && m < M) { \
             out_t o[kOutPerPiece]; \
   _Pragma("unroll") \
-            for (int e = 0; e < kOutPerPiece; ++e) o[e] = P::finish(raw[e], p, m + e, n); \
-            uint4_t pk; \
-            __builtin_memcpy(&pk, o, 16); \
-            uint4_t* const dst = reinterpret_cast<uint4_t*>((out_t*)p.C + (size_t)n * M + m); \
-            if constexpr (STREAMED_) __builtin_nontemporal_store(pk, dst); \
-            else *dst = pk; \
+            for (int e = 0; e < kOutPerPiece; ++e) o[e] = P::finish(raw[e], p, min(m + e, M - 1), n); \
+            out_t* const dst = (out_t*)p.C + (size_t)n * M + m; \
+            if ((M % kOutPerPiece) == 0) { \
+              uint4_t pk; \
+              __builtin_memcpy(&pk, o, 16); \
+              if constexpr (STREAMED_) __builtin_nontemporal_store(pk, reinterpret_cast<uint4_t*>(dst)); \
+              else *reinterpret_cast<uint4_t*>(dst) = pk; \
+            } else { \
+  _Pragma("unroll") \
+              for (int e = 0; e < kOutPerPiece; ++e) \
+                if (m + e < M) dst[e] = o[e]; \
+            } \
           } \
         } \
       } else { \
+  _Pragma("unroll 8") \
         for (int it = 0; it < 32 * kRows / 64; ++it) { \
           const int q = lane + 64 * it; \
           const int col = q / kRows, m = m_wave + q % kRows, n = n_block + col; \
