@@ -49,8 +49,10 @@ def current_stream_handle(device_type: str = "cuda", index: int | None = None) -
     return 0
 
 
-#: a kernel object's native call that its first call has yet to bind
-_unbound = object()
+def _unbound(*inputs):
+    """Stands for a kernel object's native call until the first call binds it.  A function, which a copy of the object
+    shares: the mark is told by identity."""
+    return NotImplemented
 
 
 class KernelAdapter:
@@ -84,6 +86,10 @@ class KernelAdapter:
         # bound by the first call: a kernel object that is only looked at, or made anew, pays for none
         self._native = _unbound if self._native_spec is not None else None
         self._native_new: dict = {}
+
+    def __getstate__(self):
+        # A native call is bound to the object that it was made for and cannot be copied: a copy binds its own.
+        return {**self.__dict__, "_native": _unbound if self._native_spec is not None else None, "_native_new": {}}
 
     def _bind(self, result_idx):
         """The native call with the parameters of ``result_idx`` allocated by it; None where there is none."""
