@@ -11,7 +11,9 @@ from __future__ import annotations
 import ctypes
 import os
 import subprocess
+import sys
 import threading
+import warnings
 
 _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_PKG_DIR, "libdqgemm.so")
@@ -63,11 +65,14 @@ class LibraryNotBuiltError(RuntimeError):
 
 def build_library(jobs: int = 8, clean: bool = False) -> str:
     """Compile every HIP source for gfx950 into ``libdqgemm.so`` (hipcc cross-compiles without a GPU)."""
+    make = ["make", "-C", CSRC_DIR, f"PYTHON={sys.executable}"]
     if clean:
-        subprocess.run(["make", "-C", CSRC_DIR, "clean"], check=True, capture_output=True)
-    proc = subprocess.run(["make", "-C", CSRC_DIR, f"-j{jobs}"], capture_output=True, text=True)
+        subprocess.run([*make, "clean"], check=True, capture_output=True)
+    proc = subprocess.run([*make, f"-j{jobs}"], capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"building libdqgemm.so failed:\n{proc.stdout[-4000:]}\n{proc.stderr[-4000:]}")
+    if not os.path.exists(os.path.join(_PKG_DIR, "_hostcall.so")):
+        warnings.warn(f"the native call of kernel objects is not built:\n{proc.stderr[-2000:]}", stacklevel=2)
     return LIB_PATH
 
 
