@@ -12,6 +12,7 @@ import ctypes
 import os
 import subprocess
 import sys
+import sysconfig
 import threading
 import warnings
 
@@ -71,7 +72,7 @@ def build_library(jobs: int = 8, clean: bool = False) -> str:
     proc = subprocess.run([*make, f"-j{jobs}"], capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"building libdqgemm.so failed:\n{proc.stdout[-4000:]}\n{proc.stderr[-4000:]}")
-    if not os.path.exists(os.path.join(_PKG_DIR, "_hostcall.so")):
+    if not os.path.exists(os.path.join(_PKG_DIR, "_hostcall" + sysconfig.get_config_var("EXT_SUFFIX"))):
         warnings.warn(f"the native call of kernel objects is not built:\n{proc.stderr[-2000:]}", stacklevel=2)
     return LIB_PATH
 
@@ -133,7 +134,8 @@ _host_call = None  # None: not looked for; False: not there
 
 
 def host_call():
-    """The native call of kernel objects (csrc/host_call.cpp), bound to the library; None where it is not built."""
+    """The native call of kernel objects (csrc/host_call.cpp), bound to the library; None where it is not built, or was built
+    against another torch than the one that runs: it reads the layout of torch's classes, which is that version's own."""
     global _host_call
     if _host_call is None:
         try:
@@ -142,10 +144,17 @@ def host_call():
             from . import _hostcall
 
             load_library()
-            raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-            _host_call = _hostcall if raw_stream is not None and _hostcall.open(LIB_PATH, raw_stream) else False
         except (ImportError, LibraryNotBuiltError):
             return None
+        runs = f"{torch.__version__}/{torch.version.git_version}"
+        built_for = getattr(_hostcall, "built_for", None)
+        raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        if built_for != runs:
+            warnings.warn(f"{_hostcall.__file__} was built against torch {built_for}, this is {runs}: kernel calls go through "
+                          f"the interpreter until `make -C {CSRC_DIR}` builds it anew", stacklevel=2)
+            _host_call = False
+        else:
+            _host_call = _hostcall if raw_stream is not None and _hostcall.open(LIB_PATH, raw_stream) else False
     return _host_call or None
 
 

@@ -263,6 +263,9 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_hostcall", nullptr, -1, kMethods
 
 }  // namespace
 
+#define DQ_TEXT_OF(X) #X
+#define DQ_TEXT(X) DQ_TEXT_OF(X)
+
 PyMODINIT_FUNC PyInit__hostcall(void) {
   CallType.tp_name = "tilelang_amd._hostcall.Call";
   CallType.tp_basicsize = sizeof(Call);
@@ -270,5 +273,11 @@ PyMODINIT_FUNC PyInit__hostcall(void) {
   CallType.tp_dealloc = call_dealloc;
   CallType.tp_call = call_call;
   if (PyType_Ready(&CallType) < 0) return nullptr;
-  return PyModule_Create(&kModule);
+  PyObject* const module = PyModule_Create(&kModule);
+  // the torch whose headers this was compiled against, which the caller compares before it makes a call
+  if (module && PyModule_AddStringConstant(module, "built_for", DQ_TEXT(DQ_BUILT_FOR)) < 0) {
+    Py_DECREF(module);
+    return nullptr;
+  }
+  return module;
 }
