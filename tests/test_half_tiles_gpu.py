@@ -101,6 +101,28 @@ def test_int8_int4(cuda, M, N, K, transposed):
     assert torch.equal(C, ref.int())
 
 
+# a transposed column by blocks of 32 rows (up to 47 rows left in a wave's 64), one row short of that and one beyond it
+@pytest.mark.parametrize("M", [1, 31, 33, 47, 49, 63, 65, 111, 113, 129])
+def test_transposed_rows_off_16_bytes(cuda, M):
+    N, K = 203, 256
+    gen = torch.Generator(device=cuda).manual_seed(M)
+    B = _ints(gen, 0, 255, N, K // 2, dtype=torch.uint8, device=cuda)
+    stream = torch.cuda.current_stream().cuda_stream
+    A = _ints(gen, -128, 127, M, K, dtype=torch.int8, device=cuda)
+    C = torch.full((N + 1, M), -7, dtype=torch.int32, device=cuda)
+    rc = _lib.get_library().call_gemm_int8xint4(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, 0, 0, 1, stream)
+    assert rc == 0, _lib.last_error()
+    assert torch.equal(C[:N], (_nibbles(B).double() @ A.double().t()).int()) and bool((C[N:] == -7).all())
+    A = _ints(gen, -2, 2, M, K, dtype=torch.float16, device=cuda)
+    C = torch.full((N + 1, M), float("nan"), dtype=torch.float16, device=cuda)
+    rc = _lib.get_library().call_dequant_gemm_fp16_fp4(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, 1, stream)
+    assert rc == 0, _lib.last_error()
+    code = _nibbles(B).int()
+    value = torch.exp2(((code >> 1) & 3).double() - 1) * (1 + (code & 1).double() / 2)  # bits (E + 14) << 10 | m << 9
+    W = torch.where(code > 7, -value, value)
+    assert torch.equal(C[:N], (W @ A.double().t()).half()) and bool(torch.isnan(C[N:]).all())
+
+
 @pytest.mark.parametrize("fragments", [False, True])
 @pytest.mark.parametrize("M,N,K", [(1300, 4000, 768), (1300, 4000, 512), (1281, 4072, 1280)])  # three stages, two, five
 def test_bitnet(cuda, M, N, K, fragments):

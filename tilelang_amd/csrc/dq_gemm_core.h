@@ -134,10 +134,12 @@ __device__ __forceinline__ void take_k_slice(Params& p, int& bid) {
 // transposed output, which other workgroups continue, take them where they are no whole cache lines (int8 x int4, M = 1000,
 // N = 11008, K = 1024: 34 -> 21 us, nontemporal 24).  Which of the two is asked once per tile: asked per store it cost
 // BitLinear at M = 2048, N = K = 8192 1 %.
-// Transposed, the four consecutive rows that a lane holds are one LDS write, and a wave stores whole runs of its rows; a
-// column that does not start at 16 bytes goes out by elements, consecutive lanes on consecutive elements (M = 1001,
-// N = 11008, K = 4096: 73 -> 57 us, with the better tile of that shape), or, where fewer than 48 rows are left, a lane's
-// four rows one after the other (M = 5, N = K = 4096: 15.4 us by elements, 14.9 so).
+// Transposed, the four consecutive rows that a lane holds are one LDS write.  A column that does not start at 16 bytes goes
+// out by elements, consecutive lanes on consecutive elements, eight LDS reads ahead of their stores (a read under each store's
+// condition waited for each: M = 1002, N = 11008, K = 1024 27.2 us, 23.6 so; M = 1001, K = 4096 58.4 and 53.8), or, where
+// fewer than 48 rows are left, by blocks of 32 rows, a lane's four or eight one after the other (M = 3, N = 4448, K = 1024: 7.1
+// us with all of the wave's rows walked, 6.3 so; M = 5, N = K = 4096 14.9 and 13.7).  Only the copy that needs them holds
+// these forms: the wave fetches what it does not run too.
 #define DQ_GEMM_EPILOGUE DQ_GEMM_EPILOGUE_OF(kMBW)
 #define DQ_GEMM_EPILOGUE_OF(BLOCKS_) \
   if (P::kTransposed ? M * (int)sizeof(typename P::out_t) % 128 == 0 : N * (int)sizeof(typename P::out_t) % 32 == 0) { \
@@ -183,7 +185,7 @@ __device__ __forceinline__ void take_k_slice(Params& p, int& bid) {
   _Pragma("unroll") \
           for (int e = 0; e < kOutPerPiece; ++e) o[e] = P::finish(raw[e], p, m, min(n + e, N - 1)); \
           out_t* dst = (out_t*)p.C + (size_t)m * N + n; \
-          if ((n + kOutPerPiece <= N) && ((N % kOutPerPiece) == 0)) { \
+          if (STREAMED_ || (N % kOutPerPiece) == 0) { \
             uint4_t pk; \
             __builtin_memcpy(&pk, o, 16); \
             if constexpr (STREAMED_) __builtin_nontemporal_store(pk, reinterpret_cast<uint4_t*>(dst)); \
@@ -216,7 +218,7 @@ __device__ __forceinline__ void take_k_slice(Params& p, int& bid) {
         } \
       __builtin_amdgcn_wave_barrier(); \
       const int n_block = n0 + wn * (32 * kNBW) + nb * 32; \
-      if ((M % kOutPerPiece) == 0 || M - m_wave < 48) { \
+      if (STREAMED_ || (M % kOutPerPiece) == 0) { \
         constexpr int kPiecesPerCol = kRows / kOutPerPiece; \
   _Pragma("unroll") \
         for (int it = 0; it < 32 * kPiecesPerCol / 64; ++it) { \
@@ -232,26 +234,53 @@ __device__ __forceinline__ void take_k_slice(Params& p, int& bid) {
           if (n < N && m < M) { \
             out_t o[kOutPerPiece]; \
   _Pragma("unroll") \
-            for (int e = 0; e < kOutPerPiece; ++e) o[e] = P::finish(raw[e], p, min(m + e, M - 1), n); \
+            for (int e = 0; e < kOutPerPiece; ++e) o[e] = P::finish(raw[e], p, m + e, n); \
             out_t* const dst = (out_t*)p.C + (size_t)n * M + m; \
-            if ((M % kOutPerPiece) == 0) { \
-              uint4_t pk; \
-              __builtin_memcpy(&pk, o, 16); \
-              if constexpr (STREAMED_) __builtin_nontemporal_store(pk, reinterpret_cast<uint4_t*>(dst)); \
-              else *reinterpret_cast<uint4_t*>(dst) = pk; \
-            } else { \
-  _Pragma("unroll") \
-              for (int e = 0; e < kOutPerPiece; ++e) \
-                if (m + e < M) dst[e] = o[e]; \
-            } \
+            uint4_t pk; \
+            __builtin_memcpy(&pk, o, 16); \
+            if constexpr (STREAMED_) __builtin_nontemporal_store(pk, reinterpret_cast<uint4_t*>(dst)); \
+            else *reinterpret_cast<uint4_t*>(dst) = pk; \
           } \
         } \
-      } else { \
-  _Pragma("unroll 8") \
-        for (int it = 0; it < 32 * kRows / 64; ++it) { \
-          const int q = lane + 64 * it; \
-          const int col = q / kRows, m = m_wave + q % kRows, n = n_block + col; \
-          if (n < N && m < M) ((out_t*)p.C)[(size_t)n * M + m] = P::finish(slab[col * kSlabStride + q % kRows], p, m, n); \
+      } else if constexpr (!STREAMED_) { \
+        if (M - m_wave < 48) { \
+          constexpr int kPiecesPerCol = 32 / kOutPerPiece; \
+  _Pragma("unroll") \
+          for (int mb = 0; mb < BLOCKS_; ++mb) { \
+            if (m_wave + 32 * mb >= M) break; \
+  _Pragma("unroll") \
+            for (int it = 0; it < kPiecesPerCol / 2; ++it) { \
+              const int q = lane + 64 * it; \
+              const int col = q / kPiecesPerCol, at = 32 * mb + q % kPiecesPerCol * kOutPerPiece; \
+              const int n = n_block + col, m = m_wave + at; \
+              uint32_t raw[kOutPerPiece]; \
+  _Pragma("unroll") \
+              for (int e = 0; e < kOutPerPiece; e += 4) { \
+                const uint4_t v = *reinterpret_cast<const uint4_t*>(slab + col * kSlabStride + at + e); \
+                raw[e] = v[0]; raw[e + 1] = v[1]; raw[e + 2] = v[2]; raw[e + 3] = v[3]; \
+              } \
+  _Pragma("unroll") \
+              for (int e = 0; e < kOutPerPiece; ++e) \
+                if (n < N && m + e < M) ((out_t*)p.C)[(size_t)n * M + m + e] = P::finish(raw[e], p, m + e, n); \
+            } \
+          } \
+        } else { \
+          constexpr int kBatch = 8; \
+  _Pragma("unroll 1") \
+          for (int it = 0; it < 32 * kRows / 64; it += kBatch) { \
+            uint32_t raw[kBatch]; \
+  _Pragma("unroll") \
+            for (int u = 0; u < kBatch; ++u) { \
+              const int q = lane + 64 * (it + u); \
+              raw[u] = slab[q / kRows * kSlabStride + q % kRows]; \
+            } \
+  _Pragma("unroll") \
+            for (int u = 0; u < kBatch; ++u) { \
+              const int q = lane + 64 * (it + u); \
+              const int m = m_wave + q % kRows, n = n_block + q / kRows; \
+              if (n < N && m < M) ((out_t*)p.C)[(size_t)n * M + m] = P::finish(raw[u], p, m, n); \
+            } \
+          } \
         } \
       } \
       __builtin_amdgcn_wave_barrier(); \
