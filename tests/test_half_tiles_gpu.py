@@ -124,16 +124,24 @@ def test_transposed_rows_off_16_bytes(cuda, M):
 
 
 @pytest.mark.parametrize("fragments", [False, True])
-@pytest.mark.parametrize("M,N,K", [(1300, 4000, 768), (1300, 4000, 512), (1281, 4072, 1280)])  # three stages, two, five
-def test_bitnet(cuda, M, N, K, fragments):
+@pytest.mark.parametrize("M,N,K", [
+    (1300, 4000, 768), (1300, 4000, 512), (1281, 4072, 1280), (1300, 4000, 1536),  # four waves; eight on five stages, on six
+    (1300, 7000, 768), (1300, 6000, 256), (2050, 7690, 512), (2050, 7690, 2304),  # 308, 264, 527 tiles: two workgroups per CU; rounds of four waves; of eight
+])
+def test_bitnet(cuda, M, N, K, fragments, interleaved):
     gen = torch.Generator(device=cuda).manual_seed(K)
     A = _ints(gen, -128, 127, M, K, dtype=torch.int8, device=cuda)
     codes = _ints(gen, 1, 3, N, K // 16, 4, 4, dtype=torch.uint8, device=cuda)  # element e of a word at bit 8 (e % 4) + 2 (e / 4)
-    packed = sum(codes[:, :, j] << (2 * j) for j in range(4)).reshape(N, K // 4).view(torch.int8)
+    if interleaved:
+        packed = sum(codes[:, :, j] << (2 * j) for j in range(4))
+    else:  # code e of a word at bit 2 e
+        packed = sum(codes[:, :, :, j] << (2 * j) for j in range(4))
+    packed = packed.reshape(N, K // 4).view(torch.int8)
     s_a = torch.exp2(_ints(gen, -1, 2, M, dtype=torch.float32, device=cuda))
     B = quantize.prepack_i2_fragments(packed) if fragments else packed
     out = torch.full((M, N), float("nan"), dtype=torch.float16, device=cuda)
-    layout = 1 | (2 if fragments else 0)  # interleaved words, in the operand order or row-major
+@pytest.mark.parametrize("interleaved", [True, False])
+    layout = int(interleaved) | (2 if fragments else 0)
     rc = _lib.get_library().call_gemm_int8xint2(A.data_ptr(), B.data_ptr(), out.data_ptr(), M, N, K, 1, layout, s_a.data_ptr(), 4.0,
                                                 1, torch.cuda.current_stream().cuda_stream)
     assert rc == 0, _lib.last_error()

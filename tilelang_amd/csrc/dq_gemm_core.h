@@ -1234,18 +1234,18 @@ int launch_dma_half(const Params& p, hipStream_t stream) {
 // The tile choice of every policy that can take the direct-to-LDS path: 256 x 256 tiles there when the problem has
 // enough of them, else 128 x 256 tiles there, else the register-staged kernel with the tile size launch_auto picks.
 template <class P>
-int launch_best(const Params& p, hipStream_t stream, int half_tile_min = kHalfTileMin) {
+int launch_best(const Params& p, hipStream_t stream) {
   if (dma_eligible<P>(p)) return launch_dma<P>(p, stream);
-  if (dma_half_eligible<P>(p, half_tile_min)) return launch_dma_half<P>(p, stream);
+  if (dma_half_eligible<P>(p)) return launch_dma_half<P>(p, stream);
   return launch_auto<P>(p, stream);
 }
 
 // ---- K sliced over workgroups, fp32 sums in between --------------------------------------------------
 // A few dozen to a few hundred rows: M x N gives a fraction of the CUs a tile of 128 x 256, and each of them then runs
-// all of K at the rate of its ring (8 to 13 ns per k).  Sliced, the same tiles fill the chip; what it costs is the
-// slices' sums (4 bytes an element and slice, written and read: about 5 TB/s together) and a second kernel (with the
-// pipeline's start and end about 13 us).  MXFP4, N = K = 8192: M = 96 64 -> 29 us, M = 512 93 -> 71 us; N = 4096,
-// K = 14336, M = 128: 117 -> 31 us.
+// all of K at the rate of its ring (7 to 9 ns per k).  Sliced, the same tiles fill the chip; what it costs is the slices'
+// sums (4 bytes an element and slice, written and read: 2.2 TB/s) and a second kernel (with the pipeline's start and end
+// 8 us).  MXFP4, N = K = 8192: M = 96 64 -> 25.5 us, M = 384 90 -> 55.  The sums are added in an order of their own, so
+// the cut form takes the eight waves that the uncut one (kOneOrder) may not.
 // The policy with its accumulators stored as they are: one slice's partial result.
 template <class P>
 struct PartialSums : P {

@@ -30,12 +30,16 @@ namespace {
 // operation as the mask): two instructions per dword instead of three, and the epilogue shifts the sum back by 6.
 // FRAG: B re-ordered offline by prepack_i2_fragments (whole 16-byte pieces move, so the decode is the same); the
 // direct-to-LDS kernel only.
-template <int CONV, class EPI, bool INTERLEAVED, bool TOP = false, bool FRAG = false>
+// K_ORDER (plain words, direct-to-LDS kernel): the decoded weights are transposed instead of A.  For the 128 x 256 tile, whose
+// waves side by side each read every A fragment: 16 byte shuffles a step instead of 32.
+template <int CONV, class EPI, bool INTERLEAVED, bool TOP = false, bool FRAG = false, bool K_ORDER = false>
 struct I2Policy : I8Mfma, gemm::NoScale, EPI {
   static_assert(!TOP || CONV != I2_UNSIGNED, "unsigned codes are masked in place");
+  static_assert(!K_ORDER || !INTERLEAVED, "interleaved words decode into k order");
   // the two-instruction decoder leaves a lone workgroup's waves little to overlap: M = 2477, N = 3920, K = 2560 (320 tiles of
   // 128 x 256) 47 us on 160 tiles of 256 rows, 36.7 so; M = 965, N = 9992, K = 4096 58 -> 49
   static constexpr bool kPairWorkgroups = true;
+  using HalfTile = I2Policy<CONV, EPI, INTERLEAVED, TOP, FRAG, !INTERLEAVED>;
   static constexpr int kBRowBytes = 32;
   static constexpr bool kBFragments = FRAG;
   static constexpr bool kAPacked = false;
@@ -45,9 +49,13 @@ struct I2Policy : I8Mfma, gemm::NoScale, EPI {
   __device__ static __forceinline__ Scale prep_scale(int, const Params&) { return {}; }
   using gemm::NoScale::prep_scale;
   __device__ static __forceinline__ frag_t fix_a(frag_t f) {
-    return INTERLEAVED ? f : __builtin_bit_cast(frag_t, transpose4x4_bytes(__builtin_bit_cast(uint4_t, f)));
+    return INTERLEAVED || K_ORDER ? f : __builtin_bit_cast(frag_t, transpose4x4_bytes(__builtin_bit_cast(uint4_t, f)));
   }
   __device__ static __forceinline__ frag_t decode(const uint32_t* w, int j, const Scale&) {
+    const frag_t o = decode_word(w, j);
+    return K_ORDER ? __builtin_bit_cast(frag_t, transpose4x4_bytes(__builtin_bit_cast(uint4_t, o))) : o;
+  }
+  __device__ static __forceinline__ frag_t decode_word(const uint32_t* w, int j) {
     frag_t o;
     if constexpr (TOP) {
       constexpr uint32_t flip = CONV == I2_OFFSET ? 0x80808080u : 0u;
@@ -78,13 +86,10 @@ int i2_gemm_conv(const Params& p, hipStream_t stream) {
   using Plain = I2Policy<CONV, std::conditional_t<BITNET, BitnetOut, Int32Out<0, false>>, INTERLEAVED, false, FRAG>;
   auto run = [&](auto pol) -> int {
     using Pol = decltype(pol);
-    if constexpr (FRAG) {
-      if (gemm::dma_eligible<Pol>(p)) return gemm::launch_dma<Pol>(p, stream);
-      if (gemm::dma_half_eligible<Pol>(p, kI2HalfTileMin)) return gemm::launch_dma_half<Pol>(p, stream);
-      return 1;
-    } else {
-      return gemm::launch_best<Pol>(p, stream, kI2HalfTileMin);
-    }
+    if (gemm::dma_eligible<Pol>(p)) return gemm::launch_dma<Pol>(p, stream);
+    if (gemm::dma_half_eligible<Pol>(p, kI2HalfTileMin)) return gemm::launch_dma_half<typename Pol::HalfTile>(p, stream);
+    if constexpr (FRAG) return 1;
+    else return gemm::launch_auto<Pol>(p, stream);
   };
   if constexpr (CONV != I2_UNSIGNED) {
     using Top = I2Policy<CONV, std::conditional_t<BITNET, BitnetOutS<6>, Int32Out<6, false>>, INTERLEAVED, true, FRAG>;
