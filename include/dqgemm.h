@@ -153,7 +153,7 @@ int call_dequant_gemm_bf16_mxfp4(const void* A, const void* B, const void* Scale
 /* The same product with a workspace for partial sums (the form of call_dequantize_gemv_w4a16_ws): where M x N gives
  * the CUs too few tiles, K is cut into slices, their fp32 sums go to the workspace and a second kernel adds them in
  * slice order, with the bias, and rounds once.  split: 0 the library's choice (then dq_mxfp4_workspace_bytes(M, N, K)
- * bytes are what it asks for; 0: no slices; DQ_FP4_SIMPLE leaves some of them unused), 1 none, up to 16 that many where
+ * bytes are what it asks for; 0: no slices; DQ_FP4_SIMPLE leaves some of them unused or would take more), 1 none, up to 16 that many where
  * the shape allows it (K % 128 == 0, a slice at least 128 k, M * N a multiple of four, Scale at a multiple of four bytes;
  * else the call is not cut).  A smaller workspace lowers the count.  Workspace: 16-byte aligned, contents undefined afterwards, not to be shared by calls that
  * overlap in time.

@@ -74,6 +74,15 @@ def test_mxfp4_is_not_cut_where_that_is_slower(M, N, K):
     assert _lib.load_library().dq_mxfp4_workspace_bytes(M, N, K) == 0
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (92, 726, 5632), (84, 1024, 7168), (105, 728, 6144), (85, 192, 13568), (100, 128, 15872), (113, 120, 17280),  # register-resident
+    (252, 966, 2048), (240, 1218, 1664),  # rows of sums that are stored by elements
+])
+def test_mxfp4_small_matrices_are_not_cut(M, N, K):
+    """A few row blocks of a small matrix: one round of the uncut kernel, 10 to 60 % ahead of the slices and their sum."""
+    assert _lib.load_library().dq_mxfp4_workspace_bytes(M, N, K) == 0
+
+
 def test_mxfp4_factory_without_a_library(monkeypatch):
     """A kernel object's parameters do not need the built library; its call does, and says so."""
     monkeypatch.setattr(_lib, "_lib", None)

@@ -351,18 +351,20 @@ extern "C" int call_unpack_qzeros(const void* QZeros, void* Zeros, int N, int gr
 }
 
 // Into how many slices of K the tiled MXFP4 GEMM is cut when the caller brought a workspace; 1: not cut.  The times (us)
-// are fits over 131 shapes (81 to 4096 rows, N 2048 to 28672, K 1024 to 14336, odd ones among them) and ten slice counts
-// each, and cut is what they put ahead by a twelfth: the pick takes 1.0 % more than the best count on average, 17 % at most,
-// and no cut call more than uncut (M = 96, N = K = 8192: 64 -> 25.5 us; M = 384, N = K = 8192: 90 -> 55; M = 155, N = 18624,
-// K = 12672, 146 tiles: 149 -> 112).
-// * Cut: 9 us of two launches and a start and an end of the pipeline, 5.5 for every further round of 256 workgroups; a
-//   slice's k at 7.6 ns with 64 workgroups, 9.1 with 208 and 11.5 with all CUs taken (M = 96, N = K = 8192: six slices, 192
-//   workgroups, 26.9 us, eight 30.1), 10.6 per round beyond; and the sums' way through memory at 3.3 TB/s.
-// * Uncut, on tiles of 256 rows where the kernel takes those, else of 128 from 96 of them on.  Below that the register-staged
-//   kernel's tiles of 128 x 64 (beyond 256 of them a second round); at a decode batch the register-resident kernel, which
-//   up to K = 4096 takes 0.7 of its estimate (M = 128, N = 2048: 16.5 us, cut 17.2).
-// * The "simple" format's decoder is longer, and the 128 x 256 tile spills with it: its times are 1.65 of the above there,
-//   1.3 on the other kernels (M = 166, N = 5818, K = 3072: 35.2 us, in four slices 43; e2m1 27.9 and 27.3).
+// are fits over 6178 shapes (81 to 4096 rows, N 64 to 16384, K 1024 to 28672, odd ones among them, the three formats) with
+// every slice count from 1 to 12, and cut is what they put ahead by a twelfth (up to K = 2048, where they are least sure, by a
+// tenth).  The pick takes 0.8 % more than the best count on average in e2m1 and 2.5 in the other two, and no cut call takes
+// 3 % more than uncut but one ("simple", 5 %) (M = 96, N = K = 8192: 64 -> 25.5 us; M = 384, N = K = 8192: 90 -> 55; M = 155,
+// N = 18624, K = 12672, 146 tiles: 149 -> 112).
+// * Cut: 7.9 us of two launches and a start and an end of the pipeline, 4.3 for every further round of 256 workgroups; a
+//   slice's k at 7 ns with few workgroups, 7.4 with 200 and 8.4 with all CUs taken, 9.3 per round beyond; the sums' way
+//   through memory at 2.2 TB/s; and 3.4 us ("simple" 4.6) where rows of sums are no multiple of 16 bytes and are stored by
+//   elements (M = 136, N = 957, K = 1664 in three slices 19.6 us, M = 148, N = 1136 14.0).
+// * Uncut, tiles of 128 x 256 from 96 of them on (so few are never run as tiles of 256 rows).  Below that the register-staged
+//   kernel's tiles of 128 x 64 (beyond 256 of them a second round); at a decode batch the register-resident kernel, at 0.8 of its
+//   estimate, to K = 4096 0.68 (M = 92, N = 726, K = 5632: 11.7 us, in eleven slices 19.2; M = 100, N = 128, K = 15872 16.5 and 22.2).
+// * The "simple" format's decoder is longer where 128 x 256 tiles run uncut: 1.1 of the above (M = 590, N = 4824, K = 5376:
+//   86 us, in two slices 48).
 // * More than one round from 160 tiles on only where the tile count is a multiple of the XCDs: an XCD then walks neighbouring
 //   tiles (M = 384, N = 13824, K = 8192, 162 tiles: 95 us, in three slices 112 when those were slower than they are now).
 // From 192 tiles on nothing is gained (M = 768, N = 8192, K = 14336: 174 us, in four slices 178).
@@ -373,22 +375,22 @@ static int mxfp4_ksplit(int M, int N, int K, int fp4_format) {
   const long tiles = (((long)M + 127) / 128) * (((long)N + 255) / 256);
   if (tiles >= 192) return 1;
   const int units = K / 128;
-  const long tall_tiles = (((long)M + 255) / 256) * (((long)N + 255) / 256);
   const long small_tiles = (((long)M + 127) / 128) * (((long)N + 63) / 64);  // of the register-staged kernel
   // as dq_gemm_core.h counts them: a last round of few workgroups takes two thirds of a full one
   auto rounds = [](long wgs) { return (double)(wgs / 256) + (wgs % 256 ? 0.65 + 0.35 * (double)(wgs % 256) / 256.0 : 0.0); };
   double best;
-  if (tall_tiles >= 96 && 1.85 * rounds(tall_tiles) <= rounds(tiles)) best = 11.3 + 1e-3 * K * 19.6 * rounds(tall_tiles);
-  else if (tiles >= 96) best = 5.1 + 1e-3 * K * (8.65 + 4.5 * (double)tiles / 256.0);
+  if (tiles >= 96) best = 5.1 + 1e-3 * K * (8.65 + 4.5 * (double)tiles / 256.0);
   else best = 2.0 + 1e-3 * K * (tiles <= 32 ? 7.2 : tiles <= 64 ? 8.0 : small_tiles <= 256 ? 7.6 : 9.5);
-  if (M <= 128) best = std::min(best, mxfp4_regres_time(M, N, K) * (K <= 4096 ? 0.7 : 1.0));
-  best *= fp4_format == DQ_FP4_SIMPLE && tiles < 96 ? 0.92 / 1.25 : 0.92;
+  if (M <= 128) best = std::min(best, mxfp4_regres_time(M, N, K) * (K <= 4096 ? 0.68 : 0.8));
+  best *= K <= 2048 ? 0.9 : 0.92;
+  if (fp4_format == DQ_FP4_SIMPLE && tiles >= 96) best *= 1.1;
   int split = 1;
   for (int s = 2; s <= 12 && units / s >= 4; ++s) {
     const long wgs = tiles * s;
     if (wgs > 256 && tiles >= 160 && tiles % 8 != 0) break;
-    const double rate = wgs <= 256 ? 7.0 + 0.01 * (double)wgs + 0.04 * (double)std::max(0L, wgs - 208) : 10.6 * rounds(wgs);
-    const double t = 9.0 + 5.5 * (double)((wgs - 1) / 256) + 1e-3 * rate * 128 * ((units + s - 1) / s) + (double)s * M * N * 4 / 3.3e6;
+    const double rate = wgs <= 256 ? 7.0 + 0.002 * (double)wgs + 0.016 * (double)std::max(0L, wgs - 200) : 9.3 * rounds(wgs);
+    const double t = 7.9 + 4.3 * (double)((wgs - 1) / 256) + 1e-3 * rate * 128 * ((units + s - 1) / s) + (double)s * M * N * 4 / 2.23e6 +
+                     (N % 4 == 0 ? 0.0 : fp4_format == DQ_FP4_SIMPLE ? 4.6 : 3.4);
     if (t < best) best = t, split = s;
   }
   return split;
