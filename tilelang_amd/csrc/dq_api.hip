@@ -592,12 +592,15 @@ extern "C" int call_bitnet_activation_quant(const void* X, void* Q, void* S, int
 // BitLinear's forward in one launch: whether a GEMM kernel quantises the activations itself, in every workgroup.  Against two
 // launches (us): N = K = 4096, row-major words, M = 1 6.7 -> 4.6, M = 4 7.5 -> 6.5, M = 8 8.0 -> 7.3, M = 16 8.4 against 8.5;
 // fragments M = 4 7.2 -> 5.6, M = 8 7.5 -> 6.7; N = K = 8192, M = 8 11.9 -> 11.2; N = 11008, K = 6144, M = 16 10.6 against
-// 11.3; N = 11008, K = 2048, M = 16 7.8 -> 7.1.
+// 11.3; N = 11008, K = 2048, M = 16 7.8 -> 7.1.  Row-major words beyond K = 10240: two rows stay with two launches on matrices
+// of more than 1024 rows (N = 2298, K = 15872 10.6 against 11.5; N = 512, K = 10880 7.7 -> 6.8), three on smaller ones than 2048
+// (N = 800, K = 13312 8.7 against 10.1; N = 10424, K = 11776 20.4 -> 16.5).
 static bool bitlinear_by_gemv(int M, int K, int layout) {
   return (layout & LAYOUT_FRAGMENTS) ? M == 1 && K <= 16384 : M <= 2 && (size_t)M * K <= 32768;
 }
 static bool bitlinear_in_one_kernel(int M, int N, int K, int layout) {
   if (M < 1 || M > 16 || N < 1 || K < 128 || K % 128 != 0) return false;
+  if (!(layout & LAYOUT_FRAGMENTS) && K > 10240 && ((M == 2 && N > 1024) || (M == 3 && N < 2048))) return false;
   if (bitlinear_by_gemv(M, K, layout)) return true;
   if (K % 256 != 0 || (uint64_t)(N + 32) * (uint64_t)(K >> 2) >= (1ull << 32)) return false;
   return K <= (M <= 4 ? 16384 : M <= 8 ? 10240 : 2048);
