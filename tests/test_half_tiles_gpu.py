@@ -22,13 +22,18 @@ def _nibbles(packed):
 
 @pytest.mark.parametrize("zeros", [False, True])
 @pytest.mark.parametrize("M,N,K,group", [
-    (1025, 3076, 384, 64),    # three stages of 128 k, the fewest on eight waves; one row and four columns in the last tiles
-    (1100, 3500, 256, 128),   # two: four waves
-    (1100, 3500, 640, 64),    # five
+    (1025, 3076, 384, 64),    # up to K = 1024 four waves; one row and four columns in the last tiles
+    (1100, 3500, 256, 128),
+    (1100, 3500, 640, 64),
     (1100, 3500, 1024, 128),  # a dword of scales every other stage
+    (1025, 3076, 1152, 64),   # nine stages of 128 k on eight waves, a dword of scales each
+    (1100, 3500, 1280, 128),  # every other
     (1100, 3500, 3072, 512),  # every eighth
-    (1100, 3500, 512, 32),    # one per 64 k: four waves
+    (1100, 3500, 1536, 32),   # one per 64 k: four waves
+    (1100, 3500, 512, 32),
     (897, 4104, 1024, 256),   # rows of C that are no whole lines
+    (897, 4104, 1280, 256),
+    (2600, 6200, 2048, 256), (2600, 6200, 2304, 256),  # more than 512 tiles: four waves to K = 2048, eight beyond
 ])
 def test_uint4(cuda, M, N, K, group, zeros):
     gen = torch.Generator(device=cuda).manual_seed(K + group)
@@ -44,7 +49,7 @@ def test_uint4(cuda, M, N, K, group, zeros):
     assert torch.equal(C, (A.double() @ W.t()).half())
 
 
-@pytest.mark.parametrize("K", [384, 640, 256])
+@pytest.mark.parametrize("K", [384, 640, 256, 1152, 1280])
 def test_fp4(cuda, K):
     M, N = 1100, 3500
     gen = torch.Generator(device=cuda).manual_seed(K)
@@ -79,8 +84,10 @@ def test_mxfp4_rows_keep_their_bits(cuda, M, N, K):
 
 @pytest.mark.parametrize("M,N,K", [
     (1000, 3500, 768),   # 128 x 256; columns of Ct that are no whole lines
-    (1001, 3500, 256),   # and no multiple of 16 bytes: stored by elements; two k-blocks: four waves
-    (1002, 3333, 512),   # 128 x 256 on eight waves
+    (1001, 3500, 256),   # and no multiple of 16 bytes: stored by elements; two k-blocks
+    (1002, 3333, 512),
+    (1002, 3333, 1152),  # 128 x 256 on eight waves
+    (1001, 3500, 1280),
     (1024, 3500, 1024),
     (999, 11008, 512),   # 256 x 256
     (131, 200, 384),     # register-staged

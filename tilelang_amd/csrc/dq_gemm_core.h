@@ -1213,7 +1213,11 @@ struct OneOrder : std::false_type {};
 template <class P>
 struct OneOrder<P, std::void_t<decltype(P::kOneOrder)>> : std::integral_constant<bool, P::kOneOrder> {};
 
-// Eight waves on the two halves of every stage: at least three stages, and no groups of 32 k (a dword of scales per tile)
+// Eight waves on the two halves of every stage: at least three stages, and no groups of 32 k (a dword of scales per tile).  Uncut
+// only where K is long enough for the halves' exchange of sums and the one workgroup per CU, up to 1024 four waves are ahead or
+// even: against four (us), int8 x int4, 97 to 256 tiles, K <= 1024 up to 1.06 times, K > 4096 0.97; fp16 x uint4, K <= 512 1.03,
+// K > 4096 0.87, and beyond 512 tiles, where two workgroups of four waves fill each other's ends of tiles, K <= 1024 1.12 to 1.2,
+// K <= 2048 1.06, K <= 4096 1.0.  (The slices of a cut K, one tile of 512 k and more each, were measured on eight.)
 template <class P>
 bool dma_halves_take(const Params& p) {
   if constexpr (OneOrder<P>::value) return false;
@@ -1222,6 +1226,7 @@ bool dma_halves_take(const Params& p) {
   const int shortest = UnevenSlices<P>::value && p.split > 1 ? p.K / p.kunit / p.split * p.kunit : p.K;
   const int stage_k = P::kKPerBlock * (P::kBRowBytes == 32 ? 2 : 1);
   return shortest % stage_k == 0 && shortest / stage_k >= 3 && !(P::kScaleDma >= 2 && p.p0 == 5);
+  if (p.split == 1 && shortest <= (tiles_of(p, 128) > 512 ? 2048 : 1024)) return false;
 }
 
 template <class P>
