@@ -90,6 +90,9 @@ def test_mxfp4_rows_keep_their_bits(cuda, M, N, K):
     (1001, 3500, 1280),
     (1024, 3500, 1024),
     (999, 11008, 512),   # 256 x 256
+    (2600, 6200, 384),   # 525 tiles of 128 x 256: more than 320 and no multiple of eight are dealt to the XCDs in runs too
+    (3300, 9970, 256),   # 507 of 256 x 256
+    (1100, 2490, 384),   # 351 of 128 x 64, register-staged
     (131, 200, 384),     # register-staged
     (36, 130, 256),
 ])
@@ -130,6 +133,7 @@ def test_transposed_rows_off_16_bytes(cuda, M):
     assert torch.equal(C[:N], (W @ A.double().t()).half()) and bool(torch.isnan(C[N:]).all())
 
 
+@pytest.mark.parametrize("interleaved", [True, False])
 @pytest.mark.parametrize("fragments", [False, True])
 @pytest.mark.parametrize("M,N,K", [
     (1300, 4000, 768), (1300, 4000, 512), (1281, 4072, 1280), (1300, 4000, 1536),  # four waves; eight on five stages, on six
@@ -147,7 +151,6 @@ def test_bitnet(cuda, M, N, K, fragments, interleaved):
     s_a = torch.exp2(_ints(gen, -1, 2, M, dtype=torch.float32, device=cuda))
     B = quantize.prepack_i2_fragments(packed) if fragments else packed
     out = torch.full((M, N), float("nan"), dtype=torch.float16, device=cuda)
-@pytest.mark.parametrize("interleaved", [True, False])
     layout = int(interleaved) | (2 if fragments else 0)
     rc = _lib.get_library().call_gemm_int8xint2(A.data_ptr(), B.data_ptr(), out.data_ptr(), M, N, K, 1, layout, s_a.data_ptr(), 4.0,
                                                 1, torch.cuda.current_stream().cuda_stream)

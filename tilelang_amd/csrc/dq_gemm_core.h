@@ -603,8 +603,8 @@ __device__ __forceinline__ void dma4_unless(int not_due, unsigned lds_addr, unsi
 // four waves, 2 x 2) it was busy 87 % of the time and the matrix pipe 45 %.  So scales come only when their dword is due,
 // a stage brings B in pieces of 64 bytes, and eight waves share one stage (load unit 43 %, matrix pipe 73 %).  fp16 x
 // uint4 with zeros at M = 2048, N = 4096, K = 14336: 260 -> 233 (scales when due, waves side by side) -> 211 us; M = 300,
-// N = 13824, K = 5120: 86 -> 73 -> 60; MXFP4 at M = 768, N = K = 8192: 102 -> 92 -> 83; int8 x 2-bit, M = 1024,
-// N = K = 8192: 58 -> 53.5; int8 x int4, M = 1024, N = K = 8192: 64 -> 59.5.
+// N = 13824, K = 5120: 86 -> 73 -> 60; MXFP4 at M = 768, N = K = 8192, which stays on four waves (kOneOrder): 102 -> 92; int8 x
+// 2-bit, M = 1024, N = K = 8192: 58 -> 53.5; int8 x int4, M = 1024, N = K = 8192: 64 -> 59.5.
 template <class P, int kMBW, int kNBW, int kWavesM = 2, int kKHalves = 1>
 __global__ __launch_bounds__(256 * kKHalves, 32 * kMBW * kWavesM == 128 ? 2 : 1) void gemm_kernel_dma(const Params p_in) {
   Params p = p_in;
@@ -853,6 +853,7 @@ __global__ __launch_bounds__(256 * kKHalves, 32 * kMBW * kWavesM == 128 ? 2 : 1)
     const unsigned char* base = smem + stage * kAStride;
     const unsigned char* bbase = smem + kBRing + (kPairB ? (kb & 3) : stage) * kBSlot;
     constexpr int kIterOps = !kPairB ? kTileOps : (odd ? kAOps : kSOps + kAOps + 2 * kBOps);  // issued per iteration at most
+    static_assert(kIterOps <= (kWavesM == 1 && kMBW == 4 ? 2 * kSteps : 16), "more loads than the iteration has places for");
     {
       using DoMfma = std::integral_constant<bool, !first>;
       auto dma = [&](int chunk) {
@@ -1154,7 +1155,7 @@ template <class P>
 struct PairWorkgroups<P, std::void_t<decltype(P::kPairWorkgroups)>> : std::integral_constant<bool, P::kPairWorkgroups> {};
 
 // 256 x 256 tiles, or 128 x 256.  A round of the first costs 1.85 of the second's (K = 8192: fp16 x uint4 215 and 116 us,
-// MXFP4 180 and 98, int8 x int4 84 and 57), so what decides is how either fills its rounds.  Measured on both, fp16 x uint4
+// MXFP4 180 and 98, int8 x int4 84 and 57), so what decides is how either fills its rounds (up to 128 of the first never).  Measured on both, fp16 x uint4
 // with zeros, K = 4096: M = 700, N = 11008 75 us in tiles of 256 rows, 98 in tiles of 128; M = 1000 92 and 106; M = 600 76
 // and 56; M = 1100, N = 13824 176 and 119; M = 1300, N = 8192 92 and 102; M = 1500, N = 28672 300 and 338.
 template <class P>
@@ -1162,7 +1163,7 @@ bool dma_eligible(const Params& p) {
   // fp16 scales of groups of 32 k go with every tile: not with the pairwise issue of the 32-byte-row form of this tile
   const bool scales_per_tile = P::kScaleDma >= 2 && P::kBRowBytes == 32 && p.p0 == 5;
   const long tiles = tiles_of(p, 256);
-  return !scales_per_tile && tiles >= (PairWorkgroups<P>::value ? 192 : 96) && dma_takes<P>(p) && 1.85 * dma_rounds(tiles) <= dma_rounds(tiles_of(p, 128));
+  return !scales_per_tile && (!PairWorkgroups<P>::value || tiles >= 192) && dma_takes<P>(p) && 1.85 * dma_rounds(tiles) <= dma_rounds(tiles_of(p, 128));
 }
 
 // Too few 256 x 256 tiles but at least `min_tiles` of 128 x 256: the same kernel on the half-height tile, which keeps the
@@ -1225,8 +1226,8 @@ bool dma_halves_take(const Params& p) {
     if (tiles_of(p, 128) > 256 && tiles_of(p, 128) <= 512) return false;
   const int shortest = UnevenSlices<P>::value && p.split > 1 ? p.K / p.kunit / p.split * p.kunit : p.K;
   const int stage_k = P::kKPerBlock * (P::kBRowBytes == 32 ? 2 : 1);
-  return shortest % stage_k == 0 && shortest / stage_k >= 3 && !(P::kScaleDma >= 2 && p.p0 == 5);
   if (p.split == 1 && shortest <= (tiles_of(p, 128) > 512 ? 2048 : 1024)) return false;
+  return shortest % stage_k == 0 && shortest / stage_k >= 3 && !(P::kScaleDma >= 2 && p.p0 == 5);
 }
 
 template <class P>

@@ -319,7 +319,7 @@ int int_gemv(const void* A, const void* B, void* C, int M, int N, int K, Decoder
 constexpr int kFragWaves = 16;
 constexpr int kFragActBytes = 32768;  // staged activations: MROWS * K bytes
 
-// QUANT: as in the kernel above.
+// QUANT: as in the kernel above, one row.
 template <int MROWS, int NP, bool QUANT = false>
 __global__ __launch_bounds__(64 * kFragWaves) void i2_gemv_frag_kernel(const void* __restrict__ A_any, const uint8_t* __restrict__ B,
                                                                        void* __restrict__ C, const float* __restrict__ s_a,
@@ -328,8 +328,9 @@ __global__ __launch_bounds__(64 * kFragWaves) void i2_gemv_frag_kernel(const voi
   __shared__ __align__(16) int8_t act[kFragActBytes];
   __shared__ int red[kFragWaves * 64 * MROWS];
   __shared__ int asum[MROWS];
-  __shared__ float wave_amax[MROWS][kFragWaves];
-  float scale[MROWS];  // QUANT: s_a
+  static_assert(!QUANT || MROWS == 1, "one row of fp16 activations");
+  __shared__ float wave_amax[kFragWaves];
+  float scale = 0.f;  // QUANT: s_a
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -353,26 +354,18 @@ __global__ __launch_bounds__(64 * kFragWaves) void i2_gemv_frag_kernel(const voi
   if (tid < MROWS) asum[tid] = 0;
   __syncthreads();
   const int pieces = K >> 4;  // 16-byte pieces per activation row
-  half8_t x[MROWS][2];  // the thread's piece of every row: K <= 16384 is at most 1024 pieces
+  half8_t x[2];  // the thread's piece: K <= 16384 is at most 1024 pieces
   if constexpr (QUANT) {
     const int q = min(tid, pieces - 1);
 #pragma unroll
-    for (int m = 0; m < MROWS; ++m)
-#pragma unroll
-      for (int i = 0; i < 2; ++i) x[m][i] = *reinterpret_cast<const half8_t*>((const half_t*)A_any + (size_t)min(m, M - 1) * K + q * 16 + i * 8);
-#pragma unroll
-    for (int m = 0; m < MROWS; ++m) {
-      const float amax = wave_max(amax8(x[m][1], amax8(x[m][0], 0.f)));
-      if (lane == 0) wave_amax[m][wave] = amax;
-    }
+    for (int i = 0; i < 2; ++i) x[i] = *reinterpret_cast<const half8_t*>((const half_t*)A_any + q * 16 + i * 8);
+    const float amax_here = wave_max(amax8(x[1], amax8(x[0], 0.f)));
+    if (lane == 0) wave_amax[wave] = amax_here;
     __syncthreads();
+    float amax = 0.f;
 #pragma unroll
-    for (int m = 0; m < MROWS; ++m) {
-      float amax = 0.f;
-#pragma unroll
-      for (int w = 0; w < kFragWaves; ++w) amax = fmaxf(amax, wave_amax[m][w]);
-      scale[m] = act_scale(amax);
-    }
+    for (int w = 0; w < kFragWaves; ++w) amax = fmaxf(amax, wave_amax[w]);
+    scale = act_scale(amax);
   }
 #pragma unroll
   for (int m = 0; m < MROWS; ++m) {
@@ -381,7 +374,7 @@ __global__ __launch_bounds__(64 * kFragWaves) void i2_gemv_frag_kernel(const voi
     for (int q = tid; q < pieces; q += 64 * kFragWaves) {
       uint4_t d;
       if constexpr (QUANT) {
-        const uint2_t lo = quantise8(x[m][0], scale[m]), hi = quantise8(x[m][1], scale[m]);
+        const uint2_t lo = quantise8(x[0], scale), hi = quantise8(x[1], scale);
         d = uint4_t{lo[0], lo[1], hi[0], hi[1]};
       } else {
         d = *reinterpret_cast<const uint4_t*>(ap + q * 16);
@@ -439,14 +432,8 @@ __global__ __launch_bounds__(64 * kFragWaves) void i2_gemv_frag_kernel(const voi
           ((int32_t*)C)[(size_t)m * N + row] = v;
         } else {
           float f = (float)v;
-          if constexpr (QUANT) {
-            float sa = scale[0];
-#pragma unroll
-            for (int k = 1; k < MROWS; ++k) sa = m == k ? scale[k] : sa;
-            f = f / sa;
-          } else {
-            f = f / s_a[m];
-          }
+          if constexpr (QUANT) f = f / scale;
+          else f = f / s_a[m];
           f = f / s_w;
           ((half_t*)C)[(size_t)m * N + row] = (half_t)f;
         }

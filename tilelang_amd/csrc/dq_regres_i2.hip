@@ -665,12 +665,8 @@ int i2_bitlinear_regres(const void* X, const void* B, void* C, int M, int N, int
       default: return 1;  // (six pairs spill)
     }
   }
-  switch (npw) {
-    case 1: DQ_GO(1, 8);
-    case 2: DQ_GO(2, 8);
-    case 3: DQ_GO(3, 8);
-    default: return 1;  // (four pairs spill)
-  }
+  if (npw == 1) DQ_GO(1, 8);
+  return 1;  // (the lines of 16 rows take eight times 4 registers a pair: two launches are the faster ones beyond K = 2048)
 #undef DQ_GO
 }
 
