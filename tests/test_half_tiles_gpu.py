@@ -137,6 +137,7 @@ def test_transposed_rows_off_16_bytes(cuda, M):
 @pytest.mark.parametrize("fragments", [False, True])
 @pytest.mark.parametrize("M,N,K", [
     (1300, 4000, 768), (1300, 4000, 512), (1281, 4072, 1280), (1300, 4000, 1536),  # four waves; eight on five stages, on six
+    (1800, 7000, 1024), (1800, 7000, 1280),  # 224 tiles of 256 rows, 420 of 128: the second to K = 1024, the first beyond
     (1300, 7000, 768), (1300, 6000, 256), (2050, 7690, 512), (2050, 7690, 2304),  # 308, 264, 527 tiles: two workgroups per CU; rounds of four waves; of eight
 ])
 def test_bitnet(cuda, M, N, K, fragments, interleaved):

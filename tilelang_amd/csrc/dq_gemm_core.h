@@ -601,7 +601,7 @@ __device__ __forceinline__ void dma4_unless(int not_due, unsigned lds_addr, unsi
 // What bounds the 128-row form is the CU's load unit, which takes about two cycles per 64 bytes or per row piece, if that
 // is shorter: with a 32-byte piece of B and a dword of scales and of zeros per weight row and k-block (two workgroups of
 // four waves, 2 x 2) it was busy 87 % of the time and the matrix pipe 45 %.  So scales come only when their dword is due,
-// a stage brings B in pieces of 64 bytes, and eight waves share one stage (load unit 43 %, matrix pipe 73 %).  fp16 x
+// a stage brings B in pieces of 64 bytes, and eight waves share one stage (load unit 45 %, matrix pipe 67 %).  fp16 x
 // uint4 with zeros at M = 2048, N = 4096, K = 14336: 260 -> 233 (scales when due, waves side by side) -> 211 us; M = 300,
 // N = 13824, K = 5120: 86 -> 73 -> 60; MXFP4 at M = 768, N = K = 8192, which stays on four waves (kOneOrder): 102 -> 92; int8 x
 // 2-bit, M = 1024, N = K = 8192: 58 -> 53.5; int8 x int4, M = 1024, N = K = 8192: 64 -> 59.5.
@@ -1148,7 +1148,9 @@ inline double dma_rounds(long tiles) {
   return (double)full + (rest ? 0.65 + 0.35 * (double)rest / 256.0 : 0.0);
 }
 
-// P::kPairWorkgroups: 257 to 512 tiles of 128 x 256 run as two workgroups of four waves per CU, not as rounds of eight waves
+// P::kPairWorkgroups: 257 to 512 tiles of 128 x 256 run as two workgroups of four waves per CU, not as rounds of eight waves,
+// and up to K = 1024 also where 192 tiles of 256 rows or more would fill their rounds better: int8 x 2-bit there takes 0.77 of the
+// time (median of 41 shapes; beyond, the tall tile is ahead or even).
 template <class P, class = void>
 struct PairWorkgroups : std::false_type {};
 template <class P>
@@ -1163,7 +1165,8 @@ bool dma_eligible(const Params& p) {
   // fp16 scales of groups of 32 k go with every tile: not with the pairwise issue of the 32-byte-row form of this tile
   const bool scales_per_tile = P::kScaleDma >= 2 && P::kBRowBytes == 32 && p.p0 == 5;
   const long tiles = tiles_of(p, 256);
-  return !scales_per_tile && (!PairWorkgroups<P>::value || tiles >= 192) && dma_takes<P>(p) && 1.85 * dma_rounds(tiles) <= dma_rounds(tiles_of(p, 128));
+  if (PairWorkgroups<P>::value && (tiles < 192 || (p.K <= 1024 && tiles_of(p, 128) <= 512))) return false;
+  return !scales_per_tile && dma_takes<P>(p) && 1.85 * dma_rounds(tiles) <= dma_rounds(tiles_of(p, 128));
 }
 
 // Too few 256 x 256 tiles but at least `min_tiles` of 128 x 256: the same kernel on the half-height tile, which keeps the
