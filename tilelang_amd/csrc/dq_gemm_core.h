@@ -567,7 +567,7 @@ struct BFragments<P, std::void_t<decltype(P::kBFragments)>> : std::integral_cons
 // address, so the XOR swizzle of the A rows is applied by permuting the SOURCE addresses.  These
 // loads are issued from inline assembly and tracked by hand (one s_waitcnt vmcnt per tile): the
 // kernel issues no other vector-memory load inside the main loop, so the counter only ever
-// holds these.  Requires K % 128 == 0 and A, B smaller than 4 GiB (32-bit lane offsets).
+// holds these.  Requires two k-blocks or more, whole ones, and A, B smaller than 4 GiB (32-bit lane offsets).
 //
 // M0 is written inside the statement and is not on its clobber list: clang treats M0 as a reserved register,
 // warns that a reserved register on a clobber list "may not be preserved" and promises nothing for it.  What
@@ -605,7 +605,10 @@ __device__ __forceinline__ void dma4_unless(int not_due, unsigned lds_addr, unsi
 // uint4 with zeros at M = 2048, N = 4096, K = 14336: 260 -> 233 (scales when due, waves side by side) -> 211 us; M = 300,
 // N = 13824, K = 5120: 86 -> 73 -> 60; MXFP4 at M = 768, N = K = 8192, which stays on four waves (kOneOrder): 102 -> 92; int8 x
 // 2-bit, M = 1024, N = K = 8192: 58 -> 53.5; int8 x int4, M = 1024, N = K = 8192: 64 -> 59.5.
-template <class P, int kMBW, int kNBW, int kWavesM = 2, int kKHalves = 1>
+//
+// kOdd: K may be an odd number of k-blocks and a row's scale groups an odd number.  Only policies with a scale byte per 32 k
+// have both kinds (MXFP4, M = 4096, N = K = 8192: 369 us, and 374 in the kind that asks).
+template <class P, int kMBW, int kNBW, int kWavesM = 2, int kKHalves = 1, bool kOdd = P::kScaleDma != 1>
 __global__ __launch_bounds__(256 * kKHalves, 32 * kMBW * kWavesM == 128 ? 2 : 1) void gemm_kernel_dma(const Params p_in) {
   Params p = p_in;
   int bid = blockIdx.x;
@@ -692,26 +695,31 @@ __global__ __launch_bounds__(256 * kKHalves, 32 * kMBW * kWavesM == 128 ? 2 : 1)
   }
   // fp16 scales (kScaleDma >= 2): one per 2^p0 k (p.p0 = 5 .. 12, the policy's dma_ok checks it), so a dword of a row
   // serves 2^s_ps tiles of 64 k.  Groups of 32 k (one tile per dword, the two k halves of a tile in different groups)
-  // need the scales issued with every tile: not the kPairB form, which dma_eligible keeps them away from
-  const int s_gshift = P::kScaleDma >= 2 ? p.p0 : 7;
+  // need the scales issued with every tile: not the kPairB form, which dma_eligible keeps them away from.  The two scale
+  // bytes of a tile (kScaleDma == 1) are two bytes per 64 k, placed as a group of 64 k is
+  const int s_gshift = P::kScaleDma >= 2 ? p.p0 : 6;
   const int s_ps = s_gshift - 5;
-  const unsigned s_voff = (unsigned)min(n0 + (tid & 255), N - 1) * (unsigned)(P::kScaleDma == 1 ? (p.ldk >> 5) : ((p.ldk >> s_gshift) << 1));  // waves 4..7 repeat 0..3
+  // Rows of an odd count of groups: every other row starts in the middle of a dword.  Dword i of such a row holds groups
+  // 2 i - 1 and 2 i; it is asked for one ahead, where dword i - 1 of the rows between them is, so that both kinds of row have
+  // a group by the time that its tile is due, and dword 0 goes before all others to the slot that is needed last.
+  const bool s_odd = kOdd && P::kScaleDma != 0 && ((p.ldk >> s_gshift) & 1) != 0;
+  const int s_ahead = s_odd ? -(lane & 1) : 0;  // rows of a tile start at an even one
+  const unsigned s_row = (unsigned)min(n0 + (tid & 255), N - 1) * ((unsigned)(p.ldk >> s_gshift) << 1);  // waves 4..7 repeat 0..3
+  const unsigned s_voff0 = s_row & ~3u, s_voff = s_voff0 + 4u * (s_row >> 1 & 1);
+  const int s_last = s_odd ? (p.ldk >> s_gshift) >> 1 : -1;  // the dword index from which none is ahead
 
   // One tile = kSOps + kAOps + kBOps DMA instructions per thread: first the scale dword(s) (row tid) if one is due,
   // then the A chunks, then the packed-B chunks.  Two halves: waves 0 .. 3 bring the scales and waves 4 .. 7 the zeros.
   // Two tiles of a stage share its dwords: no groups of 32 k there.
   constexpr int kTileOps = kSOps + kAOps + kBOps;
-  auto issue_op = [&](int op, int kb, int stage, bool first_tile = false) {
+  auto issue_op = [&](int op, int kb, int stage, int b_tile = -1) {
     const unsigned sbase = lds0 + stage * kAStride;
     const unsigned bbase = lds0 + kBRing + (kPairB ? (kb & 3) : stage) * kBSlot;
     if (op < kSOps) {
-      if constexpr (P::kScaleDma == 1) {
-        const int pair = kHalves ? kb : kb >> 1;
-        dma4_unless(kHalves ? kh : (first_tile ? 0 : kb & 1), lds0 + kRing + (pair & 3) * 1024 + (wave & 3) * 256, s_voff, (const unsigned char*)p.S + (size_t)pair * 4);
-      } else if constexpr (P::kScaleDma >= 2) {
+      if constexpr (P::kScaleDma != 0) {
         const int quad = (kb * kStageTiles) >> s_ps;
-        dma4_unless(kHalves && kh != op ? 1 : (first_tile ? 0 : (kb * kStageTiles) & ((1 << s_ps) - 1)),
-                    lds0 + kRing + op * 4096 + (quad & 3) * 1024 + (wave & 3) * 256, s_voff,
+        dma4_unless(kHalves && kh != op ? 1 : (kb * kStageTiles) & ((1 << s_ps) - 1),
+                    lds0 + kRing + op * 4096 + (quad & 3) * 1024 + (wave & 3) * 256, quad == s_last ? s_voff0 : s_voff,
                     (const unsigned char*)(op == 0 ? p.S : p.Z) + (size_t)quad * 4);
       }
     } else if (op < kSOps + kAOps) {
@@ -719,7 +727,14 @@ __global__ __launch_bounds__(256 * kKHalves, 32 * kMBW * kWavesM == 128 ? 2 : 1)
       dma16(sbase + (dma_wave * kAOps + i) * 1024, a_voff[i], (const unsigned char*)p.A + (size_t)kb * (128 * kStageTiles));
     } else {
       const int i = op - kSOps - kAOps;
-      dma16(bbase + (dma_wave * kBOps + i) * 1024, b_voff[i], (const unsigned char*)p.B + (size_t)kb * ((kBFrag ? 1024 : P::kBRowBytes) * kStageTiles));
+      dma16(bbase + (dma_wave * kBOps + i) * 1024, b_voff[i], (const unsigned char*)p.B + (size_t)(b_tile < 0 ? kb : b_tile) * ((kBFrag ? 1024 : P::kBRowBytes) * kStageTiles));
+    }
+  };
+  auto issue_first_scales = [&] {
+    if constexpr (P::kScaleDma != 0) {
+#pragma unroll
+      for (int op = 0; op < kSOps; ++op)
+        dma4_unless(s_odd && !(kHalves && kh != op) ? 0 : 1, lds0 + kRing + op * 4096 + 3 * 1024 + (wave & 3) * 256, s_voff0, op == 0 ? p.S : p.Z);
     }
   };
   // DMA instructions of one tile that may be outstanding while the one before is waited for: the scales come first in a
@@ -761,18 +776,25 @@ __global__ __launch_bounds__(256 * kKHalves, 32 * kMBW * kWavesM == 128 ? 2 : 1)
       bw[4 * h + 0] = v[0]; bw[4 * h + 1] = v[1]; bw[4 * h + 2] = v[2]; bw[4 * h + 3] = v[3];
     }
   };
+  // where the scale of 64-k tile kb lies from s_off on (groups of 32 k: the lane's half of the tile is in s_off)
+  auto scale_at = [&](int kb) -> int {
+    const int group = (kb << 6) >> s_gshift;
+    const int aligned = ((group >> 1) & 3) * 1024 + (group & 1) * 2;
+    if constexpr (!kOdd) return aligned;
+    const int ahead = (((group - 1) >> 1) & 3) * 1024 + ((group + 1) & 1) * 2;
+    return aligned + ((ahead - aligned) & s_ahead);
+  };
   // the LDS read of a scale and the arithmetic on it are separate steps, so that the read can be issued a
   // chunk ahead of its first use
   auto read_scale_byte = [&](int step_kb, int nb) -> int {
     const int kb = step_kb * kStageTiles + (kStageTiles == 2 ? kh : 0);
-    if constexpr (P::kScaleDma == 1) return (smem + s_off[0] + ((kb >> 1) & 3) * 1024 + (kb & 1) * 2)[nb * 128];
+    if constexpr (P::kScaleDma == 1) return (smem + s_off[0] + scale_at(kb))[nb * 128];
     else return 0;
   };
   auto read_scale1 = [&](int step_kb, int nb) -> typename P::Scale {
     const int kb = step_kb * kStageTiles + (kStageTiles == 2 ? kh : 0);  // the 64-k tile
     if constexpr (P::kScaleDma >= 2) {
-      // which of the dword's two groups: with groups of 32 k the lane's half of the tile (in s_off), else the tile's
-      const unsigned char* at = smem + s_off[0] + ((kb >> s_ps) & 3) * 1024 + (s_gshift == 5 ? 0 : (((kb << 6) >> s_gshift) & 1) * 2) + nb * 128;
+      const unsigned char* at = smem + s_off[0] + scale_at(kb) + nb * 128;
       return P::ring_scale(at, at + 4096);
     } else {
       return P::prep_scale(read_scale_byte(kb, nb), p);
@@ -788,9 +810,10 @@ __global__ __launch_bounds__(256 * kKHalves, 32 * kMBW * kWavesM == 128 ? 2 : 1)
       for (int i = 0; i < 16; ++i) acc[mb][nb][i] = 0;
 
   // ---- prologue: tiles 0 and 1 (and their scales) in flight; only tile 0 has to have landed -------
+  issue_first_scales();
   if constexpr (kPairB) {  // scales, A of tile 0, the B pairs of tiles 0 and 1, then A of tile 1
 #pragma unroll
-    for (int op = 0; op < kSOps + kAOps; ++op) issue_op(op, 0, 0, true);
+    for (int op = 0; op < kSOps + kAOps; ++op) issue_op(op, 0, 0);
 #pragma unroll
     for (int i = 0; i < kBOps; ++i) {
       issue_op(kSOps + kAOps + i, 0, 0);
@@ -801,9 +824,9 @@ __global__ __launch_bounds__(256 * kKHalves, 32 * kMBW * kWavesM == 128 ? 2 : 1)
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kAOps) : "memory");
   } else {
 #pragma unroll
-    for (int op = 0; op < kTileOps; ++op) issue_op(op, 0, 0, true);
+    for (int op = 0; op < kTileOps; ++op) issue_op(op, 0, 0);
 #pragma unroll
-    for (int op = 0; op < kTileOps; ++op) issue_op(op, 1, 1);  // KB >= 2 because K % 128 == 0
+    for (int op = 0; op < kTileOps; ++op) issue_op(op, 1, 1);  // KB >= 2
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kWaitOps) : "memory");
   }
   __syncthreads();
@@ -865,7 +888,8 @@ __global__ __launch_bounds__(256 * kKHalves, 32 * kMBW * kWavesM == 128 ? 2 : 1)
           if (has_next2 && chunk < kSOps + kAOps) issue_op(chunk, kb + 2, stage2);
           else if (has_next2 && chunk < kIterOps) {
             const int j = chunk - kSOps - kAOps;  // B instruction j / 2 of tile kb + 2 + j % 2
-            issue_op(kSOps + kAOps + (j >> 1), kb + 2 + (j & 1), stage2);
+            // (an odd count of tiles: the last pair's second half is asked for in the first one's place and never read)
+            issue_op(kSOps + kAOps + (j >> 1), kb + 2 + (j & 1), stage2, kOdd ? min(kb + 2 + (j & 1), KB - 1) : -1);
           }
         }
       };
@@ -1006,7 +1030,7 @@ __global__ __launch_bounds__(256 * kKHalves, 32 * kMBW * kWavesM == 128 ? 2 : 1)
     __syncthreads();
   };
 
-  // KB is even (K % (2 kKPerBlock) == 0): tiles come in (even, odd) pairs
+  // tiles come in (even, odd) pairs, an odd count ends with an even one
   using T = std::true_type;
   using F = std::false_type;
   int stage = 0;
@@ -1031,11 +1055,19 @@ __global__ __launch_bounds__(256 * kKHalves, 32 * kMBW * kWavesM == 128 ? 2 : 1)
       iteration(kb + 1, stage, F{}, T{}, F{});
       next_stage();
     }
-    iteration(kb, stage, F{}, T{}, T{});  // kb = KB - 3
-    next_stage();
-    iteration(kb + 1, stage, F{}, F{}, F{});
-    next_stage();
-    iteration(kb + 2, stage, F{}, F{}, T{});
+    const bool odd_count = kOdd && (KB & 1) != 0;
+    if (!odd_count) {
+      iteration(kb, stage, F{}, T{}, T{});  // kb = KB - 3
+      next_stage();
+      iteration(++kb, stage, F{}, F{}, F{});
+      next_stage();
+      ++kb;
+    }
+    iteration(kb, stage, F{}, F{}, T{});
+    if (odd_count) {
+      next_stage();
+      iteration(kb + 1, stage, F{}, F{}, F{});
+    }
   } else {  // KB == 2
     iteration(0, 0, T{}, F{}, F{});
     iteration(1, 1, F{}, F{}, T{});
@@ -1135,7 +1167,7 @@ bool dma_takes(const Params& p) {
   // 32-bit lane offsets: A rows are 128 bytes per K block, packed B rows kBRowBytes
   const size_t a_bytes = (size_t)p.M * (p.ldk / P::kKPerBlock) * kARowBytes;
   const size_t b_bytes = (size_t)p.N * (p.ldk / P::kKPerBlock) * P::kBRowBytes;
-  return P::dma_ok(p) && (p.K % (2 * P::kKPerBlock) == 0) && a_bytes < (1ull << 32) && b_bytes < (1ull << 32);
+  return P::dma_ok(p) && p.K % P::kKPerBlock == 0 && p.K >= 2 * P::kKPerBlock && a_bytes < (1ull << 32) && b_bytes < (1ull << 32);
 }
 
 inline long tiles_of(const Params& p, int rows) { return (long)((p.M + rows - 1) / rows) * ((p.N + BN - 1) / BN) * p.split; }
@@ -1179,8 +1211,10 @@ bool dma_half_eligible(const Params& p, int min_tiles = kHalfTileMin) {
   return !dma_eligible<P>(p) && dma_takes<P>(p) && tiles_of(p, 128) >= min_tiles;
 }
 
-template <class P, int kMBW, int kNBW, int kWavesM = 2, int kKHalves = 1>
+template <class P, int kMBW, int kNBW, int kWavesM = 2, int kKHalves = 1, bool kOdd = P::kScaleDma != 1>
 int launch_dma_tile(Params p, hipStream_t stream) {
+  if constexpr (!kOdd && kKHalves == 1)
+    if (p.ldk / P::kKPerBlock % 2 != 0) return launch_dma_tile<P, kMBW, kNBW, kWavesM, kKHalves, true>(p, stream);
   constexpr int kWaves = 4;
   constexpr int kTileM = 32 * kMBW * kWavesM;
   constexpr bool kPairB = P::kBRowBytes == 32 && kTileM == 256;  // as in the kernel: a fourth B slot
@@ -1191,7 +1225,7 @@ int launch_dma_tile(Params p, hipStream_t stream) {
   p.tiles_m = (p.M + kTileM - 1) / kTileM;
   p.tiles_n = (p.N + BN - 1) / BN;
   static_assert(kLds <= 160 * 1024, "LDS budget");
-  auto kern = gemm_kernel_dma<P, kMBW, kNBW, kWavesM, kKHalves>;
+  auto kern = gemm_kernel_dma<P, kMBW, kNBW, kWavesM, kKHalves, kOdd>;
   static bool lds_limit_raised[kMaxDevices];
   if (raise_lds_limit<kLds>(kern, lds_limit_raised)) return -1;
   hipLaunchKernelGGL(kern, dim3(p.tiles_m * p.tiles_n * p.split), dim3(64 * kWaves * kKHalves), kLds, stream, p);

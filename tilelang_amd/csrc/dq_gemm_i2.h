@@ -86,6 +86,8 @@ int i2_gemm_conv(const Params& p, hipStream_t stream) {
   using Plain = I2Policy<CONV, std::conditional_t<BITNET, BitnetOut, Int32Out<0, false>>, INTERLEAVED, false, FRAG>;
   auto run = [&](auto pol) -> int {
     using Pol = decltype(pol);
+    if constexpr (FRAG)
+      if (p.K % 256 != 0) return 1;  // a fragment-ordered matrix has whole pairs of k-blocks
     if (gemm::dma_eligible<Pol>(p)) return gemm::launch_dma<Pol>(p, stream);
     if (gemm::dma_half_eligible<Pol>(p, kI2HalfTileMin)) return gemm::launch_dma_half<typename Pol::HalfTile>(p, stream);
     if constexpr (FRAG) return 1;
