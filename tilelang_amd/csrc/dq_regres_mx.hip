@@ -23,8 +23,10 @@
 //     a block meet in LDS in fp32 (two buffers, one barrier per block) and 64 threads add them in slice order (the
 //     same order every run), add the bias, round to bf16 and store.
 //
-// K beyond 8192 (K % 128 == 0): slices of at most 6144 k, the kernel's body once per slice with a prologue of its own,
-// the running fp32 sums of the workgroup's blocks kept in LDS between slices (N <= 65536).
+// K beyond 8192 (beyond 6144 with a half chunk, whose lane-dependent addresses leave no registers for eight chunks per wave):
+// slices of at most 6144 k, the kernel's body once per slice with a prologue of its own, the running fp32 sums of the
+// workgroup's blocks kept in LDS between slices (N <= 65536).  Half chunks there, against the tiled kernel: M = 8, N = 4048,
+// K = 9792 73 -> 16.3 us, M = 14, N = 2168, K = 13760 102 -> 22.3; one row (the dot-product kernel), N = 10720, K = 9152 91 -> 16.2.
 //
 // Every load is unconditional and the last blocks have their own copies of the code, so that the compiler's count of
 // loads in flight is exact (see dq_regres_i2.hip).  A wave whose run is shorter than the longest loads its last chunk
@@ -700,9 +702,12 @@ int launch_mx_gemv_long(const void* A, const void* B, const void* S, const void*
 // prologue (2 us + 2.5 us per 8192 k, once per slice of K) and 0.3 us + 2.8 us per 8192 k for every block of 16
 // weight rows it visits (measured at K = 8192: N = 8192 at 16 / 32 / 48 rows 13 / 24 / 35 us, N = 28672 at 16 rows
 // 26.6 us; N = K = 2880, where the passes share a round, 16 / 32 / 64 / 128 rows 6.7 / 11 / 16 / 29 us against 24.6 us).
+// A half chunk at the end of K leaves no registers for more than six chunks per wave, whatever K.
+static bool mxfp4_k_in_slices(int K) { return K > kWaves * (K % 128 != 0 ? 6 : kMaxChunks) * 128; }
+
 double mxfp4_regres_time(int M, int N, int K) {
   const double kfrac = (double)K / 8192.0;
-  const int nslices = K > kWaves * kMaxChunks * 128 ? ((K >> 7) + kWaves * 6 - 1) / (kWaves * 6) : 1;
+  const int nslices = mxfp4_k_in_slices(K) ? (((K + 127) >> 7) + kWaves * 6 - 1) / (kWaves * 6) : 1;
   const long grid = (N + 15) / 16 < 256 ? (N + 15) / 16 : 256, blocks_each = ((N + 15) / 16 + grid - 1) / grid;
   const long rounds = (grid * ((M + 15) / 16) + 255) / 256;
   return 2.0 + 1.1 * (double)rounds * (2.0 * nslices + 2.5 * kfrac + (double)blocks_each * (0.3 * nslices + 2.8 * kfrac));
@@ -713,8 +718,8 @@ double mxfp4_regres_time(int M, int N, int K) {
 int mxfp4_gemm_regres(const void* A, const void* B, const void* S, const void* Bias, void* C, int M, int N, int K, int fmt,
                       int scale_bias, int max_rows, hipStream_t stream) {
   // 128-k chunks (the last one may be half: K % 128 == 64), at most eight per wave
-  const bool longk = K > kWaves * kMaxChunks * 128;
-  if (M < 1 || M > max_rows || K % 64 != 0 || (longk && K % 128 != 0)) return 1;
+  const bool longk = mxfp4_k_in_slices(K);
+  if (M < 1 || M > max_rows || K % 64 != 0) return 1;
   if (M > 16) {
     const double t_tiled = (N > 16384 ? 92.0 : 60.0) * ((double)K / 8192.0) + 3.0;
     if (mxfp4_regres_time(M, N, K) > 0.9 * t_tiled) return 1;
@@ -794,7 +799,6 @@ int mxfp4_gemm_regres(const void* A, const void* B, const void* S, const void* B
   // chunks per wave: the longest run (with lines, whole pairs)
   const int nchunk = (K + 127) >> 7;
   const int ncw = lines ? 2 * ((nchunk / 2 + kWaves - 1) / kWaves) : (nchunk + kWaves - 1) / kWaves;
-  if (half && ncw > 6) return 1;  // the half chunk's form with eight chunks per wave does not fit the registers
 #define DQ_MXR(FMT_, NCW_, LINES_, HALF_, LONGK_)                                                                            \
   do {                                                                                                                       \
     if (Bias) return launch_mx_regres<FMT_, true, NCW_, LINES_, HALF_, LONGK_>(A, B, S, Bias, C, M, N, K, exp_off, stream); \
@@ -804,6 +808,7 @@ int mxfp4_gemm_regres(const void* A, const void* B, const void* S, const void* B
   do {                                                                                                         \
     if (longk) { /* slices of at most 6144 k: six chunks per wave leave the registers the slice loop needs */ \
       if (lines) DQ_MXR(FMT_, 6, 1, false, true);                                                              \
+      if (half) DQ_MXR(FMT_, 6, 0, true, true);                                                                \
       DQ_MXR(FMT_, 6, 0, false, true);                                                                         \
     }                                                                                                          \
     if (lines == 2 && ncw == 4) DQ_MXR(FMT_, 4, 2, false, false);                                              \
