@@ -48,7 +48,14 @@ int fp16_fp4_gemm(const void* A, const void* B, void* C, int M, int N, int K, in
 int w4_f16_gemm(const void* A, const void* B, const void* S, const void* Z, void* C, int M, int N, int K, int group,
                 int mode, int layout, hipStream_t stream);
 int i2_gemm(const void* A, const void* B, void* C, int M, int N, int K, int convention, int layout, const void* s_a,
-            float s_w, int bitnet_epilogue, hipStream_t stream);
+            float s_w, int bitnet_epilogue, int kwaves, hipStream_t stream);
+int i2_kwaves_form(int M, int N, int K);
+double mxfp4_kwaves_time(int M, int N, int K);
+int mxfp4_gemm_kwaves(const void* A, const void* B, const void* S, const void* Bias, void* C, int M, int N, int K, int fmt,
+                      int scale_bias, hipStream_t stream);
+double w4_kwaves_time(int M, int N, int K);
+int w4_f16_gemm_kwaves(const void* A, const void* B, const void* S, const void* Z, void* C, int M, int N, int K, int group,
+                       int mode, int layout, hipStream_t stream);
 int wlow_gemv(const void* A, const void* B, const void* Scale, const void* Zeros, void* C, int M, int N, int K, int group,
               int bits, int convention, int layout, int zeros_rescale, hipStream_t stream);
 int i2_gemm_kslice(const void* A, const void* B, void* C, int M, int N, int K, int convention, int layout, const void* s_a,
@@ -68,7 +75,7 @@ int fp16_fp4_gemm_splitk(const void* A, const void* B, void* parts, void* C, int
 int mxfp4_mxfp4_gemm(const void* A, const void* SA, const void* B, const void* SB, const void* Bias, void* C, int M,
                      int N, int K, hipStream_t stream);
 int i4_gemm(const void* A, const void* B, void* C, int M, int N, int K, int decode, int a_packed, int transposed,
-            hipStream_t stream);
+            int tiled, hipStream_t stream);
 
 int unpack_qzeros(const void* QZ, void* Z, int N, int groups, int packed, hipStream_t stream);
 int mfma_rate(const void* operands, void* out, int dtype, int workgroups, int iters, hipStream_t stream);
@@ -199,6 +206,16 @@ extern "C" size_t dq_w4a16_workspace_bytes(int M, int N, int K, int group, int m
   return split > 1 ? (size_t)split * M * N * sizeof(float) : 0;
 }
 
+// K that is no multiple of 256: neither the register-resident nor the streaming kernel takes it, and from three rows on K over
+// the waves of a workgroup is ahead of the general ones (M = 8, N = 23848, K = 3968, group 64: 37 -> 21 us; M = 24, N = 6712,
+// K = 11904 84 -> 22; M = 88, N = 7952, K = 3712 42 -> 19), beyond 64 rows while the tiled GEMM's big tiles are few (its small
+// ones take some 10 us a thousand k).
+static bool w4a16_by_kwaves(int M, int N, int K) {
+  if (M < 3 || K % 256 == 0) return false;
+  if (M <= 64) return true;
+  return (((long)M + 127) / 128) * (((long)N + 255) / 256) < 96 && w4_kwaves_time(M, N, K) < 2.0 + 9.0e-3 * K;
+}
+
 static int gemv_w4a16(const char* fn, const void* A, const void* B, const void* Scale, const void* Zeros, void* C, int M, int N,
                       int K, int group, int mode, int layout, int variant, void* workspace, size_t workspace_bytes,
                       dq_stream_t stream) {
@@ -222,6 +239,10 @@ static int gemv_w4a16(const char* fn, const void* A, const void* B, const void* 
       DQ_FAIL("%s: fragment-ordered weights are read at M <= 16, N %% 16 == 0, K = 2048 / 4096 / 8192, group 128 and every mode "
               "but \"rescale\" only (got M=%d N=%d K=%d group=%d mode=%d)", fn, M, N, K, group, mode);
     return rc;
+  }
+  if (variant == -1 && w4a16_by_kwaves(M, N, K)) {
+    const int rc = w4_f16_gemm_kwaves(A, B, Scale, Zeros, C, M, N, K, group, asked_mode, layout, (hipStream_t)stream);
+    if (rc <= 0) return rc;
   }
   // prefill-sized M: the tiled MFMA GEMM (same tile-exact decoders); up to 128 rows, and beyond that against a
   // matrix of few tiles, the streaming kernel below (passes of 64 rows over the weights) is still the faster one.
@@ -396,6 +417,19 @@ static int mxfp4_ksplit(int M, int N, int K, int fp4_format) {
   return split;
 }
 
+// K over the waves of a workgroup: from 17 to 64 rows always (31 shapes: 0.98 to 3.6 times as fast as the register-resident
+// kernel's passes or the tiled GEMM; M = 64, N = K = 8192 49 -> 20 us, M = 60, N = 2976, K = 4352 21 -> 9), below where it is a
+// fifth ahead of the register-resident kernel's estimate (M = 14, N = 2168, K = 13760 22 -> 14; two rows stay with dot
+// products).  From 65 rows on with K % 128 == 0 a row keeps the bits that it has in a large product, or K is cut; otherwise,
+// and while the tiles of 128 x 256 are few, against the 7.5 us a thousand k of the register-staged kernel (M = 101, N = 4336,
+// K = 4800 39 -> 17 us, M = 254, N = 2176, K = 6336 53 -> 22, M = 282, N = 4024, K = 9408 82 -> 47).
+static bool mxfp4_by_kwaves(int M, int N, int K) {
+  if (M < 3) return false;
+  if (M > 64)
+    return K % 128 != 0 && (((long)M + 127) / 128) * (((long)N + 255) / 256) < 96 && mxfp4_kwaves_time(M, N, K) < 0.95 * (2.0 + 7.5e-3 * K);
+  return M > 16 || mxfp4_kwaves_time(M, N, K) < 0.8 * mxfp4_regres_time(M, N, K);
+}
+
 static int gemm_bf16_mxfp4(const char* fn, const void* A, const void* B, const void* Scale, const void* Bias, void* C, int M, int N,
                            int K, int scale_size, int fp4_format, int scale_bias, int split, void* workspace,
                            size_t workspace_bytes, dq_stream_t stream) {
@@ -410,6 +444,10 @@ static int gemm_bf16_mxfp4(const char* fn, const void* A, const void* B, const v
   if (scale_bias < 0 || scale_bias > 255) DQ_FAIL("%s: scale_bias must be in 0..255 (got %d)", fn, scale_bias);
   if (!aligned16(A) || !aligned16(B) || !aligned16(C) || (Bias && !aligned16(Bias)))
     DQ_FAIL("%s: A, B, Bias and C must be 16-byte aligned", fn);
+  if (split <= 1 && mxfp4_by_kwaves(M, N, K)) {
+    const int rc = mxfp4_gemm_kwaves(A, B, Scale, Bias, C, M, N, K, fp4_format, scale_bias, (hipStream_t)stream);
+    if (rc <= 0) return rc;
+  }
   if (workspace && split == 0) split = mxfp4_ksplit(M, N, K, fp4_format);
   while (split > 1 && (size_t)split * M * N * sizeof(float) > workspace_bytes) --split;
   if (split > 1) {
@@ -544,6 +582,11 @@ extern "C" int call_gemm_int8xint2(const void* A, const void* B, void* C, int M,
     if (rc > 0) DQ_FAIL("%s: the register-resident kernel needs M <= 32 (on matrices of few rows M <= 128) and K %% 256 == 0 (got M=%d N=%d K=%d)", fn, M, N, K);
     return rc;
   }
+  const int kwaves = kernel_choice || frag ? -1 : i2_kwaves_form(M, N, K);
+  if (kwaves >= 0) {
+    const int rc = i2_gemm(A, B, C, M, N, K, convention, layout, s_a, s_w, out_kind, kwaves, (hipStream_t)stream);
+    if (rc <= 0) return rc;
+  }
   // 4 to 32 rows: activations resident in registers, weights streamed once (at 4 rows ahead of the dot-product kernel
   // on fragment-ordered weights, N = 28672, K = 8192: 14.8 against 25.2 us, and on row-major ones from about 6000
   // weight rows on: N = 11008, K = 4096 7.3 against 8.7 us, N = 3072, K = 8192 8.6 against 7.1)
@@ -564,7 +607,7 @@ extern "C" int call_gemm_int8xint2(const void* A, const void* B, void* C, int M,
     const int rc = i2_gemm_kslice(A, B, C, M, N, K, convention, layout, s_a, s_w, out_kind, 0, (hipStream_t)stream);
     if (rc <= 0) return rc;
   }
-  const int rc = i2_gemm(A, B, C, M, N, K, convention, layout, s_a, s_w, out_kind, (hipStream_t)stream);
+  const int rc = i2_gemm(A, B, C, M, N, K, convention, layout, s_a, s_w, out_kind, -1, (hipStream_t)stream);
   if (rc <= 0 || !frag) return rc;
   // Fragment-ordered weights are read by the decode kernel, the K-sliced kernel and the direct-to-LDS tiled kernel;
   // a shape the tiled one does not take (too few tiles) goes to the K-sliced kernel whatever its size.
@@ -700,7 +743,8 @@ extern "C" int call_gemm_int8xint4(const void* A, const void* B, void* C, int M,
     const int rc = i4_gemv(A, B, C, M, N, K, decode, (hipStream_t)stream);
     if (rc <= 0) return rc;
   }
-  return i4_gemm(A, B, C, M, N, K, decode, a_packed, transposed & 1, (hipStream_t)stream);
+  return i4_gemm(A, B, C, M, N, K, decode, a_packed, transposed & 1,
+                 variant_bits(transposed) & DQ_I4_KERNEL_TILED, (hipStream_t)stream);
 }
 
 extern "C" int call_gemv_int8xint1(const void* A, const void* B, void* C, int M, int N, int K, int convention, int layout,

@@ -68,6 +68,7 @@ struct Params {
   int tiles_m, tiles_n;
   int p0, p1;        // policy specific integers (e.g. scale exponent offset, group shift)
   float f0;          // policy specific float (e.g. 1 / weight scale)
+  int kwaves;        // host only: the form of dq_gemm_kwaves.h that the call goes to, or -1
 };
 
 // Workgroup id -> output tile.  With T tiles and 8 XCDs, XCD x (ids x, x+8, ...) gets a
@@ -1342,6 +1343,7 @@ inline Params make_params(const void* A, const void* B, const void* S, const voi
   p.M = M; p.N = N; p.K = K;
   p.ldk = K;
   p.split = 1;
+  p.kwaves = -1;
   p.tiles_m = (M + BM - 1) / BM;
   p.tiles_n = (N + BN - 1) / BN;
   return p;

@@ -1,7 +1,7 @@
 // 16-bit operand policies of the LDS-staged dequantize GEMM (dq_gemm_core.h): MXFP4 x bf16, fp4 x bf16 and
 // "simple" fp4 x fp16 (uint4 x fp16: dq_gemm_w4.hip).
 #include "dq_fp4_codes.h"
-#include "dq_gemm_core.h"
+#include "dq_gemm_kwaves.h"
 
 namespace dq {
 
@@ -115,6 +115,30 @@ int mxfp4_gemm(const void* A, const void* B, const void* S, const void* Bias, vo
   do {                                                                     \
     if (Bias) return gemm::launch_best<MxPolicy<FMT_, true>>(p, stream);   \
     return gemm::launch_best<MxPolicy<FMT_, false>>(p, stream);            \
+  } while (0)
+  switch (fmt) {
+    case FP4_E2M1: DQ_MX(FP4_E2M1);
+    case FP4_SIMPLE: DQ_MX(FP4_SIMPLE);
+    case FP4_TWIDDLING: DQ_MX(FP4_TWIDDLING);
+    default: DQ_FAIL("mxfp4 gemm: unknown weight format %d", fmt);
+  }
+#undef DQ_MX
+}
+
+// K over the waves of a workgroup: what it would take (us), and the launch (1: not a shape of that kernel).  Times of e2m1.
+static constexpr gemm::KwavesCosts kKwavesMx = {{2.2, 0.97, 0.88, false}, {2.65, 0.77, 1.03, false}, {3.37, 0.47, 1.67, false},
+                                                {3.11, 1.54, 2.34, true}, {3.15, 2.07, 2.44, true}};
+double mxfp4_kwaves_time(int M, int N, int K) { return gemm::kwaves_pick(kKwavesMx, M, N, K).us; }
+int mxfp4_gemm_kwaves(const void* A, const void* B, const void* S, const void* Bias, void* C, int M, int N, int K, int fmt,
+                      int scale_bias, hipStream_t stream) {
+  Params p = gemm::make_params(A, B, S, nullptr, Bias, C, M, N, K);
+  p.p0 = 127 - scale_bias;
+  const int form = gemm::kwaves_pick(kKwavesMx, M, N, K).form;
+#define DQ_MX(FMT_)                                                                                \
+  do {                                                                                             \
+    if (!gemm::kwaves_takes<MxPolicy<FMT_, false>>(p)) return 1;                                   \
+    if (Bias) return gemm::launch_kwaves<MxPolicy<FMT_, true>>(p, form, stream);                   \
+    return gemm::launch_kwaves<MxPolicy<FMT_, false>>(p, form, stream);                            \
   } while (0)
   switch (fmt) {
     case FP4_E2M1: DQ_MX(FP4_E2M1);

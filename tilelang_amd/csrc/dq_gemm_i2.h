@@ -4,6 +4,7 @@
 #pragma once
 
 #include "dq_gemm_i8.h"
+#include "dq_gemm_kwaves.h"
 
 namespace dq {
 
@@ -84,6 +85,14 @@ constexpr int kI2HalfTileMin = 160;
 template <int CONV, bool INTERLEAVED, bool BITNET, bool FRAG>
 int i2_gemm_conv(const Params& p, hipStream_t stream) {
   using Plain = I2Policy<CONV, std::conditional_t<BITNET, BitnetOut, Int32Out<0, false>>, INTERLEAVED, false, FRAG>;
+  if constexpr (!FRAG) {
+    if (p.kwaves >= 0) {
+      using Waves = I2Policy<CONV, std::conditional_t<BITNET, BitnetOutS<CONV == I2_UNSIGNED ? 0 : 6>, Int32Out<CONV == I2_UNSIGNED ? 0 : 6, false>>,
+                             INTERLEAVED, CONV != I2_UNSIGNED, false>;
+      if (p.K >= 131072 || !gemm::kwaves_takes<Waves>(p)) return 1;
+      return gemm::launch_kwaves<Waves>(p, p.kwaves, stream);
+    }
+  }
   auto run = [&](auto pol) -> int {
     using Pol = decltype(pol);
     if constexpr (FRAG)
