@@ -610,14 +610,14 @@ __device__ __forceinline__ void dma4_unless(int not_due, unsigned lds_addr, unsi
 // kOdd: K may be an odd number of k-blocks and a row's scale groups an odd number.  Only policies with a scale byte per 32 k
 // have both kinds (MXFP4, M = 4096, N = K = 8192: 369 us, and 374 in the kind that asks).
 template <class P, int kMBW, int kNBW, int kWavesM = 2, int kKHalves = 1, bool kOdd = P::kScaleDma != 1>
-__global__ __launch_bounds__(256 * kKHalves, 32 * kMBW * kWavesM == 128 ? 2 : 1) void gemm_kernel_dma(const Params p_in) {
+__global__ __launch_bounds__(256 * kKHalves, 32 * kMBW * kWavesM <= 128 ? 2 : 1) void gemm_kernel_dma(const Params p_in) {
   Params p = p_in;
   int bid = blockIdx.x;
   take_k_slice<P>(p, bid);
   extern __shared__ __align__(16) unsigned char smem[];
   static_assert(P::kBRowBytes == 32 || P::kBRowBytes == 64, "direct-to-LDS variant: 32 or 64 packed bytes per weight row per tile");
-  static_assert(kWavesM == 2 ? (kMBW == 4 && kNBW == 4) : (kWavesM == 1 && (kMBW == 8 || kMBW == 4) && kNBW == 2), "one of the three forms");
-  static_assert(kKHalves == 1 || (kKHalves == 2 && kWavesM == 1 && kMBW == 4), "two halves of a stage: the 128-row form");
+  static_assert(kWavesM == 2 ? (kMBW == 4 && kNBW == 4) : (kWavesM == 1 && (kMBW <= 4 || kMBW == 6 || kMBW == 8) && kNBW == 2), "one of the forms");
+  static_assert(kKHalves == 1 || (kKHalves == 2 && kWavesM == 1 && kMBW <= 4), "two halves of a stage: 128 rows at most");
   constexpr int kWavesN = 8 / kNBW;            // waves across the 256 tile columns
   constexpr int kWaves = 4;                    // of one half
   constexpr int BM = 32 * kMBW * kWavesM;      // shadows the 256-row default
@@ -877,7 +877,10 @@ __global__ __launch_bounds__(256 * kKHalves, 32 * kMBW * kWavesM == 128 ? 2 : 1)
     const unsigned char* base = smem + stage * kAStride;
     const unsigned char* bbase = smem + kBRing + (kPairB ? (kb & 3) : stage) * kBSlot;
     constexpr int kIterOps = !kPairB ? kTileOps : (odd ? kAOps : kSOps + kAOps + 2 * kBOps);  // issued per iteration at most
-    static_assert(kIterOps <= (kWavesM == 1 && kMBW == 4 ? 2 * kSteps : 16), "more loads than the iteration has places for");
+    // waves side by side: a step is one scheduling region of at most eight matrix instructions, or two
+    constexpr int kRegions = kMBW > 4 ? 2 : 1, kRegionRows = kMBW / kRegions;
+    constexpr int kPlaces = kWavesM == 2 ? 1 : (kIterOps <= 2 * kSteps * kRegions ? 2 : 3);  // for loads, in a region
+    static_assert(kIterOps <= (kWavesM == 2 ? 16 : kPlaces * kSteps * kRegions), "more loads than the iteration has places for");
     {
       using DoMfma = std::integral_constant<bool, !first>;
       auto dma = [&](int chunk) {
@@ -905,59 +908,59 @@ __global__ __launch_bounds__(256 * kKHalves, 32 * kMBW * kWavesM == 128 ? 2 : 1)
       };
       auto nothing = [] {};
       if constexpr (kWavesM == 1) {
-        // Eight matrix instructions (four A fragments against the wave's two B fragments) and their side work per
-        // scheduling region, as a pipeline of one matrix instruction, at most one LDS read and a few vector
-        // instructions.  Skewed by one step like the 2 x 2 form below.
-        constexpr int kValu = kMBW == 4 ? 4 : 3;
+        // A region's matrix instructions (its A fragments against the wave's two B fragments) and their side work, as a
+        // pipeline of one matrix instruction, at most one LDS read and a few vector instructions: the fewer rows share a
+        // decoded fragment, the more.  Skewed by one step like the 2 x 2 form below.
+        constexpr int kValu = kMBW >= 6 ? 3 : kMBW == 4 ? 4 : kMBW == 3 ? 5 : 7;
         auto region = [&](int q0, auto do_mfma_tag, auto&& side) {
           if constexpr (decltype(do_mfma_tag)::value) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
+            for (int q = 0; q < kRegionRows; ++q)
 #pragma unroll
               for (int nb = 0; nb < 2; ++nb) acc[q0 + q][nb] = P::mfma(af_c[q0 + q], bf_c[nb], acc[q0 + q][nb]);
           }
           side();
-#define DQ_SPREAD_GROUP                                  \
-  __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);     \
-  __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);     \
-  __builtin_amdgcn_sched_group_barrier(0x002, kValu, 0);
-          DQ_SPREAD_GROUP DQ_SPREAD_GROUP DQ_SPREAD_GROUP DQ_SPREAD_GROUP
-          DQ_SPREAD_GROUP DQ_SPREAD_GROUP DQ_SPREAD_GROUP DQ_SPREAD_GROUP
-#undef DQ_SPREAD_GROUP
+#pragma unroll
+          for (int q = 0; q < 2 * kRegionRows; ++q) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, kValu, 0);
+          }
           __builtin_amdgcn_sched_barrier(0);
         };
-        if constexpr (kMBW == 4) {
-          // 128 rows: a step of the wave is one region
+        auto read_rows = [&](int j, int q0) {
+#pragma unroll
+          for (int q = q0; q < q0 + kRegionRows; ++q) af_n[q] = read_a1(base, j, q);
+        };
+        auto loads = [&](int region_of_iteration) {
+#pragma unroll
+          for (int i = 0; i < kPlaces; ++i) dma(region_of_iteration * kPlaces + i);
+        };
+        auto first_operands = [&] {
+          finish_scale(0);
+          finish_scale(1);
+          bf_n[0] = P::decode(bw_c[0], 0, sc_c[0]);
+          bf_n[1] = P::decode(bw_c[1], 0, sc_c[1]);
+        };
+        if constexpr (kRegions == 1) {
           region(0, DoMfma{}, [&] {
             fetch_b(0);
             fetch_b(1);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) af_n[q] = read_a1(base, 0, q);
-            dma(0);
-            dma(1);
-            finish_scale(0);
-            finish_scale(1);
-            bf_n[0] = P::decode(bw_c[0], 0, sc_c[0]);
-            bf_n[1] = P::decode(bw_c[1], 0, sc_c[1]);
+            read_rows(0, 0);
+            loads(0);
+            first_operands();
           });
         } else {
           region(0, DoMfma{}, [&] {
             fetch_b(0);
             fetch_b(1);
-            dma(0);
-            dma(1);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) af_n[q] = read_a1(base, 0, q);
+            loads(0);
+            read_rows(0, 0);
           });
-          region(4, DoMfma{}, [&] {
-#pragma unroll
-            for (int q = 4; q < 8; ++q) af_n[q] = read_a1(base, 0, q);
-            finish_scale(0);
-            finish_scale(1);
-            dma(2);
-            dma(3);
-            bf_n[0] = P::decode(bw_c[0], 0, sc_c[0]);
-            bf_n[1] = P::decode(bw_c[1], 0, sc_c[1]);
+          region(kRegionRows, DoMfma{}, [&] {
+            read_rows(0, kRegionRows);
+            loads(1);
+            first_operands();
           });
         }
 #pragma unroll
@@ -966,30 +969,24 @@ __global__ __launch_bounds__(256 * kKHalves, 32 * kMBW * kWavesM == 128 ? 2 : 1)
         bf_c[1] = bf_n[1];
 #pragma unroll
         for (int j = 0; j < kSteps - 1; ++j) {
-          if constexpr (kMBW == 4) {
+          if constexpr (kRegions == 1) {
             region(0, std::true_type{}, [&] {
-#pragma unroll
-              for (int q = 0; q < 4; ++q) af_n[q] = read_a1(base, j + 1, q);
-              dma(2 + 2 * j);
-              dma(3 + 2 * j);
+              read_rows(j + 1, 0);
+              loads(j + 1);
               bf_n[0] = P::decode(bw_c[0], j + 1, sc_c[0]);
               bf_n[1] = P::decode(bw_c[1], j + 1, sc_c[1]);
             });
-          } else if constexpr (kMBW == 8) {
-          region(0, std::true_type{}, [&] {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) af_n[q] = read_a1(base, j + 1, q);
-            dma(4 + 4 * j);
-            dma(5 + 4 * j);
-            bf_n[0] = P::decode(bw_c[0], j + 1, sc_c[0]);
-          });
-          region(4, std::true_type{}, [&] {
-#pragma unroll
-            for (int q = 4; q < 8; ++q) af_n[q] = read_a1(base, j + 1, q);
-            dma(6 + 4 * j);
-            dma(7 + 4 * j);
-            bf_n[1] = P::decode(bw_c[1], j + 1, sc_c[1]);
-          });
+          } else {
+            region(0, std::true_type{}, [&] {
+              read_rows(j + 1, 0);
+              loads(2 * j + 2);
+              bf_n[0] = P::decode(bw_c[0], j + 1, sc_c[0]);
+            });
+            region(kRegionRows, std::true_type{}, [&] {
+              read_rows(j + 1, kRegionRows);
+              loads(2 * j + 3);
+              bf_n[1] = P::decode(bw_c[1], j + 1, sc_c[1]);
+            });
           }
 #pragma unroll
           for (int q = 0; q < kMBW; ++q) af_c[q] = af_n[q];
@@ -1080,15 +1077,16 @@ __global__ __launch_bounds__(256 * kKHalves, 32 * kMBW * kWavesM == 128 ? 2 : 1)
     for (int nb = 0; nb < kNBW; ++nb) acc[q][nb] = P::mfma(af_c[q], bf_c[nb], acc[q][nb]);
 
   if constexpr (kKHalves == 2) {
-    // Each half hands two of its four 32-row blocks over and finishes the other two: [half][wave][block][nb][i / 4][lane]
+    // Each half hands its sums of the other's 32-row blocks over and finishes its own: [half][wave][block][nb][i / 4][lane]
+    constexpr int kOwn0 = (kMBW + 1) / 2, kOwn1 = kMBW - kOwn0;  // blocks of the first half, of the second
     typedef decltype(acc[0][0][0] + 0) elem_t;
     typedef elem_t elem4_t __attribute__((ext_vector_type(4)));
-    elem4_t* const red = reinterpret_cast<elem4_t*>(smem) + wave * (2 * 2 * 4 * 64) + lane;
-    constexpr int kHalfPieces = 4 * 2 * 2 * 4 * 64;
-    auto hand_over = [&](auto first_block) {
+    elem4_t* const red = reinterpret_cast<elem4_t*>(smem) + wave * (kOwn0 * 2 * 4 * 64) + lane;
+    constexpr int kHalfPieces = 4 * kOwn0 * 2 * 4 * 64;
+    auto hand_over = [&](auto first_block, auto blocks) {
       constexpr int q0 = decltype(first_block)::value;
 #pragma unroll
-      for (int q = 0; q < 2; ++q)
+      for (int q = 0; q < decltype(blocks)::value; ++q)
 #pragma unroll
         for (int nb = 0; nb < kNBW; ++nb)
 #pragma unroll
@@ -1096,31 +1094,47 @@ __global__ __launch_bounds__(256 * kKHalves, 32 * kMBW * kWavesM == 128 ? 2 : 1)
             red[kh * kHalfPieces + ((q * kNBW + nb) * 4 + v) * 64] =
                 elem4_t{acc[q0 + q][nb][4 * v], acc[q0 + q][nb][4 * v + 1], acc[q0 + q][nb][4 * v + 2], acc[q0 + q][nb][4 * v + 3]};
     };
+    auto take = [&](auto blocks) {
+#pragma unroll
+      for (int q = 0; q < decltype(blocks)::value; ++q)
+#pragma unroll
+        for (int nb = 0; nb < kNBW; ++nb)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            const elem4_t other = red[(1 - kh) * kHalfPieces + ((q * kNBW + nb) * 4 + v) * 64];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[q][nb][4 * v + e] += other[e];
+          }
+    };
+    using Own0 = std::integral_constant<int, kOwn0>;
+    using Own1 = std::integral_constant<int, kOwn1>;
     if (kh == 0) {
-      hand_over(std::integral_constant<int, 2>{});
+      hand_over(Own0{}, Own1{});
     } else {
-      hand_over(std::integral_constant<int, 0>{});
+      hand_over(std::integral_constant<int, 0>{}, Own0{});
 #pragma unroll
-      for (int q = 0; q < 2; ++q)
+      for (int q = 0; q < kOwn1; ++q)
 #pragma unroll
-        for (int nb = 0; nb < kNBW; ++nb) acc[q][nb] = acc[q + 2][nb];
+        for (int nb = 0; nb < kNBW; ++nb) acc[q][nb] = acc[q + kOwn0][nb];
     }
     __syncthreads();
-#pragma unroll
-    for (int q = 0; q < 2; ++q)
-#pragma unroll
-      for (int nb = 0; nb < kNBW; ++nb)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const elem4_t other = red[(1 - kh) * kHalfPieces + ((q * kNBW + nb) * 4 + v) * 64];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) acc[q][nb][4 * v + e] += other[e];
-        }
+    if constexpr (kOwn0 == kOwn1) {
+      take(Own0{});
+    } else {
+      if (kh == 0) take(Own0{});
+      else take(Own1{});
+    }
     __syncthreads();  // the epilogue's slabs lie where the sums were handed over
-    const int first_row = m0 + 64 * kh, slab_wave = wave + kWaves * kh;
+    const int first_row = m0 + 32 * kOwn0 * kh, slab_wave = wave + kWaves * kh;
     {
       const int m0 = first_row, wave = slab_wave;
-      DQ_GEMM_EPILOGUE_OF(2)
+      if constexpr (kOwn0 == kOwn1) {
+        DQ_GEMM_EPILOGUE_OF(kOwn0)
+      } else if (kh == 0) {
+        DQ_GEMM_EPILOGUE_OF(kOwn0)
+      } else {
+        DQ_GEMM_EPILOGUE_OF(kOwn1)
+      }
     }
   } else {
     DQ_GEMM_EPILOGUE
@@ -1275,12 +1289,53 @@ int launch_dma_half(const Params& p, hipStream_t stream) {
   return launch_dma_tile<P, 4, 2, 1>(p, stream);
 }
 
-// The tile choice of every policy that can take the direct-to-LDS path: 256 x 256 tiles there when the problem has
-// enough of them, else 128 x 256 tiles there, else the register-staged kernel with the tile size launch_auto picks.
+// P::kRowCosts: what a call takes on tiles of 96, 128, 192 and 256 rows (us: start + rounds x (round + K / 1000 x per_k), rounds
+// as dma_rounds counts them), for the policies that are built at 96 and 192 rows too.  Fitted over 70 shapes a policy (140 to
+// 3500 rows, N 1500 to 28500, K 1024 to 14300), where they pick tiles that are 5 % (uint4, MXFP4) and 8 % (2-bit) faster in the
+// mean than the better of 128 and 256 rows; 7 % slower in the worst (uint4).  They are taken where they save a twenty-fifth.
+// int8 x int4 gains nothing (0.5 %) and stays with the two.
+struct RowsCost {
+  double start, round, per_k;
+};
+template <class P, class = void>
+struct HasRowCosts : std::false_type {};
+template <class P>
+struct HasRowCosts<P, std::void_t<decltype(P::kRowCosts)>> : std::true_type {};
+
+// The tile's rows, or 0: not a call of the direct-to-LDS kernel.
+template <class P>
+int dma_rows(const Params& p, int min_tiles = kHalfTileMin) {
+  int rows = dma_eligible<P>(p) ? 256 : dma_half_eligible<P>(p, min_tiles) ? 128 : 0;
+  if constexpr (HasRowCosts<P>::value) {
+    if (!rows) return 0;
+    constexpr int kHeights[4] = {96, 128, 192, 256};
+    auto us = [&](int i) { return P::kRowCosts[i].start + dma_rounds(tiles_of(p, kHeights[i])) * (P::kRowCosts[i].round + P::kRowCosts[i].per_k * p.K * 1e-3); };
+    double best = 0.96 * us(rows == 256 ? 3 : 1);
+    for (int i = 0; i < 3; ++i)
+      if (kHeights[i] != rows && us(i) < best) best = us(i), rows = kHeights[i];
+  }
+  return rows;
+}
+template <class P>
+int launch_dma_rows(const Params& p, int rows, hipStream_t stream) {
+  if constexpr (HasRowCosts<P>::value) {
+    if (rows == 192) return launch_dma_tile<P, 6, 2, 1>(p, stream);
+    if (rows == 96) {
+      if constexpr (!OneOrder<P>::value)
+        if (dma_halves_take<P>(p)) return launch_dma_tile<P, 3, 2, 1, 2>(p, stream);
+      return launch_dma_tile<P, 3, 2, 1>(p, stream);
+    }
+  }
+  return launch_dma_half<P>(p, stream);
+}
+
+// The tile choice of every policy that can take the direct-to-LDS path: that kernel where the problem has tiles enough,
+// else the register-staged kernel with the tile size launch_auto picks.
 template <class P>
 int launch_best(const Params& p, hipStream_t stream) {
-  if (dma_eligible<P>(p)) return launch_dma<P>(p, stream);
-  if (dma_half_eligible<P>(p)) return launch_dma_half<P>(p, stream);
+  const int rows = dma_rows<P>(p);
+  if (rows == 256) return launch_dma<P>(p, stream);
+  if (rows) return launch_dma_rows<P>(p, rows, stream);
   return launch_auto<P>(p, stream);
 }
 
@@ -1326,7 +1381,9 @@ int launch_ksplit(Params p, void* parts, int split, hipStream_t stream) {
   using out_t = typename P::out_t;
   out_t* const C = (out_t*)p.C;
   p.C = parts;
-  if (launch_dma_half<PartialSums<P>>(p, stream)) return -1;
+  // tiles of 96 rows where they are no more than those of 128
+  const bool low = (p.M + 95) / 96 == (p.M + 127) / 128;
+  if (low ? launch_dma_rows<PartialSums<P>>(p, 96, stream) : launch_dma_half<PartialSums<P>>(p, stream)) return -1;
   const dim3 blocks((unsigned)((count + 1023) / 1024));
   if (p.Bias)
     hipLaunchKernelGGL((ksplit_sum_kernel<out_t, true>), blocks, dim3(256), 0, stream, (const float*)parts, (const out_t*)p.Bias, C, count, split);

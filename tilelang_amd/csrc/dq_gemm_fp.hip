@@ -33,6 +33,7 @@ template <int FMT, bool HAS_BIAS>
 struct MxPolicy : Bf16Mfma, gemm::PlainA {
   static constexpr int kBRowBytes = 32;
   static constexpr bool kOneOrder = true;  // the header's promise of a row's bits
+  static constexpr gemm::RowsCost kRowCosts[4] = {{4.3, 1.2, 10.4}, {5.15, 1.1, 12.8}, {-3.2, 14.7, 15.0}, {-7.2, 26.3, 16.3}};
   static constexpr bool kTransposed = false;
   using out_t = bf16_t;
   using ScaleRaw = int;

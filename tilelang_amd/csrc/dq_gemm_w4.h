@@ -29,6 +29,7 @@ struct W4F16Policy : F16Mfma {
   // 9 to 17 vector instructions per decoded operand: with two rows of waves a lone wave's instruction issue is
   // busier than its matrix pipe (fp16 x uint4 at M = 4096, N = K = 8192: 467 us; 427 us with the waves side by side)
   static constexpr bool kTallWaves = true;
+  static constexpr gemm::RowsCost kRowCosts[4] = {{2.1, 2.75, 12.4}, {1.8, 3.64, 14.6}, {-4.4, 12.9, 18.8}, {-11.0, 24.7, 21.4}};
   using out_t = half_t;
   struct ScaleRaw { half_t s, z; };
   struct Scale { half_t s, addend; };  // what the decoder multiplies by and adds (w4_cvt_addend)
