@@ -14,6 +14,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [
     (3, 130, 6208), (16, 515, 7232), (20, 64, 8128),                  # two slices, seven or eight chunks a wave without them
     (1, 1001, 8256), (2, 130, 8256), (8, 4100, 8256), (16, 33, 12352),  # two slices, three; one and two rows: dot products
+    (1, 130, 9728), (2, 65, 12288), (1, 40, 18432), (2, 33, 18240),   # whole ones: dot products in chunks of three steps
     (1, 40, 32832), (5, 64, 24640),                                   # beyond the dot-product kernel; five slices
 ])
 def test_half_chunk(cuda, fmt, with_bias, M, N, K):

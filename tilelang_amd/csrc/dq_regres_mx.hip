@@ -582,11 +582,12 @@ int launch_mx_gemv_rows(const void* A, const void* B, const void* S, const void*
   return 0;
 }
 
-// ---- one and two activation rows with K beyond 8192: the dot-product kernel over chunks of four steps ---------------------
+// ---- one and two activation rows with K beyond 8192: the dot-product kernel over chunks of three or four steps -------------
 // As mx_gemv_rows_kernel (activations in LDS, padded with zeros to whole chunks), the loop over K in chunks of four
-// steps (8192 k): a chunk's 16 loads of a batch of four weight rows are asked for, waited for and multiplied, the
-// sums carried from chunk to chunk; the other waves of the SIMD cover the wait.
-template <int FMT, bool HAS_BIAS, int MR>
+// steps (8192 k), or of three where that pads K to less (five and six steps, nine: K = 9728 is six steps, not eight): a chunk's
+// loads of a batch of four weight rows are asked for, waited for and multiplied, the sums carried from chunk to chunk; the
+// other waves of the SIMD cover the wait.
+template <int FMT, bool HAS_BIAS, int MR, int STEPS>
 __global__ __launch_bounds__(256) void mx_gemv_long_kernel(const bf16_t* __restrict__ A, const uint8_t* __restrict__ B,
                                                            const uint8_t* __restrict__ S, const bf16_t* __restrict__ Bias,
                                                            bf16_t* __restrict__ C, int M, int N, int K, int exp_off) {
@@ -595,7 +596,7 @@ __global__ __launch_bounds__(256) void mx_gemv_long_kernel(const bf16_t* __restr
   const int tid = threadIdx.x, lane = tid & 63;
   const int gw = blockIdx.x * 4 + (tid >> 6), nwaves = gridDim.x * 4;
   const int nblk = K >> 5;
-  const int nchunk = (nblk + 255) >> 8, nsteps = 4 * nchunk;  // steps of 64 blocks, padded to whole chunks
+  const int nchunk = (nblk + 64 * STEPS - 1) / (64 * STEPS), nsteps = STEPS * nchunk;  // steps of 64 blocks, padded to whole chunks
   const uint32_t w_row_bytes = (uint32_t)(K >> 1), s_row_bytes = (uint32_t)nblk;
   for (int p = tid; p < MR * nsteps * 256; p += 256) {  // piece q of block 64 s + l of row m at p = ((m nsteps + s) 64 + l) 4 + q
     const int q = p & 3, l = (p >> 2) & 63, ms = p >> 8;
@@ -611,27 +612,27 @@ __global__ __launch_bounds__(256) void mx_gemv_long_kernel(const bf16_t* __restr
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[i] = 0.f;
     for (int ch = 0; ch < nchunk; ++ch) {
-      uint4_t w[kGemvRows][4];
-      uint32_t sc[kGemvRows][4];
+      uint4_t w[kGemvRows][STEPS];
+      uint32_t sc[kGemvRows][STEPS];
 #pragma unroll
       for (int j = 0; j < kGemvRows; ++j) {
         const int n = min(b * kGemvRows + j, N - 1);
         const uint8_t* const w_row = B + (size_t)n * w_row_bytes;
         const uint8_t* const s_row = S + (size_t)n * s_row_bytes;
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          const uint32_t blk = (uint32_t)min((4 * ch + s) * 64 + lane, nblk - 1);
+        for (int s = 0; s < STEPS; ++s) {
+          const uint32_t blk = (uint32_t)min((STEPS * ch + s) * 64 + lane, nblk - 1);
           w[j][s] = __builtin_nontemporal_load(reinterpret_cast<const uint4_t*>(w_row + blk * 16));
           sc[j][s] = __builtin_nontemporal_load(s_row + blk);
         }
       }
 #pragma unroll
-      for (int s = 0; s < 4; ++s) {
+      for (int s = 0; s < STEPS; ++s) {
         uint4_t af[MR][4];
 #pragma unroll
         for (int m = 0; m < MR; ++m)
 #pragma unroll
-          for (int q = 0; q < 4; ++q) af[m][q] = *reinterpret_cast<const uint4_t*>(smem + (((m * nsteps + 4 * ch + s) * 4 + q) * 64 + lane) * 16);
+          for (int q = 0; q < 4; ++q) af[m][q] = *reinterpret_cast<const uint4_t*>(smem + (((m * nsteps + STEPS * ch + s) * 4 + q) * 64 + lane) * 16);
 #pragma unroll
         for (int j = 0; j < kGemvRows; ++j) {
           const LaneScale ls = lane_scale<FMT>(sc[j][s], exp_off);
@@ -666,21 +667,21 @@ __global__ __launch_bounds__(256) void mx_gemv_long_kernel(const bf16_t* __restr
 
 constexpr int kGemvLongMaxK = 32768;  // two rows of activations: 128 KiB of LDS
 
-template <int FMT, bool HAS_BIAS, int MR>
-int launch_mx_gemv_long(const void* A, const void* B, const void* S, const void* Bias, void* C, int M, int N, int K,
+template <int FMT, bool HAS_BIAS, int MR, int STEPS>
+int launch_mx_gemv_long_of(const void* A, const void* B, const void* S, const void* Bias, void* C, int M, int N, int K,
                         int exp_off, hipStream_t stream) {
-  auto kern = mx_gemv_long_kernel<FMT, HAS_BIAS, MR>;
+  auto kern = mx_gemv_long_kernel<FMT, HAS_BIAS, MR, STEPS>;
   static bool raised[kMaxDevices] = {};
   if (raise_lds_limit<MR * (kGemvLongMaxK / 2048) * 4096>(kern, raised)) return -1;
-  const int nchunk = ((K >> 5) + 255) >> 8;
-  const int lds = MR * 4 * nchunk * 4096;
+  const int nchunk = ((K >> 5) + 64 * STEPS - 1) / (64 * STEPS);
+  const int lds = MR * STEPS * nchunk * 4096;
   static int cus_of[kMaxDevices] = {};
   int device = 0;
   DQ_CHECK_HIP(hipGetDevice(&device));
   if (device < 0 || device >= kMaxDevices) DQ_FAIL("device index %d is beyond the %d this library keeps state for", device, kMaxDevices);
   if (!cus_of[device]) DQ_CHECK_HIP(hipDeviceGetAttribute(&cus_of[device], hipDeviceAttributeMultiprocessorCount, device));
   // workgroups per CU: depends on K through the LDS a workgroup takes (asked once per device and chunk count)
-  static int per_cu_of[kMaxDevices][kGemvLongMaxK / 8192 + 1] = {};
+  static int per_cu_of[kMaxDevices][kGemvLongMaxK / (2048 * STEPS) + 2] = {};
   int& per_cu = per_cu_of[device][nchunk];
   if (!per_cu) {
     DQ_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, 256, lds));
@@ -692,6 +693,15 @@ int launch_mx_gemv_long(const void* A, const void* B, const void* S, const void*
                      (const uint8_t*)S, (const bf16_t*)Bias, (bf16_t*)C, M, N, K, exp_off);
   DQ_CHECK_HIP(hipGetLastError());
   return 0;
+}
+
+template <int FMT, bool HAS_BIAS, int MR>
+int launch_mx_gemv_long(const void* A, const void* B, const void* S, const void* Bias, void* C, int M, int N, int K,
+                        int exp_off, hipStream_t stream) {
+  const int steps = (K + 2047) / 2048;  // at most 16
+  const bool three = (steps + 2) / 3 * 3 < (steps + 3) / 4 * 4 && (steps + 2) / 3 <= (steps + 3) / 4;
+  return three ? launch_mx_gemv_long_of<FMT, HAS_BIAS, MR, 3>(A, B, S, Bias, C, M, N, K, exp_off, stream)
+               : launch_mx_gemv_long_of<FMT, HAS_BIAS, MR, 4>(A, B, S, Bias, C, M, N, K, exp_off, stream);
 }
 
 }  // namespace
