@@ -95,7 +95,8 @@ int call_dequantize_gemv_w4a16(const void* A, const void* B, const void* Scale, 
  * (N = 4096, K = 14336: 64 workgroups of 64 rows for 256 CUs) leaves most of the chip idle at 2 <= M <= 128; with a
  * workspace of dq_w4a16_workspace_bytes(M, N, K, group, mode) bytes the default dispatch (`variant` < 0) cuts K into
  * up to 16 slices, one workgroup each, writes their fp32 sums to the workspace and adds them in slice order in a
- * second kernel: results do not depend on timing and stay within rounding of the unsplit kernel's.  A smaller
+ * second kernel: results do not depend on timing and stay within rounding of the unsplit kernel's.  So it does at more
+ * rows, on the tiled GEMM, where the scaled modes leave CUs idle there (M = 202, N = 8928, K = 10752).  A smaller
  * workspace lowers the slice count, NULL / 0 bytes is call_dequantize_gemv_w4a16.  Workspace: 16-byte aligned,
  * contents undefined afterwards, not to be shared by calls that overlap in time. */
 size_t dq_w4a16_workspace_bytes(int M, int N, int K, int group, int mode);
@@ -145,8 +146,9 @@ enum dq_fp4_format {
  * scale_bias = 127.  Bias may be NULL.  Requires K % 64 == 0, scale_size == 32.
  * The library picks the kernel by shape (one and two rows up to K = 32768: a dot-product kernel on whole weight
  * rows; up to 16 rows: the activations resident in registers and the weights streamed once, or K over the waves of a
- * workgroup, as from 17 to 64 rows from K = 512 on and, K % 128 == 64, on small matrices beyond; else the tiled GEMM).  Each adds the same products in fp32 in an order of its own: a row computed
- * in a small batch and in a large one may differ in the last bf16 bit; every call of one shape returns the same bits. */
+ * workgroup, as from 17 to 64 rows from K = 512 on and, K % 128 == 64, on small matrices beyond; else the tiled GEMM).
+ * Each adds the same products in fp32 in an order of its own: a row computed in a small batch and in a large one may
+ * differ in the last bf16 bit; every call of one shape returns the same bits. */
 int call_dequant_gemm_bf16_mxfp4(const void* A, const void* B, const void* Scale, const void* Bias, void* C, int M,
                                  int N, int K, int scale_size, int fp4_format, int scale_bias, dq_stream_t stream);
 

@@ -53,6 +53,9 @@ int i2_kwaves_form(int M, int N, int K);
 double mxfp4_kwaves_time(int M, int N, int K);
 int mxfp4_gemm_kwaves(const void* A, const void* B, const void* S, const void* Bias, void* C, int M, int N, int K, int fmt,
                       int scale_bias, hipStream_t stream);
+int w4_f16_gemm_ksplit(const void* A, const void* B, const void* S, const void* Z, void* C, void* parts, int M, int N, int K,
+                       int group, int mode, int layout, int split, hipStream_t stream);
+double w4_tiled_time(int M, int N, int K);
 double w4_kwaves_time(int M, int N, int K);
 int w4_f16_gemm_kwaves(const void* A, const void* B, const void* S, const void* Z, void* C, int M, int N, int K, int group,
                        int mode, int layout, hipStream_t stream);
@@ -155,6 +158,9 @@ extern "C" int init(void) {
   return 0;
 }
 
+// Tiles of 128 x 256
+static long half_tiles(int M, int N) { return (((long)M + 127) / 128) * (((long)N + 255) / 256); }
+
 // ---- the streaming small-batch kernel's default configuration and K split ------------------------------
 // Which configuration the default dispatch runs at M rows (see w4a16_stream for the numbering).
 static int w4a16_stream_config(int M, int N) {
@@ -200,7 +206,43 @@ static bool w4a16_few_tiles(int M, int N, int K) {
   return M <= 1024 && K % 256 == 0 && (long)((M + 255) / 256) * ((N + 255) / 256) <= 64;
 }
 
+// Into how many slices of K the tiled GEMM is cut where a workspace was brought: 65 to some thousand rows against a matrix of
+// few tiles, where neither it uncut nor the streaming kernel fills the chip.  Both sides are fits (us) over 90 shapes of 64 to
+// 1280 rows (mean error 5 %), and cut is what they put a tenth ahead: 1.08 times as fast in the mean, 0.99 in the worst (M = 202,
+// N = 8928, K = 10752 97 -> 61 us; M = 73, N = 17328, K = 7680 74 -> 37; M = 419, N = 5296, K = 7680 74 -> 52; not M = 128, N = 4096,
+// K = 14336, 28 us on the streaming kernel and 31 cut).  1: not cut.
+static int w4a16_tiled_split(int M, int N, int K, int group, int mode) {
+  const bool scaled = mode == W4_SCALE || mode == W4_USCALE || mode == W4_ZEROS_ORIGINAL || mode == W4_ZEROS_FOLDED;
+  // slices start where a dword of a row's scales does
+  if (M <= 64 || !scaled || group == K || group < 32 || group > 4096 || K % 256 != 0 || K % (2 * group) != 0 || ((size_t)M * N) % 4 != 0) return 1;
+  const long big = half_tiles(M, N);
+  if (big >= 192) return 1;
+  auto rounds = [](long wgs) { return (double)(wgs / 256) + (wgs % 256 ? 0.65 + 0.35 * (double)(wgs % 256) / 256.0 : 0.0); };
+  double best;
+  if (M <= 128 || w4a16_few_tiles(M, N, K)) {  // the streaming kernel, in passes of 64 rows and slices of its own
+    const int own = w4a16_stream_split(M, N, K, group, mode, w4a16_stream_config(M, N));
+    const long wgs = (((long)N + 127) / 128) * (((long)M + 63) / 64) * own;
+    best = 4.0 + (double)((wgs + 255) / 256) * (1.5 + 4.55e-3 * K / own) + (own > 1 ? 1.5 + 2.5e-6 * own * M * N : 0.0);
+  } else {
+    best = big < 96 ? 2.0 + 9.0e-3 * K : w4_tiled_time(M, N, K);
+  }
+  best *= 0.9;
+  const bool low = (M + 95) / 96 == (M + 127) / 128;  // tiles of 96 rows, as launch_ksplit takes them
+  const long tiles = (long)(low ? (M + 95) / 96 : (M + 127) / 128) * (((long)N + 255) / 256);
+  const int unit = std::max(128, 2 * group), units = K / unit;
+  int split = 1;
+  for (int s = 2; s <= 12 && units >= s && K / s >= 1024; ++s) {
+    const double r = rounds(tiles * s);
+    const double us = 5.7 + r * (4.5 + 12.7e-3 * unit * ((units + s - 1) / s) * (low ? 0.79 : 1.0)) + 1.02e-6 * (double)s * M * N;
+    if (us < best) best = us, split = s;
+  }
+  return split;
+}
+
 extern "C" size_t dq_w4a16_workspace_bytes(int M, int N, int K, int group, int mode) {
+  if (M < 2 || N <= 0 || K <= 0 || group <= 0) return 0;
+  const int cut = w4a16_tiled_split(M, N, K, group, mode);
+  if (cut > 1) return (size_t)cut * M * N * sizeof(float);
   if (M < 2 || N <= 0 || K <= 0 || group <= 0 || (M > 128 && !w4a16_few_tiles(M, N, K))) return 0;
   const int split = w4a16_stream_split(M, N, K, group, mode, w4a16_stream_config(M, N));
   return split > 1 ? (size_t)split * M * N * sizeof(float) : 0;
@@ -213,7 +255,7 @@ extern "C" size_t dq_w4a16_workspace_bytes(int M, int N, int K, int group, int m
 static bool w4a16_by_kwaves(int M, int N, int K) {
   if (M < 3 || K % 256 == 0) return false;
   if (M <= 64) return true;
-  return (((long)M + 127) / 128) * (((long)N + 255) / 256) < 96 && w4_kwaves_time(M, N, K) < 2.0 + 9.0e-3 * K;
+  return half_tiles(M, N) < 96 && w4_kwaves_time(M, N, K) < 2.0 + 9.0e-3 * K;
 }
 
 static int gemv_w4a16(const char* fn, const void* A, const void* B, const void* Scale, const void* Zeros, void* C, int M, int N,
@@ -240,9 +282,25 @@ static int gemv_w4a16(const char* fn, const void* A, const void* B, const void* 
               "but \"rescale\" only (got M=%d N=%d K=%d group=%d mode=%d)", fn, M, N, K, group, mode);
     return rc;
   }
+  // 52 .. 66: K cut over the workgroups of the tiled GEMM, in that many slices less 50 (measurements and tests)
+  if (variant > 51 && variant <= 66) {
+    const int split = variant - 50;
+    if ((size_t)split * M * N * sizeof(float) > workspace_bytes) DQ_FAIL("%s: %d slices need %zu bytes of workspace", fn, split, (size_t)split * M * N * sizeof(float));
+    const int rc = w4_f16_gemm_ksplit(A, B, Scale, Zeros, C, workspace, M, N, K, group, asked_mode, layout, split, (hipStream_t)stream);
+    if (rc > 0) DQ_FAIL("%s: the tiled kernel does not cut M=%d N=%d K=%d group=%d mode=%d", fn, M, N, K, group, mode);
+    return rc;
+  }
   if (variant == -1 && w4a16_by_kwaves(M, N, K)) {
     const int rc = w4_f16_gemm_kwaves(A, B, Scale, Zeros, C, M, N, K, group, asked_mode, layout, (hipStream_t)stream);
     if (rc <= 0) return rc;
+  }
+  if (variant == -1 && workspace) {
+    int cut = w4a16_tiled_split(M, N, K, group, asked_mode);
+    while (cut > 1 && (size_t)cut * M * N * sizeof(float) > workspace_bytes) --cut;
+    if (cut > 1) {
+      const int rc = w4_f16_gemm_ksplit(A, B, Scale, Zeros, C, workspace, M, N, K, group, asked_mode, layout, cut, (hipStream_t)stream);
+      if (rc <= 0) return rc;
+    }
   }
   // prefill-sized M: the tiled MFMA GEMM (same tile-exact decoders); up to 128 rows, and beyond that against a
   // matrix of few tiles, the streaming kernel below (passes of 64 rows over the weights) is still the faster one.
@@ -426,7 +484,7 @@ static int mxfp4_ksplit(int M, int N, int K, int fp4_format) {
 static bool mxfp4_by_kwaves(int M, int N, int K) {
   if (M < 3) return false;
   if (M > 64)
-    return K % 128 != 0 && (((long)M + 127) / 128) * (((long)N + 255) / 256) < 96 && mxfp4_kwaves_time(M, N, K) < 0.95 * (2.0 + 7.5e-3 * K);
+    return K % 128 != 0 && half_tiles(M, N) < 96 && mxfp4_kwaves_time(M, N, K) < 0.95 * (2.0 + 7.5e-3 * K);
   return M > 16 || mxfp4_kwaves_time(M, N, K) < 0.8 * mxfp4_regres_time(M, N, K);
 }
 

@@ -110,9 +110,10 @@ __device__ __forceinline__ void take_k_slice(Params& p, int& bid) {
       const int u0 = units * z / p.split, u1 = units * (z + 1) / p.split;
       k0 = u0 * p.kunit;
       p.K = (u1 - u0) * p.kunit;
-      // a slice starts where a dword of a row's scale bytes does (kunit is a multiple of 128 k)
-      static_assert(P::kScaleDma <= 1, "slices of fp16 group scales are not built");
+      // a slice starts where a dword of a row's scales does: kunit is a multiple of 128 k, and of two groups
       if constexpr (P::kScaleDma == 1) p.S = (const unsigned char*)p.S + (k0 >> 5);
+      if constexpr (P::kScaleDma >= 2) p.S = (const unsigned char*)p.S + ((k0 >> p.p0) << 1);
+      if constexpr (P::kScaleDma == 3) p.Z = (const unsigned char*)p.Z + ((k0 >> p.p0) << 1);
     }
     p.A = (const unsigned char*)p.A + (size_t)k0 * (kARowBytes / P::kKPerBlock);
     p.B = (const unsigned char*)p.B + (size_t)k0 * P::kBRowBytes / P::kKPerBlock;
@@ -1376,6 +1377,7 @@ int launch_ksplit(Params p, void* parts, int split, hipStream_t stream) {
   if (split < 2 || !dma_takes<P>(p)) return 1;
   const size_t count = (size_t)p.M * p.N;
   p.kunit = 2 * P::kKPerBlock;
+  if (P::kScaleDma >= 2 && (2 << p.p0) > p.kunit) p.kunit = 2 << p.p0;
   if (p.K % p.kunit != 0 || p.K / p.kunit < split || count % 4 != 0) return 1;
   p.split = split;
   using out_t = typename P::out_t;

@@ -5,6 +5,19 @@ namespace dq {
 
 using gemm::Params;
 
+// What a call takes on the direct-to-LDS kernel's tiles (us), whichever are best
+double w4_tiled_time(int M, int N, int K) {
+  using P = W4F16Policy<W4_SCALE, false>;
+  const Params p = gemm::make_params(nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, M, N, K);
+  constexpr int kHeights[4] = {96, 128, 192, 256};
+  double best = 1e30;
+  for (int i = 0; i < 4; ++i) {
+    const double us = P::kRowCosts[i].start + gemm::dma_rounds(gemm::tiles_of(p, kHeights[i])) * (P::kRowCosts[i].round + P::kRowCosts[i].per_k * K * 1e-3);
+    if (us < best) best = us;
+  }
+  return best;
+}
+
 int w4_f16_gemm(const void* A, const void* B, const void* S, const void* Z, void* C, int M, int N, int K, int group,
                 int mode, int layout, hipStream_t stream) {
   Params p = gemm::make_params(A, B, S, Z, nullptr, C, M, N, K);
