@@ -206,6 +206,12 @@ static bool w4a16_few_tiles(int M, int N, int K) {
   return M <= 1024 && K % 256 == 0 && (long)((M + 255) / 256) * ((N + 255) / 256) <= 64;
 }
 
+// What the streaming kernel takes (us) in passes of 64 rows, cut into `split` slices
+static double w4a16_stream_passes_time(int M, int N, int K, int split) {
+  const long wgs = (((long)N + 127) / 128) * (((long)M + 63) / 64) * split;
+  return 4.0 + (double)((wgs + 255) / 256) * (1.5 + 4.55e-3 * K / split) + (split > 1 ? 1.5 + 2.5e-6 * split * M * N : 0.0);
+}
+
 // Into how many slices of K the tiled GEMM is cut where a workspace was brought: 65 to some thousand rows against a matrix of
 // few tiles, where neither it uncut nor the streaming kernel fills the chip.  Both sides are fits (us) over 90 shapes of 64 to
 // 1280 rows (mean error 5 %), and cut is what they put a tenth ahead: 1.08 times as fast in the mean, 0.99 in the worst (M = 202,
@@ -220,9 +226,7 @@ static int w4a16_tiled_split(int M, int N, int K, int group, int mode) {
   auto rounds = [](long wgs) { return (double)(wgs / 256) + (wgs % 256 ? 0.65 + 0.35 * (double)(wgs % 256) / 256.0 : 0.0); };
   double best;
   if (M <= 128 || w4a16_few_tiles(M, N, K)) {  // the streaming kernel, in passes of 64 rows and slices of its own
-    const int own = w4a16_stream_split(M, N, K, group, mode, w4a16_stream_config(M, N));
-    const long wgs = (((long)N + 127) / 128) * (((long)M + 63) / 64) * own;
-    best = 4.0 + (double)((wgs + 255) / 256) * (1.5 + 4.55e-3 * K / own) + (own > 1 ? 1.5 + 2.5e-6 * own * M * N : 0.0);
+    best = w4a16_stream_passes_time(M, N, K, w4a16_stream_split(M, N, K, group, mode, w4a16_stream_config(M, N)));
   } else {
     best = big < 96 ? 2.0 + 9.0e-3 * K : w4_tiled_time(M, N, K);
   }
@@ -243,17 +247,42 @@ extern "C" size_t dq_w4a16_workspace_bytes(int M, int N, int K, int group, int m
   if (M < 2 || N <= 0 || K <= 0 || group <= 0) return 0;
   const int cut = w4a16_tiled_split(M, N, K, group, mode);
   if (cut > 1) return (size_t)cut * M * N * sizeof(float);
-  if (M < 2 || N <= 0 || K <= 0 || group <= 0 || (M > 128 && !w4a16_few_tiles(M, N, K))) return 0;
+  if (M > 128 && !w4a16_few_tiles(M, N, K)) return 0;
   const int split = w4a16_stream_split(M, N, K, group, mode, w4a16_stream_config(M, N));
   return split > 1 ? (size_t)split * M * N * sizeof(float) : 0;
+}
+
+// What the streaming kernel takes (us) to 128 rows in one round of workgroups, cut into `split` slices: fits over 84 shapes (mean
+// error 3 to 6 %).  0: not fitted.
+static double w4a16_stream_time(int M, int N, int K, int split) {
+  const int config = w4a16_stream_config(M, N);
+  const bool narrow = config >= 3 && config <= 5;
+  const int pass = config == 3 ? 16 : narrow || config == 1 ? 32 : (config == 7 ? 48 : 64);
+  const long wgs = (((long)N + (narrow ? 63 : 127)) / (narrow ? 64 : 128)) * (((long)M + pass - 1) / pass) * split;
+  if (wgs > 256) return 0.0;  // (workgroups that share a CU are not fitted)
+  const double k = 1e-3 * K / split, sums = split > 1 ? 1e-6 * split * M * N : 0.0, cut = split > 1 ? 1.0 : 0.0;
+  switch (config) {
+    case 3: return 2.3 + 2.33 * k + 2.7 * cut + 9.9 * sums;
+    case 4: return 2.3 + 2.83 * k + 1.0 * cut + 15.1 * sums;
+    case 7: return 2.4 + 4.4 * k + 1.7 * cut + 4.4 * sums;
+    case 6: return std::min(2.7 + 5.58 * k + 2.3 * cut + 4.0 * sums, M > 64 ? w4a16_stream_passes_time(M, N, K, split) : 1e30);
+    default: return 0.0;  // 17 to 32 rows of a wide matrix: the streaming kernel is ahead (N = 27632, K = 2560 16.2 against 18.3 us)
+  }
 }
 
 // K that is no multiple of 256: neither the register-resident nor the streaming kernel takes it, and from three rows on K over
 // the waves of a workgroup is ahead of the general ones (M = 8, N = 23848, K = 3968, group 64: 37 -> 21 us; M = 24, N = 6712,
 // K = 11904 84 -> 22; M = 88, N = 7952, K = 3712 42 -> 19), beyond 64 rows while the tiled GEMM's big tiles are few (its small
-// ones take some 10 us a thousand k).
-static bool w4a16_by_kwaves(int M, int N, int K) {
-  if (M < 3 || K % 256 == 0) return false;
+// ones take some 10 us a thousand k).  Multiples of 256, to 128 rows where the register-resident kernel declines: where it is a
+// seventh ahead of the streaming kernel's estimate, beyond 32 rows a fifth, which it is in a fourth of the shapes (M = 58,
+// N = 2528, K = 3840 14.2 -> 8.7 us, M = 13, N = 6224, K = 7424 14.1 -> 11.6; not M = 49, N = 5224, K = 13568, 25 us in slices
+// over workgroups and 39 so, nor M = 36, N = 15416, K = 4608, 20 and 24).
+static bool w4a16_by_kwaves(int M, int N, int K, int group, int mode, bool room) {
+  if (M < 3) return false;
+  if (K % 256 == 0) {
+    if (M > 128 || (M <= 16 && N % 16 == 0 && group == 128 && (K == 2048 || K == 4096 || K == 8192))) return false;
+    return w4_kwaves_time(M, N, K) < (M <= 32 ? 0.85 : 0.78) * w4a16_stream_time(M, N, K, room ? w4a16_stream_split(M, N, K, group, mode, w4a16_stream_config(M, N)) : 1);
+  }
   if (M <= 64) return true;
   return half_tiles(M, N) < 96 && w4_kwaves_time(M, N, K) < 2.0 + 9.0e-3 * K;
 }
@@ -290,7 +319,7 @@ static int gemv_w4a16(const char* fn, const void* A, const void* B, const void* 
     if (rc > 0) DQ_FAIL("%s: the tiled kernel does not cut M=%d N=%d K=%d group=%d mode=%d", fn, M, N, K, group, mode);
     return rc;
   }
-  if (variant == -1 && w4a16_by_kwaves(M, N, K)) {
+  if (variant == -1 && w4a16_by_kwaves(M, N, K, group, asked_mode, workspace != nullptr)) {
     const int rc = w4_f16_gemm_kwaves(A, B, Scale, Zeros, C, M, N, K, group, asked_mode, layout, (hipStream_t)stream);
     if (rc <= 0) return rc;
   }
