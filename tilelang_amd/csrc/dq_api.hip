@@ -283,6 +283,7 @@ static bool w4a16_by_kwaves(int M, int N, int K, int group, int mode, bool room)
     if (M > 128 || (M <= 16 && N % 16 == 0 && group == 128 && (K == 2048 || K == 4096 || K == 8192))) return false;
     return w4_kwaves_time(M, N, K) < (M <= 32 ? 0.85 : 0.78) * w4a16_stream_time(M, N, K, room ? w4a16_stream_split(M, N, K, group, mode, w4a16_stream_config(M, N)) : 1);
   }
+  if (M <= 4 && K <= 8192) return false;  // the dot-product kernel, which rounds no weight to fp16
   if (M <= 64) return true;
   return half_tiles(M, N) < 96 && w4_kwaves_time(M, N, K) < 2.0 + 9.0e-3 * K;
 }

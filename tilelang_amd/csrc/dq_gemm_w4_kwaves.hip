@@ -1,5 +1,5 @@
-// uint4 x fp16 with K over the waves of a workgroup (dq_gemm_kwaves.h): W4A16 at 3 to some hundreds of rows where K is no
-// multiple of 256, which the decode kernels do not take.
+// uint4 x fp16 with K over the waves of a workgroup (dq_gemm_kwaves.h): W4A16 at 3 to some hundreds of rows, where the decode
+// kernels do not take the shape or are behind.
 #include "dq_gemm_kwaves.h"
 #include "dq_gemm_w4.h"
 
