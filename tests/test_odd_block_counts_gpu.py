@@ -2,10 +2,12 @@
 tile, and every other row of scales starts in the middle of a dword.  Operands are small integers and powers of two, so that
 every product and every fp32 sum is exact and the result is one rounding of the float64 product."""
 
+import numpy as np
 import pytest
 import torch
 
 import tilelang_amd as tl
+from oracle import dq_oracle as orc
 from tilelang_amd import _lib
 
 pytestmark = pytest.mark.gpu
@@ -99,3 +101,16 @@ def test_bitnet(cuda, M, N, K):
     assert rc == 0, _lib.last_error()
     W = codes.reshape(N, K).double() - 2
     assert torch.equal(C, (A.double() @ W.t()).int())
+
+
+@pytest.mark.parametrize("transposed", [True, False])
+@pytest.mark.parametrize("K,split", [(384, 2), (640, 2), (576, 3), (512, 2)])  # the last: an even count
+def test_fp16_fp4_slices(cuda, K, split, transposed):
+    """An even number of k-blocks in all and an odd one in each equal slice."""
+    M, N = HALF[0], 3504
+    rng = np.random.default_rng(K)
+    A = rng.integers(-2, 3, size=(M, K)).astype(np.float16)
+    B = rng.integers(0, 256, size=(N, K // 2), dtype=np.uint8) & 0x33  # magnitudes to 1.5
+    out = tl.matmul_fp16_fp4(M, N, K, split=split, transposed_output=transposed)(torch.from_numpy(A).to(cuda), torch.from_numpy(B).to(cuda))
+    ref = orc.ref_fp16xfp4_splitk(A, B, split)
+    np.testing.assert_array_equal(out.cpu().numpy(), ref.T if transposed else ref)

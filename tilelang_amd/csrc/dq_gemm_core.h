@@ -608,9 +608,10 @@ __device__ __forceinline__ void dma4_unless(int not_due, unsigned lds_addr, unsi
 // N = 13824, K = 5120: 86 -> 73 -> 60; MXFP4 at M = 768, N = K = 8192, which stays on four waves (kOneOrder): 102 -> 92; int8 x
 // 2-bit, M = 1024, N = K = 8192: 58 -> 53.5; int8 x int4, M = 1024, N = K = 8192: 64 -> 59.5.
 //
-// kOdd: K may be an odd number of k-blocks and a row's scale groups an odd number.  Only policies with a scale byte per 32 k
-// have both kinds (MXFP4, M = 4096, N = K = 8192: 369 us, and 374 in the kind that asks).
-template <class P, int kMBW, int kNBW, int kWavesM = 2, int kKHalves = 1, bool kOdd = P::kScaleDma != 1>
+// kOdd: K may be an odd number of k-blocks and a row's scale groups an odd number.  Both kinds are built: the one that asks is
+// slower also where nothing is odd (MXFP4, M = 4096, N = K = 8192: 369 and 374 us; fp16 x uint4 at M = 2048, N = 4096,
+// K = 14336 203 and 206, at M = 2015, N = 24640, K = 2048 191 and 193; int8 x 2-bit, M = 2048, N = K = 8192: 109.7 and 110.2).
+template <class P, int kMBW, int kNBW, int kWavesM = 2, int kKHalves = 1, bool kOdd = false>
 __global__ __launch_bounds__(256 * kKHalves, 32 * kMBW * kWavesM <= 128 ? 2 : 1) void gemm_kernel_dma(const Params p_in) {
   Params p = p_in;
   int bid = blockIdx.x;
@@ -1227,10 +1228,14 @@ bool dma_half_eligible(const Params& p, int min_tiles = kHalfTileMin) {
   return !dma_eligible<P>(p) && dma_takes<P>(p) && tiles_of(p, 128) >= min_tiles;
 }
 
-template <class P, int kMBW, int kNBW, int kWavesM = 2, int kKHalves = 1, bool kOdd = P::kScaleDma != 1>
+template <class P, int kMBW, int kNBW, int kWavesM = 2, int kKHalves = 1, bool kOdd = false>
 int launch_dma_tile(Params p, hipStream_t stream) {
-  if constexpr (!kOdd && kKHalves == 1)
-    if (p.ldk / P::kKPerBlock % 2 != 0) return launch_dma_tile<P, kMBW, kNBW, kWavesM, kKHalves, true>(p, stream);
+  // uneven slices start and end on an even block and an even group; eight waves take any count of stages
+  if constexpr (!kOdd && !UnevenSlices<P>::value && (kKHalves == 1 || P::kScaleDma != 0)) {
+    const bool odd_blocks = kKHalves == 1 && p.K / P::kKPerBlock % 2 != 0;
+    const bool odd_groups = P::kScaleDma != 0 && ((p.ldk >> (P::kScaleDma >= 2 ? p.p0 : 6)) & 1) != 0;
+    if (odd_blocks || odd_groups) return launch_dma_tile<P, kMBW, kNBW, kWavesM, kKHalves, true>(p, stream);
+  }
   constexpr int kWaves = 4;
   constexpr int kTileM = 32 * kMBW * kWavesM;
   constexpr bool kPairB = P::kBRowBytes == 32 && kTileM == 256;  // as in the kernel: a fourth B slot
