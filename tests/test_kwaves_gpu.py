@@ -46,6 +46,7 @@ def test_int8_int4(cuda, M, N, K, decode, transposed):
     (3, 2100, 13824), (14, 2168, 6720), (17, 130, 512), (20, 1001, 576),  # the least K; a chunk in part
     (32, 8200, 2880), (33, 9000, 1088), (48, 16400, 768), (64, 20003, 832), (64, 3000, 2112),
     (101, 2000, 4800), (254, 1030, 1344),                                # passes (K % 128 == 64)
+    (81, 2004, 1024), (95, 2760, 2304), (327, 1036, 1792), (204, 2912, 3328),  # in place of the cut over workgroups
 ])
 @pytest.mark.parametrize("with_bias", [False, True])
 @pytest.mark.parametrize("fmt", ["e2m1", "simple"])

@@ -270,7 +270,7 @@ static double w4a16_stream_time(int M, int N, int K, int split) {
   }
 }
 
-// K that is no multiple of 256: neither the register-resident nor the streaming kernel takes it, and from three rows on K over
+// K that is no multiple of 256: neither the register-resident nor the streaming kernel takes it, and from five rows on K over
 // the waves of a workgroup is ahead of the general ones (M = 8, N = 23848, K = 3968, group 64: 37 -> 21 us; M = 24, N = 6712,
 // K = 11904 84 -> 22; M = 88, N = 7952, K = 3712 42 -> 19), beyond 64 rows while the tiled GEMM's big tiles are few (its small
 // ones take some 10 us a thousand k).  Multiples of 256, to 128 rows where the register-resident kernel declines: where it is a
@@ -479,9 +479,10 @@ extern "C" int call_unpack_qzeros(const void* QZeros, void* Zeros, int N, int gr
 // From 192 tiles on nothing is gained (M = 768, N = 8192, K = 14336: 174 us, in four slices 178).
 // Up to 80 rows nothing is cut.  That is a promise of the header and no crossover: up to there a call that runs on the
 // tiled kernel gives the bits that its rows have in a large product (cut, M = 80, N = K = 8192 would take 25 us, not 63).
-static int mxfp4_ksplit(int M, int N, int K, int fp4_format) {
+static int mxfp4_ksplit(int M, int N, int K, int fp4_format, double* us) {
+  *us = 0.0;
   if (M <= 80 || K % 128 != 0 || ((size_t)M * N) % 4 != 0) return 1;
-  const long tiles = (((long)M + 127) / 128) * (((long)N + 255) / 256);
+  const long tiles = half_tiles(M, N);
   if (tiles >= 192) return 1;
   const int units = K / 128;
   const long small_tiles = (((long)M + 127) / 128) * (((long)N + 63) / 64);  // of the register-staged kernel
@@ -491,6 +492,7 @@ static int mxfp4_ksplit(int M, int N, int K, int fp4_format) {
   if (tiles >= 96) best = 5.1 + 1e-3 * K * (8.65 + 4.5 * (double)tiles / 256.0);
   else best = 2.0 + 1e-3 * K * (tiles <= 32 ? 7.2 : tiles <= 64 ? 8.0 : small_tiles <= 256 ? 7.6 : 9.5);
   if (M <= 128) best = std::min(best, mxfp4_regres_time(M, N, K) * (K <= 4096 ? 0.68 : 0.8));
+  *us = best;
   best *= K <= 2048 ? 0.9 : 0.92;
   if (fp4_format == DQ_FP4_SIMPLE && tiles >= 96) best *= 1.1;
   int split = 1;
@@ -500,15 +502,33 @@ static int mxfp4_ksplit(int M, int N, int K, int fp4_format) {
     const double rate = wgs <= 256 ? 7.0 + 0.002 * (double)wgs + 0.016 * (double)std::max(0L, wgs - 200) : 9.3 * rounds(wgs);
     const double t = 7.9 + 4.3 * (double)((wgs - 1) / 256) + 1e-3 * rate * 128 * ((units + s - 1) / s) + (double)s * M * N * 4 / 2.23e6 +
                      (N % 4 == 0 ? 0.0 : fp4_format == DQ_FP4_SIMPLE ? 4.6 : 3.4);
-    if (t < best) best = t, split = s;
+    if (t < best) best = *us = t, split = s;
   }
   return split;
+}
+
+// With a workspace, which is what allows a row other bits than those of a large product: how the call runs, K over the waves
+// of a workgroup or cut in so many slices.  The former needs no second kernel and no sums in memory, which is most of what a
+// small call takes: 110 shapes of 81 to 400 rows, N 1500 to 25500, K 512 to 6100, of which 41 come here, 1.41 times as fast in the
+// mean and 0.99 in the worst (M = 101, N = 1696, K = 3456 18 -> 8.4 us, M = 204, N = 2912, K = 3328 20 -> 14).  N % 4 == 0 is
+// what the estimate was fitted on; beyond K = 6144 a workgroup's own walk is long and the slices are as fast (M = 298, N = 2528,
+// K = 9728: 31 and 30 us).  Below K = 1024 there is no workspace of two slices to name, and where nothing would be cut none is
+// asked for from K = 4096 on, where the register-resident kernel or one round of small tiles is near.
+struct Mxfp4Plan {
+  int split;
+  bool kwaves;
+};
+static Mxfp4Plan mxfp4_plan(int M, int N, int K, int fp4_format) {
+  double us;
+  const int split = mxfp4_ksplit(M, N, K, fp4_format, &us);
+  const bool kwaves = us > 0.0 && N % 4 == 0 && K >= 1024 && K <= (split > 1 ? 6144 : 4095) && mxfp4_kwaves_time(M, N, K) < 0.93 * us;
+  return {split, kwaves};
 }
 
 // K over the waves of a workgroup: from 17 to 64 rows always (31 shapes: 0.98 to 3.6 times as fast as the register-resident
 // kernel's passes or the tiled GEMM; M = 64, N = K = 8192 49 -> 20 us, M = 60, N = 2976, K = 4352 21 -> 9), below where it is a
 // fifth ahead of the register-resident kernel's estimate (M = 14, N = 2168, K = 13760 22 -> 14; two rows stay with dot
-// products).  From 65 rows on with K % 128 == 0 a row keeps the bits that it has in a large product, or K is cut; otherwise,
+// products).  From 65 rows on with K % 128 == 0 a row keeps the bits that it has in a large product, or mxfp4_plan decides; otherwise,
 // and while the tiles of 128 x 256 are few, against the 7.5 us a thousand k of the register-staged kernel (M = 101, N = 4336,
 // K = 4800 39 -> 17 us, M = 254, N = 2176, K = 6336 53 -> 22, M = 282, N = 4024, K = 9408 82 -> 47).
 static bool mxfp4_by_kwaves(int M, int N, int K) {
@@ -536,7 +556,14 @@ static int gemm_bf16_mxfp4(const char* fn, const void* A, const void* B, const v
     const int rc = mxfp4_gemm_kwaves(A, B, Scale, Bias, C, M, N, K, fp4_format, scale_bias, (hipStream_t)stream);
     if (rc <= 0) return rc;
   }
-  if (workspace && split == 0) split = mxfp4_ksplit(M, N, K, fp4_format);
+  if (workspace && split == 0) {
+    const Mxfp4Plan plan = mxfp4_plan(M, N, K, fp4_format);
+    if (plan.kwaves) {
+      const int rc = mxfp4_gemm_kwaves(A, B, Scale, Bias, C, M, N, K, fp4_format, scale_bias, (hipStream_t)stream);
+      if (rc <= 0) return rc;
+    }
+    split = plan.split;
+  }
   while (split > 1 && (size_t)split * M * N * sizeof(float) > workspace_bytes) --split;
   if (split > 1) {
     const int rc = mxfp4_gemm_ksplit(A, B, Scale, Bias, C, workspace, M, N, K, fp4_format, scale_bias, split, (hipStream_t)stream);
@@ -560,8 +587,10 @@ extern "C" int call_dequant_gemm_bf16_mxfp4(const void* A, const void* B, const 
 
 extern "C" size_t dq_mxfp4_workspace_bytes(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0 || K % 64 != 0) return 0;
-  const int split = mxfp4_ksplit(M, N, K, DQ_FP4_E2M1);
-  return split > 1 ? (size_t)split * M * N * sizeof(float) : 0;
+  const Mxfp4Plan plan = mxfp4_plan(M, N, K, DQ_FP4_E2M1);
+  // that a call comes with room is what allows an order of the sums other than a large product's: two slices' where none is used
+  const int slices = plan.split > 1 ? plan.split : plan.kwaves ? 2 : 0;
+  return (size_t)slices * M * N * sizeof(float);
 }
 
 extern "C" int call_dequant_gemm_bf16_mxfp4_ws(const void* A, const void* B, const void* Scale, const void* Bias, void* C,
