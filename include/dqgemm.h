@@ -354,6 +354,14 @@ int call_gemm_plain(const void* A, const void* B, void* C, void* Workspace, int 
  * operands hold this chip below the clock its published peak assumes, and the figure says by how much. */
 int call_mfma_rate(const void* Operands, void* Out, int in_dtype, int workgroups, int iters, dq_stream_t stream);
 
+/* What the library's choice is, for tests and measurements (host code only). */
+enum dq_operands { DQ_OPERANDS_F16_UINT4 = 0, DQ_OPERANDS_BF16_MXFP4 = 1, DQ_OPERANDS_INT8_INT4 = 2, DQ_OPERANDS_INT8_INT2 = 3 };
+
+/* The form (0 .. 4: 16, 32, 32, 48, 64 activation rows by 32, 32, 64, 64, 64 weight rows, on 8, 8, 4, 4, 4 waves) on which
+ * the default dispatch runs a call with K over the waves of a workgroup, or -1 where it runs another kernel.  group and mode:
+ * W4A16's, else 0; room: whether the call brings the workspace asked for; row-major 2-bit weights, 16-byte aligned operands. */
+int dq_kwaves_form(int operands, int M, int N, int K, int group, int mode, int room);
+
 #ifdef __cplusplus
 }
 #endif

@@ -50,13 +50,16 @@ int w4_f16_gemm(const void* A, const void* B, const void* S, const void* Z, void
 int i2_gemm(const void* A, const void* B, void* C, int M, int N, int K, int convention, int layout, const void* s_a,
             float s_w, int bitnet_epilogue, int kwaves, hipStream_t stream);
 int i2_kwaves_form(int M, int N, int K);
+int i4_kwaves_form(int M, int N, int K);
 double mxfp4_kwaves_time(int M, int N, int K);
+int mxfp4_kwaves_form(int M, int N, int K);
 int mxfp4_gemm_kwaves(const void* A, const void* B, const void* S, const void* Bias, void* C, int M, int N, int K, int fmt,
                       int scale_bias, hipStream_t stream);
 int w4_f16_gemm_ksplit(const void* A, const void* B, const void* S, const void* Z, void* C, void* parts, int M, int N, int K,
                        int group, int mode, int layout, int split, hipStream_t stream);
 double w4_tiled_time(int M, int N, int K);
 double w4_kwaves_time(int M, int N, int K);
+int w4_kwaves_form(int M, int N, int K);
 int w4_f16_gemm_kwaves(const void* A, const void* B, const void* S, const void* Z, void* C, int M, int N, int K, int group,
                        int mode, int layout, hipStream_t stream);
 int wlow_gemv(const void* A, const void* B, const void* Scale, const void* Zeros, void* C, int M, int N, int K, int group,
@@ -279,6 +282,8 @@ static double w4a16_stream_time(int M, int N, int K, int split) {
 // over workgroups and 39 so, nor M = 36, N = 15416, K = 4608, 20 and 24).
 static bool w4a16_by_kwaves(int M, int N, int K, int group, int mode, bool room) {
   if (M < 3) return false;
+  // a row of scales holds a window of eight groups (modes without scales: any)
+  if (mode >= W4_SCALE && (group == K || group < 32 || group > 4096 || K / group < 8)) return false;
   if (K % 256 == 0) {
     if (M > 128 || (M <= 16 && N % 16 == 0 && group == 128 && (K == 2048 || K == 4096 || K == 8192))) return false;
     return w4_kwaves_time(M, N, K) < (M <= 32 ? 0.85 : 0.78) * w4a16_stream_time(M, N, K, room ? w4a16_stream_split(M, N, K, group, mode, w4a16_stream_config(M, N)) : 1);
@@ -532,7 +537,7 @@ static Mxfp4Plan mxfp4_plan(int M, int N, int K, int fp4_format) {
 // and while the tiles of 128 x 256 are few, against the 7.5 us a thousand k of the register-staged kernel (M = 101, N = 4336,
 // K = 4800 39 -> 17 us, M = 254, N = 2176, K = 6336 53 -> 22, M = 282, N = 4024, K = 9408 82 -> 47).
 static bool mxfp4_by_kwaves(int M, int N, int K) {
-  if (M < 3) return false;
+  if (M < 3 || K < 512) return false;  // a row of scales holds a window
   if (M > 64)
     return K % 128 != 0 && half_tiles(M, N) < 96 && mxfp4_kwaves_time(M, N, K) < 0.95 * (2.0 + 7.5e-3 * K);
   return M > 16 || mxfp4_kwaves_time(M, N, K) < 0.8 * mxfp4_regres_time(M, N, K);
@@ -862,6 +867,19 @@ extern "C" int call_gemm_int8xint4(const void* A, const void* B, void* C, int M,
   }
   return i4_gemm(A, B, C, M, N, K, decode, a_packed, transposed & 1,
                  variant_bits(transposed) & DQ_I4_KERNEL_TILED, (hipStream_t)stream);
+}
+
+extern "C" int dq_kwaves_form(int operands, int M, int N, int K, int group, int mode, int room) {
+  if (M <= 0 || N <= 0 || K <= 0) return -1;
+  switch (operands) {
+    case DQ_OPERANDS_F16_UINT4:
+      return K % 128 == 0 && w4a16_by_kwaves(M, N, K, group, mode, room != 0) ? w4_kwaves_form(M, N, K) : -1;
+    case DQ_OPERANDS_BF16_MXFP4:
+      return K % 64 == 0 && (mxfp4_by_kwaves(M, N, K) || (room && mxfp4_plan(M, N, K, DQ_FP4_E2M1).kwaves)) ? mxfp4_kwaves_form(M, N, K) : -1;
+    case DQ_OPERANDS_INT8_INT4: return K % 128 == 0 ? i4_kwaves_form(M, N, K) : -1;
+    case DQ_OPERANDS_INT8_INT2: return K % 128 == 0 ? i2_kwaves_form(M, N, K) : -1;
+    default: return -1;
+  }
 }
 
 extern "C" int call_gemv_int8xint1(const void* A, const void* B, void* C, int M, int N, int K, int convention, int layout,

@@ -130,11 +130,12 @@ int mxfp4_gemm(const void* A, const void* B, const void* S, const void* Bias, vo
 static constexpr gemm::KwavesCosts kKwavesMx = {{2.2, 0.97, 0.88, false}, {2.65, 0.77, 1.03, false}, {3.37, 0.47, 1.67, false},
                                                 {3.11, 1.54, 2.34, true}, {3.15, 2.07, 2.44, true}};
 double mxfp4_kwaves_time(int M, int N, int K) { return gemm::kwaves_pick(kKwavesMx, M, N, K).us; }
+int mxfp4_kwaves_form(int M, int N, int K) { return gemm::kwaves_pick(kKwavesMx, M, N, K).form; }
 int mxfp4_gemm_kwaves(const void* A, const void* B, const void* S, const void* Bias, void* C, int M, int N, int K, int fmt,
                       int scale_bias, hipStream_t stream) {
   Params p = gemm::make_params(A, B, S, nullptr, Bias, C, M, N, K);
   p.p0 = 127 - scale_bias;
-  const int form = gemm::kwaves_pick(kKwavesMx, M, N, K).form;
+  const int form = mxfp4_kwaves_form(M, N, K);
 #define DQ_MX(FMT_)                                                                                \
   do {                                                                                             \
     if (!gemm::kwaves_takes<MxPolicy<FMT_, false>>(p)) return 1;                                   \

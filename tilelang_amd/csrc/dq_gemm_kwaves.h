@@ -237,7 +237,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_kernel_kwaves(const Param
   }
 }
 
-// 1: a shape that the kernel does not take.
+// Whether the kernel takes the call at all
 template <class P>
 bool kwaves_takes(const Params& p) {
   const size_t a_bytes = (size_t)p.M * (p.ldk / P::kKPerBlock) * kARowBytes;
@@ -246,6 +246,19 @@ bool kwaves_takes(const Params& p) {
   if (P::kScaleDma == 1) return p.K >= 512;  // a row of scales holds a window
   if (P::kScaleDma >= 2) return p.p0 >= 5 && p.p0 <= 12 && (p.K >> p.p0) >= 8 && (((size_t)p.S | (size_t)p.Z) & 1) == 0;
   return true;
+}
+
+// The forms that are built: activation rows / 8 and blocks of 32 weight rows of a workgroup, its waves.
+struct KwavesForm {
+  int al, nb, waves;
+};
+constexpr KwavesForm kKwavesForms[] = {{2, 1, 8}, {4, 1, 8}, {4, 2, 4}, {6, 2, 4}, {8, 2, 4}};
+constexpr int kKwavesFormCount = 5;
+
+// Workgroups of a call: passes over the rows, each of whole groups of eight sets of weight rows (one per XCD)
+inline long kwaves_workgroups(const KwavesForm& f, int M, int N) {
+  const long passes = ((long)M + 8 * f.al - 1) / (8 * f.al), sets = ((long)N + 32 * f.nb - 1) / (32 * f.nb);
+  return passes * ((sets + 7) / 8 * 8);
 }
 
 template <class P, int AL, int NB, int kWaves>
@@ -259,19 +272,15 @@ int launch_kwaves_tile(Params p, hipStream_t stream) {
   auto kern = gemm_kernel_kwaves<P, AL, NB, kWaves>;
   static bool lds_limit_raised[kMaxDevices];
   if (raise_lds_limit<kLds>(kern, lds_limit_raised)) return -1;
-  hipLaunchKernelGGL(kern, dim3((p.tiles_n + 7) / 8 * 8 * p.tiles_m), dim3(64 * kWaves), kLds, stream, p);
+  hipLaunchKernelGGL(kern, dim3((unsigned)kwaves_workgroups(KwavesForm{AL, NB, kWaves}, p.M, p.N)), dim3(64 * kWaves), kLds, stream, p);
   DQ_CHECK_HIP(hipGetLastError());
   return 0;
 }
 
-// The forms that are built, and what a call takes on each (us): start + rounds x (round + K / 1000 x per_k), fitted over some
-// hundred shapes a format (rows 2 to 500, N 1500 to 28500, K 1024 to 14300; mean error 5 to 9 %).  Two workgroups of four waves
-// share a CU, so their rounds of 256 run into each other; rounds of eight waves are counted whole.
-struct KwavesForm {
-  int al, nb, waves;
-};
-constexpr KwavesForm kKwavesForms[] = {{2, 1, 8}, {4, 1, 8}, {4, 2, 4}, {6, 2, 4}, {8, 2, 4}};
-constexpr int kKwavesFormCount = 5;
+// What a call takes on each form (us): start + rounds x (round + K / 1000 x per_k), fitted over some hundred shapes a format
+// (rows 2 to 500, N 1500 to 28500, K 1024 to 14300; mean error 5 to 9 %), where the form that they pick is 0.3 to 0.7 % slower in
+// the mean than the best of the five.  Two workgroups of four waves share a CU, so their rounds of 256 run into each other;
+// rounds of eight waves are counted whole.
 struct KwavesCost {
   double start, round, per_k;
   bool smooth;
@@ -285,9 +294,8 @@ struct KwavesPick {
 inline KwavesPick kwaves_pick(const KwavesCosts& costs, int M, int N, int K) {
   KwavesPick best{-1, 1e30};
   for (int i = 0; i < kKwavesFormCount; ++i) {
-    const KwavesForm f = kKwavesForms[i];
     if (i == 0 && M > 16) continue;  // passes of 16 rows are never the best
-    const long wgs = ((long)M + 8 * f.al - 1) / (8 * f.al) * (((long)N + 32 * f.nb - 1) / (32 * f.nb) + 7) / 8 * 8;
+    const long wgs = kwaves_workgroups(kKwavesForms[i], M, N);
     const double whole = (double)((wgs + 255) / 256);
     const double rounds = costs[i].smooth ? (wgs <= 256 ? 1.0 : 0.5 * ((double)wgs / 256.0 + whole)) : whole;
     const double us = costs[i].start + rounds * (costs[i].round + costs[i].per_k * K * 1e-3);

@@ -9,6 +9,7 @@ static constexpr gemm::KwavesCosts kKwavesW4 = {{2.55, 0.92, 1.16, true}, {2.68,
                                                 {2.81, 2.41, 2.84, true}, {3.68, 1.91, 3.1, true}};
 
 double w4_kwaves_time(int M, int N, int K) { return gemm::kwaves_pick(kKwavesW4, M, N, K).us; }
+int w4_kwaves_form(int M, int N, int K) { return gemm::kwaves_pick(kKwavesW4, M, N, K).form; }
 
 // 1: not a shape of that kernel
 int w4_f16_gemm_kwaves(const void* A, const void* B, const void* S, const void* Z, void* C, int M, int N, int K, int group,
@@ -16,7 +17,7 @@ int w4_f16_gemm_kwaves(const void* A, const void* B, const void* S, const void* 
   Params p = gemm::make_params(A, B, S, Z, nullptr, C, M, N, K);
   p.p0 = (group == K) ? 31 : (31 - __builtin_clz(group));
   p.p1 = K / group;
-  const int form = gemm::kwaves_pick(kKwavesW4, M, N, K).form;
+  const int form = w4_kwaves_form(M, N, K);
 #define DQ_W4(MODE_)                                                                                         \
   do {                                                                                                       \
     if (!gemm::kwaves_takes<W4F16Policy<MODE_, false>>(p)) return 1;                                         \
