@@ -514,8 +514,8 @@ static int mxfp4_ksplit(int M, int N, int K, int fp4_format, double* us) {
 
 // With a workspace, which is what allows a row other bits than those of a large product: how the call runs, K over the waves
 // of a workgroup or cut in so many slices.  The former needs no second kernel and no sums in memory, which is most of what a
-// small call takes: 110 shapes of 81 to 400 rows, N 1500 to 25500, K 512 to 6100, of which 41 come here, 1.41 times as fast in the
-// mean and 0.99 in the worst (M = 101, N = 1696, K = 3456 18 -> 8.4 us, M = 204, N = 2912, K = 3328 20 -> 14).  N % 4 == 0 is
+// small call takes (M = 101, N = 1696, K = 3456 18 -> 8.4 us, M = 204, N = 2912, K = 3328 20 -> 14; 4529 shapes of 65 to 600
+// rows, N 256 to 40000: 0.87 of the time without it, 0.6 % of them more than a twentieth slower).  N % 4 == 0 is
 // what the estimate was fitted on; beyond K = 6144 a workgroup's own walk is long and the slices are as fast (M = 298, N = 2528,
 // K = 9728: 31 and 30 us).  Below K = 1024 there is no workspace of two slices to name, and where nothing would be cut none is
 // asked for from K = 4096 on, where the register-resident kernel or one round of small tiles is near.
@@ -526,21 +526,23 @@ struct Mxfp4Plan {
 static Mxfp4Plan mxfp4_plan(int M, int N, int K, int fp4_format) {
   double us;
   const int split = mxfp4_ksplit(M, N, K, fp4_format, &us);
-  const bool kwaves = us > 0.0 && N % 4 == 0 && K >= 1024 && K <= (split > 1 ? 6144 : 4095) && mxfp4_kwaves_time(M, N, K) < 0.93 * us;
+  const bool kwaves = us > 0.0 && N % 4 == 0 && K >= 1024 && K <= (split > 1 ? 6144 : 4095) && mxfp4_kwaves_time(M, N, K) < 0.9 * us;
   return {split, kwaves};
 }
 
-// K over the waves of a workgroup: from 17 to 64 rows always (31 shapes: 0.98 to 3.6 times as fast as the register-resident
-// kernel's passes or the tiled GEMM; M = 64, N = K = 8192 49 -> 20 us, M = 60, N = 2976, K = 4352 21 -> 9), below where it is a
-// fifth ahead of the register-resident kernel's estimate (M = 14, N = 2168, K = 13760 22 -> 14; two rows stay with dot
-// products).  From 65 rows on with K % 128 == 0 a row keeps the bits that it has in a large product, or mxfp4_plan decides; otherwise,
-// and while the tiles of 128 x 256 are few, against the 7.5 us a thousand k of the register-staged kernel (M = 101, N = 4336,
-// K = 4800 39 -> 17 us, M = 254, N = 2176, K = 6336 53 -> 22, M = 282, N = 4024, K = 9408 82 -> 47).
+// K over the waves of a workgroup, to 64 rows: where it is a fifth ahead of the register-resident kernel's estimate, up to 2048 k,
+// where that one's is some way off, a quarter (8438 shapes of 3 to 64 rows, N 256 to 40000, K 512 to 16384: 0.86 of the time
+// of the kernels without this one, 1.4 % of them more than a twentieth slower; M = 64, N = K = 8192 49 -> 20 us, M = 14,
+// N = 2168, K = 13760 22 -> 14; not M = 29, N = 1184, K = 8192, 9.6 us there and 13.6 here, nor M = 4, N = 16384, K = 2048, 7.3
+// and 8.6).  The tiled GEMM is behind all of these.  From 65 rows on with K % 128 == 0 a row keeps the bits that it has in a
+// large product, or mxfp4_plan decides; otherwise, and while the tiles of 128 x 256 are few, against the 7.5 us a thousand k of
+// the register-staged kernel too (M = 101, N = 4336, K = 4800 39 -> 17 us, M = 254, N = 2176, K = 6336 53 -> 22; not M = 95,
+// N = 312, K = 1728, 4.2 and 5.2).
 static bool mxfp4_by_kwaves(int M, int N, int K) {
   if (M < 3 || K < 512) return false;  // a row of scales holds a window
-  if (M > 64)
-    return K % 128 != 0 && half_tiles(M, N) < 96 && mxfp4_kwaves_time(M, N, K) < 0.95 * (2.0 + 7.5e-3 * K);
-  return M > 16 || mxfp4_kwaves_time(M, N, K) < 0.8 * mxfp4_regres_time(M, N, K);
+  const double us = mxfp4_kwaves_time(M, N, K);
+  if (M <= 128 && us >= (K <= 2048 ? 0.72 : 0.8) * mxfp4_regres_time(M, N, K)) return false;
+  return M <= 64 || (K % 128 != 0 && half_tiles(M, N) < 96 && us < 0.95 * (2.0 + 7.5e-3 * K));
 }
 
 static int gemm_bf16_mxfp4(const char* fn, const void* A, const void* B, const void* Scale, const void* Bias, void* C, int M, int N,
