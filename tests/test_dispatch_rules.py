@@ -27,3 +27,12 @@ def test_a_launch_that_fills_the_chip_is_counted_as_it_runs(operands):
 ])
 def test_mxfp4_small_batches_against_the_register_resident_kernel(M, N, K, register_resident, over_waves):
     assert (form(MXFP4, M, N, K) >= 0) == (over_waves < register_resident)
+
+
+@pytest.mark.parametrize("M,N,K,neighbour,over_waves", [
+    (27, 20384, 3840, 10.3, 13.2), (18, 17864, 1792, 7.2, 8.7), (37, 3560, 2048, 5.0, 5.8),   # register-resident
+    (322, 4872, 256, 6.9, 10.4), (1251, 2160, 128, 6.0, 12.4), (70, 21400, 256, 8.3, 10.0), (483, 3800, 256, 6.9, 10.4),  # tiles
+    (20, 3000, 3200, 17, 7.7), (39, 6544, 12288, 39.7, 14.6), (33, 20592, 3328, 22.3, 14.0), (196, 3960, 1280, 9.5, 7.5),
+])
+def test_int8_int2_against_its_neighbours(M, N, K, neighbour, over_waves):
+    assert (form(INT2, M, N, K) >= 0) == (over_waves < neighbour)
