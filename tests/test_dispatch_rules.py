@@ -36,3 +36,11 @@ def test_mxfp4_small_batches_against_the_register_resident_kernel(M, N, K, regis
 ])
 def test_int8_int2_against_its_neighbours(M, N, K, neighbour, over_waves):
     assert (form(INT2, M, N, K) >= 0) == (over_waves < neighbour)
+
+
+@pytest.mark.parametrize("M,N,K,tiles,over_waves", [
+    (35, 14608, 256, 5.0, 5.8), (34, 10472, 256, 4.8, 5.5), (48, 11960, 256, 4.7, 5.4), (46, 9352, 384, 5.7, 5.9),
+    (64, 8192, 8192, 27, 13), (41, 11736, 640, 6.7, 6.3), (22, 13640, 256, 4.6, 4.5), (128, 8192, 8192, 28, 19),
+])
+def test_int8_int4_against_the_tiles(M, N, K, tiles, over_waves):
+    assert (form(INT4, M, N, K) >= 0) == (over_waves < tiles)

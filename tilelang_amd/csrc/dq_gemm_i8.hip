@@ -97,15 +97,16 @@ struct I4xI2Policy : I8Mfma, gemm::NoScale, EPI {
 
 }  // namespace
 
-// K over the waves of a workgroup instead of the tiled kernels: the form, or -1.  To 64 rows always (119 shapes of 2 to 64 rows:
-// 1.2 to 4.8 times as fast; M = 2, N = 2264, K = 8704 25 -> 7 us, M = 64, N = K = 8192 27 -> 13); beyond, where the tiled
+// K over the waves of a workgroup instead of the tiled kernels: the form, or -1.  To 32 rows, from K = 512 on to 64, always (13 000
+// shapes, N 256 to 40000: 0.57 of the time in the mean, 0.1 % more than a twentieth slower; M = 2, N = 2264, K = 8704 25 -> 7 us,
+// M = 64, N = K = 8192 27 -> 13; not M = 35, N = 14608, K = 256, 5.0 us on the tiles and 5.8 here); beyond, where the tiled
 // kernel's tiles of 128 x 64 are few (its times: 3.7 us, and 2.4 + 1.7 a round's share of tiles for a thousand k) and none of
 // 128 x 256 are taken (M = 114, N = 3432, K = 11008 32 -> 14, M = 128, N = K = 8192 28 -> 19, M = 200, N = 8192, K = 4096 18 and 17).
 static constexpr gemm::KwavesCosts kKwavesI4 = {{2.09, 1.0, 0.56, false}, {2.49, 0.89, 0.61, false}, {3.12, 0.91, 0.92, false},
-                                         {2.52, 2.25, 1.28, true}, {3.27, 1.86, 1.32, false}};
+                                                {2.52, 2.25, 1.28, true}, {3.27, 1.86, 1.32, false}};
 int i4_kwaves_form(int M, int N, int K) {
   const gemm::KwavesPick pick = gemm::kwaves_pick(kKwavesI4, M, N, K);
-  if (M <= 64) return pick.form;
+  if (M <= (K < 512 ? 32 : 64)) return pick.form;
   if (gemm::kwaves_big_tiles(M, N) >= gemm::kHalfTileMin) return -1;
   const double tiles = (double)((((long)M + 127) / 128) * (((long)N + 63) / 64));
   return pick.us < 0.95 * (3.7 + 1e-3 * K * (2.4 + 1.7 * tiles / 256.0)) ? pick.form : -1;
