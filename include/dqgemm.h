@@ -355,7 +355,12 @@ int call_gemm_plain(const void* A, const void* B, void* C, void* Workspace, int 
 int call_mfma_rate(const void* Operands, void* Out, int in_dtype, int workgroups, int iters, dq_stream_t stream);
 
 /* What the library's choice is, for tests and measurements (host code only). */
-enum dq_operands { DQ_OPERANDS_F16_UINT4 = 0, DQ_OPERANDS_BF16_MXFP4 = 1, DQ_OPERANDS_INT8_INT4 = 2, DQ_OPERANDS_INT8_INT2 = 3 };
+enum dq_operands { DQ_OPERANDS_F16_UINT4 = 0, DQ_OPERANDS_BF16_MXFP4 = 1, DQ_OPERANDS_INT8_INT4 = 2, DQ_OPERANDS_INT8_INT2 = 3,
+                   DQ_OPERANDS_FP4 = 4 /* bf16 or fp16 x fp4 without block scales */ };
+
+/* The rows of the tiles (96, 128, 192 or 256, by 256 columns) on which the tiled GEMM runs a call by direct-to-LDS loads, 0
+ * where it stages the operands through registers.  group and mode: W4A16's, else 0.  16-byte aligned operands. */
+int dq_tile_rows(int operands, int M, int N, int K, int group, int mode);
 
 /* The form (0 .. 4: 16, 32, 32, 48, 64 activation rows by 32, 32, 64, 64, 64 weight rows, on 8, 8, 4, 4, 4 waves) on which
  * the default dispatch runs a call with K over the waves of a workgroup, or -1 where it runs another kernel.  group and mode:

@@ -44,3 +44,21 @@ def test_int8_int2_against_its_neighbours(M, N, K, neighbour, over_waves):
 ])
 def test_int8_int4_against_the_tiles(M, N, K, tiles, over_waves):
     assert (form(INT4, M, N, K) >= 0) == (over_waves < tiles)
+
+
+FP4 = 4
+
+
+def tile_rows(operands, M, N, K, group=0, mode=0):
+    return _lib.load_library().dq_tile_rows(operands, M, N, K, group, mode)
+
+
+@pytest.mark.parametrize("operands,M,N,K,staged,direct", [
+    (INT4, 273, 8087, 640, 11.7, 15.3), (INT4, 1088, 2631, 1152, 15.7, 18.9), (INT4, 385, 6825, 1408, 17.1, 20.4),
+    (FP4, 409, 5890, 320, 9.7, 11.7), (FP4, 3446, 810, 320, 12.2, 14.2), (MXFP4, 110, 24823, 320, 12.1, 16.0),
+    (INT2, 317, 17954, 640, 21.4, 26.8), (INT2, 2236, 2645, 640, 21.8, 26.3), (INT2, 254, 25530, 896, 24.8, 28.5),
+])
+def test_an_odd_count_of_k_blocks_stays_register_staged(operands, M, N, K, staged, direct):
+    assert staged < direct and tile_rows(operands, M, N, K) == 0
+    # an even count is the direct-to-LDS kernel's, and so is a long K
+    assert tile_rows(operands, M, N, K + (64 if operands in (MXFP4, FP4) else 128)) and tile_rows(operands, M, N, 4224)

@@ -49,6 +49,7 @@ SIGNATURES = {
     "call_gemv_int8xint1": [_vp, _vp, _vp, _i, _i, _i, _i, _i, _vp],
     "call_gemm_plain": [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp],
     "call_mfma_rate": [_vp, _vp, _i, _i, _i, _vp],
+    "dq_tile_rows": [_i, _i, _i, _i, _i, _i],
     "dq_kwaves_form": [_i, _i, _i, _i, _i, _i, _i],
     "call_gemm_mxfp4_mxfp4": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _vp],
 }

@@ -51,6 +51,11 @@ int i2_gemm(const void* A, const void* B, void* C, int M, int N, int K, int conv
             float s_w, int bitnet_epilogue, int kwaves, hipStream_t stream);
 int i2_kwaves_form(int M, int N, int K);
 int i4_kwaves_form(int M, int N, int K);
+int w4_tile_rows(int M, int N, int K, int group, int mode);
+int mxfp4_tile_rows(int M, int N, int K);
+int fp4_tile_rows(int M, int N, int K);
+int i4_tile_rows(int M, int N, int K);
+int i2_tile_rows(int M, int N, int K);
 double mxfp4_kwaves_time(int M, int N, int K);
 int mxfp4_kwaves_form(int M, int N, int K);
 int mxfp4_gemm_kwaves(const void* A, const void* B, const void* S, const void* Bias, void* C, int M, int N, int K, int fmt,
@@ -869,6 +874,18 @@ extern "C" int call_gemm_int8xint4(const void* A, const void* B, void* C, int M,
   }
   return i4_gemm(A, B, C, M, N, K, decode, a_packed, transposed & 1,
                  variant_bits(transposed) & DQ_I4_KERNEL_TILED, (hipStream_t)stream);
+}
+
+extern "C" int dq_tile_rows(int operands, int M, int N, int K, int group, int mode) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  switch (operands) {
+    case DQ_OPERANDS_F16_UINT4: return group > 0 ? w4_tile_rows(M, N, K, group, mode) : 0;
+    case DQ_OPERANDS_BF16_MXFP4: return mxfp4_tile_rows(M, N, K);
+    case DQ_OPERANDS_INT8_INT4: return i4_tile_rows(M, N, K);
+    case DQ_OPERANDS_INT8_INT2: return i2_tile_rows(M, N, K);
+    case DQ_OPERANDS_FP4: return fp4_tile_rows(M, N, K);
+    default: return 0;
+  }
 }
 
 extern "C" int dq_kwaves_form(int operands, int M, int N, int K, int group, int mode, int room) {

@@ -1223,9 +1223,23 @@ bool dma_eligible(const Params& p) {
 // int8 x int4 31.9 against 33.4 us).  The int8 x 2-bit policy gains from 160 tiles on only (N = 8192, K = 5120: 128 tiles
 // 32 against 30.3 us, 256 tiles 36 against 45).
 constexpr int kHalfTileMin = 96;
+
+// An odd count of k-blocks, where the register-staged kernel's tiles of 128 x 128, two in place of one here, just fill their
+// rounds and K is short: it stays ahead (us, there and here: int8 x int4 to 127 tiles and 16 k-blocks, M = 273, N = 8087, K = 640
+// 11.7 and 15.3, 455 shapes 1.08 in the mean; the 16-bit operands to eight, M = 409, N = 5890, K = 320 9.7 and 11.7, 503 shapes
+// 1.04; int8 x 2-bit at 193 to 256 tiles and to eight, M = 317, N = 17954, K = 640 21.4 and 26.8, 274 shapes 1.03).
+template <class P>
+bool odd_count_stays(const Params& p) {
+  const int blocks = p.K / P::kKPerBlock;
+  const long tiles = tiles_of(p, 128);
+  if (blocks % 2 == 0) return false;
+  constexpr bool kInt = std::is_same<typename P::acc_t, int16_t_>::value;
+  if (kInt && P::kBRowBytes == 32) return tiles > 192 && tiles <= 256 && blocks <= 8;
+  return tiles < 128 && blocks <= (kInt ? 16 : 8);
+}
 template <class P>
 bool dma_half_eligible(const Params& p, int min_tiles = kHalfTileMin) {
-  return !dma_eligible<P>(p) && dma_takes<P>(p) && tiles_of(p, 128) >= min_tiles;
+  return !dma_eligible<P>(p) && dma_takes<P>(p) && tiles_of(p, 128) >= min_tiles && !odd_count_stays<P>(p);
 }
 
 template <class P, int kMBW, int kNBW, int kWavesM = 2, int kKHalves = 1, bool kOdd = false>

@@ -126,6 +126,13 @@ int mxfp4_gemm(const void* A, const void* B, const void* S, const void* Bias, vo
 #undef DQ_MX
 }
 
+int mxfp4_tile_rows(int M, int N, int K) {
+  return gemm::dma_rows<MxPolicy<FP4_E2M1, false>>(gemm::make_params(nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, M, N, K));
+}
+int fp4_tile_rows(int M, int N, int K) {
+  return gemm::dma_rows<Bf16Fp4Policy<FP4_E2M1>>(gemm::make_params(nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, M, N, K));
+}
+
 // K over the waves of a workgroup: what it would take (us), and the launch (1: not a shape of that kernel).  Times of e2m1.
 static constexpr gemm::KwavesCosts kKwavesMx = {{2.2, 0.97, 0.88, false}, {2.65, 0.77, 1.03, false}, {3.37, 0.47, 1.67, false},
                                                 {3.11, 1.54, 2.34, true}, {3.15, 2.07, 2.44, true}};

@@ -41,6 +41,11 @@ int i2_kwaves_form(int M, int N, int K) {
   return M <= 64 || pick.us < 0.94 * i2_small_tiles_time(M, N, K) ? pick.form : -1;
 }
 
+int i2_tile_rows(int M, int N, int K) {
+  return gemm::dma_rows<I2Policy<I2_OFFSET, Int32Out<0, false>, true, false, false>>(
+      gemm::make_params(nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, M, N, K), kI2HalfTileMin);
+}
+
 int i2_gemm(const void* A, const void* B, void* C, int M, int N, int K, int convention, int layout, const void* s_a,
             float s_w, int bitnet_epilogue, int kwaves, hipStream_t stream) {
   gemm::Params p = gemm::make_params(A, B, s_a, nullptr, nullptr, C, M, N, K);

@@ -112,6 +112,10 @@ int i4_kwaves_form(int M, int N, int K) {
   return pick.us < 0.95 * (3.7 + 1e-3 * K * (2.4 + 1.7 * tiles / 256.0)) ? pick.form : -1;
 }
 
+int i4_tile_rows(int M, int N, int K) {
+  return gemm::dma_rows<I4Policy<I4_TWOS, false, Int32Out<8, false>>>(gemm::make_params(nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, M, N, K));
+}
+
 int i4_gemm(const void* A, const void* B, void* C, int M, int N, int K, int decode, int a_packed, int transposed,
             int tiled, hipStream_t stream) {
   Params p = gemm::make_params(A, B, nullptr, nullptr, nullptr, C, M, N, K);

@@ -18,6 +18,14 @@ double w4_tiled_time(int M, int N, int K) {
   return best;
 }
 
+int w4_tile_rows(int M, int N, int K, int group, int mode) {
+  Params p = gemm::make_params(nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, M, N, K);
+  p.p0 = (group == K) ? 31 : (31 - __builtin_clz(group));
+  return mode >= W4_ZEROS_ORIGINAL ? gemm::dma_rows<W4F16Policy<W4_ZEROS_ORIGINAL, false>>(p)
+         : mode >= W4_SCALE        ? gemm::dma_rows<W4F16Policy<W4_SCALE, false>>(p)
+                                   : gemm::dma_rows<W4F16Policy<W4_UNSIGNED, false>>(p);
+}
+
 int w4_f16_gemm(const void* A, const void* B, const void* S, const void* Z, void* C, int M, int N, int K, int group,
                 int mode, int layout, hipStream_t stream) {
   Params p = gemm::make_params(A, B, S, Z, nullptr, C, M, N, K);
