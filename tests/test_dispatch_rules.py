@@ -62,3 +62,9 @@ def test_an_odd_count_of_k_blocks_stays_register_staged(operands, M, N, K, stage
     assert staged < direct and tile_rows(operands, M, N, K) == 0
     # an even count is the direct-to-LDS kernel's, and so is a long K
     assert tile_rows(operands, M, N, K + (64 if operands in (MXFP4, FP4) else 128)) and tile_rows(operands, M, N, 4224)
+
+
+@pytest.mark.parametrize("M,N,K", [(461, 25216, 3072), (860, 20736, 3072), (201, 17152, 4864), (213, 17856, 2304)])
+def test_uint4_groups_of_32_with_zeros_are_not_on_tiles_of_96_rows(M, N, K):
+    """104 us on tiles of 128 rows and 152 on 96 (the first), 149 and 213, 74 and 88, 37 and 44."""
+    assert tile_rows(UINT4, M, N, K, 32, ZEROS) in (128, 192)

@@ -1330,8 +1330,12 @@ int dma_rows(const Params& p, int min_tiles = kHalfTileMin) {
     if (!rows) return 0;
     constexpr int kHeights[4] = {96, 128, 192, 256};
     auto us = [&](int i) { return P::kRowCosts[i].start + dma_rounds(tiles_of(p, kHeights[i])) * (P::kRowCosts[i].round + P::kRowCosts[i].per_k * p.K * 1e-3); };
+    // Scales and zeros of groups of 32 k go with every tile, on four waves: beyond 192 tiles of 96 rows and from 1024 k on the load
+    // unit takes longer over those than the costs say (M = 461, N = 25216, K = 3072 104 us on 128 rows, 152 on 96; 143 shapes 1.02 in
+    // the mean, to 192 tiles 190 shapes 0.94)
+    const bool low = !(P::kScaleDma == 3 && p.p0 == 5 && p.K >= 1024 && tiles_of(p, 96) > 192);
     double best = 0.96 * us(rows == 256 ? 3 : 1);
-    for (int i = 0; i < 3; ++i)
+    for (int i = low ? 0 : 1; i < 3; ++i)
       if (kHeights[i] != rows && us(i) < best) best = us(i), rows = kHeights[i];
   }
   return rows;
