@@ -27,6 +27,7 @@
 #pragma once
 
 #include "dq_common.h"
+#include "dq_scale_walk.h"
 
 #include <type_traits>
 
@@ -702,14 +703,9 @@ __global__ __launch_bounds__(256 * kKHalves, 32 * kMBW * kWavesM <= 128 ? 2 : 1)
   // bytes of a tile (kScaleDma == 1) are two bytes per 64 k, placed as a group of 64 k is
   const int s_gshift = P::kScaleDma >= 2 ? p.p0 : 6;
   const int s_ps = s_gshift - 5;
-  // Rows of an odd count of groups: every other row starts in the middle of a dword.  Dword i of such a row holds groups
-  // 2 i - 1 and 2 i; it is asked for one ahead, where dword i - 1 of the rows between them is, so that both kinds of row have
-  // a group by the time that its tile is due, and dword 0 goes before all others to the slot that is needed last.
   const bool s_odd = kOdd && P::kScaleDma != 0 && ((p.ldk >> s_gshift) & 1) != 0;
   const int s_ahead = s_odd ? -(lane & 1) : 0;  // rows of a tile start at an even one
-  const unsigned s_row = (unsigned)min(n0 + (tid & 255), N - 1) * ((unsigned)(p.ldk >> s_gshift) << 1);  // waves 4..7 repeat 0..3
-  const unsigned s_voff0 = s_row & ~3u, s_voff = s_voff0 + 4u * (s_row >> 1 & 1);
-  const int s_last = s_odd ? (p.ldk >> s_gshift) >> 1 : -1;  // the dword index from which none is ahead
+  const ScaleWalk walk((unsigned)min(n0 + (tid & 255), N - 1), (unsigned)(p.ldk >> s_gshift), s_odd);  // waves 4..7 repeat 0..3
 
   // One tile = kSOps + kAOps + kBOps DMA instructions per thread: first the scale dword(s) (row tid) if one is due,
   // then the A chunks, then the packed-B chunks.  Two halves: waves 0 .. 3 bring the scales and waves 4 .. 7 the zeros.
@@ -722,7 +718,7 @@ __global__ __launch_bounds__(256 * kKHalves, 32 * kMBW * kWavesM <= 128 ? 2 : 1)
       if constexpr (P::kScaleDma != 0) {
         const int quad = (kb * kStageTiles) >> s_ps;
         dma4_unless(kHalves && kh != op ? 1 : (kb * kStageTiles) & ((1 << s_ps) - 1),
-                    lds0 + kRing + op * 4096 + (quad & 3) * 1024 + (wave & 3) * 256, quad == s_last ? s_voff0 : s_voff,
+                    lds0 + kRing + op * 4096 + (quad & 3) * 1024 + (wave & 3) * 256, walk.from(quad),
                     (const unsigned char*)(op == 0 ? p.S : p.Z) + (size_t)quad * 4);
       }
     } else if (op < kSOps + kAOps) {
@@ -737,7 +733,7 @@ __global__ __launch_bounds__(256 * kKHalves, 32 * kMBW * kWavesM <= 128 ? 2 : 1)
     if constexpr (P::kScaleDma != 0) {
 #pragma unroll
       for (int op = 0; op < kSOps; ++op)
-        dma4_unless(s_odd && !(kHalves && kh != op) ? 0 : 1, lds0 + kRing + op * 4096 + 3 * 1024 + (wave & 3) * 256, s_voff0, op == 0 ? p.S : p.Z);
+        dma4_unless(s_odd && !(kHalves && kh != op) ? 0 : 1, lds0 + kRing + op * 4096 + 3 * 1024 + (wave & 3) * 256, walk.start, op == 0 ? p.S : p.Z);
     }
   };
   // DMA instructions of one tile that may be outstanding while the one before is waited for: the scales come first in a
@@ -782,10 +778,9 @@ __global__ __launch_bounds__(256 * kKHalves, 32 * kMBW * kWavesM <= 128 ? 2 : 1)
   // where the scale of 64-k tile kb lies from s_off on (groups of 32 k: the lane's half of the tile is in s_off)
   auto scale_at = [&](int kb) -> int {
     const int group = (kb << 6) >> s_gshift;
-    const int aligned = ((group >> 1) & 3) * 1024 + (group & 1) * 2;
+    const int aligned = ScaleWalk::aligned(group);
     if constexpr (!kOdd) return aligned;
-    const int ahead = (((group - 1) >> 1) & 3) * 1024 + ((group + 1) & 1) * 2;
-    return aligned + ((ahead - aligned) & s_ahead);
+    return aligned + ((ScaleWalk::one_ahead(group) - aligned) & s_ahead);
   };
   // the LDS read of a scale and the arithmetic on it are separate steps, so that the read can be issued a
   // chunk ahead of its first use
@@ -1184,7 +1179,9 @@ bool dma_takes(const Params& p) {
   // 32-bit lane offsets: A rows are 128 bytes per K block, packed B rows kBRowBytes
   const size_t a_bytes = (size_t)p.M * (p.ldk / P::kKPerBlock) * kARowBytes;
   const size_t b_bytes = (size_t)p.N * (p.ldk / P::kKPerBlock) * P::kBRowBytes;
-  return P::dma_ok(p) && p.K % P::kKPerBlock == 0 && p.K >= 2 * P::kKPerBlock && a_bytes < (1ull << 32) && b_bytes < (1ull << 32);
+  // an odd count of groups and an odd count of rows: the last row's last dword would reach two bytes beyond the scales
+  const bool beyond = P::kScaleDma != 0 && p.N % 2 != 0 && ((p.ldk >> (P::kScaleDma >= 2 ? p.p0 : 6)) & 1) != 0;
+  return P::dma_ok(p) && !beyond && p.K % P::kKPerBlock == 0 && p.K >= 2 * P::kKPerBlock && a_bytes < (1ull << 32) && b_bytes < (1ull << 32);
 }
 
 inline long tiles_of(const Params& p, int rows) { return (long)((p.M + rows - 1) / rows) * ((p.N + BN - 1) / BN) * p.split; }
