@@ -155,15 +155,18 @@ int call_dequant_gemm_bf16_mxfp4(const void* A, const void* B, const void* Scale
 /* The same product with a workspace for partial sums (the form of call_dequantize_gemv_w4a16_ws): where M x N gives
  * the CUs too few tiles, K is cut into slices, their fp32 sums go to the workspace and a second kernel adds them in
  * slice order, with the bias, and rounds once.  split: 0 the library's choice (then dq_mxfp4_workspace_bytes(M, N, K)
- * bytes are what it asks for; 0: the kernels of the entry point without a workspace; DQ_FP4_SIMPLE leaves some of them unused or would take more), 1 none, up to 16 that many where
- * the shape allows it (K % 128 == 0, a slice at least 128 k, M * N a multiple of four, Scale at a multiple of four bytes;
- * else the call is not cut).  A smaller workspace lowers the count.  Workspace: 16-byte aligned, contents undefined afterwards, not to be shared by calls that
- * overlap in time.
+ * bytes are what it asks for; 0: the kernels of the entry point without a workspace; DQ_FP4_SIMPLE leaves some of them
+ * unused or would take more), 1 none, nor K over the waves of a workgroup, up to 16 that many where the shape allows it
+ * (K % 128 == 0, a slice at least 128 k, M * N a multiple of four, Scale at a multiple of four bytes; else the call is not
+ * cut).  A smaller workspace lowers the count.  Workspace: 16-byte aligned, contents undefined afterwards, not to be shared by
+ * calls that overlap in time.
  * A row's bits: the tiled GEMM adds a row's products in one order whatever M is, so a row of any uncut call on it has
  * the same bits.  A cut call groups the sums by slice and may differ from that in the last bf16 bit, as the kernels for
  * fewer rows do; by the library's choice (split 0) no call of up to 80 rows is cut, and the entry point without a
  * workspace never cuts.  Small calls that the choice would cut, and some it would not, run with K over the waves of a
- * workgroup instead where that is faster (81 rows and more, K 1024 to 6144; the workspace stays unused). */
+ * workgroup instead where that is faster (81 rows and more, K 1024 to 6144; the workspace stays unused).  Who wants the
+ * bits of a large product at few rows asks for split = 1, which runs what it ran before that kernel was there: up to 16 rows,
+ * more while passes of 16 stay ahead, the register-resident kernel, else the tiled GEMM. */
 size_t dq_mxfp4_workspace_bytes(int M, int N, int K);
 int call_dequant_gemm_bf16_mxfp4_ws(const void* A, const void* B, const void* Scale, const void* Bias, void* C,
                                     void* Workspace, size_t workspace_bytes, int M, int N, int K, int scale_size,

@@ -348,3 +348,22 @@ def test_scales_that_start_at_any_byte(cuda, M, N, K, split, offset):
     torch.cuda.synchronize()
     assert bool((ws == 255).all())  # neither call was cut
     assert torch.equal(results[0].view(torch.int16), results[1].view(torch.int16))
+
+
+@pytest.mark.parametrize("M,N,K", [(64, 20000, 1280), (30, 20000, 768), (254, 2176, 6336), (95, 6000, 2304)])
+def test_one_slice_asked_for_keeps_the_bits_of_a_large_product(cuda, M, N, K):
+    """split = 1: the rows of a call on the tiled GEMM have the bits that they have in a product of many rows, also where the
+    library's choice would run K over the waves of a workgroup (real-valued operands, so that another order would show)."""
+    from tilelang_amd import _lib
+
+    assert _lib.load_library().dq_kwaves_form(1, M, N, K, 0, 0, 1) >= 0
+    gen = torch.Generator(device=cuda).manual_seed(K)
+    A = torch.randn((1100, K), generator=gen, device=cuda).bfloat16()
+    B = torch.randint(0, 256, (N, K // 2), generator=gen, device=cuda).to(torch.uint8)
+    S = torch.randint(119, 128, (N, K // 32), generator=gen, device=cuda).to(torch.uint8)
+    out = []
+    for rows in (1100, M):
+        C = torch.empty((rows, N), dtype=torch.bfloat16, device=cuda)
+        assert _cut_call(A, B, S, None, C, None, 0, rows, N, K, "e2m1", 1) == 0, _lib.last_error()
+        out.append(C)
+    assert torch.equal(out[0][:M].view(torch.int16), out[1].view(torch.int16))

@@ -564,7 +564,7 @@ static int gemm_bf16_mxfp4(const char* fn, const void* A, const void* B, const v
   if (scale_bias < 0 || scale_bias > 255) DQ_FAIL("%s: scale_bias must be in 0..255 (got %d)", fn, scale_bias);
   if (!aligned16(A) || !aligned16(B) || !aligned16(C) || (Bias && !aligned16(Bias)))
     DQ_FAIL("%s: A, B, Bias and C must be 16-byte aligned", fn);
-  if (split <= 1 && mxfp4_by_kwaves(M, N, K)) {
+  if (split == 0 && mxfp4_by_kwaves(M, N, K)) {
     const int rc = mxfp4_gemm_kwaves(A, B, Scale, Bias, C, M, N, K, fp4_format, scale_bias, (hipStream_t)stream);
     if (rc <= 0) return rc;
   }
@@ -593,7 +593,7 @@ static int gemm_bf16_mxfp4(const char* fn, const void* A, const void* B, const v
 extern "C" int call_dequant_gemm_bf16_mxfp4(const void* A, const void* B, const void* Scale, const void* Bias, void* C,
                                             int M, int N, int K, int scale_size, int fp4_format, int scale_bias,
                                             dq_stream_t stream) {
-  return gemm_bf16_mxfp4("call_dequant_gemm_bf16_mxfp4", A, B, Scale, Bias, C, M, N, K, scale_size, fp4_format, scale_bias, 1, nullptr,
+  return gemm_bf16_mxfp4("call_dequant_gemm_bf16_mxfp4", A, B, Scale, Bias, C, M, N, K, scale_size, fp4_format, scale_bias, 0, nullptr,
                          0, stream);
 }
 
