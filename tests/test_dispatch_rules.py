@@ -1,11 +1,14 @@
 """The library's choice between its kernels, asked of the host code: no GPU.  Where two kernels were timed against each other,
 the shapes are some of those measured, with the times that decided (us)."""
 
+import random
+
 import pytest
 
+import tilelang_amd as tl
 from tilelang_amd import _lib
 
-UINT4, MXFP4, INT4, INT2 = range(4)
+UINT4, MXFP4, INT4, INT2, FP4 = _lib.OPERANDS_F16_UINT4, _lib.OPERANDS_BF16_MXFP4, _lib.OPERANDS_INT8_INT4, _lib.OPERANDS_INT8_INT2, _lib.OPERANDS_FP4
 SCALE, ZEROS = 3, 5
 
 
@@ -46,8 +49,6 @@ def test_int8_int4_against_the_tiles(M, N, K, tiles, over_waves):
     assert (form(INT4, M, N, K) >= 0) == (over_waves < tiles)
 
 
-FP4 = 4
-
 
 def tile_rows(operands, M, N, K, group=0, mode=0):
     return _lib.load_library().dq_tile_rows(operands, M, N, K, group, mode)
@@ -68,3 +69,33 @@ def test_an_odd_count_of_k_blocks_stays_register_staged(operands, M, N, K, stage
 def test_uint4_groups_of_32_with_zeros_are_not_on_tiles_of_96_rows(M, N, K):
     """104 us on tiles of 128 rows and 152 on 96 (the first), 149 and 213, 74 and 88, 37 and 44."""
     assert tile_rows(UINT4, M, N, K, 32, ZEROS) in (128, 192)
+
+
+@pytest.mark.parametrize("M,N,K", [(58, 2528, 3840), (100, 2000, 3712), (90, 2528, 4096)])
+def test_uint4_names_room_only_where_it_is_used(M, N, K):
+    lib = _lib.load_library()
+    takes = [form(UINT4, M, N, K, 128, mode, room) >= 0 for mode in (SCALE, ZEROS) for room in (0, 1)]
+    assert all(takes) and lib.dq_w4a16_workspace_bytes(M, N, K, 128, SCALE) == lib.dq_w4a16_workspace_bytes(M, N, K, 128, ZEROS) == 0
+
+
+def test_a_call_that_is_named_no_room_runs_as_with_it():
+    """What the workspace query and the call decide on, over the range of the layers: where K goes over the waves with room, none is
+    asked for, and the call without it goes there too."""
+    lib, rng = _lib.load_library(), random.Random(0)
+    seen = 0
+    for _ in range(4000):
+        M, N, K = rng.randint(2, 400), rng.randint(64, 3600) * 8, rng.randint(2, 100) * 128
+        group, mode = rng.choice(((128, SCALE), (128, ZEROS), (64, ZEROS), (1024, SCALE), (128, 0)))
+        if K % group:
+            continue
+        if form(UINT4, M, N, K, group, mode, 1) >= 0:
+            seen += 1
+            assert lib.dq_w4a16_workspace_bytes(M, N, K, group, mode) == 0 and form(UINT4, M, N, K, group, mode, 0) >= 0, (M, N, K, group, mode)
+    assert seen > 300
+
+
+@pytest.mark.parametrize("M,N,K,over_waves", [(101, 1696, 3456, True), (204, 2912, 3328, True), (96, 8192, 8192, False), (600, 4096, 8192, False)])
+def test_mxfp4_kernel_objects_bring_sums_room_only_where_sums_are_written(M, N, K, over_waves):
+    kernel = tl.matmul_bf16_mxfp4(M, N, K)
+    room = [p for p in kernel.params if p.name == "Workspace"]
+    assert len(room) == 1 and (room[0].shape == (16,)) == over_waves == (form(MXFP4, M, N, K) >= 0)

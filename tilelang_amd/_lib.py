@@ -54,6 +54,9 @@ SIGNATURES = {
     "call_gemm_mxfp4_mxfp4": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _vp],
 }
 
+#: dq_operands of include/dqgemm.h: what dq_tile_rows and dq_kwaves_form are asked about
+OPERANDS_F16_UINT4, OPERANDS_BF16_MXFP4, OPERANDS_INT8_INT4, OPERANDS_INT8_INT2, OPERANDS_FP4 = range(5)
+
 #: name -> argtypes of the functions that return a byte count (size_t) and launch nothing
 SIZE_QUERIES = {
     "dq_w4a16_workspace_bytes": [_i, _i, _i, _i, _i],

@@ -251,15 +251,6 @@ static int w4a16_tiled_split(int M, int N, int K, int group, int mode) {
   return split;
 }
 
-extern "C" size_t dq_w4a16_workspace_bytes(int M, int N, int K, int group, int mode) {
-  if (M < 2 || N <= 0 || K <= 0 || group <= 0) return 0;
-  const int cut = w4a16_tiled_split(M, N, K, group, mode);
-  if (cut > 1) return (size_t)cut * M * N * sizeof(float);
-  if (M > 128 && !w4a16_few_tiles(M, N, K)) return 0;
-  const int split = w4a16_stream_split(M, N, K, group, mode, w4a16_stream_config(M, N));
-  return split > 1 ? (size_t)split * M * N * sizeof(float) : 0;
-}
-
 // What the streaming kernel takes (us) to 128 rows in one round of workgroups, cut into `split` slices: fits over 84 shapes (mean
 // error 3 to 6 %).  0: not fitted.
 static double w4a16_stream_time(int M, int N, int K, int split) {
@@ -283,19 +274,33 @@ static double w4a16_stream_time(int M, int N, int K, int split) {
 // K = 11904 84 -> 22; M = 88, N = 7952, K = 3712 42 -> 19), beyond 64 rows while the tiled GEMM's big tiles are few (its small
 // ones take some 10 us a thousand k).  Multiples of 256, to 128 rows where the register-resident kernel declines: where it is a
 // seventh ahead of the streaming kernel's estimate, beyond 32 rows a fifth, which it is in a fourth of the shapes (M = 58,
-// N = 2528, K = 3840 14.2 -> 8.7 us, M = 13, N = 6224, K = 7424 14.1 -> 11.6; not M = 49, N = 5224, K = 13568, 25 us in slices
+// N = 2528, K = 3840 14.2 -> 8.7 us, M = 7, N = 6952, K = 2816 8.9 -> 7.6; not M = 49, N = 5224, K = 13568, 25 us in slices
 // over workgroups and 39 so, nor M = 36, N = 15416, K = 4608, 20 and 24).
 static bool w4a16_by_kwaves(int M, int N, int K, int group, int mode, bool room) {
   if (M < 3) return false;
   // a row of scales holds a window of eight groups (modes without scales: any)
   if (mode >= W4_SCALE && (group == K || group < 32 || group > 4096 || K / group < 8)) return false;
+  if (((size_t)N * K >> 1) >= (1ull << 32) || (size_t)M * K * 2 >= (1ull << 32)) return false;  // 32-bit lane offsets
   if (K % 256 == 0) {
     if (M > 128 || (M <= 16 && N % 16 == 0 && group == 128 && (K == 2048 || K == 4096 || K == 8192))) return false;
-    return w4_kwaves_time(M, N, K) < (M <= 32 ? 0.85 : 0.78) * w4a16_stream_time(M, N, K, room ? w4a16_stream_split(M, N, K, group, mode, w4a16_stream_config(M, N)) : 1);
+    const double us = w4_kwaves_time(M, N, K) / (M <= 32 ? 0.85 : 0.78);
+    // ahead of the slices, room or none (so no room is asked for); without room ahead of the uncut kernel, too
+    return us < w4a16_stream_time(M, N, K, w4a16_stream_split(M, N, K, group, mode, w4a16_stream_config(M, N))) ||
+           (!room && us < w4a16_stream_time(M, N, K, 1));
   }
   if (M <= 4 && K <= 8192) return false;  // the dot-product kernel, which rounds no weight to fp16
   if (M <= 64) return true;
   return half_tiles(M, N) < 96 && w4_kwaves_time(M, N, K) < 2.0 + 9.0e-3 * K;
+}
+
+extern "C" size_t dq_w4a16_workspace_bytes(int M, int N, int K, int group, int mode) {
+  if (M < 2 || N <= 0 || K <= 0 || group <= 0) return 0;
+  if (K % 128 == 0 && w4a16_by_kwaves(M, N, K, group, mode, true)) return 0;
+  const int cut = w4a16_tiled_split(M, N, K, group, mode);
+  if (cut > 1) return (size_t)cut * M * N * sizeof(float);
+  if (M > 128 && !w4a16_few_tiles(M, N, K)) return 0;
+  const int split = w4a16_stream_split(M, N, K, group, mode, w4a16_stream_config(M, N));
+  return split > 1 ? (size_t)split * M * N * sizeof(float) : 0;
 }
 
 static int gemv_w4a16(const char* fn, const void* A, const void* B, const void* Scale, const void* Zeros, void* C, int M, int N,
@@ -601,6 +606,7 @@ extern "C" size_t dq_mxfp4_workspace_bytes(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0 || K % 64 != 0) return 0;
   const Mxfp4Plan plan = mxfp4_plan(M, N, K, DQ_FP4_E2M1);
   // that a call comes with room is what allows an order of the sums other than a large product's: two slices' where none is used
+  // (sixteen bytes do where dq_kwaves_form names a form)
   const int slices = plan.split > 1 ? plan.split : plan.kwaves ? 2 : 0;
   return (size_t)slices * M * N * sizeof(float);
 }
