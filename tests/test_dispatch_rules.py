@@ -99,3 +99,10 @@ def test_mxfp4_kernel_objects_bring_sums_room_only_where_sums_are_written(M, N, 
     kernel = tl.matmul_bf16_mxfp4(M, N, K)
     room = [p for p in kernel.params if p.name == "Workspace"]
     assert len(room) == 1 and (room[0].shape == (16,)) == over_waves == (form(MXFP4, M, N, K) >= 0)
+
+
+@pytest.mark.parametrize("M,N,K,streamed,cut", [(93, 38384, 28160, 501, 679), (135, 16832, 25600, 367, 489), (138, 19706, 14080, 224, 287)])
+def test_uint4_groups_of_32_are_cut_into_one_round_at_most(M, N, K, streamed, cut):
+    room = _lib.load_library().dq_w4a16_workspace_bytes
+    tiles = -(-M // 96) * -(-N // 256)
+    assert streamed < cut and room(M, N, K, 32, ZEROS) // (4 * M * N) * tiles <= 256 < room(M, N, K, 128, ZEROS) // (4 * M * N) * tiles
