@@ -106,3 +106,12 @@ def test_uint4_groups_of_32_are_cut_into_one_round_at_most(M, N, K, streamed, cu
     room = _lib.load_library().dq_w4a16_workspace_bytes
     tiles = -(-M // 96) * -(-N // 256)
     assert streamed < cut and room(M, N, K, 32, ZEROS) // (4 * M * N) * tiles <= 256 < room(M, N, K, 128, ZEROS) // (4 * M * N) * tiles
+
+
+@pytest.mark.parametrize("operands,M,N,K,tiles,over_waves", [
+    (INT4, 3859, 256, 22272, 60, 98), (INT4, 4024, 256, 7168, 23, 35), (INT4, 2019, 592, 15616, 44, 64), (INT4, 1309, 752, 8960, 29, 42),
+    (INT2, 3998, 512, 23040, 68, 111), (INT2, 4037, 192, 20992, 56, 88), (INT2, 1245, 601, 27136, 70, 108), (MXFP4, 2416, 448, 3072, 21, 26),
+    (INT4, 847, 614, 6144, 22, 14), (INT2, 843, 413, 6912, 22, 12),
+])
+def test_many_rows_against_the_tiles(operands, M, N, K, tiles, over_waves):
+    assert (form(operands, M, N, K) >= 0) == (over_waves < tiles)

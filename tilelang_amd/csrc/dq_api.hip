@@ -58,6 +58,7 @@ int i4_tile_rows(int M, int N, int K);
 int i2_tile_rows(int M, int N, int K);
 double mxfp4_kwaves_time(int M, int N, int K);
 int mxfp4_kwaves_form(int M, int N, int K);
+double mxfp4_kwaves_margin(double margin, int M, int K);
 int mxfp4_gemm_kwaves(const void* A, const void* B, const void* S, const void* Bias, void* C, int M, int N, int K, int fmt,
                       int scale_bias, hipStream_t stream);
 int w4_f16_gemm_ksplit(const void* A, const void* B, const void* S, const void* Z, void* C, void* parts, int M, int N, int K,
@@ -539,7 +540,7 @@ struct Mxfp4Plan {
 static Mxfp4Plan mxfp4_plan(int M, int N, int K, int fp4_format) {
   double us;
   const int split = mxfp4_ksplit(M, N, K, fp4_format, &us);
-  const bool kwaves = us > 0.0 && N % 4 == 0 && K >= 1024 && K <= (split > 1 ? 6144 : 4095) && mxfp4_kwaves_time(M, N, K) < 0.9 * us;
+  const bool kwaves = us > 0.0 && N % 4 == 0 && K >= 1024 && K <= (split > 1 ? 6144 : 4095) && mxfp4_kwaves_time(M, N, K) < mxfp4_kwaves_margin(0.9, M, K) * us;
   return {split, kwaves};
 }
 
@@ -555,7 +556,7 @@ static bool mxfp4_by_kwaves(int M, int N, int K) {
   if (M < 3 || K < 512) return false;  // a row of scales holds a window
   const double us = mxfp4_kwaves_time(M, N, K);
   if (M <= 128 && us >= (K <= 2048 ? 0.72 : 0.8) * mxfp4_regres_time(M, N, K)) return false;
-  return M <= 64 || (K % 128 != 0 && half_tiles(M, N) < 96 && us < 0.95 * (2.0 + 7.5e-3 * K));
+  return M <= 64 || (K % 128 != 0 && half_tiles(M, N) < 96 && us < mxfp4_kwaves_margin(0.95, M, K) * (2.0 + 7.5e-3 * K));
 }
 
 static int gemm_bf16_mxfp4(const char* fn, const void* A, const void* B, const void* Scale, const void* Bias, void* C, int M, int N,

@@ -38,7 +38,7 @@ int i2_kwaves_form(int M, int N, int K) {
     if (tiles >= 64 && tiles <= 448 && 7.5 + 1.87e-3 * K * (double)((tiles + 255) / 256) < pick.us) return -1;
   }
   if (const double resident = i2_resident_time(M, N, K); resident > 0.0) return pick.us < 0.96 * resident ? pick.form : -1;
-  return M <= 64 || pick.us < 0.94 * i2_small_tiles_time(M, N, K) ? pick.form : -1;
+  return M <= 64 || pick.us < gemm::kwaves_margin(0.94, M, (size_t)M * K) * i2_small_tiles_time(M, N, K) ? pick.form : -1;
 }
 
 int i2_tile_rows(int M, int N, int K) {

@@ -109,7 +109,7 @@ int i4_kwaves_form(int M, int N, int K) {
   if (M <= (K < 512 ? 32 : 64)) return pick.form;
   if (gemm::kwaves_big_tiles(M, N) >= gemm::kHalfTileMin) return -1;
   const double tiles = (double)((((long)M + 127) / 128) * (((long)N + 63) / 64));
-  return pick.us < 0.95 * (3.7 + 1e-3 * K * (2.4 + 1.7 * tiles / 256.0)) ? pick.form : -1;
+  return pick.us < gemm::kwaves_margin(0.95, M, (size_t)M * K) * (3.7 + 1e-3 * K * (2.4 + 1.7 * tiles / 256.0)) ? pick.form : -1;
 }
 
 int i4_tile_rows(int M, int N, int K) {

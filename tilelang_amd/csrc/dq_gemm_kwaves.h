@@ -304,6 +304,12 @@ inline KwavesPick kwaves_pick(const KwavesCosts& costs, int M, int N, int K) {
   return best;
 }
 
+// The share of a neighbour's estimate that this kernel's has to stay below.  Every set of weight rows reads all of A again: beyond a
+// thousand rows and 8 MiB of it the L2s no longer serve that, which the costs, fitted to 600 rows, do not know (int8, 159 and 151
+// shapes: 0.64 to 0.69 of the neighbour's time where the estimates' ratio is below 0.7, 1.0 to 1.15 of it above, up to 1.6; M = 3859,
+// N = 256, K = 22272 60 us on the tiles of int8 x int4 and 98 here).
+inline double kwaves_margin(double margin, int M, size_t a_bytes) { return M > 1000 && a_bytes > (8u << 20) ? 0.7 * margin : margin; }
+
 template <class P>
 int launch_kwaves(const Params& p, int form, hipStream_t stream) {
   static_assert(sizeof(kKwavesForms) / sizeof(kKwavesForms[0]) == 5, "one case a form");
