@@ -97,7 +97,8 @@ int call_dequantize_gemv_w4a16(const void* A, const void* B, const void* Scale, 
  * up to 16 slices, one workgroup each, writes their fp32 sums to the workspace and adds them in slice order in a
  * second kernel: results do not depend on timing and stay within rounding of the unsplit kernel's.  So it does at more
  * rows, on the tiled GEMM, where the scaled modes leave CUs idle there (M = 202, N = 8928, K = 10752).  A smaller
- * workspace lowers the slice count, NULL / 0 bytes is call_dequantize_gemv_w4a16.  Workspace: 16-byte aligned,
+ * workspace lowers the slice count, NULL / 0 bytes is call_dequantize_gemv_w4a16; where dq_kwaves_form with room names a
+ * form, none is needed.  Workspace: 16-byte aligned,
  * contents undefined afterwards, not to be shared by calls that overlap in time. */
 size_t dq_w4a16_workspace_bytes(int M, int N, int K, int group, int mode);
 int call_dequantize_gemv_w4a16_ws(const void* A, const void* B, const void* Scale, const void* Zeros, void* C,

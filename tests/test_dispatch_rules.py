@@ -71,34 +71,34 @@ def test_uint4_groups_of_32_with_zeros_are_not_on_tiles_of_96_rows(M, N, K):
     assert tile_rows(UINT4, M, N, K, 32, ZEROS) in (128, 192)
 
 
-@pytest.mark.parametrize("M,N,K", [(58, 2528, 3840), (100, 2000, 3712), (90, 2528, 4096)])
-def test_uint4_names_room_only_where_it_is_used(M, N, K):
-    lib = _lib.load_library()
-    takes = [form(UINT4, M, N, K, 128, mode, room) >= 0 for mode in (SCALE, ZEROS) for room in (0, 1)]
-    assert all(takes) and lib.dq_w4a16_workspace_bytes(M, N, K, 128, SCALE) == lib.dq_w4a16_workspace_bytes(M, N, K, 128, ZEROS) == 0
-
-
-def test_a_call_that_is_named_no_room_runs_as_with_it():
-    """What the workspace query and the call decide on, over the range of the layers: where K goes over the waves with room, none is
-    asked for, and the call without it goes there too."""
-    lib, rng = _lib.load_library(), random.Random(0)
-    seen = 0
+def test_a_call_that_brings_no_room_runs_as_with_it():
+    """Over the range of the layers: where K goes over the waves of a workgroup with room, it does so without."""
+    rng, seen = random.Random(0), 0
     for _ in range(4000):
         M, N, K = rng.randint(2, 400), rng.randint(64, 3600) * 8, rng.randint(2, 100) * 128
         group, mode = rng.choice(((128, SCALE), (128, ZEROS), (64, ZEROS), (1024, SCALE), (128, 0)))
-        if K % group:
-            continue
-        if form(UINT4, M, N, K, group, mode, 1) >= 0:
+        if K % group == 0 and form(UINT4, M, N, K, group, mode, 1) >= 0:
             seen += 1
-            assert lib.dq_w4a16_workspace_bytes(M, N, K, group, mode) == 0 and form(UINT4, M, N, K, group, mode, 0) >= 0, (M, N, K, group, mode)
+            assert form(UINT4, M, N, K, group, mode, 0) >= 0, (M, N, K, group, mode)
     assert seen > 300
+
+
+def _room(kernel):
+    return [p.shape[0] for p in kernel.params if p.name == "Workspace"]
+
+
+@pytest.mark.parametrize("M,N,K,over_waves", [(58, 2528, 3840, True), (90, 2528, 4096, True), (16, 4096, 14336, False), (202, 8928, 10752, False)])
+def test_uint4_kernel_objects_bring_room_only_where_sums_are_written(M, N, K, over_waves):
+    lib = _lib.load_library()
+    asked = lib.dq_w4a16_workspace_bytes(M, N, K, 128, SCALE)
+    room = _room(tl.dequantize_gemv(M, N, K, group_size=128, source_format="int", with_scaling=True))
+    assert asked and room == ([] if over_waves else [asked]) and (form(UINT4, M, N, K, 128, SCALE) >= 0) == over_waves
 
 
 @pytest.mark.parametrize("M,N,K,over_waves", [(101, 1696, 3456, True), (204, 2912, 3328, True), (96, 8192, 8192, False), (600, 4096, 8192, False)])
 def test_mxfp4_kernel_objects_bring_sums_room_only_where_sums_are_written(M, N, K, over_waves):
-    kernel = tl.matmul_bf16_mxfp4(M, N, K)
-    room = [p for p in kernel.params if p.name == "Workspace"]
-    assert len(room) == 1 and (room[0].shape == (16,)) == over_waves == (form(MXFP4, M, N, K) >= 0)
+    asked = _lib.load_library().dq_mxfp4_workspace_bytes(M, N, K)
+    assert _room(tl.matmul_bf16_mxfp4(M, N, K)) == [16 if over_waves else asked] and (form(MXFP4, M, N, K) >= 0) == over_waves
 
 
 @pytest.mark.parametrize("M,N,K,streamed,cut", [(93, 38384, 28160, 501, 679), (135, 16832, 25600, 367, 489), (138, 19706, 14080, 224, 287)])

@@ -299,7 +299,6 @@ static bool w4a16_by_kwaves(int M, int N, int K, int group, int mode, bool room)
 
 extern "C" size_t dq_w4a16_workspace_bytes(int M, int N, int K, int group, int mode) {
   if (M < 2 || N <= 0 || K <= 0 || group <= 0) return 0;
-  if (K % 128 == 0 && w4a16_by_kwaves(M, N, K, group, mode, true)) return 0;
   const int cut = w4a16_tiled_split(M, N, K, group, mode);
   if (cut > 1) return (size_t)cut * M * N * sizeof(float);
   if (M > 128 && !w4a16_few_tiles(M, N, K)) return 0;

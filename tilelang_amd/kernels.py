@@ -187,6 +187,9 @@ def dequantize_gemv(
     ws_bytes = 0
     if variant < 0 and not weight_fragments:
         ws_bytes = int(_lib.load_library().dq_w4a16_workspace_bytes(M, N, K, group_size, mode))
+        # K over the waves of a workgroup writes no sums
+        if ws_bytes and variant == -1 and _lib.load_library().dq_kwaves_form(_lib.OPERANDS_F16_UINT4, M, N, K, group_size, mode, 1) >= 0:
+            ws_bytes = 0
     workspace_idx = []
     if ws_bytes:
         workspace_idx.append(len(params))
