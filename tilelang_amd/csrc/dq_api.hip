@@ -167,9 +167,6 @@ extern "C" int init(void) {
   return 0;
 }
 
-// Tiles of 128 x 256
-static long half_tiles(int M, int N) { return (((long)M + 127) / 128) * (((long)N + 255) / 256); }
-
 // ---- the streaming small-batch kernel's default configuration and K split ------------------------------
 // Which configuration the default dispatch runs at M rows (see w4a16_stream for the numbering).
 static int w4a16_stream_config(int M, int N) {

@@ -306,4 +306,7 @@ struct RowReduce {
   }
 };
 
+// Tiles of 128 x 256 of an M x N result, which the direct-to-LDS GEMM takes from some hundred of them on
+inline long half_tiles(int M, int N) { return (((long)M + 127) / 128) * (((long)N + 255) / 256); }
+
 }  // namespace dq

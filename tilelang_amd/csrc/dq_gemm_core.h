@@ -69,7 +69,6 @@ struct Params {
   int tiles_m, tiles_n;
   int p0, p1;        // policy specific integers (e.g. scale exponent offset, group shift)
   float f0;          // policy specific float (e.g. 1 / weight scale)
-  int kwaves;        // host only: the form of dq_gemm_kwaves.h that the call goes to, or -1
 };
 
 // Workgroup id -> output tile.  With T tiles and 8 XCDs, XCD x (ids x, x+8, ...) gets a
@@ -564,7 +563,7 @@ struct BFragments<P, std::void_t<decltype(P::kBFragments)>> : std::integral_cons
 // ---- direct-to-LDS variant ---------------------------------------------------------------------
 // For policies whose A needs no transform on its way to LDS (any per-fragment transform is P::fix_a,
 // applied after the fragment is read) and whose scales are absent, one byte per 32 k or one fp16 (plus
-// one fp16 zero) per 128 k (P::kScaleDma): the A and packed-B tiles, and the scales, travel
+// one fp16 zero) per group of 32 to 4096 k (P::kScaleDma): the A and packed-B tiles, and the scales, travel
 // global -> LDS with global_load_lds_dwordx4 / _dword, two tiles ahead of the MFMAs, without
 // passing through registers.  A lane's 16 bytes land at LDS base + lane * 16 whatever its source
 // address, so the XOR swizzle of the A rows is applied by permuting the SOURCE addresses.  These
@@ -591,7 +590,7 @@ __device__ __forceinline__ void dma4_unless(int not_due, unsigned lds_addr, unsi
   asm volatile("s_cmp_lg_u32 %0, 0\n\ts_cbranch_scc1 .Lnot_due%=\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %2, %3\n.Lnot_due%=:" ::"s"(__builtin_amdgcn_readfirstlane(not_due)), "s"(lds_addr), "v"(voff), "s"(sbase) : "memory", "scc");
 }
 
-// Three forms, on a tile of 256 columns:
+// Five forms, on a tile of 256 columns:
 // * kMBW = 4, kNBW = 4, kWavesM = 2: 256 rows on 2 x 2 waves of 128 x 128, one workgroup per CU.
 // * kMBW = 8, kNBW = 2, kWavesM = 1: 256 rows on four waves side by side, each 256 rows x 64 columns.  A wave then
 //   decodes only the 64 weight rows it alone multiplies (with two rows of waves every packed word is decoded twice per
@@ -601,6 +600,8 @@ __device__ __forceinline__ void dma4_unless(int not_due, unsigned lds_addr, unsi
 //   of 256 rows.  With kKHalves = 2 on eight waves, two per SIMD: waves 4 .. 7 multiply the other half of every stage
 //   (a second k-block, or with 64-byte rows of B the other two steps of the one k-block) into accumulators of their own,
 //   and the two halves exchange sums through LDS before the epilogue, of which each does half.
+// * kMBW = 3 and 6, kNBW = 2, kWavesM = 1: 96 rows, on four waves or (kKHalves = 2) eight, and 192 rows on four, as the two above:
+//   for the policies with P::kRowCosts, where such tiles fill their rounds better.
 // What bounds the 128-row form is the CU's load unit, which takes about two cycles per 64 bytes or per row piece, if that
 // is shorter: with a 32-byte piece of B and a dword of scales and of zeros per weight row and k-block (two workgroups of
 // four waves, 2 x 2) it was busy 87 % of the time and the matrix pipe 45 %.  So scales come only when their dword is due,
@@ -619,8 +620,8 @@ __global__ __launch_bounds__(256 * kKHalves, 32 * kMBW * kWavesM <= 128 ? 2 : 1)
   take_k_slice<P>(p, bid);
   extern __shared__ __align__(16) unsigned char smem[];
   static_assert(P::kBRowBytes == 32 || P::kBRowBytes == 64, "direct-to-LDS variant: 32 or 64 packed bytes per weight row per tile");
-  static_assert(kWavesM == 2 ? (kMBW == 4 && kNBW == 4) : (kWavesM == 1 && (kMBW <= 4 || kMBW == 6 || kMBW == 8) && kNBW == 2), "one of the forms");
-  static_assert(kKHalves == 1 || (kKHalves == 2 && kWavesM == 1 && kMBW <= 4), "two halves of a stage: 128 rows at most");
+  static_assert(kWavesM == 2 ? (kMBW == 4 && kNBW == 4) : (kWavesM == 1 && (kMBW == 3 || kMBW == 4 || kMBW == 6 || kMBW == 8) && kNBW == 2), "one of the forms");
+  static_assert(kKHalves == 1 || (kKHalves == 2 && kWavesM == 1 && kMBW <= 4), "two halves of a stage: 96 or 128 rows");
   constexpr int kWavesN = 8 / kNBW;            // waves across the 256 tile columns
   constexpr int kWaves = 4;                    // of one half
   constexpr int BM = 32 * kMBW * kWavesM;      // shadows the 256-row default
@@ -908,7 +909,7 @@ __global__ __launch_bounds__(256 * kKHalves, 32 * kMBW * kWavesM <= 128 ? 2 : 1)
         // A region's matrix instructions (its A fragments against the wave's two B fragments) and their side work, as a
         // pipeline of one matrix instruction, at most one LDS read and a few vector instructions: the fewer rows share a
         // decoded fragment, the more.  Skewed by one step like the 2 x 2 form below.
-        constexpr int kValu = kMBW >= 6 ? 3 : kMBW == 4 ? 4 : kMBW == 3 ? 5 : 7;
+        constexpr int kValu = kMBW >= 6 ? 3 : kMBW == 4 ? 4 : 5;
         auto region = [&](int q0, auto do_mfma_tag, auto&& side) {
           if constexpr (decltype(do_mfma_tag)::value) {
 #pragma unroll
@@ -1422,7 +1423,6 @@ inline Params make_params(const void* A, const void* B, const void* S, const voi
   p.M = M; p.N = N; p.K = K;
   p.ldk = K;
   p.split = 1;
-  p.kwaves = -1;
   p.tiles_m = (M + BM - 1) / BM;
   p.tiles_n = (N + BN - 1) / BN;
   return p;

@@ -10,10 +10,10 @@ namespace dq {
 
 // One translation unit each.  Return value as i2_gemm; the fragment-ordered one returns 1 where the direct-to-LDS
 // kernel does not take the shape (no other tiled kernel reads that order).
-int i2_gemm_rowmajor_bitnet(const gemm::Params& p, int convention, hipStream_t stream);
-int i2_gemm_rowmajor_int32(const gemm::Params& p, int convention, hipStream_t stream);
-int i2_gemm_interleaved_bitnet(const gemm::Params& p, int convention, hipStream_t stream);
-int i2_gemm_interleaved_int32(const gemm::Params& p, int convention, hipStream_t stream);
+int i2_gemm_rowmajor_bitnet(const gemm::Params& p, int convention, int kwaves, hipStream_t stream);
+int i2_gemm_rowmajor_int32(const gemm::Params& p, int convention, int kwaves, hipStream_t stream);
+int i2_gemm_interleaved_bitnet(const gemm::Params& p, int convention, int kwaves, hipStream_t stream);
+int i2_gemm_interleaved_int32(const gemm::Params& p, int convention, int kwaves, hipStream_t stream);
 int i2_gemm_fragments(const gemm::Params& p, int convention, bool interleaved, bool bitnet_epilogue, hipStream_t stream);
 
 namespace {
@@ -82,16 +82,16 @@ struct I2Policy : I8Mfma, gemm::NoScale, EPI {
 constexpr int kI2HalfTileMin = 160;
 
 // BITNET: out = (float(acc) / s_a[m]) / s_w -> fp16; else the raw int32.  The signed conventions use the TOP decode
-// while 128 x 128 x K stays below 2^31.
+// while 128 x 128 x K stays below 2^31.  kwaves: the form of dq_gemm_kwaves.h that the call goes to, or -1.
 template <int CONV, bool INTERLEAVED, bool BITNET, bool FRAG>
-int i2_gemm_conv(const Params& p, hipStream_t stream) {
+int i2_gemm_conv(const Params& p, int kwaves, hipStream_t stream) {
   using Plain = I2Policy<CONV, std::conditional_t<BITNET, BitnetOut, Int32Out<0, false>>, INTERLEAVED, false, FRAG>;
   if constexpr (!FRAG) {
-    if (p.kwaves >= 0) {
+    if (kwaves >= 0) {
       using Waves = I2Policy<CONV, std::conditional_t<BITNET, BitnetOutS<CONV == I2_UNSIGNED ? 0 : 6>, Int32Out<CONV == I2_UNSIGNED ? 0 : 6, false>>,
                              INTERLEAVED, CONV != I2_UNSIGNED, false>;
       if (p.K >= 131072 || !gemm::kwaves_takes<Waves>(p)) return 1;
-      return gemm::launch_kwaves<Waves>(p, p.kwaves, stream);
+      return gemm::launch_kwaves<Waves>(p, kwaves, stream);
     }
   }
   auto run = [&](auto pol) -> int {
@@ -112,11 +112,11 @@ int i2_gemm_conv(const Params& p, hipStream_t stream) {
 }
 
 template <bool INTERLEAVED, bool BITNET, bool FRAG>
-int i2_gemm_part(const Params& p, int convention, hipStream_t stream) {
+int i2_gemm_part(const Params& p, int convention, int kwaves, hipStream_t stream) {
   switch (convention) {
-    case I2_UNSIGNED: return i2_gemm_conv<I2_UNSIGNED, INTERLEAVED, BITNET, FRAG>(p, stream);
-    case I2_OFFSET: return i2_gemm_conv<I2_OFFSET, INTERLEAVED, BITNET, FRAG>(p, stream);
-    case I2_TWOS: return i2_gemm_conv<I2_TWOS, INTERLEAVED, BITNET, FRAG>(p, stream);
+    case I2_UNSIGNED: return i2_gemm_conv<I2_UNSIGNED, INTERLEAVED, BITNET, FRAG>(p, kwaves, stream);
+    case I2_OFFSET: return i2_gemm_conv<I2_OFFSET, INTERLEAVED, BITNET, FRAG>(p, kwaves, stream);
+    case I2_TWOS: return i2_gemm_conv<I2_TWOS, INTERLEAVED, BITNET, FRAG>(p, kwaves, stream);
     default: DQ_FAIL("int2 gemm: unknown code convention %d", convention);
   }
 }

@@ -30,7 +30,7 @@ static double i2_small_tiles_time(int M, int N, int K) {
   return 4.75 + 0.91 * rounds + 1e-3 * K * (2.63 * rounds + 0.76 * (double)tiles / 256.0);
 }
 int i2_kwaves_form(int M, int N, int K) {
-  if (M < (K % 256 ? 5 : 17) || gemm::kwaves_big_tiles(M, N) >= gemm::kHalfTileMin) return -1;
+  if (M < (K % 256 ? 5 : 17) || half_tiles(M, N) >= gemm::kHalfTileMin) return -1;
   const gemm::KwavesPick pick = gemm::kwaves_pick(kKwavesI2, M, N, K);
   // the K-sliced kernel keeps what its rounds of 256 tiles fill better: M = 200, N = K = 8192 28 us, 29.5 here
   if (K % 2048 == 0 && K >= 4096) {
@@ -50,13 +50,12 @@ int i2_gemm(const void* A, const void* B, void* C, int M, int N, int K, int conv
             float s_w, int bitnet_epilogue, int kwaves, hipStream_t stream) {
   gemm::Params p = gemm::make_params(A, B, s_a, nullptr, nullptr, C, M, N, K);
   p.f0 = s_w;
-  p.kwaves = kwaves;
   const bool interleaved = (layout & ~LAYOUT_FRAGMENTS) == LAYOUT_INTERLEAVED;
   if (layout & LAYOUT_FRAGMENTS) return i2_gemm_fragments(p, convention, interleaved, bitnet_epilogue != 0, stream);
   if (interleaved) {
-    return bitnet_epilogue ? i2_gemm_interleaved_bitnet(p, convention, stream) : i2_gemm_interleaved_int32(p, convention, stream);
+    return bitnet_epilogue ? i2_gemm_interleaved_bitnet(p, convention, kwaves, stream) : i2_gemm_interleaved_int32(p, convention, kwaves, stream);
   }
-  return bitnet_epilogue ? i2_gemm_rowmajor_bitnet(p, convention, stream) : i2_gemm_rowmajor_int32(p, convention, stream);
+  return bitnet_epilogue ? i2_gemm_rowmajor_bitnet(p, convention, kwaves, stream) : i2_gemm_rowmajor_int32(p, convention, kwaves, stream);
 }
 
 }  // namespace dq

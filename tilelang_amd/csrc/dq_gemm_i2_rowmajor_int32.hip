@@ -3,8 +3,8 @@
 
 namespace dq {
 
-int i2_gemm_rowmajor_int32(const gemm::Params& p, int convention, hipStream_t stream) {
-  return i2_gemm_part<false, false, false>(p, convention, stream);
+int i2_gemm_rowmajor_int32(const gemm::Params& p, int convention, int kwaves, hipStream_t stream) {
+  return i2_gemm_part<false, false, false>(p, convention, kwaves, stream);
 }
 
 }  // namespace dq

@@ -107,7 +107,7 @@ static constexpr gemm::KwavesCosts kKwavesI4 = {{2.09, 1.0, 0.56, false}, {2.49,
 int i4_kwaves_form(int M, int N, int K) {
   const gemm::KwavesPick pick = gemm::kwaves_pick(kKwavesI4, M, N, K);
   if (M <= (K < 512 ? 32 : 64)) return pick.form;
-  if (gemm::kwaves_big_tiles(M, N) >= gemm::kHalfTileMin) return -1;
+  if (half_tiles(M, N) >= gemm::kHalfTileMin) return -1;
   const double tiles = (double)((((long)M + 127) / 128) * (((long)N + 63) / 64));
   return pick.us < gemm::kwaves_margin(0.95, M, (size_t)M * K) * (3.7 + 1e-3 * K * (2.4 + 1.7 * tiles / 256.0)) ? pick.form : -1;
 }

@@ -1,8 +1,8 @@
-// Dequantize GEMM of a few dozen rows on gfx950: K over the eight waves of a workgroup.
+// Dequantize GEMM of a few dozen rows on gfx950: K over the waves of a workgroup.
 //
 // The tiled kernels of dq_gemm_core.h give M x N / (128 x 256) workgroups all of K each: at 64 rows of N = K = 8192 that is 32
-// workgroups for 256 CUs.  Here a workgroup owns few columns (32 or 64 weight rows) and as many activation rows as it
-// can hold accumulators for (to 96), and its eight waves take an eighth of K each:
+// workgroups for 256 CUs.  Here a workgroup owns few columns (32 or 64 weight rows) and few activation rows (16 to 64: what it
+// holds accumulators for, more run as passes), and its eight or four waves take an eighth or a quarter of K each:
 //   * a wave is a pipeline of its own: 4 KiB of LDS per 32 activation rows and 32 weight rows, written and read by that wave
 //     alone.  A wave's LDS operations are carried out in the order they were issued, so the loop over K has no barrier and the
 //     two waves of a SIMD run into each other's waits;
@@ -12,7 +12,7 @@
 //     in dq_gemm_core.h, by the same policies;
 //   * scales of a row travel 16 bytes at a time (a window: eight groups, or 512 k of block exponents), from whatever byte they
 //     lie at;
-//   * the eight sums of an output meet in LDS, a block of 32 activation rows at a time, and are added in slice order.
+//   * the waves' sums of an output meet in LDS, a block of 32 activation rows at a time, and are added in slice order.
 // What bounds it is the load unit and the LDS port of a CU, which take a byte of A and B once in and once out each: per tile
 // of 64 k and wave (64 rows x 64 columns) 10 KiB in and 10 KiB out beside 16 matrix instructions.
 #pragma once
@@ -42,7 +42,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_kernel_kwaves(const Param
   if (nt >= p.tiles_n) return;
   const int m0 = j_in % passes * (8 * AL), n0 = nt * (32 * NB);
 
-  // the wave's chunks; which eighth of K is its own turns with the workgroup, so that the CUs do not ask for the same
+  // the wave's chunks; which part of K is its own turns with the workgroup, so that the CUs do not ask for the same
   // stretch of every row at once
   const int KT = p.K / P::kKPerBlock, NC = (KT + T - 1) / T;
   const int kw = (wave + (nt >> 3)) & (kWaves - 1);
@@ -184,7 +184,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_kernel_kwaves(const Param
     }
   }
 
-  // ---- the eight sums: a block of 32 activation rows at a time, two buffers, one barrier per block.  A wave's sums are
+  // ---- the waves' sums: a block of 32 activation rows at a time, two buffers, one barrier per block.  A wave's sums are
   // rows of 128 NB bytes (an activation row's columns) or, transposed, of 128 (a column's activation rows).
   __syncthreads();  // every wave is done with its areas
   constexpr int kPart = 4096 * NB;
@@ -321,9 +321,6 @@ int launch_kwaves(const Params& p, int form, hipStream_t stream) {
     default: return launch_kwaves_tile<P, 8, 2, 4>(p, stream);
   }
 }
-
-// Tiles of 128 x 256 that the call would be for the direct-to-LDS kernel, which takes it from 96 of them on.
-inline long kwaves_big_tiles(int M, int N) { return (((long)M + 127) / 128) * (((long)N + 255) / 256); }
 
 }  // namespace gemm
 }  // namespace dq
