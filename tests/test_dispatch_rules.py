@@ -115,3 +115,8 @@ def test_uint4_groups_of_32_are_cut_into_one_round_at_most(M, N, K, streamed, cu
 ])
 def test_many_rows_against_the_tiles(operands, M, N, K, tiles, over_waves):
     assert (form(operands, M, N, K) >= 0) == (over_waves < tiles)
+
+
+@pytest.mark.parametrize("M,N,K,rows128,rows96", [(101, 31779, 256, 14.8, 18.5), (122, 32242, 512, 17.4, 20.1), (112, 32150, 896, 23.6, 27.1)])
+def test_tiles_of_96_rows_are_not_twice_those_of_128(M, N, K, rows128, rows96):
+    assert rows128 < rows96 and tile_rows(MXFP4, M, N, K) == 128 and tile_rows(MXFP4, 257, N, K) == 96
