@@ -242,9 +242,10 @@ static int w4a16_tiled_split(int M, int N, int K, int group, int mode) {
   const int unit = std::max(128, 2 * group), units = K / unit;
   int split = 1;
   for (int s = 2; s <= 12 && units >= s && K / s >= 1024; ++s) {
-    // groups of 32 k, whose scales go with every tile, on 96 rows: one round (M = 93, N = 38384, K = 28160 501 us on the streaming
-    // kernel, 679 in three; M = 138, N = 19706, K = 14080 224 and 287 in two)
-    if (group == 32 && low && tiles * s > 256) break;
+    // groups of 32 k, whose scales go with every tile, on 96 rows: one round, with zeros three quarters of one (M = 93, N = 38384,
+    // K = 28160 501 us on the streaming kernel, 679 in three rounds; M = 138, N = 19706, K = 14080 224 and 287 in two; M = 156,
+    // N = 10674, K = 18432 104 and 136 in 252 workgroups)
+    if (group == 32 && low && tiles * s > (mode >= W4_ZEROS_ORIGINAL ? 192 : 256)) break;
     const double r = rounds(tiles * s);
     const double us = 5.7 + r * (4.5 + 12.7e-3 * unit * ((units + s - 1) / s) * (low ? 0.79 : 1.0)) + 1.02e-6 * (double)s * M * N;
     if (us < best) best = us, split = s;
