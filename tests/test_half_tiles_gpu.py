@@ -10,6 +10,13 @@ from tilelang_amd import _lib, quantize
 
 pytestmark = pytest.mark.gpu
 
+# What the rule leaves on tiles of 128 rows, whatever K: 256 of them, or some hundreds
+ON_128 = ((1020, 8190), (2041, 4090), (2570, 8190), (1367, 13198))
+
+
+def _on_128(operands, M, N, K, group=0, mode=0):
+    return (M, N) not in ON_128 or _lib.load_library().dq_tile_rows(operands, M, N, K, group, mode) == 128
+
 
 def _ints(gen, lo, hi, *shape, dtype, device):
     return torch.randint(lo, hi + 1, shape, generator=gen, device=device).to(dtype)
@@ -34,8 +41,12 @@ def _nibbles(packed):
     (897, 4104, 1024, 256),   # rows of C that are no whole lines
     (897, 4104, 1280, 256),
     (2600, 6200, 2048, 256), (2600, 6200, 2304, 256),  # more than 512 tiles: four waves to K = 2048, eight beyond
+    (1020, 8190, 384, 64), (1020, 8190, 256, 128), (1020, 8190, 1024, 128), (2041, 4090, 640, 64),  # as above, on tiles of 128 rows
+    (1020, 8190, 1152, 64), (1020, 8190, 1280, 128), (2041, 4090, 3072, 512), (1020, 8190, 1536, 32), (1020, 8190, 512, 32),
+    (1367, 13198, 2048, 256), (1367, 13198, 2304, 256),
 ])
 def test_uint4(cuda, M, N, K, group, zeros):
+    assert _on_128(_lib.OPERANDS_F16_UINT4, M, N, K, group, 5 if zeros else 3)
     gen = torch.Generator(device=cuda).manual_seed(K + group)
     A = _ints(gen, -2, 2, M, K, dtype=torch.float16, device=cuda)
     B = _ints(gen, -128, 127, N, K // 2, dtype=torch.int8, device=cuda)
@@ -64,10 +75,11 @@ def test_fp4(cuda, K):
     assert torch.equal(C, (A.double() @ W.t()).bfloat16())
 
 
-@pytest.mark.parametrize("M,N,K", [(1100, 3500, 640), (1100, 3500, 128), (2600, 6200, 384)])
+@pytest.mark.parametrize("M,N,K", [(1100, 3500, 640), (1100, 3500, 128), (2600, 6200, 384), (1020, 8190, 640), (2570, 8190, 384)])
 def test_mxfp4_rows_keep_their_bits(cuda, M, N, K):
     """Uncut, a row's products are added in one order whatever tile the call runs on: the rows of a large product against
     a call of 80 of them (real-valued operands, so that another order would show)."""
+    assert _on_128(_lib.OPERANDS_BF16_MXFP4, M, N, K)
     gen = torch.Generator(device=cuda).manual_seed(N + K)
     A = torch.randn((M, K), generator=gen, device=cuda).bfloat16()
     B = _ints(gen, 0, 255, N, K // 2, dtype=torch.uint8, device=cuda)
@@ -139,8 +151,10 @@ def test_transposed_rows_off_16_bytes(cuda, M):
     (1300, 4000, 768), (1300, 4000, 512), (1281, 4072, 1280), (1300, 4000, 1536),  # four waves; eight on five stages, on six
     (1800, 7000, 1024), (1800, 7000, 1280),  # 224 tiles of 256 rows, 420 of 128: the second to K = 1024, the first beyond
     (1300, 7000, 768), (1300, 6000, 256), (2050, 7690, 512), (2050, 7690, 2304),  # 308, 264, 527 tiles: two workgroups per CU; rounds of four waves; of eight
+    (1020, 8190, 768), (2041, 4090, 512), (1020, 8190, 1280), (2041, 4090, 1536), (2570, 8190, 512), (2570, 8190, 2304),  # tiles of 128 rows
 ])
 def test_bitnet(cuda, M, N, K, fragments, interleaved):
+    assert _on_128(_lib.OPERANDS_INT8_INT2, M, N, K)
     gen = torch.Generator(device=cuda).manual_seed(K)
     A = _ints(gen, -128, 127, M, K, dtype=torch.int8, device=cuda)
     codes = _ints(gen, 1, 3, N, K // 16, 4, 4, dtype=torch.uint8, device=cuda)  # element e of a word at bit 8 (e % 4) + 2 (e / 4)

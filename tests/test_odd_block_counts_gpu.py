@@ -12,8 +12,13 @@ from tilelang_amd import _lib
 
 pytestmark = pytest.mark.gpu
 
-# 256 x 256 tiles, 128 x 256 tiles; ragged last tiles of odd widths
+# many tiles and few; ragged last tiles of odd widths (with an odd count of groups such a call is staged through registers)
 TALL, HALF = (2570, 5131), (1100, 3503)
+
+
+def _rows(operands, M, N, K, group=0, mode=0):
+    """The rows of the direct-to-LDS kernel's tiles that the call runs on."""
+    return _lib.load_library().dq_tile_rows(operands, M, N, K, group, mode)
 
 
 def _ints(gen, lo, hi, *shape, dtype, device):
@@ -35,6 +40,22 @@ def _nibbles(packed):
     (320, 32), (224 * 3 - 32, 32),
 ])
 def test_uint4(cuda, M, N, K, group, zeros):
+    _uint4(cuda, M, N, K, group, zeros)
+
+
+@pytest.mark.parametrize("zeros", [False, True])
+@pytest.mark.parametrize("rows,M,N,K,group", [
+    (128, 1020, 8190, 192, 64), (128, 1020, 8190, 448, 64), (128, 1020, 8190, 1088, 64), (128, 2041, 4090, 384, 128),
+    (128, 1020, 8190, 1152, 128), (128, 1020, 8190, 1792, 256), (128, 1020, 8190, 320, 32), (128, 1020, 8185, 320, 32),
+    (256, 2570, 5132, 640, 64), (256, 2570, 5132, 832, 64), (256, 2570, 5132, 1152, 128), (256, 3050, 5100, 1792, 256), (256, 3050, 5100, 1088, 64),
+    (192, 2050, 5132, 192, 64), (192, 2050, 5132, 1152, 128), (96, 257, 20002, 448, 64), (96, 257, 20002, 1408, 128),
+])
+def test_uint4_on_tiles(cuda, rows, M, N, K, group, zeros):
+    assert _rows(_lib.OPERANDS_F16_UINT4, M, N, K, group, 5 if zeros else 3) == rows
+    _uint4(cuda, M, N, K, group, zeros)
+
+
+def _uint4(cuda, M, N, K, group, zeros):
     gen = torch.Generator(device=cuda).manual_seed(K + group)
     A = _ints(gen, -2, 2, M, K, dtype=torch.float16, device=cuda)
     B = _ints(gen, -128, 127, N, K // 2, dtype=torch.int8, device=cuda)
@@ -54,6 +75,21 @@ def test_uint4(cuda, M, N, K, group, zeros):
 @pytest.mark.parametrize("K", [192, 320, 448, 576, 1088])
 @pytest.mark.parametrize("fmt", ["e2m1", "simple"])
 def test_mxfp4(cuda, M, N, K, fmt):
+    _mxfp4(cuda, M, N, K, fmt)
+
+
+@pytest.mark.parametrize("rows,M,N,K", [
+    (128, 1020, 8190, 192), (128, 1020, 8190, 448), (128, 2041, 4090, 1088), (128, 2570, 5132, 576),
+    (256, 3050, 5100, 1088), (256, 3050, 5100, 1344), (256, 2570, 5132, 1600),  # B by pairs of tiles: the last pair is half
+    (192, 2050, 5132, 1088), (96, 1100, 3504, 1088), (96, 257, 20002, 448),
+])
+@pytest.mark.parametrize("fmt", ["e2m1", "simple"])
+def test_mxfp4_on_tiles(cuda, rows, M, N, K, fmt):
+    assert _rows(_lib.OPERANDS_BF16_MXFP4, M, N, K) == rows
+    _mxfp4(cuda, M, N, K, fmt)
+
+
+def _mxfp4(cuda, M, N, K, fmt):
     gen = torch.Generator(device=cuda).manual_seed(K)
     A = _ints(gen, -2, 2, M, K, dtype=torch.bfloat16, device=cuda)
     B = _ints(gen, 0, 255, N, K // 2, dtype=torch.uint8, device=cuda)
@@ -71,10 +107,11 @@ def test_mxfp4(cuda, M, N, K, fmt):
     assert torch.equal(C, (A.double() @ W.t()).bfloat16())
 
 
-@pytest.mark.parametrize("M,N", [TALL, HALF])
+@pytest.mark.parametrize("M,N", [TALL, HALF, (1020, 8190), (1017, 8191)])
 @pytest.mark.parametrize("K", [384, 640, 896, 1408])
 @pytest.mark.parametrize("transposed", [True, False])
 def test_int8_int4(cuda, M, N, K, transposed):
+    assert _rows(_lib.OPERANDS_INT8_INT4, M, N, K) == {TALL: 256, HALF: 0}.get((M, N), 128)
     gen = torch.Generator(device=cuda).manual_seed(K)
     A = _ints(gen, -128, 127, M, K, dtype=torch.int8, device=cuda)
     B = _ints(gen, 0, 255, N, K // 2, dtype=torch.uint8, device=cuda)
@@ -91,6 +128,19 @@ def test_int8_int4(cuda, M, N, K, transposed):
 @pytest.mark.parametrize("M,N", [TALL, (2050, 5131), HALF])
 @pytest.mark.parametrize("K", [384, 640, 1152, 1408])
 def test_bitnet(cuda, M, N, K):
+    _bitnet(cuda, M, N, K)
+
+
+@pytest.mark.parametrize("rows,M,N,K", [
+    (128, 2570, 5131, 384), (128, 2570, 8190, 640), (128, 1020, 8185, 1152), (128, 2041, 4090, 1408), (128, 1020, 8190, 2432),
+    (256, 2040, 6141, 4480), (192, 1089, 10703, 3456), (96, 2050, 5131, 384), (96, 1281, 4073, 1152),
+])
+def test_bitnet_on_tiles(cuda, rows, M, N, K):
+    assert _rows(_lib.OPERANDS_INT8_INT2, M, N, K) == rows
+    _bitnet(cuda, M, N, K)
+
+
+def _bitnet(cuda, M, N, K):
     gen = torch.Generator(device=cuda).manual_seed(K)
     A = _ints(gen, -128, 127, M, K, dtype=torch.int8, device=cuda)
     codes = _ints(gen, 0, 3, N, K // 4, 4, dtype=torch.uint8, device=cuda)  # code e of a byte at bit 2 e

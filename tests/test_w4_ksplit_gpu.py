@@ -57,21 +57,34 @@ def test_named_slices(cuda, M, N, K, group, split, zeros):
     assert bool(torch.isfinite(ws.view(torch.float32)).all())
 
 
-@pytest.mark.parametrize("M,N,K,group,zeros", [(202, 2240, 10752, 128, True), (700, 1648, 8960, 64, False), (90, 5528, 7936, 128, False)])
+@pytest.mark.parametrize("M,N,K,group,zeros", [(200, 5004, 10752, 128, True), (700, 1648, 8960, 64, False), (90, 5528, 7936, 128, False)])
 def test_default(cuda, M, N, K, group, zeros):
     """Shapes that the library cuts by itself, through the kernel object, which brings the workspace."""
     room = int(_lib.load_library().dq_w4a16_workspace_bytes(M, N, K, group, 5 if zeros else 3))
     assert room and room % (M * N * 4) == 0
     A, B, S, Z, codes = _operands(cuda, M, N, K, group, 7)
-    kern = tl.matmul_w4a16(M, N, K, group_size=group, source_format="uint" if zeros else "int", with_zeros=zeros)
+    kern = tl.dequantize_gemv(M, N, K, group_size=group, source_format="uint" if zeros else "int", with_scaling=True, with_zeros=zeros)
+    assert [p.shape for p in kern.params if p.name == "Workspace"] == [(room,)]
     C = torch.full((M, N), float("nan"), dtype=torch.float16, device=cuda)
     kern(A, B, S, *([Z] if zeros else []), C)
     assert torch.equal(C, _ref(A, S, Z, codes, group, zeros))
+    # and it is the tiled GEMM that is cut: the same bits as the slices named
+    ws = torch.empty(room, dtype=torch.uint8, device=cuda)
+    A = torch.randn(A.shape, device=cuda).half()
+    out = []
+    for variant in (-1, 50 + room // (M * N * 4)):
+        C = torch.full((M, N), float("nan"), dtype=torch.float16, device=cuda)
+        rc = _lib.get_library().call_dequantize_gemv_w4a16_ws(A.data_ptr(), B.data_ptr(), S.data_ptr(), Z.data_ptr() if zeros else None, C.data_ptr(),
+                                                              ws.data_ptr(), room, M, N, K, group, 5 if zeros else 3, 0, variant,
+                                                              torch.cuda.current_stream().cuda_stream)
+        assert rc == 0, _lib.last_error()
+        out.append(C)
+    assert torch.equal(out[0], out[1])
 
 
 def test_less_room_than_asked_for(cuda):
     """A smaller workspace lowers the count, none at all leaves the call uncut."""
-    M, N, K, group = 202, 2240, 10752, 128
+    M, N, K, group = 90, 5528, 7936, 128
     lib = _lib.get_library()
     full = int(lib.dq_w4a16_workspace_bytes(M, N, K, group, 3))
     assert full >= 3 * M * N * 4

@@ -67,7 +67,7 @@ double w4_tiled_time(int M, int N, int K);
 double w4_kwaves_time(int M, int N, int K);
 int w4_kwaves_form(int M, int N, int K);
 int w4_f16_gemm_kwaves(const void* A, const void* B, const void* S, const void* Z, void* C, int M, int N, int K, int group,
-                       int mode, int layout, hipStream_t stream);
+                       int mode, int layout, int form, hipStream_t stream);
 int wlow_gemv(const void* A, const void* B, const void* Scale, const void* Zeros, void* C, int M, int N, int K, int group,
               int bits, int convention, int layout, int zeros_rescale, hipStream_t stream);
 int i2_gemm_kslice(const void* A, const void* B, void* C, int M, int N, int K, int convention, int layout, const void* s_a,
@@ -337,8 +337,14 @@ static int gemv_w4a16(const char* fn, const void* A, const void* B, const void* 
     return rc;
   }
   if (variant == -1 && w4a16_by_kwaves(M, N, K, group, asked_mode, workspace != nullptr)) {
-    const int rc = w4_f16_gemm_kwaves(A, B, Scale, Zeros, C, M, N, K, group, asked_mode, layout, (hipStream_t)stream);
+    const int rc = w4_f16_gemm_kwaves(A, B, Scale, Zeros, C, M, N, K, group, asked_mode, layout, -1, (hipStream_t)stream);
     if (rc <= 0) return rc;
+  }
+  // 80 .. 84: K over the waves of a workgroup, the form less 80 (measurements and tests)
+  if (variant >= 80 && variant <= 84) {
+    const int rc = w4_f16_gemm_kwaves(A, B, Scale, Zeros, C, M, N, K, group, asked_mode, layout, variant - 80, (hipStream_t)stream);
+    if (rc > 0) DQ_FAIL("%s: K over the waves does not cover M=%d N=%d K=%d group=%d mode=%d", fn, M, N, K, group, mode);
+    return rc;
   }
   if (variant == -1 && workspace) {
     int cut = w4a16_tiled_split(M, N, K, group, asked_mode);

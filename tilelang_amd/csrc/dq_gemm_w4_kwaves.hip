@@ -11,13 +11,13 @@ static constexpr gemm::KwavesCosts kKwavesW4 = {{2.55, 0.92, 1.16, true}, {2.68,
 double w4_kwaves_time(int M, int N, int K) { return gemm::kwaves_pick(kKwavesW4, M, N, K).us; }
 int w4_kwaves_form(int M, int N, int K) { return gemm::kwaves_pick(kKwavesW4, M, N, K).form; }
 
-// 1: not a shape of that kernel
+// form: of kKwavesForms, -1 the best by the times.  1: not a shape of that kernel
 int w4_f16_gemm_kwaves(const void* A, const void* B, const void* S, const void* Z, void* C, int M, int N, int K, int group,
-                       int mode, int layout, hipStream_t stream) {
+                       int mode, int layout, int form, hipStream_t stream) {
   Params p = gemm::make_params(A, B, S, Z, nullptr, C, M, N, K);
   p.p0 = (group == K) ? 31 : (31 - __builtin_clz(group));
   p.p1 = K / group;
-  const int form = w4_kwaves_form(M, N, K);
+  if (form < 0) form = w4_kwaves_form(M, N, K);
 #define DQ_W4(MODE_)                                                                                         \
   do {                                                                                                       \
     if (!gemm::kwaves_takes<W4F16Policy<MODE_, false>>(p)) return 1;                                         \
