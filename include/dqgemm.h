@@ -146,8 +146,9 @@ enum dq_fp4_format {
  * multiplies by 2^Scale with the raw byte (:254-267): scale_bias = 0; an E8M0 scale is
  * scale_bias = 127.  Bias may be NULL.  Requires K % 64 == 0, scale_size == 32.
  * The library picks the kernel by shape (one and two rows up to K = 32768: a dot-product kernel on whole weight
- * rows; up to 16 rows: the activations resident in registers and the weights streamed once, or K over the waves of a
- * workgroup, as from 17 to 64 rows from K = 512 on and, K % 128 == 64, on small matrices beyond; else the tiled GEMM).
+ * rows; up to 16 rows, more while passes of 16 stay ahead: the activations resident in registers and the weights streamed
+ * once; from three to 64 rows from K = 512 on, K % 128 == 64 on small matrices beyond, where that is ahead: K over the waves of
+ * a workgroup; else the tiled GEMM).
  * Each adds the same products in fp32 in an order of its own: a row computed in a small batch and in a large one may
  * differ in the last bf16 bit; every call of one shape returns the same bits. */
 int call_dequant_gemm_bf16_mxfp4(const void* A, const void* B, const void* Scale, const void* Bias, void* C, int M,
@@ -247,8 +248,9 @@ enum dq_i2_convention {
  * Replaces `call(A, B, C, stream)` of tilelang_bitnet_158_int8xint2_prefill.py:188-296 and
  * tilelang_bitnet_158_int8xint2_decode.py:66-175.  Requires K % 128 == 0.
  * The library picks the kernel by shape (M <= 4: a streaming dot-product kernel; up to 32 rows with K % 256 == 0: the
- * activations resident in registers and the weights streamed once; a few hundred rows on a long K:
- * K sliced over the waves of a workgroup; else the tiled GEMM).  All four read DQ_LAYOUT_FRAGMENTS; where the
+ * activations resident in registers and the weights streamed once; row-major words from five rows on where that is ahead,
+ * K over the waves of a workgroup; a few hundred rows on a long K: K sliced over the waves of a workgroup; else the tiled
+ * GEMM).  All but the third read DQ_LAYOUT_FRAGMENTS; where the
  * tiled GEMM does not take a fragment-ordered problem (too few tiles) the K-sliced kernel runs it whatever its size.  For tests and measurements out_kind may carry one
  * of the flags below, which names the kernel instead; all kernels return the same bits. */
 enum dq_i2_kernel {
@@ -314,7 +316,8 @@ enum dq_i4_decode {
  * path of example_dequant_gemm_fine_grained.py (DQ_I4_UNSIGNED) and the int8 branch (`use_dp4a`) of
  * example_dequant_gemv_fp16xint4.py:47-54,113-133: its slow path (DQ_I4_TWOS) and, with fast_decoding, the two
  * interleaved decoders.  M <= 4 runs as a streaming dot-product kernel (K <= 16384; 16 bytes of B per lane,
- * v_dot4_i32_i8, the decoder's constant applied through the sum of the activations), larger M on the tiled GEMM.
+ * v_dot4_i32_i8, the decoder's constant applied through the sum of the activations), larger M, and Ct at few rows, with K
+ * over the waves of a workgroup where that is ahead, else on the tiled GEMM.
  * a_packed 1: A is packed int4 too, A[M,K/2] (examples/gemm_int4/example_tilelang_gemm_int4.py:17-38), DQ_I4_TWOS
  * or DQ_I2_TO_I4, K < 131072 (the operands carry a factor 16 in the int32 accumulator).  Requires K % 128 == 0. */
 int call_gemm_int8xint4(const void* A, const void* B, void* C, int M, int N, int K, int decode, int a_packed,

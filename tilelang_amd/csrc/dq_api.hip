@@ -221,7 +221,7 @@ static double w4a16_stream_passes_time(int M, int N, int K, int split) {
 // Into how many slices of K the tiled GEMM is cut where a workspace was brought: 65 to some thousand rows against a matrix of
 // few tiles, where neither it uncut nor the streaming kernel fills the chip.  Both sides are fits (us) over 90 shapes of 64 to
 // 1280 rows (mean error 5 %), and cut is what they put a tenth ahead: 1.08 times as fast in the mean, 0.99 in the worst (M = 202,
-// N = 8928, K = 10752 97 -> 61 us; M = 73, N = 17328, K = 7680 74 -> 37; M = 419, N = 5296, K = 7680 74 -> 52; not M = 128, N = 4096,
+// N = 8928, K = 10752 107 -> 63 us; M = 73, N = 17328, K = 7680 76 -> 40; M = 419, N = 5296, K = 7680 75 -> 55; not M = 128, N = 4096,
 // K = 14336, 28 us on the streaming kernel and 31 cut).  1: not cut.
 static int w4a16_tiled_split(int M, int N, int K, int group, int mode) {
   const bool scaled = mode == W4_SCALE || mode == W4_USCALE || mode == W4_ZEROS_ORIGINAL || mode == W4_ZEROS_FOLDED;
@@ -531,7 +531,7 @@ static int mxfp4_ksplit(int M, int N, int K, int fp4_format, double* us) {
 
 // With a workspace, which is what allows a row other bits than those of a large product: how the call runs, K over the waves
 // of a workgroup or cut in so many slices.  The former needs no second kernel and no sums in memory, which is most of what a
-// small call takes (M = 101, N = 1696, K = 3456 18 -> 8.4 us, M = 204, N = 2912, K = 3328 20 -> 14; 4529 shapes of 65 to 600
+// small call takes (M = 101, N = 1696, K = 3456 15.7 -> 7.9 us, M = 204, N = 2912, K = 3328 20 -> 14; 4529 shapes of 65 to 600
 // rows, N 256 to 40000: 0.87 of the time without it, 0.6 % of them more than a twentieth slower).  N % 4 == 0 is
 // what the estimate was fitted on; beyond K = 6144 a workgroup's own walk is long and the slices are as fast (M = 298, N = 2528,
 // K = 9728: 31 and 30 us).  Below K = 1024 there is no workspace of two slices to name, and where nothing would be cut none is
@@ -549,7 +549,7 @@ static Mxfp4Plan mxfp4_plan(int M, int N, int K, int fp4_format) {
 
 // K over the waves of a workgroup, to 64 rows: where it is a fifth ahead of the register-resident kernel's estimate, up to 2048 k,
 // where that one's is some way off, a quarter (8438 shapes of 3 to 64 rows, N 256 to 40000, K 512 to 16384: 0.86 of the time
-// of the kernels without this one, 1.4 % of them more than a twentieth slower; M = 64, N = K = 8192 49 -> 20 us, M = 14,
+// of the kernels without this one, 1.4 % of them more than a twentieth slower; M = 64, N = K = 8192 49 -> 21 us, M = 14,
 // N = 2168, K = 13760 22 -> 14; not M = 29, N = 1184, K = 8192, 9.6 us there and 13.6 here, nor M = 4, N = 16384, K = 2048, 7.3
 // and 8.6).  The tiled GEMM is behind all of these.  From 65 rows on with K % 128 == 0 a row keeps the bits that it has in a
 // large product, or mxfp4_plan decides; otherwise, and while the tiles of 128 x 256 are few, against the 7.5 us a thousand k of

@@ -99,7 +99,7 @@ struct I4xI2Policy : I8Mfma, gemm::NoScale, EPI {
 
 // K over the waves of a workgroup instead of the tiled kernels: the form, or -1.  To 32 rows, from K = 512 on to 64, always (13 000
 // shapes, N 256 to 40000: 0.57 of the time in the mean, 0.1 % more than a twentieth slower; M = 2, N = 2264, K = 8704 25 -> 7 us,
-// M = 64, N = K = 8192 27 -> 13; not M = 35, N = 14608, K = 256, 5.0 us on the tiles and 5.8 here); beyond, where the tiled
+// M = 64, N = K = 8192 28.5 -> 14.4; not M = 35, N = 14608, K = 256, 5.0 us on the tiles and 5.8 here); beyond, where the tiled
 // kernel's tiles of 128 x 64 are few (its times: 3.7 us, and 2.4 + 1.7 a round's share of tiles for a thousand k) and none of
 // 128 x 256 are taken (M = 114, N = 3432, K = 11008 32 -> 14, M = 128, N = K = 8192 28 -> 19, M = 200, N = 8192, K = 4096 18 and 17).
 static constexpr gemm::KwavesCosts kKwavesI4 = {{2.09, 1.0, 0.56, false}, {2.49, 0.89, 0.61, false}, {3.12, 0.91, 0.92, false},
