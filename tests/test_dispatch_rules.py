@@ -101,6 +101,14 @@ def test_mxfp4_kernel_objects_bring_sums_room_only_where_sums_are_written(M, N, 
     assert _room(tl.matmul_bf16_mxfp4(M, N, K)) == [16 if over_waves else asked] and (form(MXFP4, M, N, K) >= 0) == over_waves
 
 
+@pytest.mark.parametrize("M,N,K", [(170, 15548, 2048), (546, 5024, 2176), (380, 8036, 2432)])
+def test_simple_mxfp4_kernel_objects_keep_room_for_the_sums(M, N, K):
+    """The "simple" format is cut here, which e2m1 is not: with less than two slices' room the call would run uncut."""
+    asked = _lib.load_library().dq_mxfp4_workspace_bytes(M, N, K)
+    assert form(MXFP4, M, N, K) >= 0 and _room(tl.matmul_bf16_mxfp4(M, N, K, weight_format="e2m1")) == [16]
+    assert _room(tl.matmul_bf16_mxfp4(M, N, K, weight_format="simple")) == [asked] and asked >= 2 * 4 * M * N
+
+
 @pytest.mark.parametrize("M,N,K,streamed,cut", [(93, 38384, 28160, 501, 679), (135, 16832, 25600, 367, 489), (138, 19706, 14080, 224, 287),
                                               (156, 10674, 18432, 104, 136), (146, 9408, 26880, 139, 166)])
 def test_uint4_groups_of_32_are_cut_into_less_than_a_round(M, N, K, streamed, cut):

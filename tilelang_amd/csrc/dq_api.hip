@@ -613,7 +613,7 @@ extern "C" size_t dq_mxfp4_workspace_bytes(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0 || K % 64 != 0) return 0;
   const Mxfp4Plan plan = mxfp4_plan(M, N, K, DQ_FP4_E2M1);
   // that a call comes with room is what allows an order of the sums other than a large product's: two slices' where none is used
-  // (sixteen bytes do where dq_kwaves_form names a form)
+  // (sixteen bytes do where dq_kwaves_form names a form, but in the "simple" format)
   const int slices = plan.split > 1 ? plan.split : plan.kwaves ? 2 : 0;
   return (size_t)slices * M * N * sizeof(float);
 }

@@ -455,8 +455,9 @@ def matmul_bf16_mxfp4(
     # some dozens to hundreds of rows: the library cuts K over workgroups when it is given room for the slices' sums
     try:
         ws_bytes = int(_lib.load_library().dq_mxfp4_workspace_bytes(M, N, K))
-        # K over the waves of a workgroup writes no sums: any room allows it
-        if ws_bytes and _lib.load_library().dq_kwaves_form(_lib.OPERANDS_BF16_MXFP4, M, N, K, 0, 0, 1) >= 0:
+        # K over the waves of a workgroup writes no sums: any room allows it ("simple" may be cut where e2m1, which is asked
+        # about, is not: its tiles take longer uncut)
+        if ws_bytes and fmt != _FP4_FORMATS["simple"] and _lib.load_library().dq_kwaves_form(_lib.OPERANDS_BF16_MXFP4, M, N, K, 0, 0, 1) >= 0:
             ws_bytes = 16
     except _lib.LibraryNotBuiltError:  # the kernel's parameters can be had without a library; its call raises this
         ws_bytes = 0
