@@ -36,6 +36,8 @@ def test_mxfp4_small_batches_against_the_register_resident_kernel(M, N, K, regis
     (27, 20384, 3840, 10.3, 13.2), (18, 17864, 1792, 7.2, 8.7), (37, 3560, 2048, 5.0, 5.8),   # register-resident
     (322, 4872, 256, 6.9, 10.4), (1251, 2160, 128, 6.0, 12.4), (70, 21400, 256, 8.3, 10.0), (483, 3800, 256, 6.9, 10.4),  # tiles
     (20, 3000, 3200, 17, 7.7), (39, 6544, 12288, 39.7, 14.6), (33, 20592, 3328, 22.3, 14.0), (196, 3960, 1280, 9.5, 7.5),
+    (117, 2592, 2048, 6.7, 5.3), (350, 2872, 2048, 11.1, 8.9), (332, 5400, 6144, 34.8, 21.6), (97, 15752, 6528, 32.8, 24.0),  # K shared out evenly
+    (1099, 2168, 11776, 67, 49), (1104, 2552, 7680, 43, 36), (3038, 176, 16384, 30, 55), (2876, 184, 16384, 30, 53),  # activations that no L2 holds
 ])
 def test_int8_int2_against_its_neighbours(M, N, K, neighbour, over_waves):
     assert (form(INT2, M, N, K) >= 0) == (over_waves < neighbour)
@@ -48,6 +50,11 @@ def test_int8_int2_against_its_neighbours(M, N, K, neighbour, over_waves):
 def test_int8_int4_against_the_tiles(M, N, K, tiles, over_waves):
     assert (form(INT4, M, N, K) >= 0) == (over_waves < tiles)
 
+
+
+def test_activations_that_no_l2_holds_are_read_by_sets_of_64_weight_rows():
+    """50 us on sets of 32 (form 1), which read them five times an XCD, and 32 on sets of 64."""
+    assert form(INT2, 776, 1136, 13056) == 4 and form(INT2, 776, 1136, 2304 + 128) != 4
 
 
 def tile_rows(operands, M, N, K, group=0, mode=0):

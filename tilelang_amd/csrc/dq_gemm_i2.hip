@@ -31,14 +31,22 @@ static double i2_small_tiles_time(int M, int N, int K) {
 }
 int i2_kwaves_form(int M, int N, int K) {
   if (M < (K % 256 ? 5 : 17) || half_tiles(M, N) >= gemm::kHalfTileMin) return -1;
-  const gemm::KwavesPick pick = gemm::kwaves_pick(kKwavesI2, M, N, K);
+  const gemm::KwavesPick pick = gemm::kwaves_pick(kKwavesI2, M, N, K, (size_t)M * K);
   // the K-sliced kernel keeps what its rounds of 256 tiles fill better: M = 200, N = K = 8192 28 us, 29.5 here
   if (K % 2048 == 0 && K >= 4096) {
     const long tiles = (((long)M + 63) / 64) * (((long)N + 127) / 128);
     if (tiles >= 64 && tiles <= 448 && 7.5 + 1.87e-3 * K * (double)((tiles + 255) / 256) < pick.us) return -1;
   }
-  if (const double resident = i2_resident_time(M, N, K); resident > 0.0) return pick.us < 0.96 * resident ? pick.form : -1;
-  return M <= 64 || pick.us < gemm::kwaves_margin(0.94, M, (size_t)M * K) * i2_small_tiles_time(M, N, K) ? pick.form : -1;
+  // where its waves share K out evenly the estimate is high, the neighbours' as well as it was fitted (M = 117, N = 2592, K = 2048
+  // 5.3 us, 6.7 on the register-resident kernel; M = 350, N = 2872 8.9, 11.1 on the tiles): 255 shapes that come here by that take
+  // 0.93 of the neighbour's time
+  const double even = M <= 1000 ? gemm::kwaves_even(pick, K, 512) : 1.0;
+  if (const double resident = i2_resident_time(M, N, K); resident > 0.0)
+    return pick.us < 0.96 * resident || even * pick.us < 0.86 * resident ? pick.form : -1;
+  // beyond a thousand rows and 8 MiB of activations the estimate of the tiles is high, too (M = 1099, N = 2168, K = 11776 67 us there
+  // and 49 here, M = 1900, N = 192, K = 20864 70 and 39, but M = 4037, N = 192, K = 20992 56 and 88)
+  const double margin = M > 1000 && (size_t)M * K > (8u << 20) ? 0.78 : 0.94;
+  return M <= 64 || even * pick.us < margin * i2_small_tiles_time(M, N, K) ? pick.form : -1;
 }
 
 int i2_tile_rows(int M, int N, int K) {

@@ -291,23 +291,43 @@ struct KwavesPick {
   int form;
   double us;
 };
-inline KwavesPick kwaves_pick(const KwavesCosts& costs, int M, int N, int K) {
+// What reading A takes (us) where no L2 holds it: once for every set of weight rows of an XCD, less the sets that run side by side,
+// at 0.9 TB/s an XCD.
+inline double kwaves_reread(const KwavesForm& f, int M, int N, size_t a_bytes) {
+  const long passes = ((long)M + 8 * f.al - 1) / (8 * f.al), sets = (((long)N + 32 * f.nb - 1) / (32 * f.nb) + 7) / 8;
+  const long beside = std::max(1L, (f.waves == 8 ? 32 : 64) / passes);
+  return (double)a_bytes * (double)((sets + beside - 1) / beside) / 0.9e6;
+}
+
+// a_bytes: of the activations, where the estimate is to know that beyond 4 MB they do not stay in an L2.  The costs, fitted to 600 rows,
+// do not (2100 shapes of int8 x 2-bit with more, calls by the ratio of reading A to their estimate: 1.0 of it to 0.75, 1.2 to 1, 1.4
+// beyond; M = 776, N = 1136, K = 13056 51 us on sets of 32, 33 on 64); 0: as fitted.
+inline KwavesPick kwaves_pick(const KwavesCosts& costs, int M, int N, int K, size_t a_bytes = 0) {
   KwavesPick best{-1, 1e30};
   for (int i = 0; i < kKwavesFormCount; ++i) {
     if (i == 0 && M > 16) continue;  // passes of 16 rows are never the best
     const long wgs = kwaves_workgroups(kKwavesForms[i], M, N);
     const double whole = (double)((wgs + 255) / 256);
     const double rounds = costs[i].smooth ? (wgs <= 256 ? 1.0 : 0.5 * ((double)wgs / 256.0 + whole)) : whole;
-    const double us = costs[i].start + rounds * (costs[i].round + costs[i].per_k * K * 1e-3);
+    double us = costs[i].start + rounds * (costs[i].round + costs[i].per_k * K * 1e-3);
+    if (a_bytes > 4000000u) us = std::max(us, 0.5 * us + 0.8 * kwaves_reread(kKwavesForms[i], M, N, a_bytes));
     if (us < best.us) best = {i, us};
   }
   return best;
 }
 
+// What a call takes of its estimate, which counts K smoothly, while the waves walk whole chunks (128 bytes of a row of B, chunk_k of
+// K): where those share out evenly less (int8 x 2-bit, 9000 shapes: 0.85 of it, 0.92 where the waves walk a fifth more than K, 1.0
+// from a half more on).
+inline double kwaves_even(const KwavesPick& pick, int K, int chunk_k) {
+  const int waves = kKwavesForms[pick.form].waves, each = ((K + chunk_k - 1) / chunk_k + waves - 1) / waves;
+  return std::min(1.0, 0.55 + 0.3 * each * waves * chunk_k / K);
+}
+
 // The share of a neighbour's estimate that this kernel's has to stay below.  Every set of weight rows reads all of A again: beyond a
 // thousand rows and 8 MiB of it the L2s no longer serve that, which the costs, fitted to 600 rows, do not know (int8, 159 and 151
 // shapes: 0.64 to 0.69 of the neighbour's time where the estimates' ratio is below 0.7, 1.0 to 1.15 of it above, up to 1.6; M = 3859,
-// N = 256, K = 22272 60 us on the tiles of int8 x int4 and 98 here).
+// N = 256, K = 22272 60 us on the tiles of int8 x int4 and 98 here).  int8 x 2-bit, whose tiles' estimate is high there, counts the reads.
 inline double kwaves_margin(double margin, int M, size_t a_bytes) { return M > 1000 && a_bytes > (8u << 20) ? 0.7 * margin : margin; }
 
 template <class P>
