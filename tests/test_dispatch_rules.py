@@ -27,8 +27,9 @@ def test_a_launch_that_fills_the_chip_is_counted_as_it_runs(operands):
     (29, 1184, 8192, 9.6, 13.6), (32, 720, 5888, 8.1, 11.6), (56, 632, 4096, 6.0, 8.6), (4, 16384, 2048, 7.3, 8.6),
     (8, 13632, 2048, 9.2, 10.2), (95, 312, 1728, 4.2, 5.2), (77, 448, 5056, 10.4, 12.8),
     (64, 8192, 8192, 49, 20), (14, 2168, 13760, 22, 14), (23, 8376, 2816, 14.5, 9.9), (101, 4336, 4800, 39, 17),
+    (106, 14536, 2048, 18.7, 14.3), (404, 3592, 3072, 23.0, 18.1), (202, 6272, 3072, 20.7, 16.9),  # K shared out evenly
 ])
-def test_mxfp4_small_batches_against_the_register_resident_kernel(M, N, K, register_resident, over_waves):
+def test_mxfp4_against_its_neighbours(M, N, K, register_resident, over_waves):
     assert (form(MXFP4, M, N, K) >= 0) == (over_waves < register_resident)
 
 

@@ -137,6 +137,10 @@ int fp4_tile_rows(int M, int N, int K) {
 static constexpr gemm::KwavesCosts kKwavesMx = {{2.2, 0.97, 0.88, false}, {2.65, 0.77, 1.03, false}, {3.37, 0.47, 1.67, false},
                                                 {3.11, 1.54, 2.34, true}, {3.15, 2.07, 2.44, true}};
 double mxfp4_kwaves_time(int M, int N, int K) { return gemm::kwaves_pick(kKwavesMx, M, N, K).us; }
+double mxfp4_kwaves_even_time(int M, int N, int K) {
+  const gemm::KwavesPick pick = gemm::kwaves_pick(kKwavesMx, M, N, K);
+  return pick.us * gemm::kwaves_even(pick, K, 256);
+}
 double mxfp4_kwaves_margin(double margin, int M, int K) { return gemm::kwaves_margin(margin, M, (size_t)M * K * 2); }
 int mxfp4_kwaves_form(int M, int N, int K) { return gemm::kwaves_pick(kKwavesMx, M, N, K).form; }
 int mxfp4_gemm_kwaves(const void* A, const void* B, const void* S, const void* Bias, void* C, int M, int N, int K, int fmt,
