@@ -1331,9 +1331,11 @@ int dma_rows(const Params& p, int min_tiles = kHalfTileMin) {
     // Scales and zeros of groups of 32 k go with every tile, on four waves: beyond 192 tiles of 96 rows and from 1024 k on the load
     // unit takes longer over those than the costs say (M = 461, N = 25216, K = 3072 104 us on 128 rows, 152 on 96; 143 shapes 1.02 in
     // the mean, to 192 tiles 190 shapes 0.94)
-    // And twice the tiles of 128 rows (97 to 128 rows of C) gain nothing: MXFP4, 108 shapes 1.00 in the mean, M = 101, N = 31779,
-    // K = 256 14.8 us on 128 rows, 18.5 on 96.
-    const bool low = !(P::kScaleDma == 3 && p.p0 == 5 && p.K >= 1024 && tiles_of(p, 96) > 192) && tiles_of(p, 96) < 2 * tiles_of(p, 128);
+    // And twice the tiles of 128 rows (97 to 128 rows of C) where a tile does little but store rows of C that are off 16 bytes (MXFP4,
+    // K < 2048, 420 shapes: 128 rows 0.94 of the time of 96, M = 101, N = 31779, K = 256 14.8 and 18.5 us; from 2048 k on, and with rows
+    // of whole 16 bytes, 1.01 to 1.14).
+    const bool twice = tiles_of(p, 96) >= 2 * tiles_of(p, 128) && p.K < 2048 && p.N % 8 != 0;
+    const bool low = !(P::kScaleDma == 3 && p.p0 == 5 && p.K >= 1024 && tiles_of(p, 96) > 192) && !twice;
     double best = 0.96 * us(rows == 256 ? 3 : 1);
     for (int i = low ? 0 : 1; i < 3; ++i)
       if (kHeights[i] != rows && us(i) < best) best = us(i), rows = kHeights[i];
