@@ -166,10 +166,10 @@ int call_dequant_gemm_bf16_mxfp4(const void* A, const void* B, const void* Scale
  * the same bits.  A cut call groups the sums by slice and may differ from that in the last bf16 bit, as the kernels for
  * fewer rows do; by the library's choice (split 0) no call of up to 80 rows is cut, and the entry point without a
  * workspace never cuts.  Small calls that the choice would cut, and some it would not, run with K over the waves of a
- * workgroup instead where that is faster (81 rows and more, K 1024 to 6144; the workspace stays unused, and
- * 16 bytes of it do where dq_kwaves_form with room names a form, but in DQ_FP4_SIMPLE, which may be cut there: its tiles
- * take longer uncut).  Who wants the bits of a large product at few rows asks for split = 1, which runs what it ran before that kernel was there: up to 16 rows,
- * more while passes of 16 stay ahead, the register-resident kernel, else the tiled GEMM. */
+ * workgroup instead where that is faster (81 rows and more, K 1024 to 6144; the workspace stays unused, and 16 bytes of it do
+ * where dq_kwaves_form with room names a form, but in DQ_FP4_SIMPLE, which may be cut there: its tiles take longer uncut).
+ * Who wants the bits of a large product at few rows asks for split = 1, which runs what it ran before that kernel was there:
+ * up to 16 rows, more while passes of 16 stay ahead, the register-resident kernel, else the tiled GEMM. */
 size_t dq_mxfp4_workspace_bytes(int M, int N, int K);
 int call_dequant_gemm_bf16_mxfp4_ws(const void* A, const void* B, const void* Scale, const void* Bias, void* C,
                                     void* Workspace, size_t workspace_bytes, int M, int N, int K, int scale_size,
